@@ -656,454 +656,329 @@ __device__ __forceinline__ void tile_of_block(Blk blk, int ntx, int nty, int ntz
 }
 
 //==================================================================================================
-// mapParticles2Grid as a gather over cell-sorted particles (FLIP_Solver.cpp:57-95,
-// ArrayHelpers.cpp:50-76). Thread (i,j,k) owns u(i,j,k), v(i,j,k), w(i,j,k); it visits the particles
-// of cells [i-1,i+1]x[j-1,j+1]x[k-1,k+1] in sorted order and keeps each particle's exact trilinear
-// weight for the face when the face is one of the particle's 8 stencil corners.
+// mapParticles2Grid over cell-sorted particles (FLIP_Solver.cpp:57-95, ArrayHelpers.cpp:50-76); with
+// kAffine the velocity carried to a node has the affine term of APIC_Solver.cpp:52-91 /
+// AFLIP_Solver.cpp:48-90.
+//
+// A thread owns one column of cells (i, j) and streams up z. A particle of cell c reaches on each axis
+// the nodes c, c+1 of a node-aligned grid and c-1 .. c+1 of a half-shifted one (one of the three with
+// weight 0), clamps included, so all of a column's contributions fall on 18 nodes of each face grid per
+// row: 2x3x3 (u), 3x2x3 (v), 3x3x2 (w). Their momentum and weight sums live in registers, a window of
+// planes that moves up with the row, and each particle costs its weights and 54 multiply-adds with no
+// memory traffic beyond its own record. When a plane of nodes is complete, the workgroup's columns
+// exchange their partial sums through LDS and each node's owner adds its 6 (u, v) or 9 (w) columns in
+// one fixed order. A node's sum is therefore: per column in (z, then particle) order, then over the
+// columns by y, then x, whatever the tile, the segment length or the batch.
+//
+// A workgroup is 16 x 16 columns around 14 x 14 owned ones (each node needs the columns next to it:
+// 1.31 visits a particle, against 1.95 for a tile of 8^3 nodes scattered into LDS, which this
+// replaces) and a segment of `seg` node planes (seg + 2 rows read). Bound by VALU issue: 214
+// instructions a particle visit, and a wavefront's row lasts as long as its fullest cell. 33M particles
+// at 256^3: 1724 -> 876 us (689 while every cell holds 8); 26k at 24^3, where the scattered tile was a
+// serial chain of 27 colour rounds in 64 wavefronts: 263 -> 33 us; affine, 1.27M: 1155 -> 180 us (a
+// gather per node column).
 //==================================================================================================
 struct FaceOut {
     float *u, *v, *w;
     uint8_t *vu, *vv, *vw;
 };
 
-__device__ __forceinline__ bool stencil_weight(float q, int i_high, int target, float& wgt) {
-    int   i;
-    float f;
-    bary(q, i_high, i, f);
-    if(target == i) {
-        wgt = 1.0f - f;
-        return true;
-    }
-    if(target == i + 1) {
-        wgt = f;
-        return true;
-    }
-    return false;
-}
+constexpr int kP2gSide = 16, kP2gOwn = kP2gSide - 2;  // columns of a workgroup per axis, and those it owns
 
-//--------------------------------------------------------------------------------------------------
-// P2G as a gather that streams along z. A thread owns the nodes (i, j, k0 .. k0+kSeg-1) of all
-// three face grids and reads each particle row z = k0-1 .. k0+kSeg once: a particle binned to
-// row z reaches only nodes z-1 .. z+1 along z (its z base is z-1 or z for the half-shifted stencil,
-// z for the node-aligned one, clamps included), which a three-node register window holds. Node k
-// still receives rows k-1, k, k+1 in that order, each row's y rows in order and each y row's
-// particles in cell-sorted order, with the weight (wx*wy)*wz and the momentum w*v rounded before
-// each add (no contraction): the per-node sums are those of a per-node gather over its 27 cells.
-//--------------------------------------------------------------------------------------------------
-// The segment length kSeg (the z extent of a thread's tile: 4, 8 or 16) changes which thread sums a
-// node, never the order of its sum, so every length gives the same bits; the batch autotuner picks it.
-
-struct P2gAcc {
-    float mu, wu, mv, wv, mw, ww;
-};
-
-// weights (1-f) at base and f at base+1; d = base - (z-1) picks the window slots (0,1) or (1,2).
-// vlo / vhi: the velocity carried to the base node and to base+1 (the particle's velocity; with the
-// affine term of APIC / AFLIP, v + dot(C_d, node - particle) per node). A zero ab (no
-// contribution) adds exact zeros.
-__device__ __forceinline__ void p2g_window_add(int d, float ab, float f, float vlo, float vhi, float& m0, float& w0, float& m1,
-                                               float& w1, float& m2, float& w2) {
+// one axis of a particle of cell c: n = node-aligned weights of the nodes c, c+1; h = half-shifted weights
+// of c-1, c, c+1. With f = x - c in [0, 1) these are bary()'s fractions without its branches: the base of
+// x - 0.5 is c-1 with fraction f + 0.5 when f < 0.5, else c with f - 0.5 (both exact), and 1 - fraction
+// rounds the same exact value either way. Outside the grid f clamps to 0 / 1 as bary's does.
+__device__ __forceinline__ void p2g_axis(float x, float c, float* n, float* h) {
 #pragma clang fp contract(off)
-    const float wl = ab * (1.0f - f), wh = ab * f;
-    const bool  lo = d == 0;
-    const float c0 = lo ? wl : 0.f, c1 = lo ? wh : wl, c2 = lo ? 0.f : wh;
-    const float v1 = lo ? vhi : vlo;
-    m0 += c0 * vlo;
-    w0 += c0;
-    m1 += c1 * v1;
-    w1 += c1;
-    m2 += c2 * vhi;
-    w2 += c2;
+    const float f = fminf(fmaxf(x - c, 0.f), 1.f);
+    n[0] = 1.0f - f;
+    n[1] = f;
+    h[0] = fmaxf(0.5f - f, 0.f);
+    h[1] = fminf(f + 0.5f, 1.5f - f);
+    h[2] = fmaxf(f - 0.5f, 0.f);
+}
+// the first (lo) / last (hi) cell of an axis: the half-shifted stencil clamps onto the cell's own node
+__device__ __forceinline__ void p2g_axis_edge(bool lo, bool hi, float* h) {
+    if(lo && h[0] > 0.f) {
+        h[0] = 0.f;
+        h[1] = 1.f;
+    }
+    if(hi) {
+        if(h[2] > 0.f) h[1] = 1.f;
+        h[2] = 0.f;
+    }
 }
 
-// v_d + dot(C_d, gpos - ppos) (APIC_Solver.cpp:73-76) for the node at grid index (xi + ex, yi + ey,
-// zi + ez): gpos = getWorldCoordinate = (index + extra) * dx + bMin, the dot product in glm's order
-__device__ __forceinline__ float affine_vel(float v, const float* c, float xi, float yi, float zi, float ex, float ey, float ez,
-                                            const GridGeom& g, float px, float py, float pz) {
+// momentum and weight of kX x kY x kZ nodes: (wx * wy) * wz as the reference forms it, added node by node
+template<int kX, int kY, int kZ>
+__device__ __forceinline__ void p2g_add(const float* wx, const float* wy, const float* wz, float v, float (*m)[kX * kY], float (*w)[kX * kY]) {
 #pragma clang fp contract(off)
-    const float gxw = (xi + ex) * g.dx + g.bminx, gyw = (yi + ey) * g.dx + g.bminy, gzw = (zi + ez) * g.dx + g.bminz;
-    return v + ((c[0] * (gxw - px) + c[1] * (gyw - py)) + c[2] * (gzw - pz));
-}
-
-__device__ __forceinline__ void p2g_emit(const P2gAcc& a, int i, int j, int k, bool uCol, bool vCol, bool wCol, const GridGeom& g,
-                                         const FaceOut& out) {
-    if(uCol && k < g.nz) {
-        const size_t id = lin3(i, j, k, g.nx + 1, g.ny);
-        const bool   ok = a.wu > kFltMin;
-        out.u[id]       = ok ? a.mu / a.wu : 0.f;
-        out.vu[id]      = ok ? 1 : 0;
-    }
-    if(vCol && k < g.nz) {
-        const size_t id = lin3(i, j, k, g.nx, g.ny + 1);
-        const bool   ok = a.wv > kFltMin;
-        out.v[id]       = ok ? a.mv / a.wv : 0.f;
-        out.vv[id]      = ok ? 1 : 0;
-    }
-    if(wCol) {
-        const size_t id = lin3(i, j, k, g.nx, g.ny);
-        const bool   ok = a.ww > kFltMin;
-        out.w[id]       = ok ? a.mw / a.ww : 0.f;
-        out.vw[id]      = ok ? 1 : 0;
-    }
-}
-
-// stencil weight of node `target` for coordinate q when no clamp can apply (q's floor is base, the
-// weights (1 - f, f) sit at base and base + 1): the operations of bary + stencil_weight without the
-// clamps, so the value is the same; 0 outside the stencil
-__device__ __forceinline__ float stencil_weight_interior(float q, float target) {
-    const float s = floorf(q), f = q - s;
-    return s == target ? 1.0f - f : (s == target - 1.0f ? f : 0.f);
-}
-
-// A particle binned to row z, seen from column (i, j): abU / abV / abW the x-y weight products of the
-// three face grids (0 when the column is not in the particle's stencil or the grid's row is off: onU
-// etc.), fh / dh and fn / dn the z weight of the half-shifted (u, v) and node-aligned (w) stencils and
-// the window slot of their base. kInterior: no barycentric clamp can apply.
-template<bool kInterior>
-__device__ __forceinline__ void p2g_col_weights(float gx, float gy, float gz, bool onU, bool onV, bool onW, const GridGeom& g, int i,
-                                                int j, int z, float fi, float fj, float& abU, float& abV, float& abW, float& fh,
-                                                float& fn, int& dh, int& dn) {
-#pragma clang fp contract(off)
-    if(kInterior) {
-        const float axn = stencil_weight_interior(gx, fi), axh = stencil_weight_interior(gx - 0.5f, fi);
-        const float byn = stencil_weight_interior(gy, fj), byh = stencil_weight_interior(gy - 0.5f, fj);
-        const float qh = gz - 0.5f, sh = floorf(qh);
-        fh  = qh - sh;
-        dh  = sh == (float)(z - 1) ? 0 : 1;
-        fn  = gz - floorf(gz);
-        dn  = 1;  // the node-aligned base is the row itself
-        abU = onU ? axn * byh : 0.f;
-        abV = onV ? axh * byn : 0.f;
-        abW = onW ? axh * byh : 0.f;
-    } else {
-        float      axn = 0.f, axh = 0.f, byn = 0.f, byh = 0.f;
-        const bool oxn = stencil_weight(gx, g.nx + 1, i, axn);
-        const bool oxh = stencil_weight(gx - 0.5f, g.nx, i, axh);
-        const bool oyn = stencil_weight(gy, g.ny + 1, j, byn);
-        const bool oyh = stencil_weight(gy - 0.5f, g.ny, j, byh);
-        int        kh, kn;
-        bary(gz - 0.5f, g.nz, kh, fh);
-        bary(gz, g.nz + 1, kn, fn);
-        dh  = kh - (z - 1);
-        dn  = kn - (z - 1);
-        abU = (onU && oxn && oyh) ? axn * byh : 0.f;
-        abV = (onV && oxh && oyn) ? axh * byn : 0.f;
-        abW = (onW && oxh && oyh) ? axh * byh : 0.f;
-    }
-}
-
-// one column segment of P2G: nodes (i, j, k0 .. k1-1). kInterior: every cell the segment reads lies
-// in [1, n-2] on each axis, so no barycentric clamp can apply to its particles.
-// FLIP / PIC: the coordinates and velocities of kBatch particles are loaded together (one memory
-// round trip per batch instead of two or more per particle) and then added in order; a batch slot
-// past the row's end repeats its last particle with every weight 0, which adds exact zeros (a sum
-// here starts at +0 and never becomes -0), so the sums are those of the particle-by-particle loop.
-template<bool kInterior, bool kAffine>
-__device__ __forceinline__ void p2g_column(const Particles& P, const Affine& A, const uint32_t* __restrict__ cell_start, const GridGeom& g,
-                                           const FaceOut& out, int i, int j, int k0, int k1) {
-#pragma clang fp contract(off)
-    constexpr int kBatch = 4;
-    const bool uCol = j < g.ny, vCol = i < g.nx, wCol = i < g.nx && j < g.ny;
-    const int  x0 = max(i - 1, 0), x1 = min(i + 1, g.nx - 1), xu = min(i, g.nx - 1);
-    const int  y0 = max(j - 1, 0), y1 = min(j + 1, g.ny - 1);
-    const int  zs = max(k0 - 1, 0), ze = min(k1, g.nz - 1);
-    const float fi = (float)i, fj = (float)j;
-    P2gAcc     a0 = {}, a1 = {}, a2 = {};  // nodes z-1, z, z+1 while row z is read
-    for(int z = zs; z <= ze; ++z) {
-        for(int y = y0; y <= y1; ++y) {
-            const size_t   r    = lin3(0, y, z, g.nx, g.ny);
-            const uint32_t pb   = cell_start[r + x0], pe = cell_start[r + x1 + 1], pu = cell_start[r + xu + 1];
-            const bool     rowU = uCol, rowV = vCol && y <= j, rowW = wCol;
-            if constexpr(!kAffine) {
-                for(uint32_t p0 = pb; p0 < pe; p0 += kBatch) {
-                    float qx[kBatch], qy[kBatch], qz[kBatch], ux[kBatch], uy[kBatch], uz[kBatch];
 #pragma unroll
-                    for(int q = 0; q < kBatch; ++q) {
-                        const uint32_t p = min(p0 + (uint32_t)q, pe - 1u);
-                        const float4   a = P.gp[p];
-                        const float2   b = P.gv[p];
-                        qx[q]            = a.x;
-                        qy[q]            = a.y;
-                        qz[q]            = a.z;
-                        ux[q]            = a.w;
-                        uy[q]            = b.x;
-                        uz[q]            = b.y;
-                    }
+    for(int y = 0; y < kY; ++y)
 #pragma unroll
-                    for(int q = 0; q < kBatch; ++q) {
-                        const uint32_t p    = p0 + (uint32_t)q;
-                        const bool     live = p < pe;
-                        float          abU, abV, abW, fh, fn;
-                        int            dh, dn;
-                        p2g_col_weights<kInterior>(qx[q], qy[q], qz[q], live && rowU && p < pu, live && rowV, live && rowW, g, i, j, z, fi,
-                                                   fj, abU, abV, abW, fh, fn, dh, dn);
-                        // a zero weight adds exact zeros with v taken as 0
-                        const float vx = abU != 0.f ? ux[q] : 0.f, vy = abV != 0.f ? uy[q] : 0.f, vz = abW != 0.f ? uz[q] : 0.f;
-                        p2g_window_add(dh, abU, fh, vx, vx, a0.mu, a0.wu, a1.mu, a1.wu, a2.mu, a2.wu);
-                        p2g_window_add(dh, abV, fh, vy, vy, a0.mv, a0.wv, a1.mv, a1.wv, a2.mv, a2.wv);
-                        p2g_window_add(dn, abW, fn, vz, vz, a0.mw, a0.ww, a1.mw, a1.ww, a2.mw, a2.ww);
-                    }
-                }
-            } else {
-                for(uint32_t p = pb; p < pe; ++p) {
-                    float abU, abV, abW, fh, fn;
-                    int   dh, dn;
-                    const float4 gq = P.gp[p];
-                    p2g_col_weights<kInterior>(gq.x, gq.y, gq.z, rowU && p < pu, rowV, rowW, g, i, j, z, fi, fj, abU, abV, abW, fh, fn, dh,
-                                               dn);
-                    // a zero weight adds exact zeros whatever v is, so v is read only when it counts
-                    const float vx = abU != 0.f ? P.vx[p] : 0.f, vy = abV != 0.f ? P.vy[p] : 0.f, vz = abW != 0.f ? P.vz[p] : 0.f;
-                    // the base node along z of the half-shifted (u, v) and node-aligned (w) stencils
-                    const float zh = (float)(z - 1 + dh), zn = (float)(z - 1 + dn);
-                    const float px = P.px[p], py = P.py[p], pz = P.pz[p];
-                    float       cu[3] = {0.f, 0.f, 0.f}, cv[3] = {0.f, 0.f, 0.f}, cw[3] = {0.f, 0.f, 0.f};
-                    if(abU != 0.f)
-                        for(int e = 0; e < 3; ++e) cu[e] = A.c[e][p];
-                    if(abV != 0.f)
-                        for(int e = 0; e < 3; ++e) cv[e] = A.c[3 + e][p];
-                    if(abW != 0.f)
-                        for(int e = 0; e < 3; ++e) cw[e] = A.c[6 + e][p];
-                    p2g_window_add(dh, abU, fh, affine_vel(vx, cu, fi, fj, zh, 0.f, 0.5f, 0.5f, g, px, py, pz),
-                                   affine_vel(vx, cu, fi, fj, zh + 1.0f, 0.f, 0.5f, 0.5f, g, px, py, pz), a0.mu, a0.wu, a1.mu, a1.wu,
-                                   a2.mu, a2.wu);
-                    p2g_window_add(dh, abV, fh, affine_vel(vy, cv, fi, fj, zh, 0.5f, 0.f, 0.5f, g, px, py, pz),
-                                   affine_vel(vy, cv, fi, fj, zh + 1.0f, 0.5f, 0.f, 0.5f, g, px, py, pz), a0.mv, a0.wv, a1.mv, a1.wv,
-                                   a2.mv, a2.wv);
-                    p2g_window_add(dn, abW, fn, affine_vel(vz, cw, fi, fj, zn, 0.5f, 0.5f, 0.f, g, px, py, pz),
-                                   affine_vel(vz, cw, fi, fj, zn + 1.0f, 0.5f, 0.5f, 0.f, g, px, py, pz), a0.mw, a0.ww, a1.mw, a1.ww,
-                                   a2.mw, a2.ww);
-                }
+        for(int x = 0; x < kX; ++x) {
+            const float ab = wx[x] * wy[y];
+#pragma unroll
+            for(int z = 0; z < kZ; ++z) {
+                const float c = ab * wz[z];
+                m[z][y * kX + x] = __builtin_fmaf(c, v, m[z][y * kX + x]);
+                w[z][y * kX + x] += c;
             }
         }
-        if(z - 1 >= k0) p2g_emit(a0, i, j, z - 1, uCol, vCol, wCol, g, out);  // node z-1 is complete
-        a0 = a1;
-        a1 = a2;
-        a2 = P2gAcc{};
-    }
-    // nodes ze and ze+1 receive no further rows
-    if(ze >= k0 && ze < k1) p2g_emit(a0, i, j, ze, uCol, vCol, wCol, g, out);
-    if(ze + 1 >= k0 && ze + 1 < k1) p2g_emit(a1, i, j, ze + 1, uCol, vCol, wCol, g, out);
 }
-
-// the 8 stencil nodes of one particle on face grid c (extent sx x sy x sz): momentum w * v and weight
-// w = (wx * wy) * wz added to the tile's sums, acc[c * 513 + node] = (momentum, weight), for the nodes
-// the tile owns; the others go to the unused slot c * 513 + 512. The 8 nodes are distinct, so all 8
-// sums are read before any is written back (one LDS round trip per component, no branches).
-__device__ __forceinline__ void p2g_tile_add(float2* acc, int c, int ix, float fx, int iy, float fy, int iz, float fz, float v, int x0, int y0,
-                                             int z0, int3 lim) {
+// the same with the node's velocity v + dot(C, node - particle), the dot product in glm's order
+// (APIC_Solver.cpp:73-76); dx, dy, dz: node - particle per axis
+template<int kX, int kY, int kZ>
+__device__ __forceinline__ void p2g_add_affine(const float* wx, const float* wy, const float* wz, float v, const float* c, const float* dx,
+                                               const float* dy, const float* dz, float (*m)[kX * kY], float (*w)[kX * kY]) {
 #pragma clang fp contract(off)
-    const float wx[2] = {1.0f - fx, fx}, wy[2] = {1.0f - fy, fy}, wz[2] = {1.0f - fz, fz};
-    // byte offset of a node within the component's 512 owned nodes, per axis; an axis the tile does
-    // not own (outside the tile or past the grid: lim = min(8, size - tile origin)) adds 4096, so the
-    // sum of the three, clamped to 4096, is the node's offset or the unused slot's
-    uint32_t ox[2], oy[2], oz[2];
+    float ez[kZ];
 #pragma unroll
-    for(int d = 0; d < 2; ++d) {
-        const uint32_t i = (uint32_t)(ix + d - x0), j = (uint32_t)(iy + d - y0), k = (uint32_t)(iz + d - z0);
-        ox[d]            = i < (uint32_t)lim.x ? i * 8u : 4096u;
-        oy[d]            = j < (uint32_t)lim.y ? j * 64u : 4096u;
-        oz[d]            = k < (uint32_t)lim.z ? k * 512u : 4096u;
-    }
-    char* const base = reinterpret_cast<char*>(acc + c * 513);
-    float2*     n[8];
-    float       w[8];
+    for(int z = 0; z < kZ; ++z) ez[z] = c[2] * dz[z];
 #pragma unroll
-    for(int e = 0; e < 8; ++e) {
-        const int dx = e & 1, dy = (e >> 1) & 1, dz = e >> 2;
-        n[e]         = reinterpret_cast<float2*>(base + min(ox[dx] + oy[dy] + oz[dz], 4096u));
-        w[e]         = (wx[dx] * wy[dy]) * wz[dz];
-    }
-    float2 a[8];
+    for(int y = 0; y < kY; ++y)
 #pragma unroll
-    for(int e = 0; e < 8; ++e) a[e] = *n[e];
+        for(int x = 0; x < kX; ++x) {
+            const float ab = wx[x] * wy[y], exy = c[0] * dx[x] + c[1] * dy[y];
 #pragma unroll
-    for(int e = 0; e < 8; ++e) {
-        a[e].x += w[e] * v;
-        a[e].y += w[e];
-    }
-#pragma unroll
-    for(int e = 0; e < 8; ++e) *n[e] = a[e];
-}
-
-//--------------------------------------------------------------------------------------------------
-// P2G (FLIP / PIC) as a deterministic scatter: one wavefront per 8^3 tile of nodes, every particle's
-// stencil weights computed once. A particle binned to cell c reaches nodes c-1 .. c+1 on each axis
-// (clamps included), so the tile's nodes [x0, x0+8) x [y0, y0+8) x [z0, z0+8) of the three face grids
-// receive only particles of the cells [x0-1, x0+8] x .. (10^3, clipped to the grid), which it
-// visits in 27 rounds, one colour class (cx mod 3, cy mod 3, cz mod 3) per round. Two cells of one
-// colour lie 3 or more cells apart on some axis and reach no common node, so in a round each lane
-// owns a cell (at most 4 x 4 x 4 per colour) and adds its particles, in their sorted order, to the
-// tile's momentum and weight sums in LDS with no other lane touching those nodes. A node's sum is
-// therefore taken in a fixed order: by colour, then by particle; each term is the reference's
-// weight (wx * wy) * wz and momentum w * v, rounded before the add (no contraction). Contributions to
-// nodes outside the tile are left to the tile that owns them.
-//--------------------------------------------------------------------------------------------------
-struct k_p2g_tile {
-    static constexpr int kThreads = 64;
-    Particles P;
-    const uint32_t* __restrict__ cell_start;
-    GridGeom g;
-    FaceOut out;
-    const uint8_t* __restrict__ occ;  // particle occupancy of the 8^3 cell bricks (binning)
-    __device__ void operator()(Blk blk) const {
-#pragma clang fp contract(off)
-        __shared__ float2 acc[3 * 513];  // [component][node (x fastest), + 1 unused]: (momentum, weight)
-        int tx, ty, tz;
-        tile_of_block(blk, (g.nx + 8) / 8, (g.ny + 8) / 8, (g.nz + 8) / 8, tx, ty, tz);
-        const int x0 = tx * 8, y0 = ty * 8, z0 = tz * 8, lane = threadIdx.x;
-        const int cx0 = max(x0 - 1, 0), cx1 = min(x0 + 8, g.nx - 1);  // cells read
-        const int cy0 = max(y0 - 1, 0), cy1 = min(y0 + 8, g.ny - 1);
-        const int cz0 = max(z0 - 1, 0), cz1 = min(z0 + 8, g.nz - 1);
-        // nodes owned per axis and component (face grids (nx+1, ny, nz), (nx, ny+1, nz), (nx, ny, nz+1));
-        // the tile origin never lies past a face grid's size, so each is in 0 .. 8
-        const int  mx = min(8, g.nx - x0), my = min(8, g.ny - y0), mz = min(8, g.nz - z0);
-        const int3 limU = make_int3(min(8, g.nx + 1 - x0), my, mz), limV = make_int3(mx, min(8, g.ny + 1 - y0), mz),
-                   limW = make_int3(mx, my, min(8, g.nz + 1 - z0));
-        for(int e = lane; e < 3 * 513; e += 64) acc[e] = make_float2(0.f, 0.f);
-        bool any = false;
-        for(int bz = cz0 >> 3; bz <= (cz1 >> 3); ++bz)
-            for(int by = cy0 >> 3; by <= (cy1 >> 3); ++by)
-                for(int bx = cx0 >> 3; bx <= (cx1 >> 3); ++bx) any |= occ[(bz * g.nby + by) * g.nbx + bx] != 0;
-        __syncthreads();
-        if(any) {
-            // the particle range of the lane's cell in a colour round (empty when the lane has no cell)
-            auto range = [&](int colour, uint32_t& pb, uint32_t& pe) {
-                const int kx = colour % 3, ky = (colour / 3) % 3, kz = colour / 9;
-                // the (lane & 3)-th, ((lane >> 2) & 3)-th, (lane >> 4)-th cell of this colour on each axis
-                const int cx = cx0 + (kx - cx0 % 3 + 3) % 3 + 3 * (lane & 3);
-                const int cy = cy0 + (ky - cy0 % 3 + 3) % 3 + 3 * ((lane >> 2) & 3);
-                const int cz = cz0 + (kz - cz0 % 3 + 3) % 3 + 3 * (lane >> 4);
-                pb = pe = 0;
-                if(cx <= cx1 && cy <= cy1 && cz <= cz1) {
-                    const size_t cell = lin3(cx, cy, cz, g.nx, g.ny);
-                    pb                = cell_start[cell];
-                    pe                = cell_start[cell + 1];
-                }
-            };
-            // up to 8 particles [p0, pe) of a cell: coordinates and velocities (a slot past pe repeats the last)
-            struct Batch {
-                float qx[8], qy[8], qz[8], ux[8], uy[8], uz[8];
-            };
-            auto load = [&](uint32_t p0, uint32_t pe, Batch& B) {
-#pragma unroll
-                for(int q = 0; q < 8; ++q) {
-                    const uint32_t p = min(p0 + (uint32_t)q, pe - 1u);
-                    const float4   a = P.gp[p];
-                    const float2   b = P.gv[p];
-                    B.qx[q]          = a.x;
-                    B.qy[q]          = a.y;
-                    B.qz[q]          = a.z;
-                    B.ux[q]          = a.w;
-                    B.uy[q]          = b.x;
-                    B.uz[q]          = b.y;
-                }
-            };
-            auto add = [&](const Batch& B, uint32_t p0, uint32_t pe) {
-#pragma unroll
-                for(int q = 0; q < 8; ++q) {
-                    if(p0 + (uint32_t)q >= pe) break;
-                    // node-aligned (n) and half-shifted (h) stencils on each axis: base and fraction
-                    int   ixn, ixh, iyn, iyh, izn, izh;
-                    float fxn, fxh, fyn, fyh, fzn, fzh;
-                    bary(B.qx[q], g.nx + 1, ixn, fxn);
-                    bary(B.qx[q] - 0.5f, g.nx, ixh, fxh);
-                    bary(B.qy[q], g.ny + 1, iyn, fyn);
-                    bary(B.qy[q] - 0.5f, g.ny, iyh, fyh);
-                    bary(B.qz[q], g.nz + 1, izn, fzn);
-                    bary(B.qz[q] - 0.5f, g.nz, izh, fzh);
-                    // u: x node-aligned, y and z half-shifted; v: y node-aligned; w: z node-aligned
-                    p2g_tile_add(acc, 0, ixn, fxn, iyh, fyh, izh, fzh, B.ux[q], x0, y0, z0, limU);
-                    p2g_tile_add(acc, 1, ixh, fxh, iyn, fyn, izh, fzh, B.uy[q], x0, y0, z0, limV);
-                    p2g_tile_add(acc, 2, ixh, fxh, iyh, fyh, izn, fzn, B.uz[q], x0, y0, z0, limW);
-                }
-            };
-            // software pipeline: a round's first batch is loaded during the round before, its cell
-            // range two rounds before
-            Batch    cur, nxt;
-            uint32_t cb, ce, nb, ne, nnb = 0, nne = 0;
-            range(0, cb, ce);
-            range(1, nb, ne);
-            if(cb < ce) load(cb, ce, cur);
-            for(int colour = 0; colour < 27; ++colour) {
-                if(colour + 1 < 27 && nb < ne) load(nb, ne, nxt);
-                if(colour + 2 < 27) range(colour + 2, nnb, nne);
-                for(uint32_t p0 = cb; p0 < ce; p0 += 8) {
-                    if(p0 != cb) load(p0, ce, cur);  // cells of more than 8 particles
-                    add(cur, p0, ce);
-                }
-                __syncthreads();
-                cur = nxt;
-                cb  = nb;
-                ce  = ne;
-                nb  = nnb;
-                ne  = nne;
+            for(int z = 0; z < kZ; ++z) {
+                const float q = ab * wz[z];
+                m[z][y * kX + x] = __builtin_fmaf(q, v + (exy + ez[z]), m[z][y * kX + x]);
+                w[z][y * kX + x] += q;
             }
         }
-        // the tile's nodes: u = momentum / weight where the weight is positive, else 0 and invalid
-        for(int e = lane; e < 512; e += 64) {
-            const int i = x0 + (e & 7), j = y0 + ((e >> 3) & 7), k = z0 + (e >> 6);
-            if(i <= g.nx && j < g.ny && k < g.nz) {
-                const size_t id = lin3(i, j, k, g.nx + 1, g.ny);
-                const float  m = acc[e].x, w = acc[e].y;
-                const bool   ok = w > kFltMin;
-                out.u[id]       = ok ? m / w : 0.f;
-                out.vu[id]      = ok ? 1 : 0;
-            }
-            if(i < g.nx && j <= g.ny && k < g.nz) {
-                const size_t id = lin3(i, j, k, g.nx, g.ny + 1);
-                const float  m = acc[513 + e].x, w = acc[513 + e].y;
-                const bool   ok = w > kFltMin;
-                out.v[id]       = ok ? m / w : 0.f;
-                out.vv[id]      = ok ? 1 : 0;
-            }
-            if(i < g.nx && j < g.ny && k <= g.nz) {
-                const size_t id = lin3(i, j, k, g.nx, g.ny);
-                const float  m = acc[1026 + e].x, w = acc[1026 + e].y;
-                const bool   ok = w > kFltMin;
-                out.w[id]       = ok ? m / w : 0.f;
-                out.vw[id]      = ok ? 1 : 0;
-            }
-        }
-    }
-};
+}
 
-template<bool kAffine, int kSeg>
-struct k_p2g_col {
-    static constexpr int kThreads = kBlock;
+template<bool kAffine>
+struct k_p2g {
+    static constexpr int kThreads = kP2gSide * kP2gSide;
+    // FLIP: 3 waves per SIMD hide a batch's load (170 registers; a batch of 4 loaded ahead of its use took
+    // 206, 2 waves, and 980 us against 890 at 256^3). Affine: a record is 18 floats, so 2 waves and the next
+    // record loaded ahead (bounded to 3 waves it spills: 657 against 181 us for 1.27M particles).
+    static constexpr int  kOneBlocks = kAffine ? 2 : 3, kManyBlocks = kOneBlocks;
+    static constexpr int  kBatch = kAffine ? 1 : 2;  // particles whose records are loaded together
+    static constexpr bool kAhead = kAffine;          // ... before the batch ahead of them is added
     Particles P;
     Affine A;
     const uint32_t* __restrict__ cell_start;
     GridGeom g;
     FaceOut out;
     const uint8_t* __restrict__ occ;  // particle occupancy of the 8^3 cell bricks (binning)
-    __device__ void operator()(Blk blk) const {
-        const int      ex = g.nx + 1, ey = g.ny + 1, ez = g.nz + 1;
-        const uint32_t cols = (uint32_t)ex * (uint32_t)ey;
-        const uint32_t nseg = (uint32_t)(ez + kSeg - 1) / kSeg;
-        // consecutive blocks (neighbouring j rows, which read the same particle rows) stay on one XCD
-        const uint32_t nblk = blk.n, b = blk.id, xcd = b % 8u, q = nblk / 8u, rr = nblk % 8u;
-        const uint32_t t    = (xcd * q + min(xcd, rr) + b / 8u) * blockDim.x + threadIdx.x;
-        if(t >= cols * nseg) return;
-        const int  i = (int)(t % (uint32_t)ex), j = (int)((t / (uint32_t)ex) % (uint32_t)ey), seg = (int)(t / cols);
-        const int  k0 = seg * kSeg, k1 = min(k0 + kSeg, ez);  // nodes [k0, k1)
-        // cells read: x in [i-1, i+1], y in [j-1, j+1], z in [k0-1, k1] (clamped to the grid). With no
-        // particle in any brick covering them every node of the segment has weight 0: u = 0, invalid.
-        {
-            const int x0 = max(i - 1, 0), x1 = min(i + 1, g.nx - 1), y0 = max(j - 1, 0), y1 = min(j + 1, g.ny - 1);
-            const int zs = max(k0 - 1, 0), ze = min(k1, g.nz - 1);
-            bool      any = false;
-            for(int bz = zs >> 3; bz <= (ze >> 3); ++bz)
-                for(int by = y0 >> 3; by <= (y1 >> 3); ++by)
-                    for(int bx = x0 >> 3; bx <= (x1 >> 3); ++bx) any |= occ[(bz * g.nby + by) * g.nbx + bx] != 0;
-            if(!any) {
-                const P2gAcc zero{};
-                for(int k = k0; k < k1; ++k) p2g_emit(zero, i, j, k, j < g.ny, i < g.nx, i < g.nx && j < g.ny, g, out);
-                return;
+    int seg;                          // node planes per workgroup
+    struct Rec {
+        float x[kBatch], y[kBatch], z[kBatch], u[kBatch], v[kBatch], w[kBatch];
+        float p[kAffine ? kBatch : 1][3], c[kAffine ? kBatch : 1][9];
+    };
+    // particles [p, p + kBatch) of a cell that ends at e (a slot past it repeats the last)
+    __device__ __forceinline__ void load(uint32_t p, uint32_t e, Rec& R) const {
+#pragma unroll
+        for(int q = 0; q < kBatch; ++q) {
+            const uint32_t at = min(p + (uint32_t)q, e - 1u);
+            const float4   a = P.gp[at];
+            const float2   b = P.gv[at];
+            R.x[q] = a.x;
+            R.y[q] = a.y;
+            R.z[q] = a.z;
+            R.u[q] = a.w;
+            R.v[q] = b.x;
+            R.w[q] = b.y;
+            if constexpr(kAffine) {
+                R.p[q][0] = P.px[at];
+                R.p[q][1] = P.py[at];
+                R.p[q][2] = P.pz[at];
+#pragma unroll
+                for(int k = 0; k < 9; ++k) R.c[q][k] = A.c[k][at];
             }
         }
-        const bool interior = i >= 2 && i <= g.nx - 3 && j >= 2 && j <= g.ny - 3 && k0 >= 2 && k1 <= g.nz - 2;
-        if(interior) p2g_column<true, kAffine>(P, A, cell_start, g, out, i, j, k0, k1);
-        else p2g_column<false, kAffine>(P, A, cell_start, g, out, i, j, k0, k1);
+    }
+    __device__ void operator()(Blk blk) const {
+#pragma clang fp contract(off)
+        __shared__ float2 part[21][kThreads];  // a complete plane's partial sums: u 2x3, v 3x2, w 3x3
+        const int ntx = (g.nx + kP2gOwn) / kP2gOwn, nty = (g.ny + kP2gOwn) / kP2gOwn, ntz = (g.nz + seg) / seg;
+        int       tx, ty, tz;
+        tile_of_block(blk, ntx, nty, ntz, tx, ty, tz);
+        const int  t = threadIdx.x, lx = t % kP2gSide, ly = t / kP2gSide;
+        const int  i = tx * kP2gOwn - 1 + lx, j = ty * kP2gOwn - 1 + ly;  // the thread's column, and the node it owns
+        const int  k0 = tz * seg, k1 = min(k0 + seg, g.nz + 1);           // node planes [k0, k1)
+        const bool column = i >= 0 && i < g.nx && j >= 0 && j < g.ny;
+        const bool own = lx >= 1 && lx <= kP2gOwn && ly >= 1 && ly <= kP2gOwn;
+        const bool ownU = own && i <= g.nx && j < g.ny, ownV = own && i < g.nx && j <= g.ny, ownW = own && i < g.nx && j < g.ny;
+        // any particle in the bricks of the cells read? One brick a thread
+        const int bx0 = max(tx * kP2gOwn - 1, 0) >> 3, bx1 = min(tx * kP2gOwn + kP2gOwn, g.nx - 1) >> 3;
+        const int by0 = max(ty * kP2gOwn - 1, 0) >> 3, by1 = min(ty * kP2gOwn + kP2gOwn, g.ny - 1) >> 3;
+        const int bz0 = max(k0 - 1, 0) >> 3, bz1 = min(k1, g.nz - 1) >> 3;
+        const int mx = bx1 - bx0 + 1, my = by1 - by0 + 1, mb = mx * my * (bz1 - bz0 + 1);
+        int       any = 0;
+        for(int b = t; b < mb; b += kThreads) any |= occ[((bz0 + b / (mx * my)) * g.nby + by0 + (b / mx) % my) * g.nbx + bx0 + b % mx];
+        if(!__syncthreads_or(any)) {
+            for(int k = k0; k < k1; ++k) {
+                emit(out.u, out.vu, make_float2(0.f, 0.f), ownU && k < g.nz, lin3(i, j, k, g.nx + 1, g.ny));
+                emit(out.v, out.vv, make_float2(0.f, 0.f), ownV && k < g.nz, lin3(i, j, k, g.nx, g.ny + 1));
+                emit(out.w, out.vw, make_float2(0.f, 0.f), ownW, lin3(i, j, k, g.nx, g.ny));
+            }
+            return;
+        }
+        const float fi = (float)i, fj = (float)j;
+        const bool  edgeXY = i == 0 || i == g.nx - 1 || j == 0 || j == g.ny - 1;
+        // world positions of the column's nodes (getWorldCoordinate: (index + extra) * dx + bMin)
+        float nodeX[2], halfX[3], nodeY[2], halfY[3];
+        if constexpr(kAffine) {
+#pragma unroll
+            for(int e = 0; e < 2; ++e) {
+                nodeX[e] = (fi + (float)e) * g.dx + g.bminx;
+                nodeY[e] = (fj + (float)e) * g.dx + g.bminy;
+            }
+#pragma unroll
+            for(int e = 0; e < 3; ++e) {
+                halfX[e] = ((fi + (float)(e - 1)) + 0.5f) * g.dx + g.bminx;
+                halfY[e] = ((fj + (float)(e - 1)) + 0.5f) * g.dx + g.bminy;
+            }
+        }
+        // sums of the planes z-1, z, z+1 (u, v) and z, z+1 (w) while row z is read
+        float mu[3][6] = {}, wu[3][6] = {}, mv[3][6] = {}, wv[3][6] = {}, mw[2][9] = {}, ww[2][9] = {};
+        auto  range = [&](int z, uint32_t& b, uint32_t& e) {
+            b = e = 0;
+            if(column && z < g.nz) {
+                const size_t c = lin3(i, j, z, g.nx, g.ny);
+                b              = cell_start[c];
+                e              = cell_start[c + 1];
+            }
+        };
+        auto add = [&](const Rec& R, uint32_t p, uint32_t e, int z) {
+#pragma unroll
+            for(int q = 0; q < kBatch; ++q) {
+                if(p + (uint32_t)q >= e) break;
+                float xn[2], xh[3], yn[2], yh[3], zn[2], zh[3];
+                p2g_axis(R.x[q], fi, xn, xh);
+                p2g_axis(R.y[q], fj, yn, yh);
+                p2g_axis(R.z[q], (float)z, zn, zh);
+                if(edgeXY) {
+                    p2g_axis_edge(i == 0, i == g.nx - 1, xh);
+                    p2g_axis_edge(j == 0, j == g.ny - 1, yh);
+                }
+                if(z == 0 || z == g.nz - 1) p2g_axis_edge(z == 0, z == g.nz - 1, zh);
+                if constexpr(kAffine) {
+                    const float fz = (float)z;
+                    float       dnx[2], dhx[3], dny[2], dhy[3], dnz[2], dhz[3];
+#pragma unroll
+                    for(int k = 0; k < 2; ++k) {
+                        dnx[k] = nodeX[k] - R.p[q][0];
+                        dny[k] = nodeY[k] - R.p[q][1];
+                        dnz[k] = ((fz + (float)k) * g.dx + g.bminz) - R.p[q][2];
+                    }
+#pragma unroll
+                    for(int k = 0; k < 3; ++k) {
+                        dhx[k] = halfX[k] - R.p[q][0];
+                        dhy[k] = halfY[k] - R.p[q][1];
+                        dhz[k] = (((fz + (float)(k - 1)) + 0.5f) * g.dx + g.bminz) - R.p[q][2];
+                    }
+                    p2g_add_affine<2, 3, 3>(xn, yh, zh, R.u[q], R.c[q], dnx, dhy, dhz, mu, wu);
+                    p2g_add_affine<3, 2, 3>(xh, yn, zh, R.v[q], R.c[q] + 3, dhx, dny, dhz, mv, wv);
+                    p2g_add_affine<3, 3, 2>(xh, yh, zn, R.w[q], R.c[q] + 6, dhx, dhy, dnz, mw, ww);
+                } else {
+                    p2g_add<2, 3, 3>(xn, yh, zh, R.u[q], mu, wu);
+                    p2g_add<3, 2, 3>(xh, yn, zh, R.v[q], mv, wv);
+                    p2g_add<3, 3, 2>(xh, yh, zn, R.w[q], mw, ww);
+                }
+            }
+        };
+        // the owned node of the planes that row k0 completes (u, v: k0 - 1; w: k0)
+        const uint32_t sU = (uint32_t)((g.nx + 1) * g.ny), sV = (uint32_t)(g.nx * (g.ny + 1)), sW = (uint32_t)(g.nx * g.ny);
+        uint32_t       atU = (uint32_t)(k0 - 1) * sU + (uint32_t)(j * (g.nx + 1) + i), atV = (uint32_t)(k0 - 1) * sV + (uint32_t)(j * g.nx + i),
+                 atW = (uint32_t)k0 * sW + (uint32_t)(j * g.nx + i);
+        const int zs = max(k0 - 1, 0), ze = min(k1, g.nz);  // row nz holds no cells: it only completes the last planes
+        uint32_t  pb, pe, nb, ne;
+        Rec       cur, nxt;
+        range(zs, pb, pe);
+        if(pb < pe) load(pb, pe, cur);
+        for(int z = zs; z <= ze; ++z) {
+            range(z + 1, nb, ne);
+            if(z == ze) ne = nb;
+            // after a batch comes the cell's next one, or the first of the next row's cell
+            if(pb < pe) {
+                do {
+                    Rec& at = kAhead ? nxt : cur;
+                    if(!kAhead) add(cur, pb, pe, z);
+                    if(pb + kBatch < pe) load(pb + kBatch, pe, at);
+                    else if(nb < ne) load(nb, ne, at);
+                    if(kAhead) {
+                        add(cur, pb, pe, z);
+                        cur = nxt;
+                    }
+                    pb += kBatch;
+                } while(pb < pe);
+            } else if(nb < ne) {
+                load(nb, ne, cur);
+            }
+            pb = nb;
+            pe = ne;
+            // planes z-1 of u and v and z of w are complete
+            if(z >= k0) {
+#pragma unroll
+                for(int e = 0; e < 6; ++e) {
+                    part[e][t]     = make_float2(mu[0][e], wu[0][e]);
+                    part[6 + e][t] = make_float2(mv[0][e], wv[0][e]);
+                }
+#pragma unroll
+                for(int e = 0; e < 9; ++e) part[12 + e][t] = make_float2(mw[0][e], ww[0][e]);
+                __syncthreads();
+                if(own) {
+                    // the column at (dx, dy) reaches this node with its own offset (-dx, -dy)
+                    if(z > k0) {
+                        float2 a = make_float2(0.f, 0.f), b = make_float2(0.f, 0.f);
+#pragma unroll
+                        for(int dy = -1; dy <= 1; ++dy)
+#pragma unroll
+                            for(int dx = -1; dx <= 0; ++dx) {
+                                const float2 s = part[(1 - dy) * 2 - dx][t + dy * kP2gSide + dx];
+                                a.x += s.x;
+                                a.y += s.y;
+                            }
+#pragma unroll
+                        for(int dy = -1; dy <= 0; ++dy)
+#pragma unroll
+                            for(int dx = -1; dx <= 1; ++dx) {
+                                const float2 s = part[6 + (-dy) * 3 + 1 - dx][t + dy * kP2gSide + dx];
+                                b.x += s.x;
+                                b.y += s.y;
+                            }
+                        emit(out.u, out.vu, a, ownU, atU);
+                        emit(out.v, out.vv, b, ownV, atV);
+                    }
+                    if(z < k1) {
+                        float2 c = make_float2(0.f, 0.f);
+#pragma unroll
+                        for(int dy = -1; dy <= 1; ++dy)
+#pragma unroll
+                            for(int dx = -1; dx <= 1; ++dx) {
+                                const float2 s = part[12 + (1 - dy) * 3 + 1 - dx][t + dy * kP2gSide + dx];
+                                c.x += s.x;
+                                c.y += s.y;
+                            }
+                        emit(out.w, out.vw, c, ownW, atW);
+                    }
+                }
+                __syncthreads();
+                atU += sU;
+                atV += sV;
+                atW += sW;
+            }
+#pragma unroll
+            for(int e = 0; e < 6; ++e) {
+                mu[0][e] = mu[1][e], wu[0][e] = wu[1][e], mu[1][e] = mu[2][e], wu[1][e] = wu[2][e], mu[2][e] = 0.f, wu[2][e] = 0.f;
+                mv[0][e] = mv[1][e], wv[0][e] = wv[1][e], mv[1][e] = mv[2][e], wv[1][e] = wv[2][e], mv[2][e] = 0.f, wv[2][e] = 0.f;
+            }
+#pragma unroll
+            for(int e = 0; e < 9; ++e) mw[0][e] = mw[1][e], ww[0][e] = ww[1][e], mw[1][e] = 0.f, ww[1][e] = 0.f;
+        }
+    }
+    // node velocity = momentum / weight where the weight is positive, else 0 and invalid
+    __device__ __forceinline__ static void emit(float* __restrict__ vel, uint8_t* __restrict__ valid, float2 s, bool mine, size_t at) {
+        if(!mine) return;
+        const bool ok = s.y > kFltMin;
+        vel[at]       = ok ? s.x / s.y : 0.f;
+        valid[at]     = ok ? 1 : 0;
     }
 };
 

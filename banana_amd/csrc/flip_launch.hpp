@@ -23,13 +23,22 @@ struct Blk {
     uint32_t id, n;  // this workgroup's index among its scene's workgroups, and their count
 };
 
+// Workgroups per CU that the single-scene form of K is compiled to leave room for: K::kOneBlocks where
+// the functor names it, else 1 (no bound).
+template<class K, class = void> struct one_blocks {
+    static constexpr int value = 1;
+};
+template<class K> struct one_blocks<K, std::void_t<decltype(K::kOneBlocks)>> {
+    static constexpr int value = K::kOneBlocks;
+};
+
 // Single scene. The functor is the kernel's only argument, so it lies at offset 0 of the
 // kernel-argument segment, and it is called in place there (constant memory, read with scalar loads
 // even where it indexes one of its arrays at run time, as k_move does with the boundary shapes). Used
 // as the by-value parameter instead, such a functor is first copied to per-lane scratch. The call is
 // inlined by force here and in k_many: the larger functors exceed the inliner's threshold, and a real
 // call doubles their registers.
-template<class K> __global__ void __launch_bounds__(K::kThreads) k_one(K k) {
+template<class K> __global__ void __launch_bounds__(K::kThreads, one_blocks<K>::value) k_one(K k) {
     (void)k;
     const K* kp = (const K*)__builtin_amdgcn_kernarg_segment_ptr();  // an address-space conversion
     [[clang::always_inline]] (*kp)(Blk{blockIdx.x, gridDim.x});

@@ -227,6 +227,7 @@ private:
         t.s->pending    = {};
         t.s->atBarrier  = false;
         t.s->prm.timing = t.savedTiming;
+        t.s->p2gSeg     = 0;  // alone the scene chooses its own
         rec->giveLane(t.lane);
         t.co.reset();
         t.next = {};
@@ -334,13 +335,8 @@ private:
     std::unordered_map<uint64_t, Entry> table;
 };
 
-// the batched launch of P2G: the affine transfer's column gather with segment seg (4, 8 or 16), or
-// the FLIP / PIC tile scatter (which has no segment)
-static inline Recorder::LaunchFn p2g_launch_fn(int seg, bool affine) {
-    if(affine)
-        return seg == 4 ? Recorder::fnOf<k_p2g_col<true, 4>>() : (seg == 16 ? Recorder::fnOf<k_p2g_col<true, 16>>() : Recorder::fnOf<k_p2g_col<true, 8>>());
-    return Recorder::fnOf<k_p2g_tile>();
-}
+// the batched launch of P2G
+static inline Recorder::LaunchFn p2g_launch_fn(bool affine) { return affine ? Recorder::fnOf<k_p2g<true>>() : Recorder::fnOf<k_p2g<false>>(); }
 
 static inline uint64_t batch_signature(const std::vector<FlipSolver*>& sc) {
     uint64_t cells = 0;

@@ -307,9 +307,9 @@ public:
     std::vector<uint32_t> rankHost;
     bool        systemValid = false;
     bool        lastRefined = false;
-    // launch shapes that leave results unchanged (set by the batch autotuner): P2G column segment
-    // length, and the PCG iterations queued before the first stop-flag poll and at most per poll
-    int      p2gSeg        = 8;
+    // launch shapes that leave results unchanged (set by the batch autotuner): P2G segment length
+    // (0: by the grid, p2gSegment), and the PCG iterations queued before the first stop-flag poll and at most per poll
+    int      p2gSeg        = 0;
     uint32_t pcgChunkFirst = 4, pcgChunkMax = 64;
 
     // stats
@@ -690,18 +690,20 @@ public:
         if(!binned) binParticles();
     }
 
-    // APIC_Solver.cpp:52-91 / AFLIP_Solver.cpp:48-90 as a column gather; the column segment length
-    // p2gSeg (4, 8 or 16) does not change the result
-    template<bool kAffine, int kSeg> void p2gLaunch(const FaceOut& out) {
-        const size_t n = (size_t)(g.nx + 1) * (g.ny + 1) * (((size_t)g.nz + 1 + kSeg - 1) / kSeg);  // columns x segments
-        launch(k_p2g_col<kAffine, kSeg>{cur->view(), kAffine ? cur->affine() : Affine{}, (const uint32_t*)cellStart.as<uint32_t>(), g, out,
-                                        (const uint8_t*)occ.as<uint8_t>()},
-               blocks(n));
+    // node planes per P2G workgroup: the segment re-reads two rows of cells, so it is as long as leaves
+    // the chip's 256 CUs with work (the result does not depend on it)
+    int p2gSegment() const {
+        const int cols = ((g.nx + kP2gOwn) / kP2gOwn) * ((g.ny + kP2gOwn) / kP2gOwn);
+        int       seg  = 16;
+        while(seg > 2 && cols * ((g.nz + seg) / seg) < 1024) seg /= 2;
+        return seg;
     }
-    template<bool kAffine> void p2gSegLaunch(const FaceOut& out) {
-        if(p2gSeg == 4) p2gLaunch<kAffine, 4>(out);
-        else if(p2gSeg == 16) p2gLaunch<kAffine, 16>(out);
-        else p2gLaunch<kAffine, 8>(out);
+    template<bool kAffine> void p2gLaunch(const FaceOut& out) {
+        const int      seg = p2gSeg ? p2gSeg : p2gSegment();
+        const uint32_t n   = (uint32_t)(((g.nx + kP2gOwn) / kP2gOwn) * ((g.ny + kP2gOwn) / kP2gOwn) * ((g.nz + seg) / seg));
+        launch(k_p2g<kAffine>{cur->view(), kAffine ? cur->affine() : Affine{}, (const uint32_t*)cellStart.as<uint32_t>(), g, out,
+                              (const uint8_t*)occ.as<uint8_t>(), seg},
+               n);
     }
     void mapParticles2Grid() {
         requireBinned();
@@ -711,12 +713,8 @@ public:
         }
         FaceOut out{u.as<float>(), v.as<float>(), w.as<float>(), vu.as<uint8_t>(), vv.as<uint8_t>(), vw.as<uint8_t>()};
         ktBegin(BNN_KT_P2G);
-        if(affineScheme()) {
-            p2gSegLaunch<true>(out);  // APIC_Solver.cpp:52-91, AFLIP_Solver.cpp:48-90
-        } else {  // FLIP_Solver.cpp:57-95: one wavefront per 8^3 tile of nodes
-            const uint32_t tiles = (uint32_t)(((g.nx + 8) / 8) * ((g.ny + 8) / 8) * ((g.nz + 8) / 8));
-            launch(k_p2g_tile{cur->view(), (const uint32_t*)cellStart.as<uint32_t>(), g, out, (const uint8_t*)occ.as<uint8_t>()}, tiles);
-        }
+        if(affineScheme()) p2gLaunch<true>(out);  // APIC_Solver.cpp:52-91, AFLIP_Solver.cpp:48-90
+        else p2gLaunch<false>(out);               // FLIP_Solver.cpp:57-95
         ktEnd(BNN_KT_P2G);
     }
 
@@ -2366,7 +2364,7 @@ bnn_status batch_call(bnn_flip_batch* b, bnn_flip* const* scenes, uint32_t n, bn
         const bnn::BatchRunner::Shape sh     = b->pinned ? b->pinnedShape : b->tuner.next(sig);
         R.setShape(sh);
         if(tuning) {
-            rec.timedFns = {bnn::p2g_launch_fn(sh.p2gSeg, false), bnn::p2g_launch_fn(sh.p2gSeg, true)};
+            rec.timedFns = {bnn::p2g_launch_fn(false), bnn::p2g_launch_fn(true)};
             rec.timedMs  = 0;
         }
         std::vector<bnn::BatchRunner::Task> tasks(n);

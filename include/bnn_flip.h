@@ -402,7 +402,7 @@ bnn_status  bnn_flip_footprint(const bnn_flip_params* p, uint64_t n_particles, u
  * with one copy and one wait; launch sequences that repeat (PCG iterations) are replayed from
  * hipGraphs. A scene's blocks compute exactly what they compute alone, so each scene's results are
  * bit-identical to stepping it alone, in any batch. Launch shapes that cannot change results (the
- * APIC / AFLIP P2G column segment, PCG iterations per stop-flag poll, scene blocks per workgroup,
+ * P2G segment, PCG iterations per stop-flag poll, scene blocks per workgroup,
  * graphs on or off)
  * are chosen by an autotuner over the first calls of each batch size, or pinned with
  * bnn_flip_batch_set_shape. The scenes stay owned by their handles; a handle must not be used
@@ -422,7 +422,7 @@ bnn_status  bnn_flip_batch_advance_frame(bnn_flip_batch* b, bnn_flip* const* sce
 bnn_status  bnn_flip_batch_pressure_projection(bnn_flip_batch* b, bnn_flip* const* scenes, const float* dts, uint32_t n,
                                                bnn_status* status);
 typedef struct bnn_batch_shape {
-    int32_t  p2g_segment;     /* z nodes per thread of the APIC / AFLIP P2G gather: 4, 8 or 16 */
+    int32_t  p2g_segment;     /* z node planes per P2G workgroup: 4, 8 or 16 */
     uint32_t pcg_chunk_first; /* PCG iterations queued before the first stop-flag poll */
     uint32_t pcg_chunk_max;   /* ... and at most per poll after it (later chunks: the iterations a geometric
                                  fit of max|r| so far says remain) */
