@@ -64,74 +64,69 @@ __device__ __forceinline__ float bilerpf(float v00, float v10, float v01, float 
     return lerpf(lerpf(v00, v10, fx), lerpf(v01, v11, fx), fy);
 }
 
-// ArrayHelpers.cpp:91-102: interpolateValueLinear on an array with dims (sx, sy, sz)
-__device__ __forceinline__ float interp3(const float* __restrict__ g, int sx, int sy, int sz, float x, float y, float z) {
-    int   i, j, k;
-    float fi, fj, fk;
-    bary(x, sx, i, fi);
-    bary(y, sy, j, fj);
-    bary(z, sz, k, fk);
-    const size_t b   = lin3(i, j, k, sx, sy);
-    const size_t sxy = (size_t)sx * sy;
-    float v000 = g[b], v100 = g[b + 1], v010 = g[b + sx], v110 = g[b + sx + 1];
-    float v001 = g[b + sxy], v101 = g[b + sxy + 1], v011 = g[b + sxy + sx], v111 = g[b + sxy + sx + 1];
-    return lerpf(bilerpf(v000, v100, v010, v110, fi, fj), bilerpf(v001, v101, v011, v111, fi, fj), fk);
+// The 2x2x2 stencil of grid coordinate (x, y, z) on an array with dims (sx, sy, sz): first corner and
+// fractions (MathHelpers.h:515-529 per axis)
+struct Stencil {
+    size_t at, sx, sxy;
+    float  fi, fj, fk;
+};
+__device__ __forceinline__ Stencil stencil3(int sx, int sy, int sz, float x, float y, float z) {
+    int     i, j, k;
+    Stencil s;
+    bary(x, sx, i, s.fi);
+    bary(y, sy, j, s.fj);
+    bary(z, sz, k, s.fk);
+    s.at  = lin3(i, j, k, sx, sy);
+    s.sx  = (size_t)sx;
+    s.sxy = (size_t)sx * sy;
+    return s;
 }
-
-// Same stencil on the difference (a - b): computeChangesGridVelocity followed by the FLIP
-// interpolation (FLIP_Solver.cpp:115-133), each corner difference formed exactly as the
-// reference's dVels array would hold it.
-__device__ __forceinline__ float interp3_diff(const float* __restrict__ a, const float* __restrict__ o, int sx, int sy, int sz,
-                                              float x, float y, float z) {
-    int   i, j, k;
-    float fi, fj, fk;
-    bary(x, sx, i, fi);
-    bary(y, sy, j, fj);
-    bary(z, sz, k, fk);
-    const size_t b   = lin3(i, j, k, sx, sy);
-    const size_t sxy = (size_t)sx * sy;
-    float v000 = a[b] - o[b], v100 = a[b + 1] - o[b + 1], v010 = a[b + sx] - o[b + sx], v110 = a[b + sx + 1] - o[b + sx + 1];
-    float v001 = a[b + sxy] - o[b + sxy], v101 = a[b + sxy + 1] - o[b + sxy + 1];
-    float v011 = a[b + sxy + sx] - o[b + sxy + sx], v111 = a[b + sxy + sx + 1] - o[b + sxy + sx + 1];
-    return lerpf(bilerpf(v000, v100, v010, v110, fi, fj), bilerpf(v001, v101, v011, v111, fi, fj), fk);
+// its eight corner values, x fastest. The particle gathers are bound by the rate of vector memory
+// instructions (about 22 cycles each per CU, whatever they hit), so the two x neighbours come from one
+// 8-byte load (4-byte aligned, which global loads allow) and each corner is loaded once.
+struct Corners {
+    float v[8];
+};
+typedef float float2u __attribute__((ext_vector_type(2), aligned(4)));
+__device__ __forceinline__ Corners corners(const float* __restrict__ g, const Stencil& s) {
+    const float2u a = *reinterpret_cast<const float2u*>(g + s.at), b = *reinterpret_cast<const float2u*>(g + s.at + s.sx);
+    const float2u c = *reinterpret_cast<const float2u*>(g + s.at + s.sxy), d = *reinterpret_cast<const float2u*>(g + s.at + s.sxy + s.sx);
+    return Corners{{a.x, a.y, b.x, b.y, c.x, c.y, d.x, d.y}};
+}
+// a - o corner by corner, as the reference's dVels array of computeChangesGridVelocity holds it
+// (FLIP_Solver.cpp:115-121)
+__device__ __forceinline__ Corners corner_diff(const Corners& a, const Corners& o) {
+    Corners d;
+#pragma unroll
+    for(int e = 0; e < 8; ++e) d.v[e] = a.v[e] - o.v[e];
+    return d;
+}
+// ArrayHelpers.cpp:91-102: interpolateValueLinear
+__device__ __forceinline__ float interp8(const Corners& c, const Stencil& s) {
+    return lerpf(bilerpf(c.v[0], c.v[1], c.v[2], c.v[3], s.fi, s.fj), bilerpf(c.v[4], c.v[5], c.v[6], c.v[7], s.fi, s.fj), s.fk);
+}
+__device__ __forceinline__ float interp3(const float* __restrict__ g, int sx, int sy, int sz, float x, float y, float z) {
+    const Stencil s = stencil3(sx, sy, sz, x, y, z);
+    return interp8(corners(g, s), s);
 }
 
 // ArrayHelpers.cpp:275-302 (interpolateGradientValue): the gradient of the trilinear interpolant of
 // the eight corner values over the cell, the corner terms added in the reference's order, divided
 // by the cell size
-__device__ __forceinline__ void grad_value8(float v000, float v001, float v010, float v011, float v100, float v101, float v110, float v111,
-                                            float fi, float fj, float fk, float dx, float& gx, float& gy, float& gz) {
+__device__ __forceinline__ void grad8(const Corners& c8, const Stencil& s, float dx, float* g) {
 #pragma clang fp contract(off)
+    const float v000 = c8.v[0], v100 = c8.v[1], v010 = c8.v[2], v110 = c8.v[3], v001 = c8.v[4], v101 = c8.v[5], v011 = c8.v[6], v111 = c8.v[7];
+    const float fi = s.fi, fj = s.fj, fk = s.fk;
     const float a = 1.0f - fi, b = 1.0f - fj, c = 1.0f - fk;
-    gx = v000 * (-b * c) + v001 * (-b * fk) + v010 * (-fj * c) + v011 * (-fj * fk) + v100 * (b * c) + v101 * (b * fk) + v110 * (fj * c) +
-         v111 * (fj * fk);
-    gy = v000 * (-a * c) + v001 * (-a * fk) + v010 * (a * c) + v011 * (a * fk) + v100 * (-fi * c) + v101 * (-fi * fk) + v110 * (fi * c) +
-         v111 * (fi * fk);
-    gz = v000 * (-a * b) + v001 * (a * b) + v010 * (-a * fj) + v011 * (a * fj) + v100 * (-fi * b) + v101 * (fi * b) + v110 * (-fi * fj) +
-         v111 * (fi * fj);
-    gx /= dx;
-    gy /= dx;
-    gz /= dx;
-}
-
-// interpolateGradientValue of grid g (dims sx, sy, sz) at grid coordinate (x, y, z); with o, of the
-// difference g - o formed per corner (the dVels array of computeChangesGridVelocity)
-__device__ __forceinline__ void interp3_grad(const float* __restrict__ g, const float* __restrict__ o, int sx, int sy, int sz, float x,
-                                             float y, float z, float dx, float& gx, float& gy, float& gz) {
-    int   i, j, k;
-    float fi, fj, fk;
-    bary(x, sx, i, fi);
-    bary(y, sy, j, fj);
-    bary(z, sz, k, fk);
-    const size_t b = lin3(i, j, k, sx, sy), sxy = (size_t)sx * sy;
-    const size_t i000 = b, i001 = b + sxy, i010 = b + sx, i011 = b + sxy + sx, i100 = b + 1, i101 = b + sxy + 1, i110 = b + sx + 1,
-                 i111 = b + sxy + sx + 1;
-    if(o) {
-        grad_value8(g[i000] - o[i000], g[i001] - o[i001], g[i010] - o[i010], g[i011] - o[i011], g[i100] - o[i100], g[i101] - o[i101],
-                    g[i110] - o[i110], g[i111] - o[i111], fi, fj, fk, dx, gx, gy, gz);
-    } else {
-        grad_value8(g[i000], g[i001], g[i010], g[i011], g[i100], g[i101], g[i110], g[i111], fi, fj, fk, dx, gx, gy, gz);
-    }
+    g[0] = v000 * (-b * c) + v001 * (-b * fk) + v010 * (-fj * c) + v011 * (-fj * fk) + v100 * (b * c) + v101 * (b * fk) + v110 * (fj * c) +
+           v111 * (fj * fk);
+    g[1] = v000 * (-a * c) + v001 * (-a * fk) + v010 * (a * c) + v011 * (a * fk) + v100 * (-fi * c) + v101 * (-fi * fk) + v110 * (fi * c) +
+           v111 * (fi * fk);
+    g[2] = v000 * (-a * b) + v001 * (a * b) + v010 * (-a * fj) + v011 * (a * fj) + v100 * (-fi * b) + v101 * (fi * b) + v110 * (-fi * fj) +
+           v111 * (fi * fj);
+    g[0] /= dx;
+    g[1] /= dx;
+    g[2] /= dx;
 }
 
 // MathHelpers.h:804-821
