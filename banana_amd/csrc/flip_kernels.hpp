@@ -2276,7 +2276,7 @@ __device__ __forceinline__ uint32_t xcd_slot(uint32_t b, uint32_t n) {
 
 // The coarse bricks a fine brick's cells and halo can have as parents: its own parent (index 6) and
 // that parent's six neighbours (-x, +x, -y, +y, -z, +z), or -1. Stored per fine slot (8 ints, the
-// last unused) when the hierarchy is built.
+// last the parities of the brick's coordinates) when the hierarchy is built.
 struct k_mg_parent_table {
     static constexpr int kThreads = kBlock;
     LevelDev F;
@@ -2290,7 +2290,7 @@ struct k_mg_parent_table {
         const int32_t cs = C.brickSlot[((bz >> 1) * C.nby + (by >> 1)) * C.nbx + (bx >> 1)];
         for(int d = 0; d < 6; ++d) tab[8 * s + d] = cs >= 0 ? C.nbr[6 * cs + d] : -1;
         tab[8 * s + 6] = cs;
-        tab[8 * s + 7] = -1;
+        tab[8 * s + 7] = (bx & 1) | (by & 1) << 1 | (bz & 1) << 2;
     }
 };
 
@@ -2379,32 +2379,6 @@ __device__ __forceinline__ void smooth_halo(const LevelDev& L, const LevelDev& C
             }
         }
         xs[c] = v;
-    }
-}
-
-// four cells of one colour: their neighbours all have the other colour, so every neighbour value is
-// read before any of the four is written (the reads need not wait for the writes)
-__device__ __forceinline__ void smooth_cells_update4(const SmoothCell* R, float* xs) {
-    float v[4][6];
-#pragma unroll
-    for(int q = 0; q < 4; ++q) {
-        v[q][0] = xs[R[q].c - 100];
-        v[q][1] = xs[R[q].c - 10];
-        v[q][2] = xs[R[q].c - 1];
-        v[q][3] = xs[R[q].c + 1];
-        v[q][4] = xs[R[q].c + 10];
-        v[q][5] = xs[R[q].c + 100];
-    }
-#pragma unroll
-    for(int q = 0; q < 4; ++q) {
-        float acc = 0.f;
-        acc += R[q].czm * v[q][0];
-        acc += R[q].cym * v[q][1];
-        acc += R[q].cxm * v[q][2];
-        acc += R[q].cxp * v[q][3];
-        acc += R[q].cyp * v[q][4];
-        acc += R[q].czp * v[q][5];
-        xs[R[q].c] = (R[q].bv - acc) * R[q].inv;
     }
 }
 
@@ -2763,63 +2737,260 @@ struct k_pcg_dot_zr {
 
 namespace bnn {
 
-// coarsest level when it is a single brick (no neighbour bricks): x = 0, then `sweeps` red-black
-// sweeps and `sweeps` black-red sweeps with x held in LDS. One wavefront: each lane owns four red and
-// four black cells (x-adjacent pairs on z = z0, z0+2, z0+4, z0+6), so a half-sweep ends with a
-// single-wave barrier. The LDS array has a zero halo, so couplings to cells outside the brick (zero)
-// are added unconditionally and change nothing.
-struct k_mg_coarsest1 {
-    static constexpr int kThreads = 64;
-    LevelDev L;
-    int sweeps;
+// The V-cycle's smallest levels in one launch. On levels of a few bricks every kernel of the cycle costs
+// its own dependent loads and its launch (5-7 us each, three a level, 11 for a coarsest solve by one
+// wavefront), whatever its work. Here one workgroup takes the levels lv[0] (at most 8 bricks) to the
+// coarsest (one brick): all their x tiles (a brick and its one-cell halo) stay in LDS, a right-hand side
+// goes to the next level through that level's tile, and the coefficients of the first two levels are
+// loaded once, at the start. Four groups of 256 threads own a brick each (on lv[0] up to two in turn;
+// thread = an x-adjacent pair of cells, one of each colour). Same arithmetic, in the same order, as
+// k_mg_smooth_brick, k_mg_residual_restrict and (coarsest: x = 0, `coarsest` red-black and as many
+// black-red sweeps) their per-level launches, so the results are the same bits. Input lv[0].b, output
+// lv[0].x. Bound by the chain of half-sweeps (about 0.17 us each, 32 of them on the coarsest level):
+// 17 us for two levels, 28 for three, against 27 and 42 in separate kernels plus 4 or 7 launches; a
+// whole substep at 24^3 1116 -> 1048 us, at 64^3 2867 -> 2606.
+struct k_mg_tail {
+    static constexpr int kThreads = 1024;
+    static constexpr int kLevels = 5, kTop = 8, kRest = 4, kTiles = 16;  // levels; bricks on lv[0], on each other level, in all
+    LevelDev lv[kLevels];
+    int      nLev;
+    float    omega;
+    int      sweeps, coarsest;
     const PcgState* __restrict__ st;
-    __device__ void operator()(Blk blk) const {
-        __shared__ float xs[10 * 10 * 10];
-        if(st && st->done) return;
-        const int t = threadIdx.x, px = 2 * (t & 3), ly = (t >> 2) & 7, lz0 = t >> 5;
-        const int shift = (ly + lz0) & 1;  // colour of the even-x cell of every pair of this lane
-        for(int c = t; c < 1000; c += 64) xs[c] = 0.f;
-        SmoothCell R[4], K[4];  // red (colour 0) and black cells
-    #pragma unroll
-        for(int q = 0; q < 4; ++q) {
-            const int lz = lz0 + 2 * q;
-    #pragma unroll
-            for(int e = 0; e < 2; ++e) {
-                const int  lx = px + e, l = (lz * 8 + ly) * 8 + lx;
-                SmoothCell C;
-                C.c   = ((lz + 1) * 10 + (ly + 1)) * 10 + (lx + 1);
-                C.czm = lz > 0 ? L.cz[l - 64] : 0.f;
-                C.cym = ly > 0 ? L.cy[l - 8] : 0.f;
-                C.cxm = lx > 0 ? L.cx[l - 1] : 0.f;
-                C.cxp = lx < 7 ? L.cx[l] : 0.f;
-                C.cyp = ly < 7 ? L.cy[l] : 0.f;
-                C.czp = lz < 7 ? L.cz[l] : 0.f;
-                C.bv  = L.b[l];
-                C.inv = L.invdiag[l];
-                if((e ^ shift) == 0) R[q] = C;
-                else K[q] = C;
-            }
+
+    struct Row {  // a cell's row of A (couplings to missing neighbours 0), right-hand side and 1/diagonal
+        float czm, cym, cxm, cxp, cyp, czp, bv, inv, diag;
+    };
+    static __device__ __forceinline__ int tile_at(int l) { return (((l >> 6) + 1) * 10 + ((l >> 3) & 7) + 1) * 10 + (l & 7) + 1; }
+    // nb: the brick's six neighbour slots
+    static __device__ __forceinline__ Row row(const LevelDev& L, const int32_t* nb, int s, int l) {
+        const int     lx = l & 7, ly = (l >> 3) & 7, lz = l >> 6;
+        const int32_t o = s * 512 + l;
+        const int32_t nx = nb[0], ny = nb[2], nz = nb[4];
+        const bool    hx = lx > 0 || nx >= 0, hy = ly > 0 || ny >= 0, hz = lz > 0 || nz >= 0;
+        const int32_t ix = lx > 0 ? o - 1 : (hx ? nx * 512 + l + 7 : o), iy = ly > 0 ? o - 8 : (hy ? ny * 512 + l + 56 : o),
+                      iz = lz > 0 ? o - 64 : (hz ? nz * 512 + l + 448 : o);
+        const float czm = L.cz[iz], cym = L.cy[iy], cxm = L.cx[ix], cxp = L.cx[o], cyp = L.cy[o], czp = L.cz[o];
+        Row         R;
+        R.inv  = L.invdiag[o];
+        R.diag = L.diag[o];
+        R.czm  = hz ? czm : 0.f;
+        R.cym  = hy ? cym : 0.f;
+        R.cxm  = hx ? cxm : 0.f;
+        R.cxp  = lx < 7 || nb[1] >= 0 ? cxp : 0.f;
+        R.cyp  = ly < 7 || nb[3] >= 0 ? cyp : 0.f;
+        R.czp  = lz < 7 || nb[5] >= 0 ? czp : 0.f;
+        R.bv   = 0.f;
+        return R;
+    }
+    static __device__ __forceinline__ float off_sum(const Row& R, const float* x) {
+        float acc = 0.f;
+        acc += R.czm * x[-100];
+        acc += R.cym * x[-10];
+        acc += R.cxm * x[-1];
+        acc += R.cxp * x[1];
+        acc += R.cyp * x[10];
+        acc += R.czp * x[100];
+        return acc;
+    }
+    // one half-sweep over the group's n bricks (4 tiles apart): cells of one colour read only the other
+    template<int kTurns> static __device__ __forceinline__ void half(const Row* R, float* x, int n) {
+        float v[kTurns];
+#pragma unroll
+        for(int q = 0; q < kTurns; ++q)
+            if(q < n) v[q] = (R[q].bv - off_sum(R[q], x + 4000 * q)) * R[q].inv;
+#pragma unroll
+        for(int q = 0; q < kTurns; ++q)
+            if(q < n) x[4000 * q] = v[q];
+    }
+    // the tiles' halos from the neighbouring bricks (0 where there is none)
+    static __device__ __forceinline__ void halos(float* xs, const int32_t (*nb)[8], int nSlots) {
+        for(int h = threadIdx.x; h < 384 * nSlots; h += kThreads) {
+            const int s = h / 384, d = (h - 384 * s) >> 6, p = h & 63, a = p & 7, e = p >> 3;
+            // the halo entry, and the cell it mirrors in the neighbour's tile
+            const int     to = d < 2 ? ((e + 1) * 10 + a + 1) * 10 + (d == 0 ? 0 : 9)
+                                     : (d < 4 ? ((e + 1) * 10 + (d == 2 ? 0 : 9)) * 10 + a + 1 : ((d == 4 ? 0 : 9) * 10 + e + 1) * 10 + a + 1);
+            const int     step = (d < 2 ? 1 : (d < 4 ? 10 : 100)) * ((d & 1) ? -8 : 8);
+            const int32_t n    = nb[s][d];
+            xs[1000 * s + to]  = n >= 0 ? xs[1000 * n + to + step] : 0.f;
         }
+    }
+    // the thread's pair of cells: local indices of the red (colour 0) and the black one, their tile entries
+    struct Pair {
+        int  ly, lz, px, lr, lb, cr, cb;
+        // the parent of the pair's 2x2x2 group in the parent brick, for a brick with coordinate parities odd
+        __device__ __forceinline__ int parent(int odd) const {
+            return (((odd >> 2 & 1) * 4 + lz / 2) * 8 + (odd >> 1 & 1) * 4 + ly / 2) * 8 + (odd & 1) * 4 + px;
+        }
+    };
+    // pre-smoother from x = 0 on the level's tiles, then the residual's 2x2x2 sums to the next level's tiles
+    // (its right-hand side) and to its b (for the way up)
+    template<int kTurns>
+    __device__ __forceinline__ void down(const Row* R, const Row* K, const Pair& c, float* xs, const int32_t (*nb)[8], int S, int grp, const LevelDev& C) const {
+        const int n = (S - grp + 3) >> 2;  // bricks grp, grp + 4, ..
+        float*    x = xs + 1000 * grp;
         __syncthreads();
-        for(int it = 0; it < 2 * sweeps; ++it) {
-            if(it < sweeps) {  // red-black (uniform branch)
-                smooth_cells_update4(R, xs);
-                __syncthreads();
-                smooth_cells_update4(K, xs);
-            } else {  // black-red
-                smooth_cells_update4(K, xs);
-                __syncthreads();
-                smooth_cells_update4(R, xs);
-            }
+        for(int it = 0; it < sweeps; ++it) {
+            half<kTurns>(R, x + c.cr, n);
+            __syncthreads();
+            half<kTurns>(K, x + c.cb, n);
             __syncthreads();
         }
-    #pragma unroll
-        for(int q = 0; q < 4; ++q) {
-            const int lz = lz0 + 2 * q;
-    #pragma unroll
-            for(int e = 0; e < 2; ++e) {
-                const int lx = px + e;
-                L.x[(lz * 8 + ly) * 8 + lx] = xs[((lz + 1) * 10 + (ly + 1)) * 10 + (lx + 1)];
+        halos(xs, nb, S);
+        __syncthreads();
+#pragma unroll
+        for(int q = 0; q < kTurns; ++q)
+            if(q < n) {
+                const float* y  = x + 4000 * q;
+                const float  rr = R[q].bv - (R[q].diag * y[c.cr] + off_sum(R[q], y + c.cr));
+                const float  rk = K[q].bv - (K[q].diag * y[c.cb] + off_sum(K[q], y + c.cb));
+                // the x pair is this thread's, the odd y lies in lane ^ 4, the odd z in lane ^ 32
+                const float e0 = c.lr < c.lb ? rr : rk, e1 = c.lr < c.lb ? rk : rr;
+                const float y0 = __shfl_xor(e0, 4), y1 = __shfl_xor(e1, 4);
+                const float z0 = __shfl_xor(e0, 32), z1 = __shfl_xor(e1, 32), w0 = __shfl_xor(y0, 32), w1 = __shfl_xor(y1, 32);
+                const int   par = nb[grp + 4 * q][6];
+                if(!(c.ly & 1) && !(c.lz & 1) && par >= 0) {
+                    const float sum = ((((((e0 + e1) + y0) + y1) + z0) + z1) + w0) + w1;
+                    const int   cl  = c.parent(nb[grp + 4 * q][7]);
+                    xs[1000 * (S + par) + tile_at(cl)] = sum;
+                    C.b[par * 512 + cl]                = sum;
+                }
+            }
+        __syncthreads();
+    }
+    // coarse-grid correction, then the post-smoother
+    template<int kTurns>
+    __device__ __forceinline__ void up(const Row* R, const Row* K, const Pair& c, float* xs, const int32_t (*nb)[8], int S, int grp) const {
+        const int n = (S - grp + 3) >> 2;
+        float*    x = xs + 1000 * grp;
+#pragma unroll
+        for(int q = 0; q < kTurns; ++q)
+            if(q < n) {
+                const int par = nb[grp + 4 * q][6];
+                if(par >= 0) {
+                    const float xc = xs[1000 * (S + par) + tile_at(c.parent(nb[grp + 4 * q][7]))];
+                    float*      y  = x + 4000 * q;
+                    if(R[q].inv != 0.f) y[c.cr] = y[c.cr] + omega * xc;
+                    if(K[q].inv != 0.f) y[c.cb] = y[c.cb] + omega * xc;
+                }
+            }
+        __syncthreads();
+        halos(xs, nb, S);
+        __syncthreads();
+        for(int it = 0; it < sweeps; ++it) {
+            half<kTurns>(K, x + c.cb, n);
+            __syncthreads();
+            half<kTurns>(R, x + c.cr, n);
+            __syncthreads();
+        }
+    }
+    __device__ void operator()(Blk) const {
+        __shared__ float   xs[kTiles * 1000];
+        __shared__ int32_t nb[kTiles][8];  // per brick: six neighbour slots, parent slot, parities of its coordinates
+        if(st && st->done) return;
+        const int t = threadIdx.x, grp = t >> 8, tt = t & 255;
+        Pair      c;
+        c.ly = (tt >> 2) & 7;
+        c.lz = tt >> 5;
+        c.px = tt & 3;
+        const int l0 = (c.lz * 8 + c.ly) * 8 + 2 * c.px, o0 = (c.ly + c.lz) & 1;  // even x; its colour
+        c.lr = l0 + o0;
+        c.lb = l0 + 1 - o0;
+        c.cr = tile_at(c.lr);
+        c.cb = tile_at(c.lb);
+        int base = 0;
+        for(int l = 0; l < nLev; ++l) {
+            const int S = (int)lv[l].nSlots;
+            if(t < 8 * S) {
+                const int s = t >> 3, d = t & 7;
+                nb[base + s][d] = d < 6 ? lv[l].nbr[6 * s + d] : (l + 1 < nLev ? lv[l].ptab[8 * s + d] : -1);
+            }
+            base += S;
+        }
+        for(int e = t; e < base * 1000; e += kThreads) xs[e] = 0.f;
+        __syncthreads();
+        const int S0 = nLev > 1 ? (int)lv[0].nSlots : 0;
+        Row       R0[2], K0[2], R1[1], K1[1];
+#pragma unroll
+        for(int q = 0; q < 2; ++q) {
+            const int s = grp + 4 * q;
+            if(s < S0) {
+                R0[q]    = row(lv[0], nb[s], s, c.lr);
+                K0[q]    = row(lv[0], nb[s], s, c.lb);
+                R0[q].bv = lv[0].b[s * 512 + c.lr];
+                K0[q].bv = lv[0].b[s * 512 + c.lb];
+            }
+        }
+        auto rows = [&](int l, int at) {
+            if(grp < (int)lv[l].nSlots) {
+                R1[0] = row(lv[l], nb[at + grp], grp, c.lr);
+                K1[0] = row(lv[l], nb[at + grp], grp, c.lb);
+            }
+        };
+        auto take = [&](int l, int at) {  // the right-hand side that the finer level left in the tile; x starts from 0
+            if(grp < (int)lv[l].nSlots) {
+                float* x = xs + 1000 * (at + grp);
+                R1[0].bv = x[c.cr];
+                K1[0].bv = x[c.cb];
+                x[c.cr] = x[c.cb] = 0.f;
+            }
+        };
+        rows(nLev > 1 ? 1 : 0, S0);
+        if(nLev > 1) down<2>(R0, K0, c, xs, nb, S0, grp, lv[1]);
+        base = S0;
+        for(int l = 1; l + 1 < nLev; ++l) {
+            const int S = (int)lv[l].nSlots;
+            if(l > 1) rows(l, base);
+            take(l, base);
+            down<1>(R1, K1, c, xs + 1000 * base, nb + base, S, grp, lv[l + 1]);
+            base += S;
+        }
+        {  // coarsest level, one brick
+            const int n = grp == 0 ? 1 : 0;
+            float*    x = xs + 1000 * base;
+            if(nLev > 2) rows(nLev - 1, base);
+            if(nLev > 1) take(nLev - 1, base);
+            else if(n) {
+                R1[0].bv = lv[0].b[c.lr];
+                K1[0].bv = lv[0].b[c.lb];
+            }
+            __syncthreads();
+            for(int it = 0; it < coarsest; ++it) {
+                half<1>(R1, x + c.cr, n);
+                __syncthreads();
+                half<1>(K1, x + c.cb, n);
+                __syncthreads();
+            }
+            for(int it = 0; it < coarsest; ++it) {
+                half<1>(K1, x + c.cb, n);
+                __syncthreads();
+                half<1>(R1, x + c.cr, n);
+                __syncthreads();
+            }
+            if(n && nLev == 1) {
+                lv[0].x[c.lr] = x[c.cr];
+                lv[0].x[c.lb] = x[c.cb];
+            }
+        }
+        for(int l = nLev - 2; l >= 1; --l) {
+            const int S = (int)lv[l].nSlots;
+            base -= S;
+            rows(l, base);
+            if(grp < S) {
+                R1[0].bv = lv[l].b[grp * 512 + c.lr];
+                K1[0].bv = lv[l].b[grp * 512 + c.lb];
+            }
+            up<1>(R1, K1, c, xs + 1000 * base, nb + base, S, grp);
+        }
+        if(nLev > 1) {
+            up<2>(R0, K0, c, xs, nb, S0, grp);
+#pragma unroll
+            for(int q = 0; q < 2; ++q) {
+                const int s = grp + 4 * q;
+                if(s < S0) {
+                    lv[0].x[s * 512 + c.lr] = xs[1000 * s + c.cr];
+                    lv[0].x[s * 512 + c.lb] = xs[1000 * s + c.cb];
+                }
             }
         }
     }

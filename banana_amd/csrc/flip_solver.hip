@@ -955,7 +955,9 @@ public:
     bool vcycle(const PcgState* stp, bool finePreDone = false) {
         const int   nu    = prm.mg_sweeps;
         const float omega = prm.mg_omega;
-        for(int l = 0; l + 1 < mgLevels; ++l) {
+        const int   tail  = mgTail();
+        const int   down  = std::min(tail, mgLevels - 1);  // levels with their own launches
+        for(int l = 0; l < down; ++l) {
             const LevelDev L = levelDev(l), C = levelDev(l + 1);
             const unsigned G = std::max<uint32_t>(L.nSlots, 1u);
             if(!(l == 0 && finePreDone)) {
@@ -967,15 +969,20 @@ public:
             launch(k_mg_residual_restrict{L, C, stp}, G);
             ktEnd(l == 0 ? BNN_KT_MG_RESTRICT : BNN_KT_MG_COARSE);
         }
-        const LevelDev Lc = levelDev(mgLevels - 1);
         ktBegin(BNN_KT_MG_COARSE);
-        if(Lc.nSlots == 1) {
-            launch(k_mg_coarsest1{Lc, prm.mg_coarsest_sweeps, stp}, 1);
+        if(tail < mgLevels) {
+            k_mg_tail k{};
+            for(int l = tail; l < mgLevels; ++l) k.lv[k.nLev++] = levelDev(l);
+            k.omega    = omega;
+            k.sweeps   = nu;
+            k.coarsest = prm.mg_coarsest_sweeps;
+            k.st       = stp;
+            launch(k, 1);
         } else {
-            launch(k_mg_coarsest{Lc, prm.mg_coarsest_sweeps, stp}, 1);
+            launch(k_mg_coarsest{levelDev(mgLevels - 1), prm.mg_coarsest_sweeps, stp}, 1);
         }
         ktEnd(BNN_KT_MG_COARSE);
-        for(int l = mgLevels - 2; l >= 0; --l) {
+        for(int l = down - 1; l >= 0; --l) {
             const LevelDev L = levelDev(l), C = levelDev(l + 1);
             const uint32_t G = std::max<uint32_t>(L.nSlots, 1u);
             if(l == 0) {  // finest level: correction as its own streaming pass, then smooth and form z.r
@@ -992,6 +999,18 @@ public:
             }
         }
         return mgLevels > 1;
+    }
+    // the first level whose bricks and all coarser levels' fit k_mg_tail (below the finest, whose smoothers
+    // are fused with the PCG's own passes, unless it is the only level); mgLevels when the coarsest level
+    // holds more than one brick
+    int mgTail() {
+        if(levelDev(mgLevels - 1).nSlots != 1) return mgLevels;
+        int      l     = mgLevels - 1;
+        uint32_t tiles = 1;
+        while(l > 1 && mgLevels - l < k_mg_tail::kLevels && mg[l - 1]->nSlots <= (uint32_t)k_mg_tail::kTop &&
+              mg[l]->nSlots <= (uint32_t)k_mg_tail::kRest && tiles + mg[l - 1]->nSlots <= (uint32_t)k_mg_tail::kTiles)
+            tiles += mg[--l]->nSlots;
+        return l;
     }
 
     // IC(0) of the reference, one launch per hyperplane i + j + k = h (h = 0 .. nx + ny + nz - 3)
