@@ -1634,6 +1634,41 @@ __device__ __forceinline__ double fold(const double* __restrict__ p, int n, bool
     return isMax ? block_max<1024>(a, sh) : block_sum<1024>(a, sh);
 }
 
+// The same fold by every workgroup of a consumer kernel (NT threads), for n <= kFoldMax partials: valid
+// in all threads and, with fold()'s order (64 consecutive partials per wavefront sum, then the sums in
+// order), the same bits. On small systems it replaces a one-block launch (2.5-3.5 us of an iteration of
+// about 90 at 64^3); reading the partials in every workgroup costs more than that launch on large ones.
+constexpr int kFoldMax = 512;
+template<int NT> __device__ __forceinline__ double fold_all(const double* __restrict__ p, int n, bool isMax, double* sh) {
+#pragma unroll
+    for(int k = 0; k < kFoldMax / NT; ++k) {
+        const int    i = k * NT + (int)threadIdx.x;
+        double       v = i < n ? p[i] : 0.0;
+        v = isMax ? wave_maxd(v) : wave_sum(v);
+        if((threadIdx.x & 63) == 0) sh[k * (NT / 64) + (threadIdx.x >> 6)] = v;
+    }
+    __syncthreads();
+    double t = 0;
+    for(int w = 0; w < kFoldMax / 64; ++w) t = isMax ? fmax(t, sh[w]) : t + sh[w];
+    __syncthreads();
+    return t;
+}
+
+// the end of an iteration (PCGSolver.cpp:182-194): A = z.r, B = max|r|; stop test, beta, next rho
+__device__ __forceinline__ void pcg_end_iteration(PcgState& st, double A, double B) {
+    st.iter += 1;
+    st.res = (float)B;
+    if((float)B < st.tol) {
+        st.done    = 1;
+        st.success = 1;
+    } else if(st.iter >= st.maxIter) {
+        st.done = 1;
+    } else {
+        st.beta = A / st.rho;
+        st.rho  = A;
+    }
+}
+
 // init: x = 0, r = b, s = 0, z = M^-1 r; partials of z.r and max|b|
 struct k_pcg_init {
     static constexpr int kThreads = 512;
@@ -1718,6 +1753,9 @@ __device__ __forceinline__ void block_chunk(Blk blk, uint32_t n, uint32_t& s0, u
     s1               = (uint32_t)(((uint64_t)n * (v + 1)) / G);
 }
 
+// kFold (small systems): the last iteration's end (k_pcg_beta) runs here, from st to the other state
+// `next` (null: it has run), over nPart <= kFoldMax partials rz of z.r and rm of max|r|
+template<bool kFold>
 struct k_pcg_spmv {
     static constexpr int kThreads = 512;
     const int32_t* __restrict__ nbr;
@@ -1730,12 +1768,28 @@ struct k_pcg_spmv {
     const float* __restrict__ cy;
     const float* __restrict__ cz;
     uint32_t nSlots;
-    const PcgState* __restrict__ st;
+    const PcgState* st;
     double* __restrict__ pa;
+    PcgState* next;
+    const double* __restrict__ rz;
+    const double* __restrict__ rm;
+    int nPart;
     __device__ void operator()(Blk blk) const {
         __shared__ double sh[8];
-        if(st && st->done) return;
-        const float beta = (float)st->beta;
+        float             beta;
+        if(kFold && next) {
+            PcgState cur = *st;
+            if(!cur.done) {
+                const double A = fold_all<512>(rz, nPart, false, sh), B = fold_all<512>(rm, nPart, true, sh);
+                pcg_end_iteration(cur, A, B);
+            }
+            if(blk.id == 0 && threadIdx.x == 0) *next = cur;
+            if(cur.done) return;
+            beta = (float)cur.beta;
+        } else {
+            if(st->done) return;
+            beta = (float)st->beta;
+        }
         const int   l    = threadIdx.x;
         double      d    = 0;
         uint32_t    s0, s1;
@@ -1850,17 +1904,9 @@ struct k_pcg_beta {
         const double A = fold(pa, na, false, sh);
         const double B = fold(pb, nb, true, sh);
         if(threadIdx.x != 0) return;
-        st->iter += 1;
-        st->res = (float)B;
-        if((float)B < st->tol) {
-            st->done    = 1;
-            st->success = 1;
-        } else if(st->iter >= st->maxIter) {
-            st->done = 1;
-        } else {
-            st->beta = A / st->rho;
-            st->rho  = A;
-        }
+        PcgState n = *st;
+        pcg_end_iteration(n, A, B);
+        *st = n;
     }
 };
 
@@ -2483,6 +2529,8 @@ struct k_mg_smooth_brick {
 // pre-smoother on b = r, which reads only the brick's own cells (it starts from x = 0). The finest
 // level's r array is the PCG's q buffer: this brick's q is read before the smoother overwrites it.
 // Per cell the same arithmetic as k_pcg_update followed by k_mg_smooth_brick<0, 0>.
+// kFold (small systems): alpha (k_pcg_alpha) is formed here from nPart <= kFoldMax partials of s.q.
+template<bool kFold>
 struct k_pcg_update_pre {
     static constexpr int kThreads = 256;
     const float* __restrict__ s;
@@ -2490,14 +2538,36 @@ struct k_pcg_update_pre {
     LevelDev L;  // the finest level: L.b = r, L.r = q
     float omega;
     int sweeps;
-    const PcgState* __restrict__ st;
+    PcgState* st;
     double* __restrict__ pm;
+    const double* __restrict__ sq;
+    int nPart;
     __device__ void operator()(Blk blk) const {
         __shared__ float  xs[10 * 10 * 10];
-        __shared__ double sh[4];
-        if(st && st->done) return;
-        const float alpha = (float)st->alpha;
-        const int   t     = threadIdx.x;
+        __shared__ double sh[8];
+        if(st->done) return;
+        const int t     = threadIdx.x;
+        float     alpha = 0.f;
+        if(kFold) {
+            // the first workgroup records it in the state; the others read only rho, which stays, and a
+            // stop flag set meanwhile ends them just as their own sum does
+            const double A  = fold_all<256>(sq, nPart, false, sh);
+            const bool   ok = !(A < (double)kFltMin);
+            const double al = st->rho / A;
+            if(blk.id == 0 && t == 0) {
+                st->tmp = A;
+                if(ok) st->alpha = al;
+                else {
+                    st->done    = 1;
+                    st->success = 1;
+                    st->iter += 1;
+                }
+            }
+            if(!ok) return;
+            alpha = (float)al;
+        } else {
+            alpha = (float)st->alpha;
+        }
         for(uint32_t v = blk.id; v < L.nSlots; v += blk.n) {
             const int slot = (int)xcd_slot(v, L.nSlots);
             double    m    = 0;

@@ -422,7 +422,7 @@ public:
         occ.reserve((size_t)(nb + 3) / 4 * 4);
         bscan.reserve(nb * 4);
         brickSlot.reserve(nb * 4);
-        pst.reserve(sizeof(PcgState));
+        pst.reserve(2 * sizeof(PcgState));
         ost.reserve(sizeof(OuterState));
         // zero everything the reference zero-fills at resize (PIC_Data.cpp:101-117)
         for(auto* b : {&u, &v, &w, &ut, &vt, &wt, &uo, &vo, &wo, &wu, &wv, &ww, &vu, &vv, &vw, &eu, &ev_, &ew, &phi, &bsdf,
@@ -952,6 +952,10 @@ public:
     // Returns true when the fine level's post-smoother also wrote the per-brick partials of z.r to pz
     // (false when the fine level is the coarsest: the caller then forms z.r itself).
     // finePreDone: the finest level's pre-smoother already ran (fused with the PCG update).
+    // The finest level's correction: formed by the post-smoother itself up to kProlongInPost bricks alone
+    // (a launch less), else as a streaming pass of its own (at 9600 bricks 14 us against the dependent
+    // loads; in a batch the launch is shared).
+    static constexpr uint32_t kProlongInPost = 1024;
     bool vcycle(const PcgState* stp, bool finePreDone = false) {
         const int   nu    = prm.mg_sweeps;
         const float omega = prm.mg_omega;
@@ -985,7 +989,11 @@ public:
         for(int l = down - 1; l >= 0; --l) {
             const LevelDev L = levelDev(l), C = levelDev(l + 1);
             const uint32_t G = std::max<uint32_t>(L.nSlots, 1u);
-            if(l == 0) {  // finest level: correction as its own streaming pass, then smooth and form z.r
+            if(l == 0 && !rec && L.nSlots <= kProlongInPost) {
+                ktBegin(BNN_KT_MG_POST);
+                launch(k_mg_smooth_brick<1, 1>{L, C, omega, nu, stp, pz.as<double>()}, G);
+                ktEnd(BNN_KT_MG_POST);
+            } else if(l == 0) {  // correction as its own streaming pass, then smooth and form z.r
                 ktBegin(BNN_KT_MG_PROLONG);
                 launch(k_mg_prolong{L, C, omega, stp}, G);
                 ktEnd(BNN_KT_MG_PROLONG);
@@ -1051,6 +1059,7 @@ public:
     // FP32 PCG on b -> x (PCGSolver.cpp:143-199); returns success
     Co<bool> pcg32(const float* b, float relTol, uint32_t maxIter, uint32_t& iters, float& res, float& bmax) {
         PcgState*      dst = pst.as<PcgState>();
+        PcgState*      alt_ = dst + 1;  // the state an SpMV that ends the last iteration writes
         double*        dpa = pa.as<double>();
         double*        dpb = pb.as<double>();
         float *        sA = s0.as<float>(), *sB = s1.as<float>();
@@ -1077,6 +1086,10 @@ public:
         // multigrid over several levels: the update is fused with the finest pre-smoother, and its
         // max|r| partials are per brick
         const bool fuseUpdate = !jac && !ic0 && mgLevels > 1;
+        // small systems alone: the folds of alpha and beta run inside the kernels that use them. In a batch
+        // a launch is shared by all scenes, and mixing both forms splits it: 48 scenes took 13.65 ms a
+        // substep with the folds inside against 13.42
+        const bool folded = fuseUpdate && !rec && nSlots <= (uint32_t)kFoldMax;
         launch(k_pcg_init_fin{dst, rz, nrz, (const double*)dpb, (int)G, relTol, maxIter}, 1);
         // the first chunk is queued without a poll (the stop flag ends it early when the system is
         // already solved); each later poll sizes the next chunk from max|r| at iteration 0, which is
@@ -1093,19 +1106,31 @@ public:
             const uint32_t left = first ? maxIter : (hostSt->maxIter > hostSt->iter ? hostSt->maxIter - hostSt->iter : 1u);
             const uint32_t n    = std::min(chunk, left);
             for(uint32_t c = 0; c < n; ++c) {
+                const bool endLast = folded && c > 0;
                 ktBegin(BNN_KT_PCG_SPMV);
-                launch(k_pcg_spmv{(const int32_t*)nbrTab.as<int32_t>(), (const float*)z.as<float>(), (const float*)sA, sB, q.as<float>(), (const float*)diag32.as<float>(), (const float*)cx32.as<float>(), (const float*)cy32.as<float>(), (const float*)cz32.as<float>(), nSlots, (const PcgState*)dst, dpa}, G);
+                auto spmv = [&](auto k) {
+                    k = {nbrTab.as<int32_t>(), z.as<float>(), sA, sB, q.as<float>(), diag32.as<float>(), cx32.as<float>(), cy32.as<float>(),
+                         cz32.as<float>(), nSlots, dst, dpa, endLast ? alt_ : nullptr, rz, dpb, (int)nSlots};
+                    launch(k, G);
+                };
+                if(folded) spmv(k_pcg_spmv<true>{});
+                else spmv(k_pcg_spmv<false>{});
                 ktEnd(BNN_KT_PCG_SPMV);
-                launch(k_pcg_alpha{dst, (const double*)dpa, (int)G}, 1);
+                if(endLast) std::swap(dst, alt_);
+                if(!folded) launch(k_pcg_alpha{dst, (const double*)dpa, (int)G}, 1);
                 ktBegin(BNN_KT_PCG_UPDATE);
-                if(fuseUpdate)
-                    launch(k_pcg_update_pre{(const float*)sB, x.as<float>(), fineLevel(), prm.mg_omega, prm.mg_sweeps, (const PcgState*)dst, dpb},
-                           std::max<uint32_t>(nSlots, 1u));
+                auto updatePre = [&](auto k) {
+                    k = {sB, x.as<float>(), fineLevel(), prm.mg_omega, prm.mg_sweeps, dst, dpb, dpa, (int)G};
+                    launch(k, std::max<uint32_t>(nSlots, 1u));
+                };
+                if(folded) updatePre(k_pcg_update_pre<true>{});
+                else if(fuseUpdate) updatePre(k_pcg_update_pre<false>{});
                 else
                     launch(k_pcg_update{(const float*)sB, (const float*)q.as<float>(), (const float*)invd.as<float>(), x.as<float>(), r.as<float>(), z.as<float>(), nSlots, (const PcgState*)dst, dpa, dpb, jac}, G);
                 ktEnd(BNN_KT_PCG_UPDATE);
                 if(!jac) zr(dst, fuseUpdate);
-                launch(k_pcg_beta{dst, rz, nrz, (const double*)dpb, fuseUpdate ? (int)nSlots : (int)G}, 1);
+                if(!folded || c + 1 == n)
+                    launch(k_pcg_beta{dst, rz, nrz, (const double*)dpb, fuseUpdate ? (int)nSlots : (int)G}, 1);
                 std::swap(sA, sB);
             }
             launched += n;
