@@ -987,136 +987,185 @@ struct k_p2g {
 // invalid face that is not on the array's outer layer with the mean of its neighbours valid before
 // the layer (order +x, -x, +y, -y, +z, -z) and makes it valid and extrapolated.
 //
-// One workgroup per 8^3 brick of faces. A face changes only through faces within 4 face steps, so
-// the brick and a halo of 4 faces on every side (a 16^3 tile) are read into LDS once and the four
-// layers run there, in place with layer stamps: 0 invalid, 1 valid on entry, l + 2 filled in layer l;
-// layer l reads the stamps 1 .. l + 1, so a face filled in the same layer is never read by it and the
-// values equal the two-buffer Jacobi's bit for bit. A halo face at distance d from the brick can go
-// wrong (its own neighbours beyond the tile are missing) only from layer 4 - d on, too late to reach
-// the brick. Faces on the tile's outer shell are never computed.
+// One workgroup per 8^3 brick of faces, the three components' bricks in one launch. A face changes only
+// through faces within 4 face steps, so the brick and a halo of 4 faces on every side (a 16^3 tile) are
+// read into LDS once and the four layers run there; they equal the two-buffer Jacobi's bit for bit. A
+// halo face at distance d from the brick can go wrong (its own neighbours beyond the tile are missing)
+// only from layer 4 - d on, too late to reach the brick. Faces on the tile's outer shell are never
+// computed.
+//
+// Validity is held as one 16-bit mask per (x, y) column of the tile (bit z), in LDS for the neighbour
+// columns: the faces a layer fills in a column are the invalid ones next to a set bit, a handful of bit
+// operations for all 16. Those few faces go to a list that the whole workgroup then shares (they lie on
+// a surface: without the list 14 threads had 14 each). Each thread reads the flags of 4 x 1 x 4 faces
+// (four 4-byte loads; the columns' masks are put together in LDS) and writes back those of the same
+// faces. Bound by latency: a surface brick's dependent steps (15 us at 24^3, where all run at once) and
+// the flags' load of the idle ones. Both extrapolations of a substep, against one launch a component that
+// tested its neighbours face by face: 116 -> 31 us at 24^3, 124 -> 41 at 64^3, 891 -> 532 at 256^3, 48
+// scenes 1303 -> 654.
 //
 // Other workgroups read this brick's faces as their halo while it runs, so what they read as valid
 // on entry is never changed: a face filled here gets its value, ext = 1 and val = gen (2 or 3, the
 // host alternates it per call), which this launch's loaders read as invalid; the other generation,
 // left by the previous call, reads as valid and is rewritten as 1. Every other face of the brick gets
-// ext = 0. Any nonzero val therefore means valid.
+// ext = 0. Any nonzero val therefore means valid; val holds 0 .. 3.
 //==================================================================================================
+typedef uint32_t uint32u __attribute__((aligned(1)));  // 4 neighbouring flags, at any address
+
+struct ExtrapComp {
+    float*   a;
+    uint8_t *val, *ext;
+    int      sx, sy, sz;
+    uint32_t first;  // its first block, a multiple of 8; its bricks follow
+    uint32_t bricks() const { return (uint32_t)(((sx + 7) / 8) * ((sy + 7) / 8) * ((sz + 7) / 8)); }
+};
+
 struct k_extrap_tile {
-    static constexpr int kThreads = 256;  // one (x, y) column of the tile per thread, its 16 faces in z
-    static constexpr int kManyBlocks = 4;  // batched: at most 128 registers (a tighter bound spills)
-    float* __restrict__ a;
-    uint8_t* __restrict__ val;
-    uint8_t* __restrict__ ext;
-    int sx;
-    int sy;
-    int sz;
-    uint8_t gen;
+    static constexpr int kThreads = 256;
+    static constexpr int kList = 1024;  // a longer list (scattered faces) is not made; 20 KB of LDS, 8 workgroups a CU
+    static constexpr int kOneBlocks = 8, kManyBlocks = 7;  // 64 and 72 registers: 287 -> 266 us at 256^3, 48 scenes 372 -> 327
+    ExtrapComp comp[3];
+    uint8_t    gen;
     __device__ void operator()(Blk blk) const {
-        __shared__ float   as[4096];  // 16^3, x fastest
-        __shared__ uint8_t ss[4096];
+        __shared__ float    as[4096];       // 16^3, x fastest
+        __shared__ union {
+            uint32_t nib[4][16][4];     // [z / 4][y][x / 4]: a byte per x, a bit per z
+            uint16_t list[kList];       // a layer's faces
+        } u;
+        __shared__ uint16_t col[256];   // the columns' valid masks
+        __shared__ uint16_t fil[256];   // ... and the faces filled
+        __shared__ uint32_t count[4];   // faces on the list, per layer
+        const int         ci = blk.id >= comp[2].first ? 2 : (blk.id >= comp[1].first ? 1 : 0);
+        const ExtrapComp& C  = comp[ci];
+        const int   sx = C.sx, sy = C.sy, sz = C.sz, nbx = (sx + 7) / 8, nby = (sy + 7) / 8, nbz = (sz + 7) / 8;
+        const uint32_t id = blk.id - C.first, nbk = (uint32_t)(nbx * nby * nbz);
+        if(id >= nbk) return;
         int bx, by, bz;
-        tile_of_block(blk, (sx + 7) / 8, (sy + 7) / 8, (sz + 7) / 8, bx, by, bz);
-        const int    t = threadIdx.x, x = t & 15, y = t >> 4;  // faces (x, y, 0 .. 15)
-        const int    gi = bx * 8 - 4 + x, gj = by * 8 - 4 + y, gk0 = bz * 8 - 4;
-        const bool   inXY = gi >= 0 && gi < sx && gj >= 0 && gj < sy;
-        const bool   brickXY = x >= 4 && x < 12 && y >= 4 && y < 12;
-        const size_t sxy = (size_t)sx * (size_t)sy, col = (size_t)gj * (size_t)sx + (size_t)gi;
-        auto         off = [&](int z) { return (size_t)(gk0 + z) * sxy + col; };
-        uint8_t      v0[16];  // val on entry
-        // the thread's own column: mark (0 not valid, 1 valid on entry, layer + 2 filled by that layer)
-        // and value; its z neighbours are read from here, its x and y neighbours from the LDS copy
-        uint8_t      cs[16];
-        float        ca[16];
-        int          anyValid = 0, anyOpen = 0;
+        tile_of_block(Blk{id, nbk}, nbx, nby, nbz, bx, by, bz);
+        const int      t = threadIdx.x, gi0 = bx * 8 - 4, gj0 = by * 8 - 4, gk0 = bz * 8 - 4;
+        const uint32_t sxy = (uint32_t)sx * (uint32_t)sy, g4 = gen * 0x01010101u;
+        // flags: faces (4 q4 .. 4 q4 + 3, fy, 4 z4 .. 4 z4 + 3) of the tile
+        const int q4 = t & 3, fy = (t >> 2) & 15, z4 = t >> 6, fi = gi0 + 4 * q4, fj = gj0 + fy;
+        const bool rowIn = fj >= 0 && fj < sy, whole = fi >= 0 && fi + 4 <= sx;
+        auto       at = [&](int q) { return (uint32_t)(gk0 + 4 * z4 + q) * sxy + (uint32_t)fj * (uint32_t)sx + (uint32_t)fi; };
+        auto       zIn = [&](int q) { return rowIn && (uint32_t)(gk0 + 4 * z4 + q) < (uint32_t)sz; };
+        uint32_t   v0[4], ok[4], acc = 0;  // flags on entry; 1 per valid face, per byte
 #pragma unroll
-        for(int z = 0; z < 16; ++z) {
-            const int gk = gk0 + z;
-            v0[z]        = (inXY && gk >= 0 && gk < sz) ? val[off(z)] : (uint8_t)0;
+        for(int q = 0; q < 4; ++q) {
+            v0[q] = 0;
+            if(!zIn(q)) continue;
+            if(whole) v0[q] = *reinterpret_cast<const uint32u*>(C.val + at(q));
+            else
+                for(int e = 0; e < 4; ++e)
+                    if((uint32_t)(fi + e) < (uint32_t)sx) v0[q] |= (uint32_t)C.val[at(q) + e] << (8 * e);
         }
 #pragma unroll
-        for(int z = 0; z < 16; ++z) {
-            const uint8_t st = (v0[z] != 0 && v0[z] != gen) ? 1 : 0;
-            ss[(z << 8) | (y << 4) | x] = st;
-            cs[z]                       = st;
-            ca[z]                       = 0.f;
-            anyValid |= st;
-            if(!st && brickXY && z >= 4 && z < 12 && gk0 + z < sz && inXY) anyOpen = 1;
+        for(int q = 0; q < 4; ++q) {
+            const uint32_t x = v0[q] ^ g4;
+            ok[q]            = (v0[q] | v0[q] >> 1) & (x | x >> 1) & 0x01010101u;  // neither 0 nor gen
+            acc |= ok[q] << q;
         }
-        const bool work = __syncthreads_or(anyValid) != 0 && __syncthreads_or(anyOpen) != 0;
+        u.nib[z4][fy][q4] = acc;
+        if(t < 4) count[t] = 0;
+        bool work = __syncthreads_or(acc != 0) != 0;
+        // the thread's column of the tile
+        const int x = t & 15, y = t >> 4, gi = gi0 + x, gj = gj0 + y;
+        uint32_t  m = 0;  // valid faces
         if(work) {
+#pragma unroll
+            for(int k = 0; k < 4; ++k) m |= (u.nib[k][y][x >> 2] >> (8 * (x & 3)) & 15u) << (4 * k);
+            col[t] = (uint16_t)m;
+            const uint32_t inZ = (gk0 < 0 ? 0xFFF0u : 0xFFFFu) & (sz - gk0 < 16 ? (1u << (sz - gk0)) - 1u : 0xFFFFu);
+            const bool     open = x >= 4 && x < 12 && y >= 4 && y < 12 && gi < sx && gj < sy && (~m & inZ & 0x0FF0u) != 0;
+            work                = __syncthreads_or(open) != 0;
+        }
+        if(work) {
+            // faces that can be filled: not on the tile's outer shell, not on the array's outer layer
+            const int zl = max(1, 1 - gk0), zh = min(14, sz - 2 - gk0);
+            uint32_t  can = zl <= zh ? ((2u << zh) - 1u) & ~((1u << zl) - 1u) & ~m : 0u;
+            if(x < 1 || x > 14 || y < 1 || y > 14 || gi < 1 || gi > sx - 2 || gj < 1 || gj > sy - 2) can = 0;
             // the values of the faces valid on entry (the others are written before they are read)
+            const uint32_t c0 = (uint32_t)gj * (uint32_t)sx + (uint32_t)gi;
 #pragma unroll
             for(int z = 0; z < 16; ++z)
-                if(cs[z]) {
-                    ca[z]                       = a[off(z)];
-                    as[(z << 8) | (y << 4) | x] = ca[z];
-                }
-            __syncthreads();
-            // faces that can be filled: not on the tile's outer shell, not on the array's outer layer
-            uint32_t open = 0;
-#pragma unroll
-            for(int z = 1; z <= 14; ++z) {
-                const int gk = gk0 + z;
-                if(x >= 1 && x <= 14 && y >= 1 && y <= 14 && gi >= 1 && gi <= sx - 2 && gj >= 1 && gj <= sy - 2 && gk >= 1 && gk <= sz - 2 && !cs[z])
-                    open |= 1u << z;
-            }
-            // Layer l (0 .. 3) updates only the faces within 3 - l cells (per axis) of the brick: a face
+                if(m >> z & 1u) as[(z << 8) | t] = C.a[(uint32_t)(gk0 + z) * sxy + c0];
+            uint32_t filled = 0;
+            // Layer l (0 .. 3) fills only the faces within 3 - l cells (per axis) of the brick: a face
             // farther out reaches the brick through fewer than the layers left, so leaving it unfilled
             // changes no brick face, and every face a layer reads lies within the previous layer's region.
-#pragma unroll
             for(int layer = 0; layer < 4; ++layer) {
-                const uint8_t  lim = (uint8_t)(layer + 1);
-                const int      lo = layer + 1, hi = 14 - layer;
-                const uint32_t act = (x >= lo && x <= hi && y >= lo && y <= hi) ? open & (((2u << hi) - 1u) & ~((1u << lo) - 1u)) : 0u;
-                float          res[16];
-                uint32_t       fill = 0;
-                // all reads of the layer first (a face this layer fills is never read by it), then the writes
+                const int lo = layer + 1, hi = 14 - layer;
+                uint32_t  fill = 0;
+                if(x >= lo && x <= hi && y >= lo && y <= hi)
+                    fill = ((uint32_t)col[t + 1] | col[t - 1] | col[t + 16] | col[t - 16] | m >> 1 | m << 1) & can & ((2u << hi) - 1u) & ~((1u << lo) - 1u);
+                // list positions: the lanes before this one in the wavefront, one LDS atomic a wavefront
+                uint32_t n = __popc(fill), pre = n;
 #pragma unroll
-                for(int z = 1; z <= 14; ++z) {
-                    res[z] = 0.f;
-                    if(!(act & (1u << z))) continue;
-                    const int q   = (z << 8) | (y << 4) | x;
-                    float     sum = 0.f;  // starts at +0 and never becomes -0, so adding +0 for a neighbour not taken is exact
-                    uint32_t  count = 0;
-                    // neighbours in the order +x, -x, +y, -y, +z, -z
-                    const uint8_t m[6]  = {ss[q + 1], ss[q - 1], ss[q + 16], ss[q - 16], cs[z + 1], cs[z - 1]};
-                    const float   av[6] = {as[q + 1], as[q - 1], as[q + 16], as[q - 16], ca[z + 1], ca[z - 1]};
-#pragma unroll
-                    for(int e = 0; e < 6; ++e) {
-                        const bool ok = m[e] >= 1 && m[e] <= lim;
-                        sum += ok ? av[e] : 0.f;
-                        count += ok ? 1u : 0u;
-                    }
-                    if(count > 0) {
-                        res[z] = sum / (float)count;
-                        fill |= 1u << z;
-                    }
+                for(int o = 1; o < 64; o <<= 1) {
+                    const uint32_t up = __shfl_up(pre, o, 64);
+                    if((t & 63) >= o) pre += up;
                 }
+                uint32_t base = 0;
+                if((t & 63) == 63 && pre) base = atomicAdd(&count[layer], pre);
+                uint32_t pos = __shfl(base, 63, 64) + pre - n;
+                for(uint32_t f = fill; f && pos < (uint32_t)kList; f &= f - 1u) u.list[pos++] = (uint16_t)(__builtin_ctz(f) << 8 | t);
+                __syncthreads();
+                auto face = [&](int q) {
+                    const int      z = q >> 8, c = q & 255;
+                    // neighbours in the order +x, -x, +y, -y, +z, -z, those valid before the layer
+                    const uint32_t own = col[c];
+                    const uint32_t k[6] = {(uint32_t)col[c + 1] >> z & 1u, (uint32_t)col[c - 1] >> z & 1u, (uint32_t)col[c + 16] >> z & 1u,
+                                           (uint32_t)col[c - 16] >> z & 1u, own >> (z + 1) & 1u, own >> (z - 1) & 1u};
+                    const float    v[6] = {as[q + 1], as[q - 1], as[q + 16], as[q - 16], as[q + 256], as[q - 256]};
+                    float          sum = 0.f;  // starts at +0 and never becomes -0, so adding +0 for a neighbour not taken is exact
+                    uint32_t       num = 0;
 #pragma unroll
-                for(int z = 1; z <= 14; ++z) {
-                    if(!(fill & (1u << z))) continue;
-                    const int q = (z << 8) | (y << 4) | x;
-                    as[q]       = res[z];
-                    ss[q]       = (uint8_t)(layer + 2);
-                    ca[z]       = res[z];
-                    cs[z]       = (uint8_t)(layer + 2);
-                }
-                open &= ~fill;
-                if(layer < 3) __syncthreads();
+                    for(int d = 0; d < 6; ++d) {
+                        sum += k[d] ? v[d] : 0.f;
+                        num += k[d];
+                    }
+                    as[q] = sum / (float)num;  // a face filled by a layer is not read by it
+                };
+                const uint32_t total = count[layer];
+                if(total <= (uint32_t)kList)
+                    for(uint32_t e = t; e < total; e += kThreads) face(u.list[e]);
+                else
+                    for(uint32_t f = fill; f; f &= f - 1u) face(__builtin_ctz(f) << 8 | t);
+                __syncthreads();
+                m |= fill;
+                can &= ~fill;
+                filled |= fill;
+                col[t] = (uint16_t)m;
+                if(total == 0) break;  // nothing left within reach
+                __syncthreads();
             }
+            fil[t] = (uint16_t)filled;
+            if(x >= 4 && x < 12 && y >= 4 && y < 12)
+                for(uint32_t f = filled & 0x0FF0u; f; f &= f - 1u) {
+                    const int z = __builtin_ctz(f);
+                    C.a[(uint32_t)(gk0 + z) * sxy + c0] = as[(z << 8) | t];
+                }
+            __syncthreads();
         }
-        if(!brickXY || !inXY) return;
+        // flags of the brick's faces
+        if(q4 < 1 || q4 > 2 || fy < 4 || fy >= 12 || z4 < 1 || z4 > 2) return;
 #pragma unroll
-        for(int z = 4; z < 12; ++z) {
-            if(gk0 + z >= sz) continue;
-            const size_t  o  = off(z);
-            const uint8_t st = cs[z];
-            ext[o]           = st >= 2 ? 1 : 0;
-            if(st >= 2) {
-                a[o]   = ca[z];
-                val[o] = gen;
-            } else if(st == 1 && v0[z] != 1) {
-                val[o] = 1;
+        for(int q = 0; q < 4; ++q) {
+            if(!zIn(q)) continue;
+            uint32_t f = 0;
+            if(work)
+#pragma unroll
+                for(int e = 0; e < 4; ++e) f |= ((uint32_t)fil[fy * 16 + 4 * q4 + e] >> (4 * z4 + q) & 1u) << (8 * e);
+            const uint32_t set = (ok[q] | f) * 255u, nv = (v0[q] & ~set) | ok[q] | f * gen;
+            if(whole) {
+                *reinterpret_cast<uint32u*>(C.ext + at(q)) = f;
+                if(nv != v0[q]) *reinterpret_cast<uint32u*>(C.val + at(q)) = nv;
+            } else {
+                for(int e = 0; e < 4; ++e)
+                    if((uint32_t)(fi + e) < (uint32_t)sx) {
+                        C.ext[at(q) + e] = (uint8_t)(f >> (8 * e));
+                        if((nv ^ v0[q]) >> (8 * e) & 255u) C.val[at(q) + e] = (uint8_t)(nv >> (8 * e));
+                    }
             }
         }
     }

@@ -718,21 +718,23 @@ public:
         ktEnd(BNN_KT_P2G);
     }
 
-    // PIC_Solver.cpp:985-1090: the 4 Jacobi layers of each component in one launch over its 8^3 face
-    // bricks. Faces filled by this call are marked valid with the generation value extGen (2 or 3,
+    // PIC_Solver.cpp:985-1090: the 4 Jacobi layers of the three components in one launch over their 8^3
+    // face bricks. Faces filled by this call are marked valid with the generation value extGen (2 or 3,
     // alternating per call), which the same launch reads as invalid on entry.
     void extrapolateVelocity() {
-        struct C {
-            DevBuf *a, *val, *ext;
-            int     sx, sy, sz;
-        } comps[3] = {{&u, &vu, &eu, g.nx + 1, g.ny, g.nz}, {&v, &vv, &ev_, g.nx, g.ny + 1, g.nz}, {&w, &vw, &ew, g.nx, g.ny, g.nz + 1}};
         extGen = extGen == 2 ? 3 : 2;
-        for(auto& c : comps) {
-            const uint32_t nbk = (uint32_t)(((c.sx + 7) / 8) * ((c.sy + 7) / 8) * ((c.sz + 7) / 8));
-            ktBegin(BNN_KT_EXTRAP);
-            launch(k_extrap_tile{c.a->as<float>(), c.val->as<uint8_t>(), c.ext->as<uint8_t>(), c.sx, c.sy, c.sz, extGen}, nbk);
-            ktEnd(BNN_KT_EXTRAP);
+        k_extrap_tile k{{{u.as<float>(), vu.as<uint8_t>(), eu.as<uint8_t>(), g.nx + 1, g.ny, g.nz, 0},
+                         {v.as<float>(), vv.as<uint8_t>(), ev_.as<uint8_t>(), g.nx, g.ny + 1, g.nz, 0},
+                         {w.as<float>(), vw.as<uint8_t>(), ew.as<uint8_t>(), g.nx, g.ny, g.nz + 1, 0}},
+                        extGen};
+        uint32_t n = 0;
+        for(auto& c : k.comp) {
+            c.first = n;
+            n       = (n + c.bricks() + 7u) & ~7u;
         }
+        ktBegin(BNN_KT_EXTRAP);
+        launch(k, n);
+        ktEnd(BNN_KT_EXTRAP);
     }
 
     Co<void> ensureWeights() {

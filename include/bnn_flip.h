@@ -215,7 +215,7 @@ typedef enum bnn_kernel_timer {
     BNN_KT_MG_PROLONG  = 8,  /* coarse-grid correction, finest level */
     BNN_KT_MG_POST     = 9,  /* post-smoother (and z.r partials), finest level */
     BNN_KT_MG_COARSE   = 10, /* every V-cycle launch on the coarser levels */
-    BNN_KT_EXTRAP      = 11, /* extrapolation, one launch per face component (all four layers) */
+    BNN_KT_EXTRAP      = 11, /* extrapolation (three components, four layers) in one launch */
     BNN_KT_PERMUTE     = 12  /* binning payload permute */
 } bnn_kernel_timer;
 
