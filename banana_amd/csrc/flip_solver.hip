@@ -100,7 +100,7 @@ struct ParticleBufs {
     DevBuf px, py, pz, vx, vy, vz, gp, gv, id;
     DevBuf c[9];  // APIC / AFLIP affine matrices (allocated only for those schemes)
     void   reserve(size_t n, bool affine) {
-        for(DevBuf* b : {&px, &py, &pz, &vx, &vy, &vz}) b->reserve(n * 4);
+        for(DevBuf* b : {&px, &py, &pz, &vx, &vy, &vz}) b->reserve(n * 4 + 32);  // 8-wide reads may run past the last
         gp.reserve(n * 16);
         gv.reserve(n * 8);
         id.reserve(n * 4);
