@@ -530,20 +530,19 @@ public:
         }
     }
 
+    // through the spare particle buffer's records (16 bytes a particle), one array of triples after the
+    // other on the scene's stream
     void getParticles(float* pos, float* vel) {
         if(!np) return;
-        std::vector<float>    a(np);
-        std::vector<uint32_t> ids(np);
-        HIP_OK(hipMemcpyAsync(ids.data(), cur->id.p, np * 4, hipMemcpyDeviceToHost, stream));
+        float* stage = alt->gp.as<float>();
+        auto   read  = [&](const DevBuf& x, const DevBuf& y, const DevBuf& z, float* out) {
+            if(!out) return;
+            launch(k_user_order{x.as<float>(), y.as<float>(), z.as<float>(), cur->id.as<uint32_t>(), (uint32_t)np, stage}, blocks(np));
+            HIP_OK(hipMemcpyAsync(out, stage, np * 12, hipMemcpyDeviceToHost, stream));
+        };
+        read(cur->px, cur->py, cur->pz, pos);
+        read(cur->vx, cur->vy, cur->vz, vel);
         HIP_OK(hipStreamSynchronize(stream));
-        const DevBuf* src[6] = {&cur->px, &cur->py, &cur->pz, &cur->vx, &cur->vy, &cur->vz};
-        for(int k = 0; k < 6; ++k) {
-            float* out = k < 3 ? pos : vel;
-            if(!out) continue;
-            HIP_OK(hipMemcpyAsync(a.data(), src[k]->p, np * 4, hipMemcpyDeviceToHost, stream));
-            HIP_OK(hipStreamSynchronize(stream));
-            for(uint64_t i = 0; i < np; ++i) out[3 * (uint64_t)ids[i] + (k % 3)] = a[i];
-        }
     }
 
     // ---------------------------------------------------------------------------------------------
