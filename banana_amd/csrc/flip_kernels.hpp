@@ -1778,8 +1778,10 @@ template<int NT> __device__ __forceinline__ double fold_all(const double* __rest
     return t;
 }
 
-// the end of an iteration (PCGSolver.cpp:182-194): A = z.r, B = max|r|; stop test, beta, next rho
-__device__ __forceinline__ void pcg_end_iteration(PcgState& st, double A, double B) {
+// the stop test of an iteration (PCGSolver.cpp:182-187), B = max|r|. With the multigrid preconditioner it
+// runs before the V-cycle: the last iteration of a solve needs none (two thirds of an iteration's time, and
+// a solve has 5 to 10 iterations).
+__device__ __forceinline__ void pcg_stop_test(PcgState& st, double B) {
     st.iter += 1;
     st.res = (float)B;
     if((float)B < st.tol) {
@@ -1787,12 +1789,8 @@ __device__ __forceinline__ void pcg_end_iteration(PcgState& st, double A, double
         st.success = 1;
     } else if(st.iter >= st.maxIter) {
         st.done = 1;
-    } else {
-        st.beta = A / st.rho;
-        st.rho  = A;
     }
 }
-
 // init: x = 0, r = b, s = 0, z = M^-1 r; partials of z.r and max|b|
 struct k_pcg_init {
     static constexpr int kThreads = 512;
@@ -1877,8 +1875,8 @@ __device__ __forceinline__ void block_chunk(Blk blk, uint32_t n, uint32_t& s0, u
     s1               = (uint32_t)(((uint64_t)n * (v + 1)) / G);
 }
 
-// kFold (small systems): the last iteration's end (k_pcg_beta) runs here, from st to the other state
-// `next` (null: it has run), over nPart <= kFoldMax partials rz of z.r and rm of max|r|
+// kFold (small systems): the last iteration's beta (k_pcg_beta) is formed here, from st to the other
+// state `next` (null: it has been), over nPart <= kFoldMax partials rz of z.r
 template<bool kFold>
 struct k_pcg_spmv {
     static constexpr int kThreads = 512;
@@ -1896,20 +1894,22 @@ struct k_pcg_spmv {
     double* __restrict__ pa;
     PcgState* next;
     const double* __restrict__ rz;
-    const double* __restrict__ rm;
     int nPart;
     __device__ void operator()(Blk blk) const {
         __shared__ double sh[8];
         float             beta;
         if(kFold && next) {
-            PcgState cur = *st;
-            if(!cur.done) {
-                const double A = fold_all<512>(rz, nPart, false, sh), B = fold_all<512>(rm, nPart, true, sh);
-                pcg_end_iteration(cur, A, B);
+            const bool   done = st->done != 0;
+            const double A = done ? 0.0 : fold_all<512>(rz, nPart, false, sh), be = A / st->rho;
+            if(blk.id == 0 && threadIdx.x == 0) {
+                *next = *st;
+                if(!done) {
+                    next->beta = be;
+                    next->rho  = A;
+                }
             }
-            if(blk.id == 0 && threadIdx.x == 0) *next = cur;
-            if(cur.done) return;
-            beta = (float)cur.beta;
+            if(done) return;
+            beta = (float)be;
         } else {
             if(st->done) return;
             beta = (float)st->beta;
@@ -2013,8 +2013,8 @@ struct k_pcg_update {
     }
 };
 
-// res = max|r| ; stop test (PCGSolver.cpp:182-187) ; beta = rz / rho (:190-194)
-// pa: na partials of z.r, pb: nb partials of max|r|
+// res = max|r| from nb partials pb and the stop test (PCGSolver.cpp:182-187), when pb is given; then beta =
+// rz / rho (:190-194) from na partials pa of z.r, when pa is given
 struct k_pcg_beta {
     static constexpr int kThreads = 1024;
     PcgState* st;
@@ -2025,12 +2025,14 @@ struct k_pcg_beta {
     __device__ void operator()(Blk blk) const {
         __shared__ double sh[16];
         if(st && st->done) return;
-        const double A = fold(pa, na, false, sh);
-        const double B = fold(pb, nb, true, sh);
+        const double A = pa ? fold(pa, na, false, sh) : 0.0;
+        const double B = pb ? fold(pb, nb, true, sh) : 0.0;
         if(threadIdx.x != 0) return;
-        PcgState n = *st;
-        pcg_end_iteration(n, A, B);
-        *st = n;
+        if(pb) pcg_stop_test(*st, B);
+        if(pa && !st->done) {
+            st->beta = A / st->rho;
+            st->rho  = A;
+        }
     }
 };
 
@@ -2715,15 +2717,26 @@ struct k_pcg_update_pre {
 // the coarse right-hand side (P^T r). A group's eight cells lie in one fine brick, so the block of a
 // fine brick writes the 64 coarse cells it covers; r itself is never stored. Coarse cells without an
 // active child brick keep the zeros they get when the hierarchy is built. 256 threads, two cells each.
+// kStop (finest level, small systems): first the iteration's stop test over nPart <= kFoldMax partials rm
+// of max|r|; the first workgroup records it, the others read only what it leaves alone.
+template<bool kStop>
 struct k_mg_residual_restrict {
     static constexpr int kThreads = 256;
     LevelDev F;
     LevelDev C;
-    const PcgState* __restrict__ st;
+    PcgState* st;
+    const double* __restrict__ rm;
+    int nPart;
     __device__ void operator()(Blk blk) const {
         __shared__ float rs[512];
         if(st && st->done) return;
         const int t = threadIdx.x;
+        if(kStop) {
+            __shared__ double sh[8];
+            const double      B = fold_all<256>(rm, nPart, true, sh);
+            if(blk.id == 0 && t == 0) pcg_stop_test(*st, B);
+            if((float)B < st->tol) return;
+        }
         for(uint32_t v = blk.id; v < F.nSlots; v += blk.n) {
             const int s = (int)xcd_slot(v, F.nSlots);
             const int b = F.slotBrick[s];

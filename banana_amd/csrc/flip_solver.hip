@@ -952,12 +952,13 @@ public:
     // One block per brick. On each level the pre-smoothed x lives in L.r and the final x in L.x.
     // Returns true when the fine level's post-smoother also wrote the per-brick partials of z.r to pz
     // (false when the fine level is the coarsest: the caller then forms z.r itself).
-    // finePreDone: the finest level's pre-smoother already ran (fused with the PCG update).
+    // finePreDone: the finest level's pre-smoother already ran (fused with the PCG update). stopPart: the
+    // iteration's stop test runs in the finest restriction, over these per-brick partials of max|r|.
     // The finest level's correction: formed by the post-smoother itself up to kProlongInPost bricks alone
     // (a launch less), else as a streaming pass of its own (at 9600 bricks 14 us against the dependent
     // loads; in a batch the launch is shared).
     static constexpr uint32_t kProlongInPost = 1024;
-    bool vcycle(const PcgState* stp, bool finePreDone = false) {
+    bool vcycle(PcgState* stp, bool finePreDone = false, const double* stopPart = nullptr) {
         const int   nu    = prm.mg_sweeps;
         const float omega = prm.mg_omega;
         const int   tail  = mgTail();
@@ -971,7 +972,8 @@ public:
                 ktEnd(l == 0 ? BNN_KT_MG_PRE : BNN_KT_MG_COARSE);
             }
             ktBegin(l == 0 ? BNN_KT_MG_RESTRICT : BNN_KT_MG_COARSE);
-            launch(k_mg_residual_restrict{L, C, stp}, G);
+            if(l == 0 && stopPart) launch(k_mg_residual_restrict<true>{L, C, stp, stopPart, (int)L.nSlots}, G);
+            else launch(k_mg_residual_restrict<false>{L, C, stp, nullptr, 0}, G);
             ktEnd(l == 0 ? BNN_KT_MG_RESTRICT : BNN_KT_MG_COARSE);
         }
         ktBegin(BNN_KT_MG_COARSE);
@@ -1072,11 +1074,11 @@ public:
         int           nrz = (int)G;
         const bool    ic0 = prm.preconditioner == BNN_PRECOND_IC0;
         if(ic0) formIC0();
-        auto          zr  = [&](const PcgState* stp, bool finePreDone) {
+        auto          zr  = [&](PcgState* stp, bool finePreDone, const double* stopPart = nullptr) {
             if(ic0) {
                 applyIC0(r.as<float>(), z.as<float>(), stp);
                 launch(k_pcg_dot_zr{(const float*)z.as<float>(), (const float*)r.as<float>(), nSlots, stp, dpa}, G);
-            } else if(vcycle(stp, finePreDone)) {
+            } else if(vcycle(stp, finePreDone, stopPart)) {
                 rz  = pz.as<double>();
                 nrz = (int)nSlots;
             } else {
@@ -1111,7 +1113,7 @@ public:
                 ktBegin(BNN_KT_PCG_SPMV);
                 auto spmv = [&](auto k) {
                     k = {nbrTab.as<int32_t>(), z.as<float>(), sA, sB, q.as<float>(), diag32.as<float>(), cx32.as<float>(), cy32.as<float>(),
-                         cz32.as<float>(), nSlots, dst, dpa, endLast ? alt_ : nullptr, rz, dpb, (int)nSlots};
+                         cz32.as<float>(), nSlots, dst, dpa, endLast ? alt_ : nullptr, rz, (int)nSlots};
                     launch(k, G);
                 };
                 if(folded) spmv(k_pcg_spmv<true>{});
@@ -1129,9 +1131,14 @@ public:
                 else
                     launch(k_pcg_update{(const float*)sB, (const float*)q.as<float>(), (const float*)invd.as<float>(), x.as<float>(), r.as<float>(), z.as<float>(), nSlots, (const PcgState*)dst, dpa, dpb, jac}, G);
                 ktEnd(BNN_KT_PCG_UPDATE);
-                if(!jac) zr(dst, fuseUpdate);
-                if(!folded || c + 1 == n)
-                    launch(k_pcg_beta{dst, rz, nrz, (const double*)dpb, fuseUpdate ? (int)nSlots : (int)G}, 1);
+                if(fuseUpdate) {  // the stop test comes before the V-cycle
+                    if(!folded) launch(k_pcg_beta{dst, nullptr, 0, (const double*)dpb, (int)nSlots}, 1);
+                    zr(dst, true, folded ? (const double*)dpb : nullptr);
+                    if(!folded || c + 1 == n) launch(k_pcg_beta{dst, rz, nrz, nullptr, 0}, 1);
+                } else {
+                    if(!jac) zr(dst, false);
+                    launch(k_pcg_beta{dst, rz, nrz, (const double*)dpb, (int)G}, 1);
+                }
                 std::swap(sA, sB);
             }
             launched += n;
