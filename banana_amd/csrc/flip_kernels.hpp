@@ -1548,70 +1548,127 @@ struct k_fluid_sdf {
 //==================================================================================================
 // Pressure bricks
 //==================================================================================================
-// one block (512 threads) per brick: flag bricks holding a fluid cell, count fluid cells
+// Fluid cells per brick, one wavefront a brick (two 4-cell loads a lane), and the coarse levels' flags: a
+// coarse brick is active when a fluid brick lies below it, and the level-l brick of (bx, by, bz) is
+// (bx >> l, by >> l, bz >> l). Each writes the value 1, so concurrent writes to one flag agree.
+constexpr int kMaxMgLevels = 16;
 struct k_brick_flags {
-    static constexpr int kThreads = 512;
+    static constexpr int kThreads = kBlock;
     const float* __restrict__ phi;
-    GridGeom g;
-    uint32_t* __restrict__ flag;
-    uint32_t* __restrict__ nFluid;
+    GridGeom  g;
+    uint32_t* count;   // per brick
+    int       nLevels; // coarse levels 1 .. nLevels, their flags cleared before
+    int       cnbx[kMaxMgLevels], cnby[kMaxMgLevels];
+    uint32_t* flag[kMaxMgLevels];
+    static uint32_t blocks(uint32_t nb) { return (nb + kThreads / 64 - 1) / (kThreads / 64); }
     __device__ void operator()(Blk blk) const {
-        const int b  = blk.id;
+        const int lane = threadIdx.x & 63, b = blk.id * (kThreads / 64) + (threadIdx.x >> 6);
+        if(b >= g.nbx * g.nby * g.nbz) return;
         const int bx = b % g.nbx, by = (b / g.nbx) % g.nby, bz = b / (g.nbx * g.nby);
-        const int l  = threadIdx.x;
-        const int i = bx * 8 + (l & 7), j = by * 8 + ((l >> 3) & 7), k = bz * 8 + (l >> 6);
-        int fluid = 0;
-        if(i < g.nx && j < g.ny && k < g.nz) fluid = phi[lin3(i, j, k, g.nx, g.ny)] < 0.f;
-        const int cnt = __syncthreads_count(fluid);
-        if(l == 0) {
-            flag[b] = cnt > 0 ? 1u : 0u;
-            if(cnt) atomicAdd(nFluid, (uint32_t)cnt);
+        uint32_t  n = 0;
+#pragma unroll
+        for(int h = 0; h < 2; ++h) {
+            const int e = lane + 64 * h, i = bx * 8 + 4 * (e & 1), j = by * 8 + ((e >> 1) & 7), k = bz * 8 + (e >> 4);
+            float4u   v = {0.f, 0.f, 0.f, 0.f};
+            if(j < g.ny && k < g.nz) {
+                const size_t at = lin3(i, j, k, g.nx, g.ny);
+                if(i + 4 <= g.nx) v = *reinterpret_cast<const float4u*>(phi + at);
+                else
+                    for(int q = 0; q < 4; ++q)
+                        if(i + q < g.nx) v[q] = phi[at + q];
+            }
+#pragma unroll
+            for(int q = 0; q < 4; ++q) n += (uint32_t)__popcll(__ballot(v[q] < 0.f));
+        }
+        if(lane != 0) return;
+        count[b] = n;
+        if(n)
+            for(int l = 1; l <= nLevels; ++l) flag[l][((bz >> l) * cnby[l] + (by >> l)) * cnbx[l] + (bx >> l)] = 1u;
+    }
+};
+
+// Slots of the active bricks of every level, one workgroup a level (with the flags and tables 3 launches and
+// one host wait where a three-launch scan, slot, neighbour and parent table kernel per level and two waits
+// took 150 us of a 64^3 substep's 2350, and the cell counts' one atomic 121 us at 256^3): slots in ascending brick order, the
+// brick -> slot (-1: inactive) and slot -> brick tables, and the level's count to out[1 + l]. Level 0 reads
+// the cell counts and adds them up to out[0]; the coarse levels' flags return to 0 for the next time.
+struct k_brick_index {
+    static constexpr int kThreads = 1024, kItems = 8;
+    uint32_t* flag[kMaxMgLevels];
+    int32_t * brickSlot[kMaxMgLevels], *slotBrick[kMaxMgLevels];
+    uint32_t  nb[kMaxMgLevels];
+    uint32_t* out;
+    __device__ void operator()(Blk blk) const {
+        __shared__ uint32_t sh[kThreads / 64];
+        const int           l = (int)blk.id;
+        const uint32_t      n = nb[l];
+        uint32_t*           f = flag[l];
+        uint32_t            carry = 0, cells = 0;
+        for(uint32_t b0 = 0; b0 < n; b0 += kThreads * kItems) {
+            const uint32_t b = b0 + threadIdx.x * kItems;
+            uint32_t       v[kItems], s = 0;
+#pragma unroll
+            for(int q = 0; q < kItems; ++q) {
+                v[q] = b + q < n ? f[b + q] : 0u;
+                s += v[q] ? 1u : 0u;
+                cells += v[q];
+            }
+            uint32_t total, at = 0;
+            at = carry + block_exclusive_scan(s, sh, total);
+#pragma unroll
+            for(int q = 0; q < kItems; ++q)
+                if(b + q < n) {
+                    brickSlot[l][b + q] = v[q] ? (int32_t)at : -1;
+                    if(v[q]) {
+                        slotBrick[l][at++] = (int32_t)(b + q);
+                        if(l) f[b + q] = 0;
+                    }
+                }
+            carry += total;
+        }
+        uint32_t total;
+        block_exclusive_scan(cells, sh, total);
+        if(threadIdx.x == 0) {
+            out[1 + l] = carry;
+            if(l == 0) out[0] = total;
         }
     }
 };
 
-struct k_brick_slots {
+// The active bricks' tables, all levels in one launch. nbr: the six neighbours' slots (-x, +x, -y, +y, -z,
+// +z; -1: none). ptab (8 ints, not on the coarsest level): the coarse bricks that a brick's cells and halo
+// can have as parents, its own parent's six neighbours and (index 6) the parent; then the parities of the
+// brick's coordinates.
+struct k_brick_tables {
     static constexpr int kThreads = kBlock;
-    const uint32_t* __restrict__ flag;
-    const uint32_t* __restrict__ scan;
-    uint32_t nb;
-    int32_t* __restrict__ brickSlot;
-    int32_t* __restrict__ slotBrick;
+    int            nLevels;
+    uint32_t       first[kMaxMgLevels], nSlots[kMaxMgLevels];  // first block
+    int            nbx[kMaxMgLevels], nby[kMaxMgLevels], nbz[kMaxMgLevels];
+    const int32_t *brickSlot[kMaxMgLevels], *slotBrick[kMaxMgLevels];
+    int32_t *      nbr[kMaxMgLevels], *ptab[kMaxMgLevels];
     __device__ void operator()(Blk blk) const {
-        const uint32_t b = blk.id * blockDim.x + threadIdx.x;
-        if(b >= nb) return;
-        if(flag[b]) {
-            brickSlot[b]        = (int32_t)scan[b];
-            slotBrick[scan[b]] = (int32_t)b;
-        } else {
-            brickSlot[b] = -1;
-        }
-    }
-};
-
-// neighbour slots per active brick: -x, +x, -y, +y, -z, +z
-struct k_brick_nbrs {
-    static constexpr int kThreads = kBlock;
-    const int32_t* __restrict__ slotBrick;
-    uint32_t nSlots;
-    const int32_t* __restrict__ brickSlot;
-    GridGeom g;
-    int32_t* __restrict__ nbr;
-    __device__ void operator()(Blk blk) const {
-        const uint32_t s = blk.id * blockDim.x + threadIdx.x;
-        if(s >= nSlots) return;
-        const int b  = slotBrick[s];
-        const int bx = b % g.nbx, by = (b / g.nbx) % g.nby, bz = b / (g.nbx * g.nby);
-        auto      at = [&](int x, int y, int z) -> int32_t {
-            if(x < 0 || y < 0 || z < 0 || x >= g.nbx || y >= g.nby || z >= g.nbz) return -1;
-            return brickSlot[(z * g.nby + y) * g.nbx + x];
+        int l = 0;
+        while(l + 1 < nLevels && blk.id >= first[l + 1]) ++l;
+        const uint32_t s = (blk.id - first[l]) * blockDim.x + threadIdx.x;
+        if(s >= nSlots[l]) return;
+        const int b = slotBrick[l][s], bx = b % nbx[l], by = (b / nbx[l]) % nby[l], bz = b / (nbx[l] * nby[l]);
+        auto      slots = [&](int m, int x, int y, int z, int32_t* out) {
+            const int       X = nbx[m], Y = nby[m], Z = nbz[m];
+            const int32_t * t = brickSlot[m], o = (z * Y + y) * X + x;
+            out[0] = x > 0 ? t[o - 1] : -1;
+            out[1] = x + 1 < X ? t[o + 1] : -1;
+            out[2] = y > 0 ? t[o - X] : -1;
+            out[3] = y + 1 < Y ? t[o + X] : -1;
+            out[4] = z > 0 ? t[o - X * Y] : -1;
+            out[5] = z + 1 < Z ? t[o + X * Y] : -1;
         };
-        nbr[6 * s + 0] = at(bx - 1, by, bz);
-        nbr[6 * s + 1] = at(bx + 1, by, bz);
-        nbr[6 * s + 2] = at(bx, by - 1, bz);
-        nbr[6 * s + 3] = at(bx, by + 1, bz);
-        nbr[6 * s + 4] = at(bx, by, bz - 1);
-        nbr[6 * s + 5] = at(bx, by, bz + 1);
+        slots(l, bx, by, bz, nbr[l] + 6 * s);
+        if(l + 1 < nLevels) {
+            int32_t* t = ptab[l] + 8 * s;
+            slots(l + 1, bx >> 1, by >> 1, bz >> 1, t);
+            t[6] = brickSlot[l + 1][((bz >> 1) * nby[l + 1] + (by >> 1)) * nbx[l + 1] + (bx >> 1)];
+            t[7] = (bx & 1) | (by & 1) << 1 | (bz & 1) << 2;
+        }
     }
 };
 
@@ -2349,30 +2406,6 @@ __device__ __forceinline__ int32_t level_cell_index(const LevelDev& L, int i, in
     return s < 0 ? -1 : s * 512 + ((k & 7) * 8 + (j & 7)) * 8 + (i & 7);
 }
 
-// Every coarse level's active-brick flags in one pass: a brick of level l is active when a finest
-// active brick lies below it (the parent of an active brick is active, level by level), and the
-// level-l brick of finest brick (bx, by, bz) is (bx >> l, by >> l, bz >> l). Each writes the value 1,
-// so concurrent writes to one flag agree.
-constexpr int kMaxMgLevels = 16;
-struct k_mg_flag_levels {
-    static constexpr int kThreads = kBlock;
-    const int32_t* __restrict__ fineSlotBrick;
-    uint32_t nFine;
-    int fnbx;
-    int fnby;
-    int nLevels;  // coarse levels 1 .. nLevels
-    int cnbx[kMaxMgLevels];
-    int cnby[kMaxMgLevels];
-    uint32_t* flag[kMaxMgLevels];
-    __device__ void operator()(Blk blk) const {
-        const uint32_t s = blk.id * blockDim.x + threadIdx.x;
-        if(s >= nFine) return;
-        const int b = fineSlotBrick[s];
-        const int bx = b % fnbx, by = (b / fnbx) % fnby, bz = b / (fnbx * fnby);
-        for(int l = 1; l <= nLevels; ++l) flag[l][((bz >> l) * cnby[l] + (by >> l)) * cnbx[l] + (bx >> l)] = 1u;
-    }
-};
-
 // Galerkin coefficients of the coarse level (one block per coarse brick, thread = coarse cell)
 struct k_mg_coarsen {
     static constexpr int kThreads = 512;
@@ -2383,6 +2416,7 @@ struct k_mg_coarsen {
     float* __restrict__ ccy;
     float* __restrict__ ccz;
     float* __restrict__ cinv;
+    float* __restrict__ cb;  // the right-hand side: the restriction writes only cells under an active fine brick
     __device__ void operator()(Blk blk) const {
         const int s = blk.id, l = threadIdx.x;
         const int b = C.slotBrick[s];
@@ -2408,6 +2442,7 @@ struct k_mg_coarsen {
         ccy[o]         = cy;
         ccz[o]         = cz;
         cinv[o]        = d > 0.f ? 1.0f / d : 0.f;
+        cb[o]          = 0.f;
     }
 };
 
@@ -2445,26 +2480,6 @@ __device__ __forceinline__ uint32_t xcd_slot(uint32_t b, uint32_t n) {
     const uint32_t xcd = b % 8u, q = n / 8u, r = n % 8u;
     return xcd * q + min(xcd, r) + b / 8u;
 }
-
-// The coarse bricks a fine brick's cells and halo can have as parents: its own parent (index 6) and
-// that parent's six neighbours (-x, +x, -y, +y, -z, +z), or -1. Stored per fine slot (8 ints, the
-// last the parities of the brick's coordinates) when the hierarchy is built.
-struct k_mg_parent_table {
-    static constexpr int kThreads = kBlock;
-    LevelDev F;
-    LevelDev C;
-    int32_t* __restrict__ tab;
-    __device__ void operator()(Blk blk) const {
-        const uint32_t s = blk.id * blockDim.x + threadIdx.x;
-        if(s >= F.nSlots) return;
-        const int     b  = F.slotBrick[s];
-        const int     bx = b % F.nbx, by = (b / F.nbx) % F.nby, bz = b / (F.nbx * F.nby);
-        const int32_t cs = C.brickSlot[((bz >> 1) * C.nby + (by >> 1)) * C.nbx + (bx >> 1)];
-        for(int d = 0; d < 6; ++d) tab[8 * s + d] = cs >= 0 ? C.nbr[6 * cs + d] : -1;
-        tab[8 * s + 6] = cs;
-        tab[8 * s + 7] = (bx & 1) | (by & 1) << 1 | (bz & 1) << 2;
-    }
-};
 
 // xpre + omega * x_coarse(parent) for an unknown, xpre otherwise (x + omega P x_c). cs is the coarse
 // brick holding the parent of fine cell (i, j, k) (-1: none). An unknown's parent always lies inside

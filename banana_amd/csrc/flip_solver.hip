@@ -287,7 +287,7 @@ public:
 
     // bricks + pressure system
     uint32_t nb = 0, nSlots = 0, slotCap = 0, nFluid = 0;
-    DevBuf   bflag, bscan, brickSlot, slotBrick, nbrTab;
+    DevBuf   bflag, brickSlot, slotBrick, nbrTab;
     DevBuf   x, r, z, s0, s1, q, rhs32, diag32, cx32, cy32, cz32, invd;
     DevBuf   rhs64, diag64, cx64, cy64, cz64, x64;
     DevBuf   x64prev, prevBrickSlot;  // the last refined solve's pressure and brick -> slot table
@@ -360,7 +360,7 @@ public:
         allocGrid();
         HIP_OK(hipHostMalloc((void**)&hostSt, sizeof(PcgState), hipHostMallocDefault));
         HIP_OK(hipHostMalloc((void**)&hostOst, sizeof(OuterState), hipHostMallocDefault));
-        HIP_OK(hipHostMalloc((void**)&hostU32, 64, hipHostMallocDefault));
+        HIP_OK(hipHostMalloc((void**)&hostU32, 256, hipHostMallocDefault));
         if(prm.boundary_sdf_at_init) computeBoundarySDF();
         HIP_OK(hipStreamSynchronize(stream));
     }
@@ -420,7 +420,7 @@ public:
         counters.reserve(256);
         bflag.reserve(nb * 4);
         occ.reserve((size_t)(nb + 3) / 4 * 4);
-        bscan.reserve(nb * 4);
+        slotBrick.reserve(nb * 4);
         brickSlot.reserve(nb * 4);
         pst.reserve(2 * sizeof(PcgState));
         ost.reserve(sizeof(OuterState));
@@ -447,7 +447,6 @@ public:
         const uint32_t c  = std::max<uint32_t>(n + n / 4 + 16, 64);
         const size_t   nv = (size_t)c * 512;
         for(auto* b : {&x, &r, &z, &s0, &s1, &q, &rhs32, &diag32, &cx32, &cy32, &cz32, &invd}) b->reserve(nv * 4);
-        slotBrick.reserve(c * 4);
         nbrTab.reserve((size_t)c * 6 * 4);
         pa.reserve((size_t)kMaxRedBlocks * 8);
         pb.reserve((size_t)std::max<uint32_t>(kMaxRedBlocks, c) * 8);  // per block, or per brick (k_pcg_update_pre)
@@ -815,26 +814,52 @@ public:
             x64prev.swapWith(x64);
         }
         prevPressure = false;
-        fill32(counters.p, 0, 16);
-        uint32_t* cnt = counters.as<uint32_t>();
-        launch(k_brick_flags{(const float*)phi.as<float>(), g, bflag.as<uint32_t>(), cnt + 1}, nb);
-        scan(bflag.as<uint32_t>(), bscan.as<uint32_t>(), nb, cnt + 2);
-        readback(hostU32, counters.p, 16);
+        // the active bricks of every level, counted with one wait
+        const bool mgp = prm.preconditioner == BNN_PRECOND_MG;
+        if(mgp) setupLevels();
+        const int nCand = mgp ? (int)mg.size() - 1 : 0;
+        uint32_t* cnt   = counters.as<uint32_t>();
+        {
+            k_brick_flags f{};
+            k_brick_index x_{};
+            f.phi             = phi.as<float>();
+            f.g               = g;
+            f.count           = bflag.as<uint32_t>();
+            f.nLevels         = nCand;
+            x_.flag[0]        = bflag.as<uint32_t>();
+            x_.brickSlot[0]   = brickSlot.as<int32_t>();
+            x_.slotBrick[0]   = slotBrick.as<int32_t>();
+            x_.nb[0]          = nb;
+            x_.out            = cnt;
+            for(int l = 1; l <= nCand; ++l) {
+                MgLevel& L      = *mg[l];
+                f.cnbx[l]       = L.nbx;
+                f.cnby[l]       = L.nby;
+                f.flag[l]       = x_.flag[l] = L.flag.as<uint32_t>();
+                x_.brickSlot[l] = L.brickSlot.as<int32_t>();
+                x_.slotBrick[l] = L.slotBrick.as<int32_t>();
+                x_.nb[l]        = L.nb;
+            }
+            launch(f, k_brick_flags::blocks(nb));
+            launch(x_, (uint32_t)nCand + 1);
+        }
+        readback(hostU32, cnt, (size_t)(nCand + 2) * 4);
         co_await syncPoint();
-        nFluid = hostU32[1];
-        nSlots = hostU32[2];
+        nFluid = hostU32[0];
+        nSlots = hostU32[1];
         if(nSlots > nb) throw Error(BNN_ERR_DEVICE, "active brick count exceeds the brick grid");
         ensureSlots(std::max<uint32_t>(nSlots, 1));
         // the warm start swapped x64 with the previous-pressure buffer, which may be smaller than the
         // slot capacity (or not yet allocated): ensureSlots only grows buffers when the capacity grows
         if(prm.pressure_mode == BNN_PRESSURE_REFINED) x64.reserve((size_t)slotCap * 512 * 8);
-        launch(k_brick_slots{(const uint32_t*)bflag.as<uint32_t>(), (const uint32_t*)bscan.as<uint32_t>(), nb, brickSlot.as<int32_t>(), slotBrick.as<int32_t>()}, blocks(nb));
         if(nSlots == 0) {
             warmNext    = false;
             systemValid = true;
             co_return;
         }
-        launch(k_brick_nbrs{(const int32_t*)slotBrick.as<int32_t>(), nSlots, (const int32_t*)brickSlot.as<int32_t>(), g, nbrTab.as<int32_t>()}, blocks(nSlots));
+        if(mgp) sizeLevels(nCand);
+        else mgLevels = 1;
+        buildTables();
         const bool refined = prm.pressure_mode == BNN_PRESSURE_REFINED;
         SystemOut  S{rhs64.as<double>(), refined ? diag64.as<double>() : nullptr, refined ? cx64.as<double>() : nullptr,
                     refined ? cy64.as<double>() : nullptr, refined ? cz64.as<double>() : nullptr, rhs32.as<float>(), diag32.as<float>(),
@@ -849,7 +874,10 @@ public:
                                 (const double*)x64prev.as<double>(), (const float*)phi.as<float>(), g, nSlots, x64.as<double>()},
                    redBlocks());
         }
-        if(prm.preconditioner == BNN_PRECOND_MG) co_await buildHierarchy();
+        for(int l = 1; l < mgLevels; ++l) {
+            MgLevel& L = *mg[l];
+            launch(k_mg_coarsen{levelDev(l - 1), levelDev(l), L.diag.as<float>(), L.cx.as<float>(), L.cy.as<float>(), L.cz.as<float>(), L.inv.as<float>(), L.b.as<float>()}, L.nSlots);
+        }
         systemValid = true;
     }
 
@@ -858,7 +886,7 @@ public:
     struct MgLevel {
         int      nx = 0, ny = 0, nz = 0, nbx = 0, nby = 0, nbz = 0;
         uint32_t nb = 0, nSlots = 0, slotCap = 0;
-        DevBuf   flag, scan, brickSlot, slotBrick, nbr, diag, cx, cy, cz, inv, x, b, r, ptab;
+        DevBuf   flag, brickSlot, slotBrick, nbr, diag, cx, cy, cz, inv, x, b, r, ptab;
     };
     DevBuf                                ptab0;  // parent table of the fine level
     std::vector<std::unique_ptr<MgLevel>> mg;  // mg[0] unused (the fine level lives in the PCG buffers)
@@ -878,23 +906,14 @@ public:
                         L.x.as<float>(), L.b.as<float>(), L.r.as<float>(), L.nSlots, L.ptab.as<int32_t>()};
     }
 
-    // Coarse levels halve the grid until one brick remains (or every axis fits one brick). All levels'
-    // active bricks are flagged in one pass from the finest level's and counted together, so the
-    // host waits once for the whole hierarchy.
-    Co<void> buildHierarchy() {
-        mgLevels = 1;
-        if(mg.empty()) mg.emplace_back(nullptr);
-        if(nSlots <= kCoarsestSlots) co_return;
-        k_mg_flag_levels fl{};
-        fl.fineSlotBrick = slotBrick.as<int32_t>();
-        fl.nFine         = nSlots;
-        fl.fnbx          = g.nbx;
-        fl.fnby          = g.nby;
-        int nx = g.nx, ny = g.ny, nz = g.nz, nCand = 0;
-        while((nx > 8 || ny > 8 || nz > 8) && nCand + 1 < kMaxMgLevels) {
-            const int l = ++nCand;
-            if((int)mg.size() <= l) mg.emplace_back(new MgLevel());
-            MgLevel& L = *mg[l];
+    // the coarse levels' grids: each halves the one before until every axis fits one brick
+    void setupLevels() {
+        if(!mg.empty()) return;
+        mg.emplace_back(nullptr);
+        int nx = g.nx, ny = g.ny, nz = g.nz;
+        while((nx > 8 || ny > 8 || nz > 8) && (int)mg.size() < kMaxMgLevels) {
+            mg.emplace_back(new MgLevel());
+            MgLevel& L = *mg.back();
             nx = (nx + 1) / 2;
             ny = (ny + 1) / 2;
             nz = (nz + 1) / 2;
@@ -902,50 +921,51 @@ public:
             L.nbx = (nx + 7) / 8; L.nby = (ny + 7) / 8; L.nbz = (nz + 7) / 8;
             L.nb  = (uint32_t)(L.nbx * L.nby * L.nbz);
             L.flag.reserve(L.nb * 4);
-            L.scan.reserve(L.nb * 4);
             L.brickSlot.reserve(L.nb * 4);
+            L.slotBrick.reserve(L.nb * 4);
             fill32(L.flag.p, 0, L.nb * 4);
-            fl.cnbx[l] = L.nbx;
-            fl.cnby[l] = L.nby;
-            fl.flag[l] = L.flag.as<uint32_t>();
         }
-        if(nCand == 0) co_return;
-        fl.nLevels = nCand;
-        launch(fl, blocks(nSlots));
-        uint32_t* count = counters.as<uint32_t>() + 16;  // level l's active brick count at count[l]
-        for(int l = 1; l <= nCand; ++l) scan(mg[l]->flag.as<uint32_t>(), mg[l]->scan.as<uint32_t>(), mg[l]->nb, count + l);
-        readback(hostU32, count, (size_t)(nCand + 1) * 4);
-        co_await syncPoint();
+    }
+    // the levels in use (until one brick remains) and their buffers, from the counts in hostU32[1 + l]
+    void sizeLevels(int nCand) {
+        mgLevels           = 1;
         uint32_t prevSlots = nSlots;
         for(int l = 1; l <= nCand && prevSlots > kCoarsestSlots; ++l) {
-            MgLevel&       L    = *mg[l];
-            const LevelDev prev = levelDev(l - 1);
-            L.nSlots            = hostU32[l];
+            MgLevel& L = *mg[l];
+            L.nSlots   = hostU32[1 + l];
             if(L.nSlots == 0 || L.nSlots > L.nb) throw Error(BNN_ERR_DEVICE, "multigrid level has an invalid brick count");
             if(L.nSlots > L.slotCap) {
                 const uint32_t c  = L.nSlots + L.nSlots / 4 + 4;
                 const size_t   nv = (size_t)c * 512 * 4;
                 for(DevBuf* b : {&L.diag, &L.cx, &L.cy, &L.cz, &L.inv, &L.x, &L.b, &L.r}) b->reserve(nv);
-                L.slotBrick.reserve(c * 4);
                 L.nbr.reserve((size_t)c * 24);
                 L.slotCap = c;
             }
-            GridGeom lg = g;
-            lg.nx = L.nx; lg.ny = L.ny; lg.nz = L.nz;
-            lg.nbx = L.nbx; lg.nby = L.nby; lg.nbz = L.nbz;
-            launch(k_brick_slots{(const uint32_t*)L.flag.as<uint32_t>(), (const uint32_t*)L.scan.as<uint32_t>(), L.nb, L.brickSlot.as<int32_t>(), L.slotBrick.as<int32_t>()}, blocks(L.nb));
-            launch(k_brick_nbrs{(const int32_t*)L.slotBrick.as<int32_t>(), L.nSlots, (const int32_t*)L.brickSlot.as<int32_t>(), lg, L.nbr.as<int32_t>()}, blocks(L.nSlots));
-            const LevelDev cur = levelDev(l);
-            launch(k_mg_coarsen{prev, cur, L.diag.as<float>(), L.cx.as<float>(), L.cy.as<float>(), L.cz.as<float>(), L.inv.as<float>()}, L.nSlots);
-            // the restriction writes only coarse cells under an active fine brick; the others stay 0
-            fill32(L.b.p, 0, (size_t)L.nSlots * 512 * 4);
             // the finer level's parent table (its bricks' parents in this level)
             DevBuf& pt = l == 1 ? ptab0 : mg[l - 1]->ptab;
-            pt.reserve((size_t)std::max<uint32_t>(prev.nSlots, 1u) * 32);
-            launch(k_mg_parent_table{prev, levelDev(l), pt.as<int32_t>()}, blocks(prev.nSlots));
+            pt.reserve((size_t)std::max<uint32_t>(prevSlots, 1u) * 32);
             prevSlots = L.nSlots;
             ++mgLevels;
         }
+    }
+    void buildTables() {
+        k_brick_tables t{};
+        uint32_t       n = 0;
+        t.nLevels        = mgLevels;
+        for(int l = 0; l < mgLevels; ++l) {
+            MgLevel* L     = l ? mg[l].get() : nullptr;
+            t.first[l]     = n;
+            t.nSlots[l]    = L ? L->nSlots : nSlots;
+            t.nbx[l]       = L ? L->nbx : g.nbx;
+            t.nby[l]       = L ? L->nby : g.nby;
+            t.nbz[l]       = L ? L->nbz : g.nbz;
+            t.brickSlot[l] = (L ? L->brickSlot : brickSlot).as<int32_t>();
+            t.slotBrick[l] = (L ? L->slotBrick : slotBrick).as<int32_t>();
+            t.nbr[l]       = (L ? L->nbr : nbrTab).as<int32_t>();
+            t.ptab[l]      = l + 1 < mgLevels ? (L ? L->ptab : ptab0).as<int32_t>() : nullptr;
+            n += blocks(t.nSlots[l]);
+        }
+        launch(t, n);
     }
 
     // z = M^-1 r on the fine level (b = r, x = z); symmetric V-cycle with the brick-hybrid smoother.
