@@ -1210,25 +1210,51 @@ __device__ __forceinline__ void interp_gradient(const float* __restrict__ b, int
     gz = bilerpf(v001 - v000, v101 - v100, v011 - v010, v111 - v110, fi, fj);
 }
 
+// A face is constrained where the extrapolation filled it and its weight is 0. The new value of such a face
+// goes to tmp first: the interpolation around one face reads its neighbours, which must hold the values
+// from before this component's pass, but those of the components passed before it (components u, v, w in
+// turn): they are taken from their tmp. One pass over the faces applies all three afterwards (k_faces).
+struct FaceComp {
+    float*         vel;
+    float*         tmp;
+    const uint8_t* ext;
+    const float*   weight;
+};
+__device__ __forceinline__ bool constrained(uint8_t ext, float weight) { return ext == 1 && weight < kFltMin; }
+
+// the stencil's corners of a component whose new values may still lie in tmp
+__device__ __forceinline__ Corners corners_constrained(const FaceComp& c, const Stencil& s) {
+    Corners r = corners(c.vel, s);
+    const Corners t = corners(c.tmp, s), w = corners(c.weight, s);
+    const size_t  at[8] = {s.at, s.at + 1, s.at + s.sx, s.at + s.sx + 1, s.at + s.sxy, s.at + s.sxy + 1, s.at + s.sxy + s.sx, s.at + s.sxy + s.sx + 1};
+#pragma unroll
+    for(int e = 0; e < 8; ++e) r.v[e] = constrained(c.ext[at[e]], w.v[e]) ? t.v[e] : r.v[e];
+    return r;
+}
+
+// The few faces to constrain (about one in a thousand) are listed by the workgroup's first look at the flags
+// and weights of its 1024 faces and then shared by its threads, one each: four in turn in the thread that
+// found them took 11 us a component at 24^3, this takes 7.
 struct k_constrain {
     static constexpr int kThreads = kBlock;
-    VelGrid G;
+    FaceComp c[3];
     GridGeom g;
     int d;
-    const uint8_t* __restrict__ ext;
-    const float* __restrict__ weight;
     const float* __restrict__ bsdf;
-    float* __restrict__ out;
-    // the new velocity of face t (extrapolated, zero weight) into out[t]
-    __device__ void face(size_t t, int sx, int sy) const {
-        const float* cur = d == 0 ? G.u : (d == 1 ? G.v : G.w);
-        float        val = cur[t];
+    // the new velocity of face t
+    __device__ __forceinline__ float face(uint32_t t, int sx, int sy) const {
+        float val = c[d].vel[t];
         int i, j, k;
-        unlin3((uint32_t)t, sx, sy, i, j, k);
+        unlin3(t, sx, sy, i, j, k);
         float gp[3] = {(float)i + 0.5f, (float)j + 0.5f, (float)k + 0.5f};
         gp[d]       = d == 0 ? (float)i : (d == 1 ? (float)j : (float)k);
-        float vx, vy, vz, nx, ny, nz;
-        vel_from_grid(G, g, gp[0], gp[1], gp[2], vx, vy, vz);
+        const Stencil su = stencil3(g.nx + 1, g.ny, g.nz, gp[0], gp[1] - 0.5f, gp[2] - 0.5f);
+        const Stencil sv = stencil3(g.nx, g.ny + 1, g.nz, gp[0] - 0.5f, gp[1], gp[2] - 0.5f);
+        const Stencil sw = stencil3(g.nx, g.ny, g.nz + 1, gp[0] - 0.5f, gp[1] - 0.5f, gp[2]);
+        float vx = interp8(d > 0 ? corners_constrained(c[0], su) : corners(c[0].vel, su), su);
+        float vy = interp8(d > 1 ? corners_constrained(c[1], sv) : corners(c[1].vel, sv), sv);
+        float vz = interp8(corners(c[2].vel, sw), sw);
+        float nx, ny, nz;
         interp_gradient(bsdf, g.nx + 1, g.ny + 1, g.nz + 1, gp[0], gp[1], gp[2], nx, ny, nz);
         const float m2 = nx * nx + ny * ny + nz * nz;
         if(m2 > kFltMin) {
@@ -1242,57 +1268,95 @@ struct k_constrain {
             vz -= dt * nz;
             val = d == 0 ? vx : (d == 1 ? vy : vz);
         }
-        out[t] = val;
+        return val;
     }
-    // four faces per thread: the flags and weights read as one 4-byte and one 16-byte load
     __device__ void operator()(Blk blk) const {
-        const int    sx = g.nx + (d == 0), sy = g.ny + (d == 1), sz = g.nz + (d == 2);
-        const size_t N  = (size_t)sx * sy * sz;
-        const size_t t0 = 4 * ((size_t)blk.id * blockDim.x + threadIdx.x);
-        if(t0 >= N) return;
+        __shared__ uint16_t list[4 * kThreads];
+        __shared__ uint32_t count;
+        const int      sx = g.nx + (d == 0), sy = g.ny + (d == 1), sz = g.nz + (d == 2), t = threadIdx.x;
+        const uint32_t N = (uint32_t)sx * (uint32_t)sy * (uint32_t)sz, b0 = blk.id * 4u * kThreads, t0 = b0 + 4u * (uint32_t)t;
+        uint32_t       hit = 0;
         if(t0 + 4 <= N) {
-            const uchar4 e = *reinterpret_cast<const uchar4*>(ext + t0);
-            const float4 w = *reinterpret_cast<const float4*>(weight + t0);
-            if(e.x == 1 && w.x < kFltMin) face(t0, sx, sy);
-            if(e.y == 1 && w.y < kFltMin) face(t0 + 1, sx, sy);
-            if(e.z == 1 && w.z < kFltMin) face(t0 + 2, sx, sy);
-            if(e.w == 1 && w.w < kFltMin) face(t0 + 3, sx, sy);
+            const uchar4 e = *reinterpret_cast<const uchar4*>(c[d].ext + t0);
+            if(e.x == 1 || e.y == 1 || e.z == 1 || e.w == 1) {
+                const float4 w = *reinterpret_cast<const float4*>(c[d].weight + t0);
+                hit = (constrained(e.x, w.x) ? 1u : 0u) | (constrained(e.y, w.y) ? 2u : 0u) | (constrained(e.z, w.z) ? 4u : 0u) |
+                      (constrained(e.w, w.w) ? 8u : 0u);
+            }
         } else {
-            for(size_t t = t0; t < N; ++t)
-                if(ext[t] == 1 && weight[t] < kFltMin) face(t, sx, sy);
+            for(uint32_t f = t0; f < N; ++f)
+                if(constrained(c[d].ext[f], c[d].weight[f])) hit |= 1u << (f - t0);
+        }
+        if(t == 0) count = 0;
+        if(!__syncthreads_or((int)hit)) return;
+        if(hit) {
+            uint32_t at = atomicAdd(&count, (uint32_t)__popc(hit));
+            for(uint32_t h = hit; h; h &= h - 1u) list[at++] = (uint16_t)(4 * t + __builtin_ctz(h));
+        }
+        __syncthreads();
+        for(uint32_t e = t; e < count; e += kThreads) {
+            const uint32_t f = b0 + list[e];
+            c[d].tmp[f]      = face(f, sx, sy);
         }
     }
 };
 
-// the second half of a component's constrain: the faces k_constrain computed (extrapolated, zero
-// weight) take their new values; every other face keeps its velocity
-struct k_constrain_apply {
+// One pass over all faces for what a substep does to each on its own: the constrained faces take their new
+// values (apply), the velocities are backed up (old, FLIP_Data.h:48-52) and a constant gravity is added
+// (add[d]; PIC_Solver.cpp:505-529). Four faces a thread.
+struct k_faces {
     static constexpr int kThreads = kBlock;
-    float* __restrict__ vel;
-    const float* __restrict__ tmp;
-    const uint8_t* __restrict__ ext;
-    const float* __restrict__ weight;
-    size_t n;
-    // four faces per thread, as in k_constrain
+    FaceComp c[3];
+    float*   old[3];     // null: no backup
+    uint32_t n[3], first[3];  // faces, first block
+    int      apply, gravity;  // gravity: bit d, add[d] to component d
+    float    add[3];
+    static uint32_t blocks(uint32_t n) { return (n + 4 * kThreads - 1) / (4 * kThreads); }
     __device__ void operator()(Blk blk) const {
-        const size_t t0 = 4 * ((size_t)blk.id * blockDim.x + threadIdx.x);
-        if(t0 >= n) return;
-        if(t0 + 4 <= n) {
-            const uchar4 e = *reinterpret_cast<const uchar4*>(ext + t0);
-            const float4 w = *reinterpret_cast<const float4*>(weight + t0);
-            if(e.x == 1 && w.x < kFltMin) vel[t0] = tmp[t0];
-            if(e.y == 1 && w.y < kFltMin) vel[t0 + 1] = tmp[t0 + 1];
-            if(e.z == 1 && w.z < kFltMin) vel[t0 + 2] = tmp[t0 + 2];
-            if(e.w == 1 && w.w < kFltMin) vel[t0 + 3] = tmp[t0 + 3];
+        const int      d  = blk.id >= first[2] ? 2 : (blk.id >= first[1] ? 1 : 0);
+        const uint32_t t0 = 4u * ((blk.id - first[d]) * kThreads + threadIdx.x), N = n[d];
+        if(t0 >= N) return;
+        const FaceComp C = c[d];
+        const float    a = add[d];
+        const bool     on = gravity >> d & 1;
+        if(t0 + 4 <= N) {
+            const bool whole = old[d] || on;
+            uint32_t   hit = 0;
+            if(apply) {
+                const uchar4 e = *reinterpret_cast<const uchar4*>(C.ext + t0);
+                if(e.x == 1 || e.y == 1 || e.z == 1 || e.w == 1) {
+                    const float4 w = *reinterpret_cast<const float4*>(C.weight + t0);
+                    hit = (constrained(e.x, w.x) ? 1u : 0u) | (constrained(e.y, w.y) ? 2u : 0u) | (constrained(e.z, w.z) ? 4u : 0u) |
+                          (constrained(e.w, w.w) ? 8u : 0u);
+                }
+            }
+            if(!whole && !hit) return;
+            float4 v = *reinterpret_cast<const float4*>(C.vel + t0);
+            if(hit & 1u) v.x = C.tmp[t0];
+            if(hit & 2u) v.y = C.tmp[t0 + 1];
+            if(hit & 4u) v.z = C.tmp[t0 + 2];
+            if(hit & 8u) v.w = C.tmp[t0 + 3];
+            if(old[d]) *reinterpret_cast<float4*>(old[d] + t0) = v;
+            if(on) {
+                v.x += a;
+                v.y += a;
+                v.z += a;
+                v.w += a;
+            }
+            if(hit || on) *reinterpret_cast<float4*>(C.vel + t0) = v;
         } else {
-            for(size_t t = t0; t < n; ++t)
-                if(ext[t] == 1 && weight[t] < kFltMin) vel[t] = tmp[t];
+            for(uint32_t t = t0; t < N; ++t) {
+                float v = C.vel[t];
+                if(apply && constrained(C.ext[t], C.weight[t])) v = C.tmp[t];
+                if(old[d]) old[d][t] = v;
+                C.vel[t] = on ? v + a : v;
+            }
         }
     }
 };
 
 //==================================================================================================
-// addGravity (PIC_Solver.cpp:505-529): Earth / Directional add a constant per component
+// addGravity (PIC_Solver.cpp:505-529): Earth / Directional add a constant per component (k_faces)
 //==================================================================================================
 // c = a * b elementwise
 struct k_mul_arrays {
@@ -1304,20 +1368,6 @@ struct k_mul_arrays {
     __device__ void operator()(Blk blk) const {
         const size_t i = (size_t)blk.id * blockDim.x + threadIdx.x;
         if(i < n) c[i] = a[i] * b[i];
-    }
-};
-
-struct k_add_const {
-    static constexpr int kThreads = kBlock;
-    float* __restrict__ a;
-    size_t n;
-    float add;
-    int subtract;
-    __device__ void operator()(Blk blk) const {
-        const size_t t = (size_t)blk.id * blockDim.x + threadIdx.x;
-        if(t >= n) return;
-        if(subtract) a[t] -= add;
-        else a[t] += add;
     }
 };
 
@@ -2219,41 +2269,73 @@ template<class PT> __device__ __forceinline__ PT pressure_at(const PressView<PT>
     return pv.x[(size_t)s * 512 + ((k & 7) * 8 + (j & 7)) * 8 + (i & 7)];
 }
 
+// The three components in one launch, four faces a thread: where no fluid cell touches the four (three
+// quarters of the grid at 256^3), velocities and weights are not even read. 326 -> 243 us there.
 template<class PT>
 struct k_update_velocity {
     static constexpr int kThreads = kBlock;
-    float* __restrict__ vel;
-    uint8_t* __restrict__ valid;
-    const float* __restrict__ weight;
+    float*         vel[3];
+    uint8_t*       valid[3];
+    const float*   weight[3];
+    uint32_t       n[3], first[3];  // faces, first block
     const float* __restrict__ phi;
     PressView<PT> pv;
     GridGeom g;
-    int d;
     float dt;
+    static uint32_t blocks(uint32_t n) { return (n + 4 * kThreads - 1) / (4 * kThreads); }
     __device__ void operator()(Blk blk) const {
-        const int    sx = g.nx + (d == 0), sy = g.ny + (d == 1), sz = g.nz + (d == 2);
-        const size_t t  = (size_t)blk.id * blockDim.x + threadIdx.x;
-        if(t >= (size_t)sx * sy * sz) return;
-        int i, j, k;
-        unlin3((uint32_t)t, sx, sy, i, j, k);
-        const int ai = d == 0 ? i : (d == 1 ? j : k);       // index along the face normal
+        const int      d  = blk.id >= first[2] ? 2 : (blk.id >= first[1] ? 1 : 0);
+        const uint32_t t0 = 4u * ((blk.id - first[d]) * kThreads + threadIdx.x), N = n[d];
+        if(t0 >= N) return;
+        const int sx = g.nx + (d == 0), sy = g.ny + (d == 1), m = (int)min(4u, N - t0);
         const int an = d == 0 ? g.nx : (d == 1 ? g.ny : g.nz);
-        bool      upd = false;
-        if(ai > 0 && ai < an && weight[t] > 0.f) {
-            const int   li = i - (d == 0), lj = j - (d == 1), lk = k - (d == 2);
-            const float pc = phi[lin3(i, j, k, g.nx, g.ny)];
-            const float pl = phi[lin3(li, lj, lk, g.nx, g.ny)];
-            if(pc < 0 || pl < 0) {
-                const PT prc = pc < 0 ? pressure_at(pv, g, i, j, k) : PT(0);
-                const PT prl = pl < 0 ? pressure_at(pv, g, li, lj, lk) : PT(0);
-                PT       th  = fraction_inside2((PT)pl, (PT)pc);
-                th           = th > PT(0.01) ? th : PT(0.01);  // std::max(0.01, th)
-                vel[t]       = (float)((PT)vel[t] - (PT)dt * (prc - prl) / th);
-                upd          = true;
+        const uint32_t back = d == 0 ? 1u : (d == 1 ? (uint32_t)g.nx : (uint32_t)g.nx * (uint32_t)g.ny);  // to the cell before the face
+        int   i[4], j[4], k[4];
+        float pc[4], pl[4];
+        bool  fluid[4], any = false;
+        unlin3(t0, sx, sy, i[0], j[0], k[0]);
+#pragma unroll
+        for(int q = 1; q < 4; ++q) {  // along x, into the next row where it ends
+            const bool row = i[q - 1] + 1 == sx, slab = row && j[q - 1] + 1 == sy;
+            i[q] = row ? 0 : i[q - 1] + 1;
+            j[q] = slab ? 0 : j[q - 1] + (row ? 1 : 0);
+            k[q] = k[q - 1] + (slab ? 1 : 0);
+        }
+#pragma unroll
+        for(int q = 0; q < 4; ++q) {
+            const int ai = d == 0 ? i[q] : (d == 1 ? j[q] : k[q]);  // index along the face normal
+            pc[q] = pl[q] = 0.f;
+            if(q < m && ai > 0 && ai < an) {
+                const uint32_t c = (uint32_t)lin3(i[q], j[q], k[q], g.nx, g.ny);
+                pc[q]            = phi[c];
+                pl[q]            = phi[c - back];
             }
         }
-        if(!upd) vel[t] = 0.f;
-        valid[t] = upd ? 1 : 0;
+#pragma unroll
+        for(int q = 0; q < 4; ++q) any |= fluid[q] = pc[q] < 0 || pl[q] < 0;
+        float v[4] = {0.f, 0.f, 0.f, 0.f};
+        uint8_t ok[4] = {0, 0, 0, 0};
+        if(any) {
+#pragma unroll
+            for(int q = 0; q < 4; ++q)
+                if(fluid[q] && weight[d][t0 + q] > 0.f) {
+                    const PT prc = pc[q] < 0 ? pressure_at(pv, g, i[q], j[q], k[q]) : PT(0);
+                    const PT prl = pl[q] < 0 ? pressure_at(pv, g, i[q] - (d == 0), j[q] - (d == 1), k[q] - (d == 2)) : PT(0);
+                    PT       th  = fraction_inside2((PT)pl[q], (PT)pc[q]);
+                    th           = th > PT(0.01) ? th : PT(0.01);  // std::max(0.01, th)
+                    v[q]         = (float)((PT)vel[d][t0 + q] - (PT)dt * (prc - prl) / th);
+                    ok[q]        = 1;
+                }
+        }
+        if(m == 4) {
+            *reinterpret_cast<float4*>(vel[d] + t0)   = make_float4(v[0], v[1], v[2], v[3]);
+            *reinterpret_cast<uchar4*>(valid[d] + t0) = make_uchar4(ok[0], ok[1], ok[2], ok[3]);
+        } else {
+            for(int q = 0; q < m; ++q) {
+                vel[d][t0 + q]   = v[q];
+                valid[d][t0 + q] = ok[q];
+            }
+        }
     }
 };
 

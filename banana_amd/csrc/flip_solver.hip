@@ -746,47 +746,55 @@ public:
         weightsComputed = true;
     }
 
+    FaceComp faceComp(int d) {
+        DevBuf *vel[3] = {&u, &v, &w}, *tmp[3] = {&ut, &vt, &wt}, *ext[3] = {&eu, &ev_, &ew}, *wgt[3] = {&wu, &wv, &ww};
+        return FaceComp{vel[d]->as<float>(), tmp[d]->as<float>(), ext[d]->as<uint8_t>(), wgt[d]->as<float>()};
+    }
+    // one pass over the faces: apply constrained values, back up (FLIP_Data.h:48-52), add a constant gravity
+    void facesPass(bool apply, bool backup, const float* gravity) {
+        if(!apply && !backup && !gravity) return;
+        const size_t cnt[3] = {nU, nV, nW};
+        DevBuf*      old[3] = {&uo, &vo, &wo};
+        k_faces      k{};
+        uint32_t     nb_ = 0;
+        for(int d = 0; d < 3; ++d) {
+            k.c[d]     = faceComp(d);
+            k.old[d]   = backup ? old[d]->as<float>() : nullptr;
+            k.n[d]     = (uint32_t)cnt[d];
+            k.first[d] = nb_;
+            k.add[d]   = gravity ? gravity[d] : 0.f;
+            nb_ += k_faces::blocks(k.n[d]);
+        }
+        k.apply   = apply;
+        k.gravity = gravity ? (prm.gravity_type == 0 ? 2 : 7) : 0;  // Earth: v only
+        launch(k, nb_);
+    }
+
     // PIC_Solver.cpp:1094-1115. Uses the weights as they stand: before the first pressure projection
     // they are the zero fill of PIC_Data.cpp:109 (FLIP_Solver.cpp:45 constrains before
     // computeCellWeights runs), so every extrapolated face qualifies then. A no-op while the boundary
-    // SDF is identically zero (zero gradient) or no face has weight < FLT_MIN.
-    void constrainGridVelocity() {
-        if(!bsdfNonzero) return;
-        if(weightsComputed && solidFaces == 0) return;
-        DevBuf* vel[3] = {&u, &v, &w};
-        DevBuf* tmp[3] = {&ut, &vt, &wt};
-        DevBuf* ext[3] = {&eu, &ev_, &ew};
-        DevBuf* wgt[3] = {&wu, &wv, &ww};
-        size_t  cnt[3] = {nU, nV, nW};
-        for(int d = 0; d < 3; ++d) {
-            VelGrid G{u.as<float>(), v.as<float>(), w.as<float>()};
-            // the new values of the faces that change go to tmp first: the interpolation around one
-            // face reads its neighbours, which must still hold the values before this component's pass
-            launch(k_constrain{G, g, d, (const uint8_t*)ext[d]->as<uint8_t>(),
-                               (const float*)wgt[d]->as<float>(), (const float*)bsdf.as<float>(), tmp[d]->as<float>()}, blocks((cnt[d] + 3) / 4));
-            launch(k_constrain_apply{vel[d]->as<float>(), (const float*)tmp[d]->as<float>(), (const uint8_t*)ext[d]->as<uint8_t>(),
-                                     (const float*)wgt[d]->as<float>(), cnt[d]},
-                   blocks((cnt[d] + 3) / 4));
-        }
+    // SDF is identically zero (zero gradient) or no face has weight < FLT_MIN. Returns whether new values
+    // wait in tmp for facesPass.
+    bool constrainedValues() {
+        if(!bsdfNonzero) return false;
+        if(weightsComputed && solidFaces == 0) return false;
+        const size_t cnt[3] = {nU, nV, nW};
+        for(int d = 0; d < 3; ++d)
+            launch(k_constrain{{faceComp(0), faceComp(1), faceComp(2)}, g, d, (const float*)bsdf.as<float>()}, blocks((cnt[d] + 3) / 4));
+        return true;
     }
+    void constrainGridVelocity() { facesPass(constrainedValues(), false, nullptr); }
 
-    void backupGridVelocity() {  // FLIP_Data.h:48-52
-        copy32(uo.p, u.p, nU * 4);
-        copy32(vo.p, v.p, nV * 4);
-        copy32(wo.p, w.p, nW * 4);
-    }
-
-    void addGravity(float dt) {  // PIC_Solver.cpp:505-529
-        if(!prm.apply_gravity) return;
-        if(prm.gravity_type == 0) {
-            const float gdt = 9.81f * dt;
-            launch(k_add_const{v.as<float>(), nV, gdt, 1}, blocks(nV));
-        } else if(prm.gravity_type == 1) {
-            DevBuf* vel[3] = {&u, &v, &w};
-            size_t  cnt[3] = {nU, nV, nW};
-            for(int d = 0; d < 3; ++d)
-                launch(k_add_const{vel[d]->as<float>(), cnt[d], grav[d] * dt, 0}, blocks(cnt[d]));
-        } else {
+    // PIC_Solver.cpp:505-529; backup: the velocities before it are kept (FLIP, AFLIP). constrained: new
+    // values wait in tmp (constrainedValues)
+    void addGravity(float dt, bool backup = false, bool constrained = false) {
+        float       c[3] = {0.f, 0.f, 0.f};
+        const bool  on = prm.apply_gravity != 0, center = prm.gravity_type >= 2;
+        if(prm.gravity_type == 0) c[1] = -(9.81f * dt);
+        else
+            for(int d = 0; d < 3; ++d) c[d] = grav[d] * dt;
+        facesPass(constrained, backup, on && !center ? c : nullptr);
+        if(on && center) {
             DevBuf* vel[3] = {&u, &v, &w};
             for(int d = 0; d < 3; ++d)
                 launch(k_gravity_center{vel[d]->as<float>(), g, d,
@@ -1244,20 +1252,31 @@ public:
     }
 
     void updateProjectedVelocity(float dt) {  // PIC_Solver.cpp:911-981
-        DevBuf* vel[3] = {&u, &v, &w};
-        DevBuf* val[3] = {&vu, &vv, &vw};
-        DevBuf* wgt[3] = {&wu, &wv, &ww};
-        size_t  cnt[3] = {nU, nV, nW};
-        for(int d = 0; d < 3; ++d) {
-            if(lastRefined && nSlots) {
-                PressView<double> pv{x64.as<double>(), brickSlot.as<int32_t>()};
-                launch(k_update_velocity<double>{vel[d]->as<float>(),
-                                   val[d]->as<uint8_t>(), (const float*)wgt[d]->as<float>(), (const float*)phi.as<float>(), pv, g, d, dt}, blocks(cnt[d]));
-            } else {
-                PressView<float> pv{x.as<float>(), brickSlot.as<int32_t>()};
-                launch(k_update_velocity<float>{vel[d]->as<float>(),
-                                   val[d]->as<uint8_t>(), (const float*)wgt[d]->as<float>(), (const float*)phi.as<float>(), pv, g, d, dt}, blocks(cnt[d]));
+        const size_t cnt[3] = {nU, nV, nW};
+        DevBuf *     vel[3] = {&u, &v, &w}, *val[3] = {&vu, &vv, &vw}, *wgt[3] = {&wu, &wv, &ww};
+        auto         run = [&](auto k) {
+            uint32_t nb_ = 0;
+            for(int d = 0; d < 3; ++d) {
+                k.vel[d]    = vel[d]->as<float>();
+                k.valid[d]  = val[d]->as<uint8_t>();
+                k.weight[d] = wgt[d]->as<float>();
+                k.n[d]      = (uint32_t)cnt[d];
+                k.first[d]  = nb_;
+                nb_ += k.blocks(k.n[d]);
             }
+            k.phi = phi.as<float>();
+            k.g   = g;
+            k.dt  = dt;
+            launch(k, nb_);
+        };
+        if(lastRefined && nSlots) {
+            k_update_velocity<double> k{};
+            k.pv = {x64.as<double>(), brickSlot.as<int32_t>()};
+            run(k);
+        } else {
+            k_update_velocity<float> k{};
+            k.pv = {x.as<float>(), brickSlot.as<int32_t>()};
+            run(k);
         }
     }
 
@@ -1327,9 +1346,10 @@ public:
         extrapolateVelocity();
         stageEnd(BNN_STAGE_EXTRAPOLATE);
         stageBegin(BNN_STAGE_CONSTRAIN);
-        constrainGridVelocity();
-        backupGridVelocity();
-        addGravity(dt);
+        {
+            const bool waiting = constrainedValues();
+            addGravity(dt, true, waiting);
+        }
         stageEnd(BNN_STAGE_CONSTRAIN);
         bool ok = co_await pressureProjection(dt);
         stageBegin(BNN_STAGE_EXTRAPOLATE);
