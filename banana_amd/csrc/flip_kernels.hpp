@@ -2149,6 +2149,14 @@ struct k_pcg_beta {
 struct OuterState {
     double res, bmax;
 };
+// what the host reads back of a solve: the inner solve's two states and the outer one's
+struct SolveState {
+    PcgState   inner[2];
+    OuterState outer;
+};
+// The end of an outer pass (accumulate, next residual) can be queued behind the inner iterations before the
+// host knows that they suffice: with a gate it runs only when the inner solve has stopped.
+__device__ __forceinline__ bool gated(const PcgState* gate) { return gate && !gate->done; }
 
 struct k_residual64 {
     static constexpr int kThreads = 512;
@@ -2164,8 +2172,10 @@ struct k_residual64 {
     double* __restrict__ pa;
     double* __restrict__ pb;
     int first;
+    const PcgState* gate;
     __device__ void operator()(Blk blk) const {
         __shared__ double sh[8];
+        if(gated(gate)) return;
         const int         l = threadIdx.x;
         double            m = 0, bm = 0;
         for(uint32_t slot = blk.id; slot < nSlots; slot += blk.n) {
@@ -2205,8 +2215,10 @@ struct k_residual64_fin {
     const double* __restrict__ pa;
     const double* __restrict__ pb;
     int n;
+    const PcgState* gate;
     __device__ void operator()(Blk blk) const {
         __shared__ double sh[16];
+        if(gated(gate)) return;
         const double      M  = fold(pa, n, true, sh);
         const double      BM = fold(pb, n, true, sh);
         if(threadIdx.x == 0) {
@@ -2247,7 +2259,9 @@ struct k_accumulate64 {
     const float* __restrict__ d;
     uint32_t nSlots;
     int first;
+    const PcgState* gate;
     __device__ void operator()(Blk blk) const {
+        if(gated(gate)) return;
         for(uint32_t slot = blk.id; slot < nSlots; slot += blk.n) {
             const size_t o = (size_t)slot * 512 + threadIdx.x;
             x64[o]         = first ? (double)d[o] : x64[o] + (double)d[o];

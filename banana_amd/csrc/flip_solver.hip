@@ -293,10 +293,9 @@ public:
     DevBuf   x64prev, prevBrickSlot;  // the last refined solve's pressure and brick -> slot table
     bool     prevPressure = false;   // they hold a converged pressure of this grid
     bool     warmNext     = false;   // this solve starts from them (x64 filled by k_warm_start)
-    DevBuf   pa, pb, pz, pst, ost;  // PCG partials (per block: pa, pb; per brick: pz), device states
+    DevBuf   pa, pb, pz, pst;       // PCG partials (per block: pa, pb; per brick: pz), device states
     DevBuf   icInv, icLx, icLy, icLz;  // IC(0) factor (BNN_PRECOND_IC0 only)
-    PcgState*   hostSt  = nullptr;  // pinned
-    OuterState* hostOst = nullptr;
+    SolveState* hostSolve = nullptr;  // pinned
     uint32_t*   hostU32 = nullptr;
     int         device  = 0;  // the device current at creation (owns the stream and every buffer)
     // ParticleSimulationData::objectIndex / nObjects: the generator of each particle, in user order
@@ -358,8 +357,7 @@ public:
         HIP_OK(hipGetDevice(&device));
         HIP_OK(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
         allocGrid();
-        HIP_OK(hipHostMalloc((void**)&hostSt, sizeof(PcgState), hipHostMallocDefault));
-        HIP_OK(hipHostMalloc((void**)&hostOst, sizeof(OuterState), hipHostMallocDefault));
+        HIP_OK(hipHostMalloc((void**)&hostSolve, sizeof(SolveState), hipHostMallocDefault));
         HIP_OK(hipHostMalloc((void**)&hostU32, 256, hipHostMallocDefault));
         if(prm.boundary_sdf_at_init) computeBoundarySDF();
         HIP_OK(hipStreamSynchronize(stream));
@@ -368,8 +366,7 @@ public:
     ~FlipSolver() {
         if(stream) (void)hipStreamSynchronize(stream);
         for(hipEvent_t e : evPool) (void)hipEventDestroy(e);
-        if(hostSt) (void)hipHostFree(hostSt);
-        if(hostOst) (void)hipHostFree(hostOst);
+        if(hostSolve) (void)hipHostFree(hostSolve);
         if(hostU32) (void)hipHostFree(hostU32);
         if(stream) (void)hipStreamDestroy(stream);
     }
@@ -422,11 +419,10 @@ public:
         occ.reserve((size_t)(nb + 3) / 4 * 4);
         slotBrick.reserve(nb * 4);
         brickSlot.reserve(nb * 4);
-        pst.reserve(2 * sizeof(PcgState));
-        ost.reserve(sizeof(OuterState));
+        pst.reserve(sizeof(SolveState));
         // zero everything the reference zero-fills at resize (PIC_Data.cpp:101-117)
         for(auto* b : {&u, &v, &w, &ut, &vt, &wt, &uo, &vo, &wo, &wu, &wv, &ww, &vu, &vv, &vw, &eu, &ev_, &ew, &phi, &bsdf,
-                       &cellStart, &cellCount, &counters, &pst, &ost})
+                       &cellStart, &cellCount, &counters, &pst})
             HIP_OK(hipMemsetAsync(b->p, 0, b->bytes, stream));
         weightsDirty = true;
     }
@@ -1087,9 +1083,22 @@ public:
         return (uint32_t)std::min<double>(need, (double)pcgChunkMax);
     }
 
-    // FP32 PCG on b -> x (PCGSolver.cpp:143-199); returns success
-    Co<bool> pcg32(const float* b, float relTol, uint32_t maxIter, uint32_t& iters, float& res, float& bmax) {
-        PcgState*      dst = pst.as<PcgState>();
+    // the outer pass around an inner solve: x64 += (or =, zeroX) x, then the residual's fold
+    void residualPass(int zeroX, const PcgState* gate) {
+        const unsigned G = redBlocks();
+        launch(k_residual64{(const int32_t*)nbrTab.as<int32_t>(), (const double*)x64.as<double>(), (const double*)rhs64.as<double>(), (const double*)diag64.as<double>(), (const double*)cx64.as<double>(), (const double*)cy64.as<double>(), (const double*)cz64.as<double>(), rhs32.as<float>(), nSlots, pa.as<double>(), pb.as<double>(), zeroX, gate}, G);
+        launch(k_residual64_fin{&pst.as<SolveState>()->outer, (const double*)pa.as<double>(), (const double*)pb.as<double>(), (int)G, gate}, 1);
+    }
+    void accumulatePass(int zeroX, const PcgState* gate) {
+        launch(k_accumulate64{x64.as<double>(), (const float*)x.as<float>(), nSlots, zeroX, gate}, redBlocks());
+    }
+
+    // FP32 PCG on b -> x (PCGSolver.cpp:143-199); returns success. endPass >= 0 (alone only): the outer
+    // pass's end is queued behind every chunk of iterations, gated on the inner solve having stopped, with
+    // zeroX = endPass: when the chunk sufficed, the host has the next residual with the same wait.
+    Co<bool> pcg32(const float* b, float relTol, uint32_t maxIter, uint32_t& iters, float& res, float& bmax, int endPass = -1) {
+        PcgState*      dst = pst.as<SolveState>()->inner;
+        const PcgState* hostSt = hostSolve->inner;
         PcgState*      alt_ = dst + 1;  // the state an SpMV that ends the last iteration writes
         double*        dpa = pa.as<double>();
         double*        dpb = pb.as<double>();
@@ -1126,9 +1135,23 @@ public:
         // already solved); each later poll sizes the next chunk from max|r| at iteration 0, which is
         // max|b| since x starts at 0
         uint32_t chunk = pcgChunkFirst, launched = 0;
+        // alone, with the multigrid: as many as the last inner solve's mean reduction says (its system was the
+        // same one or the previous substep's); each wait saved is 10 to 20 us of an idle GPU, and an iteration
+        // too many costs about as much
+        if(fuseUpdate && !rec && pcgRate < 0.0 && relTol > 0.f && relTol < 1.f)
+            chunk = (uint32_t)std::min(std::max(std::ceil(std::log((double)relTol) / pcgRate), 1.0), (double)pcgChunkMax);
         for(bool first = true;; first = false) {
             if(!first) {
-                readback(hostSt, dst, sizeof(PcgState));
+                if(rec) {
+                    readback(&hostSolve->inner[0], dst, sizeof(PcgState));
+                } else {
+                    if(endPass >= 0) {
+                        accumulatePass(endPass, dst);
+                        residualPass(0, dst);
+                    }
+                    readback(hostSolve, pst.p, sizeof(SolveState));
+                    hostSt = &hostSolve->inner[dst - pst.as<SolveState>()->inner];
+                }
                 co_await syncPoint();
                 if(hostSt->done) break;
                 chunk = pcgNextChunk(hostSt->bmax, hostSt->res, hostSt->tol, hostSt->iter, chunk);
@@ -1175,8 +1198,10 @@ public:
         iters = hostSt->iter;
         res   = hostSt->res;
         bmax  = hostSt->bmax;
+        if(iters > 0 && res > 0.f && res < bmax) pcgRate = std::log((double)res / (double)bmax) / (double)iters;
         co_return hostSt->success != 0;
     }
+    double pcgRate = 0.0;  // log of max|r|'s mean reduction per iteration in the last inner solve (0: none yet)
 
     Co<bool> solveSystem() {  // PIC_Solver.cpp:897-907
         lastRefined = prm.pressure_mode == BNN_PRESSURE_REFINED;
@@ -1203,19 +1228,19 @@ public:
         const double   tol      = prm.refine_tolerance > 0 ? prm.refine_tolerance : 1e-10;
         const float    innerTol = prm.refine_inner_tolerance;
         const uint32_t maxOuter = 30;
-        const unsigned G        = redBlocks();
         uint32_t       total = 0, outer = 0;
         bool           ok = false;
         double         bmax = 0, res = 0;
         for(int first = 1;; first = 0) {
             co_await barrier();  // the scenes' outer passes start together
             const int zeroX = first && !warmNext;  // x = 0 (else x64 holds the warm start or the sum so far)
-            launch(k_residual64{(const int32_t*)nbrTab.as<int32_t>(), (const double*)x64.as<double>(), (const double*)rhs64.as<double>(), (const double*)diag64.as<double>(), (const double*)cx64.as<double>(), (const double*)cy64.as<double>(), (const double*)cz64.as<double>(), rhs32.as<float>(), nSlots, pa.as<double>(), pb.as<double>(), zeroX}, G);
-            launch(k_residual64_fin{ost.as<OuterState>(), (const double*)pa.as<double>(), (const double*)pb.as<double>(), (int)G}, 1);
-            readback(hostOst, ost.p, sizeof(OuterState));
-            co_await syncPoint();
+            if(first || rec) {  // else the inner solve's last wait brought the residual
+                residualPass(zeroX, nullptr);
+                readback(&hostSolve->outer, &pst.as<SolveState>()->outer, sizeof(OuterState));
+                co_await syncPoint();
+            }
             if(first) {
-                bmax = hostOst->bmax;
+                bmax = hostSolve->outer.bmax;
                 if(bmax < 1.17549435e-38) {
                     fill32(x64.p, 0, (size_t)nSlots * 512 * 8);
                     ok  = true;
@@ -1223,7 +1248,7 @@ public:
                     break;
                 }
             }
-            res = hostOst->res;
+            res = hostSolve->outer.res;
             if(res <= tol * bmax) {
                 if(zeroX) fill32(x64.p, 0, (size_t)nSlots * 512 * 8);
                 ok = true;
@@ -1236,9 +1261,9 @@ public:
             const float  passTol = missing > 4.0 * innerTol ? (float)std::min(0.25 * missing, 0.5) : innerTol;
             uint32_t     it;
             float        r32, b32;
-            co_await pcg32(rhs32.as<float>(), passTol, prm.max_cg_iteration, it, r32, b32);
+            co_await pcg32(rhs32.as<float>(), passTol, prm.max_cg_iteration, it, r32, b32, rec ? -1 : zeroX);
             total += it;
-            launch(k_accumulate64{x64.as<double>(), (const float*)x.as<float>(), nSlots, zeroX}, G);
+            if(rec) accumulatePass(zeroX, nullptr);
             ++outer;
             if(it == 0) break;  // inner solve made no progress
         }
