@@ -2590,16 +2590,20 @@ __device__ __forceinline__ float mg_prolonged(const LevelDev& F, const float* __
     return un ? xv + omega * xc : xv;
 }
 
-// one cell of the brick smoother: its LDS index and its row of A (a coupling to a missing neighbour
-// is 0 and that neighbour's halo entry holds 0, so the six terms are added unconditionally)
+// One cell of the brick smoother: its LDS index and its row of A, divided by the diagonal and with the sign
+// of the update x = b/d - sum (a/d) x (a coupling to a missing neighbour is 0 and that neighbour's halo
+// entry holds 0, so all six terms are added unconditionally). The thread owns an x-adjacent pair of cells,
+// one of each colour: the coupling between them takes the other's value from a register (`in`), the one
+// out of the pair lies at LDS offset `off`. Five LDS reads and seven multiply-adds in two chains, against
+// six reads and fourteen operations in one: the half-sweeps are a serial chain.
 struct SmoothCell {
-    int   c;
-    float czm, cym, cxm, cxp, cyp, czp, bv, inv;
+    int   c, off;
+    float zm, ym, out, in, yp, zp, bs;
 };
 
 template<int kProlong>
 __device__ __forceinline__ SmoothCell smooth_cell_setup(const LevelDev& L, const LevelDev& C, int32_t parent, float omega, int s, int l,
-                                                        int bx, int by, int bz, float* xs) {
+                                                        int bx, int by, int bz, float* xs, float& bv) {
     const int     lx = l & 7, ly = (l >> 3) & 7, lz = l >> 6;
     const int     c  = ((lz + 1) * 10 + (ly + 1)) * 10 + (lx + 1);
     const size_t  o  = (size_t)s * 512 + l;
@@ -2610,14 +2614,16 @@ __device__ __forceinline__ SmoothCell smooth_cell_setup(const LevelDev& L, const
     R.c   = c;
     const float   czm = L.cz[izm >= 0 ? izm : (int32_t)o], cym = L.cy[iym >= 0 ? iym : (int32_t)o];
     const float   cxm = L.cx[ixm >= 0 ? ixm : (int32_t)o], cxp = L.cx[o], cyp = L.cy[o], czp = L.cz[o];
-    R.czm = izm >= 0 ? czm : 0.f;
-    R.cym = iym >= 0 ? cym : 0.f;
-    R.cxm = ixm >= 0 ? cxm : 0.f;
-    R.cxp = ixp >= 0 ? cxp : 0.f;
-    R.cyp = iyp >= 0 ? cyp : 0.f;
-    R.czp = izp >= 0 ? czp : 0.f;
-    R.bv  = L.b[o];
-    R.inv = L.invdiag[o];
+    const float   inv = L.invdiag[o], xm = ixm >= 0 ? -cxm * inv : 0.f, xp = ixp >= 0 ? -cxp * inv : 0.f;
+    bv    = L.b[o];
+    R.zm  = izm >= 0 ? -czm * inv : 0.f;
+    R.ym  = iym >= 0 ? -cym * inv : 0.f;
+    R.yp  = iyp >= 0 ? -cyp * inv : 0.f;
+    R.zp  = izp >= 0 ? -czp * inv : 0.f;
+    R.in  = lx & 1 ? xm : xp;
+    R.out = lx & 1 ? xp : xm;
+    R.off = lx & 1 ? 1 : -1;
+    R.bs  = bv * inv;
     xs[c] = kProlong == 1 ? mg_prolonged(L, L.r, C, parent, omega, (int32_t)o, bx * 8 + lx, by * 8 + ly, bz * 8 + lz)
                           : (kProlong == 2 ? L.r[o] : 0.f);
     return R;
@@ -2665,15 +2671,12 @@ __device__ __forceinline__ void smooth_halo(const LevelDev& L, const LevelDev& C
     }
 }
 
-__device__ __forceinline__ void smooth_cell_update(const SmoothCell& R, float* xs) {
-    float acc = 0.f;
-    acc += R.czm * xs[R.c - 100];
-    acc += R.cym * xs[R.c - 10];
-    acc += R.cxm * xs[R.c - 1];
-    acc += R.cxp * xs[R.c + 1];
-    acc += R.cyp * xs[R.c + 10];
-    acc += R.czp * xs[R.c + 100];
-    xs[R.c] = (R.bv - acc) * R.inv;
+// the cell's new value; pair: the other cell of its pair
+__device__ __forceinline__ float smooth_cell_update(const SmoothCell& R, float* xs, float pair) {
+    const float p = __builtin_fmaf(R.out, xs[R.c + R.off], __builtin_fmaf(R.ym, xs[R.c - 10], __builtin_fmaf(R.zm, xs[R.c - 100], R.bs)));
+    const float v = p + __builtin_fmaf(R.zp, xs[R.c + 100], __builtin_fmaf(R.yp, xs[R.c + 10], R.in * pair));
+    xs[R.c]       = v;
+    return v;
 }
 
 // coarse-grid correction in place: L.r (the pre-smoothed x) += omega * P x_coarse on every unknown.
@@ -2722,22 +2725,25 @@ __device__ __forceinline__ void mg_smooth_one(const LevelDev& L, const LevelDev&
     const int     b      = L.slotBrick[s];
     const int     bx     = b % L.nbx, by = (b / L.nbx) % L.nby, bz = b / (L.nbx * L.nby);
     const int32_t parent = kProlong == 1 ? L.ptab[8 * s + 6] : -1;
-    const SmoothCell R = smooth_cell_setup<kProlong>(L, C, parent, omega, s, lr, bx, by, bz, xs);
-    const SmoothCell K = smooth_cell_setup<kProlong>(L, C, parent, omega, s, lb, bx, by, bz, xs);
+    float            br, bb;
+    const SmoothCell R = smooth_cell_setup<kProlong>(L, C, parent, omega, s, lr, bx, by, bz, xs, br);
+    const SmoothCell K = smooth_cell_setup<kProlong>(L, C, parent, omega, s, lb, bx, by, bz, xs, bb);
     smooth_halo<kProlong>(L, C, parent, omega, s, bx, by, bz, xs);
+    float zr = xs[R.c], zb = xs[K.c];
     __syncthreads();
     for(int it = 0; it < sweeps; ++it) {
-        smooth_cell_update(kProlong ? K : R, xs);
+        if(kProlong) zb = smooth_cell_update(K, xs, zr);
+        else zr = smooth_cell_update(R, xs, zb);
         __syncthreads();
-        smooth_cell_update(kProlong ? R : K, xs);
+        if(kProlong) zr = smooth_cell_update(R, xs, zb);
+        else zb = smooth_cell_update(K, xs, zr);
         __syncthreads();
     }
     float*      out             = kProlong ? L.x : L.r;
-    const float zr = xs[R.c], zb = xs[K.c];
     out[(size_t)s * 512 + lr]   = zr;
     out[(size_t)s * 512 + lb]   = zb;
     if(kDot) {
-        const double d = block_sum<256>((double)zr * (double)R.bv + (double)zb * (double)K.bv, sh);
+        const double d = block_sum<256>((double)zr * (double)br + (double)zb * (double)bb, sh);
         if(t == 0) pz[s] = d;
     }
     __syncthreads();  // xs is reused by the workgroup's next brick
@@ -3059,14 +3065,12 @@ namespace bnn {
 // its own dependent loads and its launch (5-7 us each, three a level, 11 for a coarsest solve by one
 // wavefront), whatever its work. Here one workgroup takes the levels lv[0] (at most 8 bricks) to the
 // coarsest (one brick): all their x tiles (a brick and its one-cell halo) stay in LDS, a right-hand side
-// goes to the next level through that level's tile, and the coefficients of the first two levels are
-// loaded once, at the start. Four groups of 256 threads own a brick each (on lv[0] up to two in turn;
-// thread = an x-adjacent pair of cells, one of each colour). Same arithmetic, in the same order, as
-// k_mg_smooth_brick, k_mg_residual_restrict and (coarsest: x = 0, `coarsest` red-black and as many
-// black-red sweeps) their per-level launches, so the results are the same bits. Input lv[0].b, output
-// lv[0].x. Bound by the chain of half-sweeps (about 0.17 us each, 32 of them on the coarsest level):
-// 17 us for two levels, 28 for three, against 27 and 42 in separate kernels plus 4 or 7 launches; a
-// whole substep at 24^3 1116 -> 1048 us, at 64^3 2867 -> 2606.
+// goes to the next level through that level's tile, and the coefficients of the first two levels and the
+// coarsest are loaded once, at the start. Four groups of 256 threads own a brick each (on lv[0] up to two in turn;
+// thread = an x-adjacent pair of cells, one of each colour). The steps are those of k_mg_smooth_brick and
+// k_mg_residual_restrict; coarsest level: x = 0, `coarsest` red-black and as many black-red sweeps. Input
+// lv[0].b, output lv[0].x. Bound by the chain of half-sweeps (32 of them on the coarsest level): 16 us for
+// two levels, 25 for three, against 27 and 42 in separate kernels plus 4 or 7 launches.
 struct k_mg_tail {
     static constexpr int kThreads = 1024;
     static constexpr int kLevels = 5, kTop = 8, kRest = 4, kTiles = 16;  // levels; bricks on lv[0], on each other level, in all
@@ -3076,8 +3080,10 @@ struct k_mg_tail {
     int      sweeps, coarsest;
     const PcgState* __restrict__ st;
 
-    struct Row {  // a cell's row of A (couplings to missing neighbours 0), right-hand side and 1/diagonal
-        float czm, cym, cxm, cxp, cyp, czp, bv, inv, diag;
+    // a cell's row of A as in SmoothCell (divided by the diagonal, signed), its diagonal
+    struct Row {
+        float zm, ym, out, in, yp, zp, bs, diag;
+        __device__ __forceinline__ void rhs(float b) { bs = diag > 0.f ? b / diag : 0.f; }
     };
     static __device__ __forceinline__ int tile_at(int l) { return (((l >> 6) + 1) * 10 + ((l >> 3) & 7) + 1) * 10 + (l & 7) + 1; }
     // nb: the brick's six neighbour slots
@@ -3088,38 +3094,34 @@ struct k_mg_tail {
         const bool    hx = lx > 0 || nx >= 0, hy = ly > 0 || ny >= 0, hz = lz > 0 || nz >= 0;
         const int32_t ix = lx > 0 ? o - 1 : (hx ? nx * 512 + l + 7 : o), iy = ly > 0 ? o - 8 : (hy ? ny * 512 + l + 56 : o),
                       iz = lz > 0 ? o - 64 : (hz ? nz * 512 + l + 448 : o);
-        const float czm = L.cz[iz], cym = L.cy[iy], cxm = L.cx[ix], cxp = L.cx[o], cyp = L.cy[o], czp = L.cz[o];
+        const float czm = L.cz[iz], cym = L.cy[iy], cxm = L.cx[ix], cxp = L.cx[o], cyp = L.cy[o], czp = L.cz[o], inv = L.invdiag[o];
+        const float xm = hx ? -cxm * inv : 0.f, xp = lx < 7 || nb[1] >= 0 ? -cxp * inv : 0.f;
         Row         R;
-        R.inv  = L.invdiag[o];
         R.diag = L.diag[o];
-        R.czm  = hz ? czm : 0.f;
-        R.cym  = hy ? cym : 0.f;
-        R.cxm  = hx ? cxm : 0.f;
-        R.cxp  = lx < 7 || nb[1] >= 0 ? cxp : 0.f;
-        R.cyp  = ly < 7 || nb[3] >= 0 ? cyp : 0.f;
-        R.czp  = lz < 7 || nb[5] >= 0 ? czp : 0.f;
-        R.bv   = 0.f;
+        R.zm   = hz ? -czm * inv : 0.f;
+        R.ym   = hy ? -cym * inv : 0.f;
+        R.yp   = ly < 7 || nb[3] >= 0 ? -cyp * inv : 0.f;
+        R.zp   = lz < 7 || nb[5] >= 0 ? -czp * inv : 0.f;
+        R.in   = lx & 1 ? xm : xp;
+        R.out  = lx & 1 ? xp : xm;
+        R.bs   = 0.f;
         return R;
     }
-    static __device__ __forceinline__ float off_sum(const Row& R, const float* x) {
-        float acc = 0.f;
-        acc += R.czm * x[-100];
-        acc += R.cym * x[-10];
-        acc += R.cxm * x[-1];
-        acc += R.cxp * x[1];
-        acc += R.cyp * x[10];
-        acc += R.czp * x[100];
-        return acc;
+    // b/d - sum (a/d) x over the neighbours of the cell at x; pair: the other cell of its pair, off: the
+    // offset out of the pair
+    static __device__ __forceinline__ float solved(const Row& R, const float* x, int off, float pair) {
+        const float p = __builtin_fmaf(R.out, x[off], __builtin_fmaf(R.ym, x[-10], __builtin_fmaf(R.zm, x[-100], R.bs)));
+        return p + __builtin_fmaf(R.zp, x[100], __builtin_fmaf(R.yp, x[10], R.in * pair));
     }
-    // one half-sweep over the group's n bricks (4 tiles apart): cells of one colour read only the other
-    template<int kTurns> static __device__ __forceinline__ void half(const Row* R, float* x, int n) {
-        float v[kTurns];
+    // one half-sweep over the group's n bricks (4 tiles apart): cells of one colour read only the other.
+    // own: the cells' values, pair: those of the other colour
+    template<int kTurns> static __device__ __forceinline__ void half(const Row* R, float* x, int off, float* own, const float* pair, int n) {
 #pragma unroll
         for(int q = 0; q < kTurns; ++q)
-            if(q < n) v[q] = (R[q].bv - off_sum(R[q], x + 4000 * q)) * R[q].inv;
+            if(q < n) own[q] = solved(R[q], x + 4000 * q, off, pair[q]);
 #pragma unroll
         for(int q = 0; q < kTurns; ++q)
-            if(q < n) x[4000 * q] = v[q];
+            if(q < n) x[4000 * q] = own[q];
     }
     // the tiles' halos from the neighbouring bricks (0 where there is none)
     static __device__ __forceinline__ void halos(float* xs, const int32_t (*nb)[8], int nSlots) {
@@ -3135,7 +3137,7 @@ struct k_mg_tail {
     }
     // the thread's pair of cells: local indices of the red (colour 0) and the black one, their tile entries
     struct Pair {
-        int  ly, lz, px, lr, lb, cr, cb;
+        int  ly, lz, px, lr, lb, cr, cb, offR, offB;  // offR, offB: tile offsets out of the pair
         // the parent of the pair's 2x2x2 group in the parent brick, for a brick with coordinate parities odd
         __device__ __forceinline__ int parent(int odd) const {
             return (((odd >> 2 & 1) * 4 + lz / 2) * 8 + (odd >> 1 & 1) * 4 + ly / 2) * 8 + (odd & 1) * 4 + px;
@@ -3147,11 +3149,12 @@ struct k_mg_tail {
     __device__ __forceinline__ void down(const Row* R, const Row* K, const Pair& c, float* xs, const int32_t (*nb)[8], int S, int grp, const LevelDev& C) const {
         const int n = (S - grp + 3) >> 2;  // bricks grp, grp + 4, ..
         float*    x = xs + 1000 * grp;
+        float     vr[kTurns] = {}, vb[kTurns] = {};
         __syncthreads();
         for(int it = 0; it < sweeps; ++it) {
-            half<kTurns>(R, x + c.cr, n);
+            half<kTurns>(R, x + c.cr, c.offR, vr, vb, n);
             __syncthreads();
-            half<kTurns>(K, x + c.cb, n);
+            half<kTurns>(K, x + c.cb, c.offB, vb, vr, n);
             __syncthreads();
         }
         halos(xs, nb, S);
@@ -3160,8 +3163,8 @@ struct k_mg_tail {
         for(int q = 0; q < kTurns; ++q)
             if(q < n) {
                 const float* y  = x + 4000 * q;
-                const float  rr = R[q].bv - (R[q].diag * y[c.cr] + off_sum(R[q], y + c.cr));
-                const float  rk = K[q].bv - (K[q].diag * y[c.cb] + off_sum(K[q], y + c.cb));
+                const float  rr = R[q].diag * (solved(R[q], y + c.cr, c.offR, vb[q]) - vr[q]);
+                const float  rk = K[q].diag * (solved(K[q], y + c.cb, c.offB, vr[q]) - vb[q]);
                 // the x pair is this thread's, the odd y lies in lane ^ 4, the odd z in lane ^ 32
                 const float e0 = c.lr < c.lb ? rr : rk, e1 = c.lr < c.lb ? rk : rr;
                 const float y0 = __shfl_xor(e0, 4), y1 = __shfl_xor(e1, 4);
@@ -3181,24 +3184,27 @@ struct k_mg_tail {
     __device__ __forceinline__ void up(const Row* R, const Row* K, const Pair& c, float* xs, const int32_t (*nb)[8], int S, int grp) const {
         const int n = (S - grp + 3) >> 2;
         float*    x = xs + 1000 * grp;
+        float     vr[kTurns] = {}, vb[kTurns] = {};
 #pragma unroll
         for(int q = 0; q < kTurns; ++q)
             if(q < n) {
                 const int par = nb[grp + 4 * q][6];
+                float*    y   = x + 4000 * q;
+                vr[q]         = y[c.cr];
+                vb[q]         = y[c.cb];
                 if(par >= 0) {
                     const float xc = xs[1000 * (S + par) + tile_at(c.parent(nb[grp + 4 * q][7]))];
-                    float*      y  = x + 4000 * q;
-                    if(R[q].inv != 0.f) y[c.cr] = y[c.cr] + omega * xc;
-                    if(K[q].inv != 0.f) y[c.cb] = y[c.cb] + omega * xc;
+                    if(R[q].diag > 0.f) y[c.cr] = vr[q] = vr[q] + omega * xc;
+                    if(K[q].diag > 0.f) y[c.cb] = vb[q] = vb[q] + omega * xc;
                 }
             }
         __syncthreads();
         halos(xs, nb, S);
         __syncthreads();
         for(int it = 0; it < sweeps; ++it) {
-            half<kTurns>(K, x + c.cb, n);
+            half<kTurns>(K, x + c.cb, c.offB, vb, vr, n);
             __syncthreads();
-            half<kTurns>(R, x + c.cr, n);
+            half<kTurns>(R, x + c.cr, c.offR, vr, vb, n);
             __syncthreads();
         }
     }
@@ -3206,7 +3212,9 @@ struct k_mg_tail {
         __shared__ float   xs[kTiles * 1000];
         __shared__ int32_t nb[kTiles][8];  // per brick: six neighbour slots, parent slot, parities of its coordinates
         if(st && st->done) return;
-        const int t = threadIdx.x, grp = t >> 8, tt = t & 255;
+        int t = threadIdx.x;
+        asm volatile("" : "+v"(t));  // keeps the batched form's loop over scenes from holding the lane's constants in registers
+        const int grp = t >> 8, tt = t & 255;
         Pair      c;
         c.ly = (tt >> 2) & 7;
         c.lz = tt >> 5;
@@ -3216,6 +3224,8 @@ struct k_mg_tail {
         c.lb = l0 + 1 - o0;
         c.cr = tile_at(c.lr);
         c.cb = tile_at(c.lb);
+        c.offR = c.lr & 1 ? 1 : -1;
+        c.offB = -c.offR;
         int base = 0;
         for(int l = 0; l < nLev; ++l) {
             const int S = (int)lv[l].nSlots;
@@ -3228,15 +3238,15 @@ struct k_mg_tail {
         for(int e = t; e < base * 1000; e += kThreads) xs[e] = 0.f;
         __syncthreads();
         const int S0 = nLev > 1 ? (int)lv[0].nSlots : 0;
-        Row       R0[2], K0[2], R1[1], K1[1];
+        Row       R0[2], K0[2], R1[1], K1[1], RC, KC;  // the first level, the second (or a later one), the coarsest
 #pragma unroll
         for(int q = 0; q < 2; ++q) {
             const int s = grp + 4 * q;
             if(s < S0) {
-                R0[q]    = row(lv[0], nb[s], s, c.lr);
-                K0[q]    = row(lv[0], nb[s], s, c.lb);
-                R0[q].bv = lv[0].b[s * 512 + c.lr];
-                K0[q].bv = lv[0].b[s * 512 + c.lb];
+                R0[q] = row(lv[0], nb[s], s, c.lr);
+                K0[q] = row(lv[0], nb[s], s, c.lb);
+                R0[q].rhs(lv[0].b[s * 512 + c.lr]);
+                K0[q].rhs(lv[0].b[s * 512 + c.lb]);
             }
         }
         auto rows = [&](int l, int at) {
@@ -3245,58 +3255,64 @@ struct k_mg_tail {
                 K1[0] = row(lv[l], nb[at + grp], grp, c.lb);
             }
         };
-        auto take = [&](int l, int at) {  // the right-hand side that the finer level left in the tile; x starts from 0
-            if(grp < (int)lv[l].nSlots) {
-                float* x = xs + 1000 * (at + grp);
-                R1[0].bv = x[c.cr];
-                K1[0].bv = x[c.cb];
-                x[c.cr] = x[c.cb] = 0.f;
-            }
+        // the right-hand side that the finer level left in the tile; x starts from 0
+        auto take = [&](Row& R, Row& K, int at) {
+            float* x = xs + 1000 * at;
+            R.rhs(x[c.cr]);
+            K.rhs(x[c.cb]);
+            x[c.cr] = x[c.cb] = 0.f;
         };
-        rows(nLev > 1 ? 1 : 0, S0);
+        const int last = nLev - 1, lastAt = base - 1;  // the coarsest level's only tile
+        if(nLev > 2) rows(1, S0);
+        if(grp == 0) {
+            RC = row(lv[last], nb[lastAt], 0, c.lr);
+            KC = row(lv[last], nb[lastAt], 0, c.lb);
+        }
         if(nLev > 1) down<2>(R0, K0, c, xs, nb, S0, grp, lv[1]);
         base = S0;
-        for(int l = 1; l + 1 < nLev; ++l) {
+        for(int l = 1; l < last; ++l) {
             const int S = (int)lv[l].nSlots;
             if(l > 1) rows(l, base);
-            take(l, base);
+            if(grp < S) take(R1[0], K1[0], base + grp);
             down<1>(R1, K1, c, xs + 1000 * base, nb + base, S, grp, lv[l + 1]);
             base += S;
         }
         {  // coarsest level, one brick
             const int n = grp == 0 ? 1 : 0;
-            float*    x = xs + 1000 * base;
-            if(nLev > 2) rows(nLev - 1, base);
-            if(nLev > 1) take(nLev - 1, base);
+            float*    x = xs + 1000 * lastAt;
+            float     vr[1] = {0.f}, vb[1] = {0.f};
+            if(n && nLev > 1) take(RC, KC, lastAt);
             else if(n) {
-                R1[0].bv = lv[0].b[c.lr];
-                K1[0].bv = lv[0].b[c.lb];
+                RC.rhs(lv[0].b[c.lr]);
+                KC.rhs(lv[0].b[c.lb]);
             }
             __syncthreads();
             for(int it = 0; it < coarsest; ++it) {
-                half<1>(R1, x + c.cr, n);
+                half<1>(&RC, x + c.cr, c.offR, vr, vb, n);
                 __syncthreads();
-                half<1>(K1, x + c.cb, n);
+                half<1>(&KC, x + c.cb, c.offB, vb, vr, n);
                 __syncthreads();
             }
             for(int it = 0; it < coarsest; ++it) {
-                half<1>(K1, x + c.cb, n);
+                half<1>(&KC, x + c.cb, c.offB, vb, vr, n);
                 __syncthreads();
-                half<1>(R1, x + c.cr, n);
+                half<1>(&RC, x + c.cr, c.offR, vr, vb, n);
                 __syncthreads();
             }
             if(n && nLev == 1) {
-                lv[0].x[c.lr] = x[c.cr];
-                lv[0].x[c.lb] = x[c.cb];
+                lv[0].x[c.lr] = vr[0];
+                lv[0].x[c.lb] = vb[0];
             }
         }
-        for(int l = nLev - 2; l >= 1; --l) {
+        for(int l = last - 1; l >= 1; --l) {
             const int S = (int)lv[l].nSlots;
             base -= S;
-            rows(l, base);
-            if(grp < S) {
-                R1[0].bv = lv[l].b[grp * 512 + c.lr];
-                K1[0].bv = lv[l].b[grp * 512 + c.lb];
+            if(last > 2 && l < last - 1) {  // the way down used the registers for a later level
+                rows(l, base);
+                if(grp < S) {
+                    R1[0].rhs(lv[l].b[grp * 512 + c.lr]);
+                    K1[0].rhs(lv[l].b[grp * 512 + c.lb]);
+                }
             }
             up<1>(R1, K1, c, xs + 1000 * base, nb + base, S, grp);
         }

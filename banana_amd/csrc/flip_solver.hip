@@ -1136,10 +1136,12 @@ public:
         // max|b| since x starts at 0
         uint32_t chunk = pcgChunkFirst, launched = 0;
         // alone, with the multigrid: as many as the last inner solve's mean reduction says (its system was the
-        // same one or the previous substep's); each wait saved is 10 to 20 us of an idle GPU, and an iteration
-        // too many costs about as much
-        if(fuseUpdate && !rec && pcgRate < 0.0 && relTol > 0.f && relTol < 1.f)
-            chunk = (uint32_t)std::min(std::max(std::ceil(std::log((double)relTol) / pcgRate), 1.0), (double)pcgChunkMax);
+        // same one or the previous substep's). A wait costs 15 to 20 us of an idle GPU, the empty launches of
+        // an iteration too many 15 us at 64^3 and 35 at 256^3: rounded up on small systems, else down.
+        if(fuseUpdate && !rec && pcgRate < 0.0 && relTol > 0.f && relTol < 1.f) {
+            const double need = std::log((double)relTol) / pcgRate;
+            chunk = (uint32_t)std::min(std::max(folded ? std::ceil(need) : std::floor(need), 1.0), (double)pcgChunkMax);
+        }
         for(bool first = true;; first = false) {
             if(!first) {
                 if(rec) {
