@@ -945,9 +945,11 @@ public:
                 L.nbr.reserve((size_t)c * 24);
                 L.slotCap = c;
             }
-            // the finer level's parent table (its bricks' parents in this level)
+            // the finer level's parent table (its bricks' parents in this level), as large as that level's
+            // other buffers: sized by its bricks it was freed and allocated, with a wait for the device (and a
+            // flush of the whole batch), at every substep that added one
             DevBuf& pt = l == 1 ? ptab0 : mg[l - 1]->ptab;
-            pt.reserve((size_t)std::max<uint32_t>(prevSlots, 1u) * 32);
+            pt.reserve((size_t)(l == 1 ? slotCap : mg[l - 1]->slotCap) * 32);
             prevSlots = L.nSlots;
             ++mgLevels;
         }
