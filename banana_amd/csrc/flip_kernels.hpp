@@ -2653,6 +2653,13 @@ __device__ __forceinline__ float mg_prolonged(const LevelDev& F, const float* __
     return un ? xv + omega * xc : xv;
 }
 
+// A brick's x with its one-cell halo in LDS (smoothers), x fastest. Rows of 12 and planes of 120 floats
+// where 10 and 100 would do: a wave's accesses in a half-sweep (4 cells two apart in 8 rows of two planes)
+// then fall on different banks, against two to a bank (a half-sweep of k_mg_tail over 8 bricks: 1110 ->
+// 700 cycles).
+constexpr int kTileRow = 12, kTilePlane = 120, kTile = 1200;
+__device__ __forceinline__ int tile_index(int lx, int ly, int lz) { return (lz + 1) * kTilePlane + (ly + 1) * kTileRow + lx + 1; }
+
 // One cell of the brick smoother: its LDS index and its row of A, divided by the diagonal and with the sign
 // of the update x = b/d - sum (a/d) x (a coupling to a missing neighbour is 0 and that neighbour's halo
 // entry holds 0, so all six terms are added unconditionally). The thread owns an x-adjacent pair of cells,
@@ -2668,7 +2675,7 @@ template<int kProlong>
 __device__ __forceinline__ SmoothCell smooth_cell_setup(const LevelDev& L, const LevelDev& C, int32_t parent, float omega, int s, int l,
                                                         int bx, int by, int bz, float* xs, float& bv, bool uni) {
     const int     lx = l & 7, ly = (l >> 3) & 7, lz = l >> 6;
-    const int     c  = ((lz + 1) * 10 + (ly + 1)) * 10 + (lx + 1);
+    const int     c  = tile_index(lx, ly, lz);
     const size_t  o  = (size_t)s * 512 + l;
     const int32_t ixm = nbr_index(L.nbr, s, l, 0), ixp = nbr_index(L.nbr, s, l, 1);
     const int32_t iym = nbr_index(L.nbr, s, l, 2), iyp = nbr_index(L.nbr, s, l, 3);
@@ -2722,7 +2729,7 @@ __device__ __forceinline__ void smooth_halo(const LevelDev& L, const LevelDev& C
             lz = d == 4 ? 0 : 7;
         }
         const int sx = d == 0 ? -1 : d == 1 ? 1 : 0, sy = d == 2 ? -1 : d == 3 ? 1 : 0, sz = d == 4 ? -1 : d == 5 ? 1 : 0;
-        const int c  = ((lz + 1 + sz) * 10 + (ly + 1 + sy)) * 10 + (lx + 1 + sx);
+        const int c  = tile_index(lx + sx, ly + sy, lz + sz);
         float     v  = 0.f;
         if(kProlong == 2) {
             const int32_t n = nbr_index(L.nbr, s, (lz * 8 + ly) * 8 + lx, d);
@@ -2744,8 +2751,8 @@ __device__ __forceinline__ void smooth_halo(const LevelDev& L, const LevelDev& C
 
 // the cell's new value; pair: the other cell of its pair
 __device__ __forceinline__ float smooth_cell_update(const SmoothCell& R, float* xs, float pair) {
-    const float p = __builtin_fmaf(R.out, xs[R.c + R.off], __builtin_fmaf(R.ym, xs[R.c - 10], __builtin_fmaf(R.zm, xs[R.c - 100], R.bs)));
-    const float v = p + __builtin_fmaf(R.zp, xs[R.c + 100], __builtin_fmaf(R.yp, xs[R.c + 10], R.in * pair));
+    const float p = __builtin_fmaf(R.out, xs[R.c + R.off], __builtin_fmaf(R.ym, xs[R.c - kTileRow], __builtin_fmaf(R.zm, xs[R.c - kTilePlane], R.bs)));
+    const float v = p + __builtin_fmaf(R.zp, xs[R.c + kTilePlane], __builtin_fmaf(R.yp, xs[R.c + kTileRow], R.in * pair));
     xs[R.c]       = v;
     return v;
 }
@@ -2832,7 +2839,7 @@ struct k_mg_smooth_brick {
     const PcgState* __restrict__ st;
     double* __restrict__ pz;
     __device__ void operator()(Blk blk) const {
-        __shared__ float xs[10 * 10 * 10];  // the brick and a one-cell halo, x-fastest
+        __shared__ float xs[kTile];  // the brick and a one-cell halo
         __shared__ double sh[4];
         if(st && st->done) return;
         for(uint32_t v = blk.id; v < L.nSlots; v += blk.n)
@@ -2859,7 +2866,7 @@ struct k_pcg_update_pre {
     const double* __restrict__ sq;
     int nPart;
     __device__ void operator()(Blk blk) const {
-        __shared__ float  xs[10 * 10 * 10];
+        __shared__ float  xs[kTile];
         __shared__ double sh[8];
         if(st->done) return;
         const int t     = threadIdx.x;
@@ -3143,8 +3150,12 @@ namespace bnn {
 // coarsest are loaded once, at the start. Four groups of 256 threads own a brick each (on lv[0] up to two in turn;
 // thread = an x-adjacent pair of cells, one of each colour). The steps are those of k_mg_smooth_brick and
 // k_mg_residual_restrict; coarsest level: x = 0, `coarsest` red-black and as many black-red sweeps. Input
-// lv[0].b, output lv[0].x. Bound by the chain of half-sweeps (32 of them on the coarsest level): 16 us for
-// two levels, 25 for three, against 27 and 42 in separate kernels plus 4 or 7 launches.
+// lv[0].b, output lv[0].x. The first red half-sweep from x = 0 and the black one that would repeat the one
+// before it are left out. Bound by what four waves a SIMD issue (16 cycles an instruction on lv[0]) and by
+// the chain of half-sweeps (260 cycles each on the coarsest level): so pairs of coefficients are loaded as
+// one, tables and own coefficients before anything waits, a halo's face and neighbour are scalars. 13 us
+// for two levels, 20 for three (16 and 25 before that and the tile's strides), against 27 and 42 in
+// separate kernels plus 4 or 7 launches.
 struct k_mg_tail {
     static constexpr int kThreads = 1024;
     static constexpr int kLevels = 5, kTop = 8, kRest = 4, kTiles = 16;  // levels; bricks on lv[0], on each other level, in all
@@ -3159,75 +3170,97 @@ struct k_mg_tail {
         float zm, ym, out, in, yp, zp, bs, diag;
         __device__ __forceinline__ void rhs(float b) { bs = diag > 0.f ? b / diag : 0.f; }
     };
-    static __device__ __forceinline__ int tile_at(int l) { return (((l >> 6) + 1) * 10 + ((l >> 3) & 7) + 1) * 10 + (l & 7) + 1; }
-    // nb: the brick's six neighbour slots
-    static __device__ __forceinline__ Row row(const LevelDev& L, const int32_t* nb, int s, int l) {
-        const int     lx = l & 7, ly = (l >> 3) & 7, lz = l >> 6;
-        const int32_t o = s * 512 + l;
+    static __device__ __forceinline__ int tile_at(int l) { return tile_index(l & 7, (l >> 3) & 7, l >> 6); }
+    // the thread's pair of cells: local indices of the red (colour 0) and the black one, their tile entries
+    struct Pair {
+        int  ly, lz, px, le, lr, lb, cr, cb, offR, offB;  // le: the even one; offR, offB: tile offsets out of the pair
+        // the parent of the pair's 2x2x2 group in the parent brick, for a brick with coordinate parities odd
+        __device__ __forceinline__ int parent(int odd) const {
+            return (((odd >> 2 & 1) * 4 + lz / 2) * 8 + (odd >> 1 & 1) * 4 + ly / 2) * 8 + (odd & 1) * 4 + px;
+        }
+    };
+    // the x-adjacent pair's own coefficients, a load each (the even cell's offset is even)
+    struct Own {
+        float2 diag, inv, cx, cy, cz;
+    };
+    static __device__ __forceinline__ float2 two(const float* __restrict__ v, int32_t o) { return *(const float2*)(v + o); }
+    static __device__ __forceinline__ Own own(const LevelDev& L, int32_t o) {
+        return Own{two(L.diag, o), two(L.invdiag, o), two(L.cx, o), two(L.cy, o), two(L.cz, o)};
+    }
+    // the rows of the pair's red and black cell; nb: the brick's six neighbour slots
+    static __device__ __forceinline__ void rows(const LevelDev& L, const int32_t* nb, const Own& w, int32_t s, const Pair& c, Row& R, Row& K) {
+        const int     l  = c.le;
+        const int32_t o  = s * 512 + l;
         const int32_t nx = nb[0], ny = nb[2], nz = nb[4];
-        const bool    hx = lx > 0 || nx >= 0, hy = ly > 0 || ny >= 0, hz = lz > 0 || nz >= 0;
-        const int32_t ix = lx > 0 ? o - 1 : (hx ? nx * 512 + l + 7 : o), iy = ly > 0 ? o - 8 : (hy ? ny * 512 + l + 56 : o),
-                      iz = lz > 0 ? o - 64 : (hz ? nz * 512 + l + 448 : o);
-        const float czm = L.cz[iz], cym = L.cy[iy], cxm = L.cx[ix], cxp = L.cx[o], cyp = L.cy[o], czp = L.cz[o], inv = L.invdiag[o];
-        const float xm = hx ? -cxm * inv : 0.f, xp = lx < 7 || nb[1] >= 0 ? -cxp * inv : 0.f;
-        Row         R;
-        R.diag = L.diag[o];
-        R.zm   = hz ? -czm * inv : 0.f;
-        R.ym   = hy ? -cym * inv : 0.f;
-        R.yp   = ly < 7 || nb[3] >= 0 ? -cyp * inv : 0.f;
-        R.zp   = lz < 7 || nb[5] >= 0 ? -czp * inv : 0.f;
-        R.in   = lx & 1 ? xm : xp;
-        R.out  = lx & 1 ? xp : xm;
-        R.bs   = 0.f;
-        return R;
+        const bool    hx = c.px > 0 || nx >= 0, hy = c.ly > 0 || ny >= 0, hz = c.lz > 0 || nz >= 0;
+        const float   cxm = L.cx[c.px > 0 ? o - 1 : (hx ? nx * 512 + l + 7 : o)];
+        const float2  cym = two(L.cy, c.ly > 0 ? o - 8 : (hy ? ny * 512 + l + 56 : o));
+        const float2  czm = two(L.cz, c.lz > 0 ? o - 64 : (hz ? nz * 512 + l + 448 : o));
+        const bool    hX = c.px < 3 || nb[1] >= 0, hY = c.ly < 7 || nb[3] >= 0, hZ = c.lz < 7 || nb[5] >= 0;
+        const Row     E{hz ? -czm.x * w.inv.x : 0.f, hy ? -cym.x * w.inv.x : 0.f, hx ? -cxm * w.inv.x : 0.f, -w.cx.x * w.inv.x,
+                    hY ? -w.cy.x * w.inv.x : 0.f, hZ ? -w.cz.x * w.inv.x : 0.f, 0.f, w.diag.x};
+        const Row     O{hz ? -czm.y * w.inv.y : 0.f, hy ? -cym.y * w.inv.y : 0.f, hX ? -w.cx.y * w.inv.y : 0.f, -w.cx.x * w.inv.y,
+                    hY ? -w.cy.y * w.inv.y : 0.f, hZ ? -w.cz.y * w.inv.y : 0.f, 0.f, w.diag.y};
+        R = c.lr == c.le ? E : O;
+        K = c.lr == c.le ? O : E;
     }
     // b/d - sum (a/d) x over the neighbours of the cell at x; pair: the other cell of its pair, off: the
     // offset out of the pair
     static __device__ __forceinline__ float solved(const Row& R, const float* x, int off, float pair) {
-        const float p = __builtin_fmaf(R.out, x[off], __builtin_fmaf(R.ym, x[-10], __builtin_fmaf(R.zm, x[-100], R.bs)));
-        return p + __builtin_fmaf(R.zp, x[100], __builtin_fmaf(R.yp, x[10], R.in * pair));
+        const float p = __builtin_fmaf(R.out, x[off], __builtin_fmaf(R.ym, x[-kTileRow], __builtin_fmaf(R.zm, x[-kTilePlane], R.bs)));
+        return p + __builtin_fmaf(R.zp, x[kTilePlane], __builtin_fmaf(R.yp, x[kTileRow], R.in * pair));
     }
     // one half-sweep over the group's n bricks (4 tiles apart): cells of one colour read only the other.
     // own: the cells' values, pair: those of the other colour
     template<int kTurns> static __device__ __forceinline__ void half(const Row* R, float* x, int off, float* own, const float* pair, int n) {
 #pragma unroll
         for(int q = 0; q < kTurns; ++q)
-            if(q < n) own[q] = solved(R[q], x + 4000 * q, off, pair[q]);
+            if(q < n) own[q] = solved(R[q], x + 4 * kTile * q, off, pair[q]);
 #pragma unroll
         for(int q = 0; q < kTurns; ++q)
-            if(q < n) x[4000 * q] = own[q];
+            if(q < n) x[4 * kTile * q] = own[q];
     }
-    // the tiles' halos from the neighbouring bricks (0 where there is none)
-    static __device__ __forceinline__ void halos(float* xs, const int32_t (*nb)[8], int nSlots) {
-        for(int h = threadIdx.x; h < 384 * nSlots; h += kThreads) {
-            const int s = h / 384, d = (h - 384 * s) >> 6, p = h & 63, a = p & 7, e = p >> 3;
-            // the halo entry, and the cell it mirrors in the neighbour's tile
-            const int     to = d < 2 ? ((e + 1) * 10 + a + 1) * 10 + (d == 0 ? 0 : 9)
-                                     : (d < 4 ? ((e + 1) * 10 + (d == 2 ? 0 : 9)) * 10 + a + 1 : ((d == 4 ? 0 : 9) * 10 + e + 1) * 10 + a + 1);
-            const int     step = (d < 2 ? 1 : (d < 4 ? 10 : 100)) * ((d & 1) ? -8 : 8);
-            const int32_t n    = nb[s][d];
-            xs[1000 * s + to]  = n >= 0 ? xs[1000 * n + to + step] : 0.f;
+    // the first red half-sweep, from x = 0
+    template<int kTurns> static __device__ __forceinline__ void first(const Row* R, float* x, float* own, int n) {
+#pragma unroll
+        for(int q = 0; q < kTurns; ++q)
+            if(q < n) x[4 * kTile * q] = own[q] = R[q].bs;
+    }
+    // the tiles' halos from the neighbouring bricks (where there is none they stay 0): a wave a face, so the
+    // face and its neighbour are scalars
+    static __device__ __forceinline__ void halos(float* xs, const int32_t (*nb)[8], int S) {
+        constexpr int kWaves = kThreads / 64, kFaces = 6 * kTop / kWaves;
+        const int     w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), a = threadIdx.x & 7, e = threadIdx.x >> 3 & 7;
+        int32_t       n[kFaces];
+#pragma unroll
+        for(int q = 0; q < kFaces; ++q) {
+            const int f = w + kWaves * q;
+            n[q]        = f < 6 * S ? nb[f / 6][f % 6] : -1;
+        }
+#pragma unroll
+        for(int q = 0; q < kFaces; ++q) {
+            const int f = w + kWaves * q, s = f / 6, d = f % 6, m = __builtin_amdgcn_readfirstlane(n[q]);
+            if(m < 0) continue;
+            // along the face's two axes; across it the halo entry and, step further, the cell it mirrors
+            const int sa = d < 2 ? kTileRow : 1, se = d < 4 ? kTilePlane : kTileRow, sd = d < 2 ? 1 : (d < 4 ? kTileRow : kTilePlane);
+            const int to = (1 + a) * sa + (1 + e) * se + (d & 1 ? 9 : 0) * sd;
+            xs[kTile * s + to] = xs[kTile * m + (d & 1 ? -8 : 8) * sd + to];
         }
     }
-    // the thread's pair of cells: local indices of the red (colour 0) and the black one, their tile entries
-    struct Pair {
-        int  ly, lz, px, lr, lb, cr, cb, offR, offB;  // offR, offB: tile offsets out of the pair
-        // the parent of the pair's 2x2x2 group in the parent brick, for a brick with coordinate parities odd
-        __device__ __forceinline__ int parent(int odd) const {
-            return (((odd >> 2 & 1) * 4 + lz / 2) * 8 + (odd >> 1 & 1) * 4 + ly / 2) * 8 + (odd & 1) * 4 + px;
-        }
-    };
     // pre-smoother from x = 0 on the level's tiles, then the residual's 2x2x2 sums to the next level's tiles
     // (its right-hand side) and to its b (for the way up)
     template<int kTurns>
     __device__ __forceinline__ void down(const Row* R, const Row* K, const Pair& c, float* xs, const int32_t (*nb)[8], int S, int grp, const LevelDev& C) const {
         const int n = (S - grp + 3) >> 2;  // bricks grp, grp + 4, ..
-        float*    x = xs + 1000 * grp;
+        float*    x = xs + kTile * grp;
         float     vr[kTurns] = {}, vb[kTurns] = {};
+        first<kTurns>(R, x + c.cr, vr, n);
         __syncthreads();
         for(int it = 0; it < sweeps; ++it) {
-            half<kTurns>(R, x + c.cr, c.offR, vr, vb, n);
-            __syncthreads();
+            if(it) {
+                half<kTurns>(R, x + c.cr, c.offR, vr, vb, n);
+                __syncthreads();
+            }
             half<kTurns>(K, x + c.cb, c.offB, vb, vr, n);
             __syncthreads();
         }
@@ -3236,18 +3269,15 @@ struct k_mg_tail {
 #pragma unroll
         for(int q = 0; q < kTurns; ++q)
             if(q < n) {
-                const float* y  = x + 4000 * q;
+                const float* y  = x + 4 * kTile * q;
                 const float  rr = R[q].diag * (solved(R[q], y + c.cr, c.offR, vb[q]) - vr[q]);
                 const float  rk = K[q].diag * (solved(K[q], y + c.cb, c.offB, vr[q]) - vb[q]);
                 // the x pair is this thread's, the odd y lies in lane ^ 4, the odd z in lane ^ 32
-                const float e0 = c.lr < c.lb ? rr : rk, e1 = c.lr < c.lb ? rk : rr;
-                const float y0 = __shfl_xor(e0, 4), y1 = __shfl_xor(e1, 4);
-                const float z0 = __shfl_xor(e0, 32), z1 = __shfl_xor(e1, 32), w0 = __shfl_xor(y0, 32), w1 = __shfl_xor(y1, 32);
+                const float e = rr + rk, ey = e + __shfl_xor(e, 4), sum = ey + __shfl_xor(ey, 32);
                 const int   par = nb[grp + 4 * q][6];
                 if(!(c.ly & 1) && !(c.lz & 1) && par >= 0) {
-                    const float sum = ((((((e0 + e1) + y0) + y1) + z0) + z1) + w0) + w1;
                     const int   cl  = c.parent(nb[grp + 4 * q][7]);
-                    xs[1000 * (S + par) + tile_at(cl)] = sum;
+                    xs[kTile * (S + par) + tile_at(cl)] = sum;
                     C.b[par * 512 + cl]                = sum;
                 }
             }
@@ -3257,17 +3287,17 @@ struct k_mg_tail {
     template<int kTurns>
     __device__ __forceinline__ void up(const Row* R, const Row* K, const Pair& c, float* xs, const int32_t (*nb)[8], int S, int grp) const {
         const int n = (S - grp + 3) >> 2;
-        float*    x = xs + 1000 * grp;
+        float*    x = xs + kTile * grp;
         float     vr[kTurns] = {}, vb[kTurns] = {};
 #pragma unroll
         for(int q = 0; q < kTurns; ++q)
             if(q < n) {
                 const int par = nb[grp + 4 * q][6];
-                float*    y   = x + 4000 * q;
+                float*    y   = x + 4 * kTile * q;
                 vr[q]         = y[c.cr];
                 vb[q]         = y[c.cb];
                 if(par >= 0) {
-                    const float xc = xs[1000 * (S + par) + tile_at(c.parent(nb[grp + 4 * q][7]))];
+                    const float xc = xs[kTile * (S + par) + tile_at(c.parent(nb[grp + 4 * q][7]))];
                     if(R[q].diag > 0.f) y[c.cr] = vr[q] = vr[q] + omega * xc;
                     if(K[q].diag > 0.f) y[c.cb] = vb[q] = vb[q] + omega * xc;
                 }
@@ -3283,9 +3313,8 @@ struct k_mg_tail {
         }
     }
     __device__ void operator()(Blk) const {
-        __shared__ float   xs[kTiles * 1000];
+        __shared__ __align__(16) float xs[kTiles * kTile];
         __shared__ int32_t nb[kTiles][8];  // per brick: six neighbour slots, parent slot, parities of its coordinates
-        if(st && st->done) return;
         int t = threadIdx.x;
         asm volatile("" : "+v"(t));  // keeps the batched form's loop over scenes from holding the lane's constants in registers
         const int grp = t >> 8, tt = t & 255;
@@ -3293,83 +3322,106 @@ struct k_mg_tail {
         c.ly = (tt >> 2) & 7;
         c.lz = tt >> 5;
         c.px = tt & 3;
-        const int l0 = (c.lz * 8 + c.ly) * 8 + 2 * c.px, o0 = (c.ly + c.lz) & 1;  // even x; its colour
-        c.lr = l0 + o0;
-        c.lb = l0 + 1 - o0;
+        c.le = (c.lz * 8 + c.ly) * 8 + 2 * c.px;
+        const int o0 = (c.ly + c.lz) & 1;  // the even cell's colour
+        c.lr = c.le + o0;
+        c.lb = c.le + 1 - o0;
         c.cr = tile_at(c.lr);
         c.cb = tile_at(c.lb);
         c.offR = c.lr & 1 ? 1 : -1;
         c.offB = -c.offR;
-        int base = 0;
-        for(int l = 0; l < nLev; ++l) {
-            const int S = (int)lv[l].nSlots;
-            if(t < 8 * S) {
-                const int s = t >> 3, d = t & 7;
-                nb[base + s][d] = d < 6 ? lv[l].nbr[6 * s + d] : (l + 1 < nLev ? lv[l].ptab[8 * s + d] : -1);
+        // the brick tables and the pairs' own coefficients of the first two levels and the coarsest, before
+        // anything waits: the lower neighbours' follow when the tables are in LDS
+        int32_t tab[kLevels];
+#pragma unroll
+        for(int l = 0; l < kLevels; ++l) {
+            const int s = t >> 3, d = t & 7;
+            tab[l] = -1;
+            if(l < nLev && s < (int)lv[l].nSlots) {
+                if(d < 6) tab[l] = lv[l].nbr[6 * s + d];
+                else if(l + 1 < nLev) tab[l] = lv[l].ptab[8 * s + d];
             }
-            base += S;
         }
-        for(int e = t; e < base * 1000; e += kThreads) xs[e] = 0.f;
+        const int last = nLev - 1;
+        const int S0   = nLev > 1 ? (int)lv[0].nSlots : 0;
+        Own       own0[2], own1, ownC;
+        float2    b0[2];
+#pragma unroll
+        for(int q = 0; q < 2; ++q)
+            if(grp + 4 * q < S0) {
+                own0[q] = own(lv[0], (grp + 4 * q) * 512 + c.le);
+                b0[q]   = two(lv[0].b, (grp + 4 * q) * 512 + c.le);
+            }
+        if(nLev > 2 && grp < (int)lv[1].nSlots) own1 = own(lv[1], grp * 512 + c.le);
+        if(grp == 0) ownC = own(lv[last], c.le);
+        if(st && st->done) return;
+        int base = 0;
+#pragma unroll
+        for(int l = 0; l < kLevels; ++l)
+            if(l < nLev) {
+                const int S = (int)lv[l].nSlots;
+                if(t < 8 * S) nb[base + (t >> 3)][t & 7] = tab[l];
+                base += S;
+            }
+        for(int e = t; e < base * (kTile / 4); e += kThreads) ((float4*)xs)[e] = make_float4(0.f, 0.f, 0.f, 0.f);
         __syncthreads();
-        const int S0 = nLev > 1 ? (int)lv[0].nSlots : 0;
-        Row       R0[2], K0[2], R1[1], K1[1], RC, KC;  // the first level, the second (or a later one), the coarsest
+        Row R0[2], K0[2], R1[1], K1[1], RC, KC;  // the first level, the second (or a later one), the coarsest
 #pragma unroll
         for(int q = 0; q < 2; ++q) {
             const int s = grp + 4 * q;
             if(s < S0) {
-                R0[q] = row(lv[0], nb[s], s, c.lr);
-                K0[q] = row(lv[0], nb[s], s, c.lb);
-                R0[q].rhs(lv[0].b[s * 512 + c.lr]);
-                K0[q].rhs(lv[0].b[s * 512 + c.lb]);
+                rows(lv[0], nb[s], own0[q], s, c, R0[q], K0[q]);
+                R0[q].rhs(c.lr == c.le ? b0[q].x : b0[q].y);
+                K0[q].rhs(c.lr == c.le ? b0[q].y : b0[q].x);
             }
         }
-        auto rows = [&](int l, int at) {
-            if(grp < (int)lv[l].nSlots) {
-                R1[0] = row(lv[l], nb[at + grp], grp, c.lr);
-                K1[0] = row(lv[l], nb[at + grp], grp, c.lb);
-            }
+        const int lastAt = base - 1;  // the coarsest level's only tile
+        if(nLev > 2 && grp < (int)lv[1].nSlots) rows(lv[1], nb[S0 + grp], own1, grp, c, R1[0], K1[0]);
+        if(grp == 0) rows(lv[last], nb[lastAt], ownC, 0, c, RC, KC);
+        // a later level's rows, when it is its turn
+        auto later = [&](int l, int at) {
+            if(grp < (int)lv[l].nSlots) rows(lv[l], nb[at + grp], own(lv[l], grp * 512 + c.le), grp, c, R1[0], K1[0]);
         };
         // the right-hand side that the finer level left in the tile; x starts from 0
         auto take = [&](Row& R, Row& K, int at) {
-            float* x = xs + 1000 * at;
+            float* x = xs + kTile * at;
             R.rhs(x[c.cr]);
             K.rhs(x[c.cb]);
             x[c.cr] = x[c.cb] = 0.f;
         };
-        const int last = nLev - 1, lastAt = base - 1;  // the coarsest level's only tile
-        if(nLev > 2) rows(1, S0);
-        if(grp == 0) {
-            RC = row(lv[last], nb[lastAt], 0, c.lr);
-            KC = row(lv[last], nb[lastAt], 0, c.lb);
-        }
         if(nLev > 1) down<2>(R0, K0, c, xs, nb, S0, grp, lv[1]);
         base = S0;
         for(int l = 1; l < last; ++l) {
             const int S = (int)lv[l].nSlots;
-            if(l > 1) rows(l, base);
+            if(l > 1) later(l, base);
             if(grp < S) take(R1[0], K1[0], base + grp);
-            down<1>(R1, K1, c, xs + 1000 * base, nb + base, S, grp, lv[l + 1]);
+            down<1>(R1, K1, c, xs + kTile * base, nb + base, S, grp, lv[l + 1]);
             base += S;
         }
         {  // coarsest level, one brick
             const int n = grp == 0 ? 1 : 0;
-            float*    x = xs + 1000 * lastAt;
+            float*    x = xs + kTile * lastAt;
             float     vr[1] = {0.f}, vb[1] = {0.f};
             if(n && nLev > 1) take(RC, KC, lastAt);
             else if(n) {
                 RC.rhs(lv[0].b[c.lr]);
                 KC.rhs(lv[0].b[c.lb]);
             }
+            first<1>(&RC, x + c.cr, vr, n);
             __syncthreads();
             for(int it = 0; it < coarsest; ++it) {
-                half<1>(&RC, x + c.cr, c.offR, vr, vb, n);
-                __syncthreads();
+                if(it) {
+                    half<1>(&RC, x + c.cr, c.offR, vr, vb, n);
+                    __syncthreads();
+                }
                 half<1>(&KC, x + c.cb, c.offB, vb, vr, n);
                 __syncthreads();
             }
             for(int it = 0; it < coarsest; ++it) {
-                half<1>(&KC, x + c.cb, c.offB, vb, vr, n);
-                __syncthreads();
+                if(it) {  // the black cells hold their solution already
+                    half<1>(&KC, x + c.cb, c.offB, vb, vr, n);
+                    __syncthreads();
+                }
                 half<1>(&RC, x + c.cr, c.offR, vr, vb, n);
                 __syncthreads();
             }
@@ -3382,13 +3434,13 @@ struct k_mg_tail {
             const int S = (int)lv[l].nSlots;
             base -= S;
             if(last > 2 && l < last - 1) {  // the way down used the registers for a later level
-                rows(l, base);
+                later(l, base);
                 if(grp < S) {
                     R1[0].rhs(lv[l].b[grp * 512 + c.lr]);
                     K1[0].rhs(lv[l].b[grp * 512 + c.lb]);
                 }
             }
-            up<1>(R1, K1, c, xs + 1000 * base, nb + base, S, grp);
+            up<1>(R1, K1, c, xs + kTile * base, nb + base, S, grp);
         }
         if(nLev > 1) {
             up<2>(R0, K0, c, xs, nb, S0, grp);
@@ -3396,8 +3448,8 @@ struct k_mg_tail {
             for(int q = 0; q < 2; ++q) {
                 const int s = grp + 4 * q;
                 if(s < S0) {
-                    lv[0].x[s * 512 + c.lr] = xs[1000 * s + c.cr];
-                    lv[0].x[s * 512 + c.lb] = xs[1000 * s + c.cb];
+                    lv[0].x[s * 512 + c.lr] = xs[kTile * s + c.cr];
+                    lv[0].x[s * 512 + c.lb] = xs[kTile * s + c.cb];
                 }
             }
         }
