@@ -2599,22 +2599,14 @@ struct k_mg_coarsen {
 
 // sum of the six couplings times x. A missing neighbour reads the cell's own x (finite) with a zero
 // coupling, which adds exactly nothing, so every load is issued before the first use.
-__device__ __forceinline__ float level_offdiag_sum(const LevelDev& L, int s, int l, const float* __restrict__ x, bool uni = false) {
+__device__ __forceinline__ float level_offdiag_sum(const LevelDev& L, int s, int l, const float* __restrict__ x) {
     const int32_t ixm = nbr_index(L.nbr, s, l, 0), ixp = nbr_index(L.nbr, s, l, 1);
     const int32_t iym = nbr_index(L.nbr, s, l, 2), iyp = nbr_index(L.nbr, s, l, 3);
     const int32_t izm = nbr_index(L.nbr, s, l, 4), izp = nbr_index(L.nbr, s, l, 5);
     const int32_t o   = s * 512 + l;
     const int32_t jxm = ixm >= 0 ? ixm : o, jxp = ixp >= 0 ? ixp : o, jym = iym >= 0 ? iym : o;
     const int32_t jyp = iyp >= 0 ? iyp : o, jzm = izm >= 0 ? izm : o, jzp = izp >= 0 ? izp : o;
-    float         czm = L.uni.c, cym = L.uni.c, cxm = L.uni.c, cxp = L.uni.c, cyp = L.uni.c, czp = L.uni.c;
-    if(!uni) {
-        czm = L.cz[jzm];
-        cym = L.cy[jym];
-        cxm = L.cx[jxm];
-        cxp = L.cx[o];
-        cyp = L.cy[o];
-        czp = L.cz[o];
-    }
+    const float   czm = L.cz[jzm], cym = L.cy[jym], cxm = L.cx[jxm], cxp = L.cx[o], cyp = L.cy[o], czp = L.cz[o];
     const float   xzm = x[jzm], xym = x[jym], xxm = x[jxm], xxp = x[jxp], xyp = x[jyp], xzp = x[jzp];
     float         acc = 0.f;
     acc += (izm >= 0 ? czm : 0.f) * xzm;
@@ -2640,19 +2632,6 @@ __device__ __forceinline__ uint32_t xcd_slot(uint32_t b, uint32_t n) {
     return xcd * q + min(xcd, r) + b / 8u;
 }
 
-// xpre + omega * x_coarse(parent) for an unknown, xpre otherwise (x + omega P x_c). cs is the coarse
-// brick holding the parent of fine cell (i, j, k) (-1: none). An unknown's parent always lies inside
-// the coarse grid; for other cells the coarse value is loaded but not used. The loads are
-// unconditional (coarse cell 0 stands in when there is no parent brick).
-__device__ __forceinline__ float mg_prolonged(const LevelDev& F, const float* __restrict__ xpre, const LevelDev& C, int32_t cs,
-                                              float omega, int32_t o, int i, int j, int k, bool uni = false) {
-    const int32_t c  = cs < 0 ? 0 : cs * 512 + (((k >> 1) & 7) * 8 + ((j >> 1) & 7)) * 8 + ((i >> 1) & 7);
-    const float   xc = C.x[c];
-    const float   xv = xpre[o];
-    const bool    un = cs >= 0 && (uni || F.invdiag[o] != 0.f);
-    return un ? xv + omega * xc : xv;
-}
-
 // A brick's x with its one-cell halo in LDS (smoothers), x fastest. Rows of 12 and planes of 120 floats
 // where 10 and 100 would do: a wave's accesses in a half-sweep (4 cells two apart in 8 rows of two planes)
 // then fall on different banks, against two to a bank (a half-sweep of k_mg_tail over 8 bricks: 1110 ->
@@ -2660,105 +2639,148 @@ __device__ __forceinline__ float mg_prolonged(const LevelDev& F, const float* __
 constexpr int kTileRow = 12, kTilePlane = 120, kTile = 1200;
 __device__ __forceinline__ int tile_index(int lx, int ly, int lz) { return (lz + 1) * kTilePlane + (ly + 1) * kTileRow + lx + 1; }
 
-// One cell of the brick smoother: its LDS index and its row of A, divided by the diagonal and with the sign
-// of the update x = b/d - sum (a/d) x (a coupling to a missing neighbour is 0 and that neighbour's halo
-// entry holds 0, so all six terms are added unconditionally). The thread owns an x-adjacent pair of cells,
-// one of each colour: the coupling between them takes the other's value from a register (`in`), the one
-// out of the pair lies at LDS offset `off`. Five LDS reads and seven multiply-adds in two chains, against
-// six reads and fourteen operations in one: the half-sweeps are a serial chain.
-struct SmoothCell {
-    int   c, off;
-    float zm, ym, out, in, yp, zp, bs;
+// The smoothers, the restriction and the prolongation work on pairs of cells: their loads, a cell each, were
+// what bounded them (a load of 64 floats costs a CU 10 to 20 cycles however few bytes it moves; a pair takes
+// half as many), and below some hundred bricks the steps from brick to parent in a launch. As pairs, with
+// the parities and parents of the brick tables: at 216 / 9593 bricks update with pre-smoother 7.3 / 35.2 ->
+// 5.8 / 31.9 us, restriction 6.4 / 18.6 -> 4.6 / 14.1, post-smoother 6.9 / 33.7 -> 6.0 / 33.3,
+// prolongation (9593) 14.7 -> 13.2, the 64^3 step 1.90 -> 1.83 ms, 256^3 14.15 -> 13.85.
+
+// The x-adjacent pair of cells that thread t of a brick's 256 owns, one of each colour: even is the first
+// one's index in the brick, cr and cb the red (colour 0) and the black one's tile entries, offR the tile
+// offset out of the pair from the red one (the black one's is -offR), swap: the first one is black.
+struct BrickPair {
+    int  px, ly, lz, even, cr, cb, offR;
+    bool swap;
+    __device__ __forceinline__ explicit BrickPair(int t) {
+        px   = t & 3;
+        ly   = (t >> 2) & 7;
+        lz   = t >> 5;
+        even = (lz * 8 + ly) * 8 + 2 * px;
+        swap = (ly + lz) & 1;
+        const int c = tile_index(2 * px, ly, lz);
+        cr   = swap ? c + 1 : c;
+        cb   = swap ? c : c + 1;
+        offR = swap ? 1 : -1;
+    }
+    // the pair's parent in the parent brick, for a brick whose coordinates' parities are odd's bits
+    __device__ __forceinline__ int parent(int odd) const {
+        return (((odd >> 2 & 1) * 4 + lz / 2) * 8 + (odd >> 1 & 1) * 4 + ly / 2) * 8 + (odd & 1) * 4 + px;
+    }
+    __device__ __forceinline__ float red(float2 v) const { return swap ? v.y : v.x; }
+    __device__ __forceinline__ float black(float2 v) const { return swap ? v.x : v.y; }
+    __device__ __forceinline__ float2 cells(float r, float k) const { return swap ? make_float2(k, r) : make_float2(r, k); }
 };
 
-template<int kProlong>
-__device__ __forceinline__ SmoothCell smooth_cell_setup(const LevelDev& L, const LevelDev& C, int32_t parent, float omega, int s, int l,
-                                                        int bx, int by, int bz, float* xs, float& bv, bool uni) {
-    const int     lx = l & 7, ly = (l >> 3) & 7, lz = l >> 6;
-    const int     c  = tile_index(lx, ly, lz);
-    const size_t  o  = (size_t)s * 512 + l;
-    const int32_t ixm = nbr_index(L.nbr, s, l, 0), ixp = nbr_index(L.nbr, s, l, 1);
-    const int32_t iym = nbr_index(L.nbr, s, l, 2), iyp = nbr_index(L.nbr, s, l, 3);
-    const int32_t izm = nbr_index(L.nbr, s, l, 4), izp = nbr_index(L.nbr, s, l, 5);
-    SmoothCell    R;
-    R.c   = c;
-    float czm = L.uni.c, cym = L.uni.c, cxm = L.uni.c, cxp = L.uni.c, cyp = L.uni.c, czp = L.uni.c, inv = L.uni.inv;
-    if(!uni) {
-        czm = L.cz[izm >= 0 ? izm : (int32_t)o];
-        cym = L.cy[iym >= 0 ? iym : (int32_t)o];
-        cxm = L.cx[ixm >= 0 ? ixm : (int32_t)o];
-        cxp = L.cx[o];
-        cyp = L.cy[o];
-        czp = L.cz[o];
-        inv = L.invdiag[o];
+// a pair of floats at an even index, one load
+__device__ __forceinline__ float2 load2(const float* __restrict__ v, int32_t o) { return *(const float2*)(v + o); }
+__device__ __forceinline__ void   store2(float* __restrict__ v, int32_t o, float2 x) { *(float2*)(v + o) = x; }
+
+// where a pair's neighbours lie, for brick s with the neighbour slots nb[0..5]: o the pair, xm and xp the
+// cells before and after it, ym .. zp the adjacent pairs (o where there is no neighbour), h: which there are
+struct PairNeighbours {
+    int32_t o, xm, xp, ym, yp, zm, zp;
+    bool    hxm, hxp, hym, hyp, hzm, hzp;
+    __device__ __forceinline__ PairNeighbours(const int32_t* __restrict__ nb, int32_t s, const BrickPair& c) {
+        const int l = c.even;
+        o   = s * 512 + l;
+        hxm = c.px > 0 || nb[0] >= 0;
+        hxp = c.px < 3 || nb[1] >= 0;
+        hym = c.ly > 0 || nb[2] >= 0;
+        hyp = c.ly < 7 || nb[3] >= 0;
+        hzm = c.lz > 0 || nb[4] >= 0;
+        hzp = c.lz < 7 || nb[5] >= 0;
+        xm  = c.px > 0 ? o - 1 : (hxm ? nb[0] * 512 + l + 7 : o);
+        xp  = c.px < 3 ? o + 2 : (hxp ? nb[1] * 512 + l - 6 : o);
+        ym  = c.ly > 0 ? o - 8 : (hym ? nb[2] * 512 + l + 56 : o);
+        yp  = c.ly < 7 ? o + 8 : (hyp ? nb[3] * 512 + l - 56 : o);
+        zm  = c.lz > 0 ? o - 64 : (hzm ? nb[4] * 512 + l + 448 : o);
+        zp  = c.lz < 7 ? o + 64 : (hzp ? nb[5] * 512 + l - 448 : o);
     }
-    const float xm = ixm >= 0 ? -cxm * inv : 0.f, xp = ixp >= 0 ? -cxp * inv : 0.f;
-    bv    = L.b[o];
-    R.zm  = izm >= 0 ? -czm * inv : 0.f;
-    R.ym  = iym >= 0 ? -cym * inv : 0.f;
-    R.yp  = iyp >= 0 ? -cyp * inv : 0.f;
-    R.zp  = izp >= 0 ? -czp * inv : 0.f;
-    R.in  = lx & 1 ? xm : xp;
-    R.out = lx & 1 ? xp : xm;
-    R.off = lx & 1 ? 1 : -1;
-    R.bs  = bv * inv;
-    xs[c] = kProlong == 1 ? mg_prolonged(L, L.r, C, parent, omega, (int32_t)o, bx * 8 + lx, by * 8 + ly, bz * 8 + lz)
-                          : (kProlong == 2 ? L.r[o] : 0.f);
-    return R;
+};
+
+// a pair's couplings: cx, cy, cz its own (upwards), xm, ym, zm those of its lower neighbours
+struct PairCoupling {
+    float2 cx, cy, cz, ym, zm;
+    float  xm;
+};
+template<class L> __device__ __forceinline__ PairCoupling pair_coupling(const L& A, const PairNeighbours& n, bool uni) {
+    const float  c = A.uni.c;
+    const float2 c2 = make_float2(c, c);
+    PairCoupling w{c2, c2, c2, c2, c2, c};
+    if(!uni) {
+        w.cx = load2(A.cx, n.o);
+        w.cy = load2(A.cy, n.o);
+        w.cz = load2(A.cz, n.o);
+        w.ym = load2(A.cy, n.ym);
+        w.zm = load2(A.cz, n.zm);
+        w.xm = A.cx[n.xm];
+    }
+    return w;
 }
 
-// the brick's one-cell halo (6 faces x 64 cells) in LDS: the neighbouring bricks' starting values
-// (0 for the pre-smoother and for missing neighbours). A wave's 64 entries share one face.
+// A cell's row of A in the brick smoothers, divided by the diagonal and with the sign of the update
+// x = b/d - sum (a/d) x (a coupling to a missing neighbour is 0 and that neighbour's halo entry holds 0, so
+// all six terms are added unconditionally). The coupling inside the pair (`in`) takes the other cell's value
+// from a register. Five LDS reads and seven multiply-adds in two chains, against six reads and fourteen
+// operations in one: the half-sweeps are a serial chain.
+struct SmoothRow {
+    float zm, ym, out, in, yp, zp, bs;
+    // the cell's new value, x at its tile entry; pair: the other cell of its pair
+    __device__ __forceinline__ float solved(const float* x, int off, float pair) const {
+        const float p = __builtin_fmaf(out, x[off], __builtin_fmaf(ym, x[-kTileRow], __builtin_fmaf(zm, x[-kTilePlane], bs)));
+        return p + __builtin_fmaf(zp, x[kTilePlane], __builtin_fmaf(yp, x[kTileRow], in * pair));
+    }
+};
+// the rows of the pair's red and black cell (bs left 0)
+__device__ __forceinline__ void smooth_rows(const PairCoupling& w, float2 inv, const PairNeighbours& n, const BrickPair& c, SmoothRow& R, SmoothRow& K) {
+    const SmoothRow E{n.hzm ? -w.zm.x * inv.x : 0.f, n.hym ? -w.ym.x * inv.x : 0.f, n.hxm ? -w.xm * inv.x : 0.f, -w.cx.x * inv.x,
+                      n.hyp ? -w.cy.x * inv.x : 0.f, n.hzp ? -w.cz.x * inv.x : 0.f, 0.f};
+    const SmoothRow O{n.hzm ? -w.zm.y * inv.y : 0.f, n.hym ? -w.ym.y * inv.y : 0.f, n.hxp ? -w.cx.y * inv.y : 0.f, -w.cx.x * inv.y,
+                      n.hyp ? -w.cy.y * inv.y : 0.f, n.hzp ? -w.cz.y * inv.y : 0.f, 0.f};
+    R = c.swap ? O : E;
+    K = c.swap ? E : O;
+}
+
+// xpre + omega * x_coarse(parent) for an unknown, xpre otherwise (x + omega P x_c); xc: the coarse value,
+// any where the parent brick is missing (has: it is there)
+__device__ __forceinline__ float mg_prolonged(float xpre, float xc, bool has, float inv, float omega) {
+    return has && inv != 0.f ? xpre + omega * xc : xpre;
+}
+
+// the brick's one-cell halo (6 faces x 64 cells) in LDS: the neighbouring bricks' starting values, 0 where
+// there is none. A wave a face, so the face and its neighbour are scalars. kProlong as in mg_smooth_one;
+// the parent of the neighbour brick is this brick's parent, or that one's neighbour across the face when
+// this brick is on the parent's face.
 template<int kProlong>
-__device__ __forceinline__ void smooth_halo(const LevelDev& L, const LevelDev& C, int32_t parent, float omega, int s, int bx, int by,
-                                            int bz, float* xs) {
-    for(int h = threadIdx.x; h < 384; h += blockDim.x) {
-        const int d = h >> 6, p = h & 63, a = p & 7, e = p >> 3;
-        int       lx, ly, lz;  // the brick cell next to the halo entry
-        if(d < 2) {
-            lx = d == 0 ? 0 : 7;
-            ly = a;
-            lz = e;
-        } else if(d < 4) {
-            lx = a;
-            ly = d == 2 ? 0 : 7;
-            lz = e;
-        } else {
-            lx = a;
-            ly = e;
-            lz = d == 4 ? 0 : 7;
-        }
-        const int sx = d == 0 ? -1 : d == 1 ? 1 : 0, sy = d == 2 ? -1 : d == 3 ? 1 : 0, sz = d == 4 ? -1 : d == 5 ? 1 : 0;
-        const int c  = tile_index(lx + sx, ly + sy, lz + sz);
-        float     v  = 0.f;
-        if(kProlong == 2) {
-            const int32_t n = nbr_index(L.nbr, s, (lz * 8 + ly) * 8 + lx, d);
-            if(n >= 0) v = L.r[n];
-        } else if(kProlong == 1) {
-            const int32_t n = nbr_index(L.nbr, s, (lz * 8 + ly) * 8 + lx, d);
-            if(n >= 0) {
-                // the neighbour brick's parent: this brick's parent, or its neighbour across the face
-                // when this brick is on the parent's face (both uniform over the wave)
-                const int  i = bx * 8 + lx + sx, j = by * 8 + ly + sy, k = bz * 8 + lz + sz;
-                const bool cross = ((i >> 4) != (bx >> 1)) || ((j >> 4) != (by >> 1)) || ((k >> 4) != (bz >> 1));
-                const int32_t cs = cross ? L.ptab[8 * s + d] : parent;
-                v = mg_prolonged(L, L.r, C, cs, omega, n, i, j, k);
+__device__ __forceinline__ void smooth_halo(const LevelDev& L, const LevelDev& C, float omega, int s, float* xs) {
+    const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), a = threadIdx.x & 7, e = threadIdx.x >> 3 & 7;
+#pragma unroll
+    for(int q = 0; q < 2; ++q) {
+        const int d = w + 4 * q;
+        if(d >= 6) break;
+        const int32_t n  = L.nbr[6 * s + d];
+        const int     sa = d < 2 ? kTileRow : 1, se = d < 4 ? kTilePlane : kTileRow, sd = d < 2 ? 1 : (d < 4 ? kTileRow : kTilePlane);
+        float         v  = 0.f;
+        if(n >= 0) {
+            // the cell's coordinates in the neighbour: m across the face, a and e along it
+            const int     m = d & 1 ? 0 : 7, lx = d < 2 ? m : a, ly = d < 2 ? a : (d < 4 ? m : e), lz = d < 4 ? e : m;
+            const int32_t o = n * 512 + (lz * 8 + ly) * 8 + lx;
+            v               = L.r[o];
+            if(kProlong == 1) {
+                const int     own = L.ptab[8 * s + 7], odd = own ^ 1 << (d >> 1);  // parities of the brick's, the neighbour's coordinates
+                const bool    cross = (own >> (d >> 1) & 1) == (d & 1);
+                const int32_t cs = L.ptab[8 * s + (cross ? d : 6)];
+                const int     cl = (((odd >> 2 & 1) * 4 + lz / 2) * 8 + (odd >> 1 & 1) * 4 + ly / 2) * 8 + (odd & 1) * 4 + lx / 2;
+                v                = mg_prolonged(v, C.x[cs < 0 ? 0 : cs * 512 + cl], cs >= 0, L.invdiag[o], omega);
             }
         }
-        xs[c] = v;
+        xs[(1 + a) * sa + (1 + e) * se + (d & 1 ? 9 : 0) * sd] = v;
     }
-}
-
-// the cell's new value; pair: the other cell of its pair
-__device__ __forceinline__ float smooth_cell_update(const SmoothCell& R, float* xs, float pair) {
-    const float p = __builtin_fmaf(R.out, xs[R.c + R.off], __builtin_fmaf(R.ym, xs[R.c - kTileRow], __builtin_fmaf(R.zm, xs[R.c - kTilePlane], R.bs)));
-    const float v = p + __builtin_fmaf(R.zp, xs[R.c + kTilePlane], __builtin_fmaf(R.yp, xs[R.c + kTileRow], R.in * pair));
-    xs[R.c]       = v;
-    return v;
 }
 
 // coarse-grid correction in place: L.r (the pre-smoothed x) += omega * P x_coarse on every unknown.
-// One block per brick, two cells per thread; each cell's parent lies in the brick's parent brick.
+// One block per brick, a pair of cells per thread with one parent, which lies in the brick's parent brick.
 struct k_mg_prolong {
     static constexpr int kThreads = 256;
     LevelDev F;
@@ -2767,17 +2789,13 @@ struct k_mg_prolong {
     const PcgState* __restrict__ st;
     __device__ void operator()(Blk blk) const {
         if(st && st->done) return;
+        const BrickPair c(threadIdx.x);
         for(uint32_t v = blk.id; v < F.nSlots; v += blk.n) {
-            const int     s      = (int)xcd_slot(v, F.nSlots);
-            const int     b      = F.slotBrick[s];
-            const int     bx     = b % F.nbx, by = (b / F.nbx) % F.nby, bz = b / (F.nbx * F.nby);
-            const int32_t parent = F.ptab[8 * s + 6];
-            const bool    uni    = F.uni.is(s);
-            for(int h = 0; h < 2; ++h) {
-                const int    l = (int)threadIdx.x + 256 * h;
-                const size_t o = (size_t)s * 512 + l;
-                F.r[o]         = mg_prolonged(F, F.r, C, parent, omega, (int32_t)o, bx * 8 + (l & 7), by * 8 + ((l >> 3) & 7), bz * 8 + (l >> 6), uni);
-            }
+            const int     s   = (int)xcd_slot(v, F.nSlots);
+            const int32_t cs  = F.ptab[8 * s + 6], o = s * 512 + c.even;
+            const float   xc  = C.x[cs < 0 ? 0 : cs * 512 + c.parent(F.ptab[8 * s + 7])];
+            const float2  inv = F.uni.is(s) ? make_float2(F.uni.inv, F.uni.inv) : load2(F.invdiag, o), xv = load2(F.r, o);
+            store2(F.r, o, make_float2(mg_prolonged(xv.x, xc, cs >= 0, inv.x, omega), mg_prolonged(xv.y, xc, cs >= 0, inv.y, omega)));
         }
     }
 };
@@ -2797,33 +2815,49 @@ struct k_mg_prolong {
 // r = L.b) to pz[slot], the PCG's next rho.
 template<int kProlong, int kDot>
 __device__ __forceinline__ void mg_smooth_one(const LevelDev& L, const LevelDev& C, float omega, int sweeps, double* __restrict__ pz, int s,
-                                              float* xs, double* sh) {
-    const int t = threadIdx.x, ly = (t >> 2) & 7, lz = t >> 5;
-    const int l0 = (lz * 8 + ly) * 8 + 2 * (t & 3);        // even x; its colour is (ly + lz) & 1
-    const int lr = ((ly + lz) & 1) ? l0 + 1 : l0, lb = ((ly + lz) & 1) ? l0 : l0 + 1;  // red (colour 0), black
-    const int     b      = L.slotBrick[s];
-    const int     bx     = b % L.nbx, by = (b / L.nbx) % L.nby, bz = b / (L.nbx * L.nby);
-    const int32_t parent = kProlong == 1 ? L.ptab[8 * s + 6] : -1;
-    const bool       uni = L.uni.is(s);
-    float            br, bb;
-    const SmoothCell R = smooth_cell_setup<kProlong>(L, C, parent, omega, s, lr, bx, by, bz, xs, br, uni);
-    const SmoothCell K = smooth_cell_setup<kProlong>(L, C, parent, omega, s, lb, bx, by, bz, xs, bb, uni);
-    smooth_halo<kProlong>(L, C, parent, omega, s, bx, by, bz, xs);
-    float zr = xs[R.c], zb = xs[K.c];
-    __syncthreads();
-    for(int it = 0; it < sweeps; ++it) {
-        if(kProlong) zb = smooth_cell_update(K, xs, zr);
-        else zr = smooth_cell_update(R, xs, zb);
-        __syncthreads();
-        if(kProlong) zr = smooth_cell_update(R, xs, zb);
-        else zb = smooth_cell_update(K, xs, zr);
+                                              const BrickPair& c, float2 b, float* xs, double* sh) {
+    const int            t = threadIdx.x;
+    const PairNeighbours n(L.nbr + 6 * s, s, c);
+    const bool           uni = L.uni.is(s);
+    const PairCoupling   w   = pair_coupling(L, n, uni);
+    const float2         inv = uni ? make_float2(L.uni.inv, L.uni.inv) : load2(L.invdiag, n.o);
+    float                zr, zb;
+    SmoothRow            R, K;
+    if(kProlong) {
+        float2 xv = load2(L.r, n.o);
+        if(kProlong == 1) {
+            const int32_t cs = L.ptab[8 * s + 6];
+            const float   xc = C.x[cs < 0 ? 0 : cs * 512 + c.parent(L.ptab[8 * s + 7])];
+            xv = make_float2(mg_prolonged(xv.x, xc, cs >= 0, inv.x, omega), mg_prolonged(xv.y, xc, cs >= 0, inv.y, omega));
+        }
+        smooth_halo<kProlong>(L, C, omega, s, xs);
+        xs[c.cr] = zr = c.red(xv);
+        xs[c.cb] = zb = c.black(xv);
+    } else {  // x = 0, and 0 around it
+        for(int e = t; e < kTile / 4; e += 256) ((float4*)xs)[e] = make_float4(0.f, 0.f, 0.f, 0.f);
         __syncthreads();
     }
-    float*      out             = kProlong ? L.x : L.r;
-    out[(size_t)s * 512 + lr]   = zr;
-    out[(size_t)s * 512 + lb]   = zb;
+    smooth_rows(w, inv, n, c, R, K);
+    R.bs = c.red(b) * c.red(inv);
+    K.bs = c.black(b) * c.black(inv);
+    if(!kProlong) {
+        xs[c.cr] = zr = R.bs;  // the first red half-sweep
+        zb            = 0.f;
+    }
+    auto red   = [&] { xs[c.cr] = zr = R.solved(xs + c.cr, c.offR, zb); };
+    auto black = [&] { xs[c.cb] = zb = K.solved(xs + c.cb, -c.offR, zr); };
+    __syncthreads();
+    for(int it = 0; it < sweeps; ++it) {
+        if(kProlong) black();
+        else if(it) red();
+        if(kProlong || it) __syncthreads();
+        if(kProlong) red();
+        else black();
+        __syncthreads();
+    }
+    store2(kProlong ? L.x : L.r, n.o, c.cells(zr, zb));
     if(kDot) {
-        const double d = block_sum<256>((double)zr * (double)br + (double)zb * (double)bb, sh);
+        const double d = block_sum<256>((double)zr * (double)c.red(b) + (double)zb * (double)c.black(b), sh);
         if(t == 0) pz[s] = d;
     }
     __syncthreads();  // xs is reused by the workgroup's next brick
@@ -2839,11 +2873,14 @@ struct k_mg_smooth_brick {
     const PcgState* __restrict__ st;
     double* __restrict__ pz;
     __device__ void operator()(Blk blk) const {
-        __shared__ float xs[kTile];  // the brick and a one-cell halo
+        __shared__ __align__(16) float xs[kTile];  // the brick and a one-cell halo
         __shared__ double sh[4];
         if(st && st->done) return;
-        for(uint32_t v = blk.id; v < L.nSlots; v += blk.n)
-            mg_smooth_one<kProlong, kDot>(L, C, omega, sweeps, pz, (int)xcd_slot(v, L.nSlots), xs, sh);
+        const BrickPair c(threadIdx.x);
+        for(uint32_t v = blk.id; v < L.nSlots; v += blk.n) {
+            const int s = (int)xcd_slot(v, L.nSlots);
+            mg_smooth_one<kProlong, kDot>(L, C, omega, sweeps, pz, s, c, load2(L.b, s * 512 + c.even), xs, sh);
+        }
     }
 };
 
@@ -2866,7 +2903,7 @@ struct k_pcg_update_pre {
     const double* __restrict__ sq;
     int nPart;
     __device__ void operator()(Blk blk) const {
-        __shared__ float  xs[kTile];
+        __shared__ __align__(16) float xs[kTile];
         __shared__ double sh[8];
         if(st->done) return;
         const int t     = threadIdx.x;
@@ -2891,21 +2928,19 @@ struct k_pcg_update_pre {
         } else {
             alpha = (float)st->alpha;
         }
+        const BrickPair c(t);
         for(uint32_t v = blk.id; v < L.nSlots; v += blk.n) {
-            const int slot = (int)xcd_slot(v, L.nSlots);
-            double    m    = 0;
-            for(int h = 0; h < 2; ++h) {
-                const size_t o  = (size_t)slot * 512 + t + 256 * h;
-                const float  xv = x[o] + alpha * s[o];
-                const float  rv = L.b[o] + (-alpha) * L.r[o];
-                x[o]            = xv;
-                L.b[o]          = rv;
-                m               = fmax(m, (double)fabsf(rv));
-            }
-            m = block_max<256>(m, sh);
+            const int     slot = (int)xcd_slot(v, L.nSlots);
+            const int32_t o    = slot * 512 + c.even;
+            const float2  sv = load2(s, o), qv = load2(L.r, o);
+            float2        xv = load2(x, o), rv = load2(L.b, o);
+            xv = make_float2(xv.x + alpha * sv.x, xv.y + alpha * sv.y);
+            rv = make_float2(rv.x + (-alpha) * qv.x, rv.y + (-alpha) * qv.y);
+            store2(x, o, xv);
+            store2(L.b, o, rv);
+            const double m = block_max<256>(fmax((double)fabsf(rv.x), (double)fabsf(rv.y)), sh);
             if(t == 0) pm[slot] = m;
-            __syncthreads();  // the brick's r, written by other threads of the workgroup, is the smoother's b
-            mg_smooth_one<0, 0>(L, L, omega, sweeps, nullptr, slot, xs, sh);
+            mg_smooth_one<0, 0>(L, L, omega, sweeps, nullptr, slot, c, rv, xs, sh);
         }
     }
 };
@@ -2913,7 +2948,8 @@ struct k_pcg_update_pre {
 // r = b - A x on level F with the pre-smoothed x (held in F.r), summed over each 2x2x2 group into
 // the coarse right-hand side (P^T r). A group's eight cells lie in one fine brick, so the block of a
 // fine brick writes the 64 coarse cells it covers; r itself is never stored. Coarse cells without an
-// active child brick keep the zeros they get when the hierarchy is built. 256 threads, two cells each.
+// active child brick keep the zeros they get when the hierarchy is built. A thread's pair of cells and its
+// partners in the group, lanes ^ 4 and ^ 32, form the sum.
 // kStop (finest level, small systems): first the iteration's stop test over nPart <= kFoldMax partials rm
 // of max|r|; the first workgroup records it, the others read only what it leaves alone.
 template<bool kStop>
@@ -2925,7 +2961,6 @@ struct k_mg_residual_restrict {
     const double* __restrict__ rm;
     int nPart;
     __device__ void operator()(Blk blk) const {
-        __shared__ float rs[512];
         if(st && st->done) return;
         const int t = threadIdx.x;
         if(kStop) {
@@ -2934,30 +2969,33 @@ struct k_mg_residual_restrict {
             if(blk.id == 0 && t == 0) pcg_stop_test(*st, B);
             if((float)B < st->tol) return;
         }
+        const BrickPair c(t);
         for(uint32_t v = blk.id; v < F.nSlots; v += blk.n) {
-            const int s = (int)xcd_slot(v, F.nSlots);
-            const int b = F.slotBrick[s];
-            const int bx = b % F.nbx, by = (b / F.nbx) % F.nby, bz = b / (F.nbx * F.nby);
-            const bool uni = F.uni.is(s);
-            for(int h = 0; h < 2; ++h) {
-                const int    l = t + 256 * h;
-                const size_t o = (size_t)s * 512 + l;
-                rs[l]          = F.b[o] - ((uni ? F.uni.d : F.diag[o]) * F.r[o] + level_offdiag_sum(F, s, l, F.r, uni));
-            }
-            __syncthreads();
-            if(t < 64) {
-                const int32_t cs = F.ptab[8 * s + 6];  // the parent brick
-                const int qx = t & 3, qy = (t >> 2) & 3, qz = t >> 4;  // coarse cell inside the brick's 4x4x4
-                const int I = bx * 4 + qx, J = by * 4 + qy, K = bz * 4 + qz;
-                float     sum = 0.f;
-                for(int ch = 0; ch < 8; ++ch) {
-                    const int fi = 2 * I + (ch & 1), fj = 2 * J + ((ch >> 1) & 1), fk = 2 * K + ((ch >> 2) & 1);
-                    if(fi >= F.nx || fj >= F.ny || fk >= F.nz) continue;
-                    sum += rs[((fk & 7) * 8 + (fj & 7)) * 8 + (fi & 7)];
-                }
-                if(cs >= 0 && I < C.nx && J < C.ny && K < C.nz) C.b[(size_t)cs * 512 + ((K & 7) * 8 + (J & 7)) * 8 + (I & 7)] = sum;
-            }
-            __syncthreads();  // rs is reused by the block's next brick
+            const int            s = (int)xcd_slot(v, F.nSlots);
+            const PairNeighbours n(F.nbr + 6 * s, s, c);
+            const bool           uni = F.uni.is(s);
+            const PairCoupling   w   = pair_coupling(F, n, uni);
+            const float2         dia = uni ? make_float2(F.uni.d, F.uni.d) : load2(F.diag, n.o);
+            const float2         b = load2(F.b, n.o), x = load2(F.r, n.o), ym = load2(F.r, n.ym), yp = load2(F.r, n.yp), zm = load2(F.r, n.zm),
+                         zp = load2(F.r, n.zp);
+            const float xm = F.r[n.xm], xp = F.r[n.xp];
+            // a missing neighbour adds its zero coupling times the pair's own x
+            auto offdiag = [&](float czm, float vzm, float cym, float vym, float cxm, float vxm, float cxp, float vxp, float cyp, float vyp, float czp, float vzp) {
+                float acc = 0.f;
+                acc += (n.hzm ? czm : 0.f) * vzm;
+                acc += (n.hym ? cym : 0.f) * vym;
+                acc += cxm * vxm;
+                acc += cxp * vxp;
+                acc += (n.hyp ? cyp : 0.f) * vyp;
+                acc += (n.hzp ? czp : 0.f) * vzp;
+                return acc;
+            };
+            const float r0 = b.x - (dia.x * x.x + offdiag(w.zm.x, zm.x, w.ym.x, ym.x, n.hxm ? w.xm : 0.f, xm, w.cx.x, x.y, w.cy.x, yp.x, w.cz.x, zp.x));
+            const float r1 = b.y - (dia.y * x.y + offdiag(w.zm.y, zm.y, w.ym.y, ym.y, w.cx.x, x.x, n.hxp ? w.cx.y : 0.f, xp, w.cy.y, yp.y, w.cz.y, zp.y));
+            // the odd y of the 2x2x2 group lies in lane ^ 4, the odd z in lane ^ 32
+            const float   e = r0 + r1, ey = e + __shfl_xor(e, 4), sum = ey + __shfl_xor(ey, 32);
+            const int32_t cs = F.ptab[8 * s + 6];
+            if(!(c.ly & 1) && !(c.lz & 1) && cs >= 0) C.b[cs * 512 + c.parent(F.ptab[8 * s + 7])] = sum;
         }
     }
 };
@@ -3165,57 +3203,32 @@ struct k_mg_tail {
     int      sweeps, coarsest;
     const PcgState* __restrict__ st;
 
-    // a cell's row of A as in SmoothCell (divided by the diagonal, signed), its diagonal
-    struct Row {
-        float zm, ym, out, in, yp, zp, bs, diag;
+    // a cell's row of A and its diagonal
+    struct Row : SmoothRow {
+        float diag;
         __device__ __forceinline__ void rhs(float b) { bs = diag > 0.f ? b / diag : 0.f; }
     };
     static __device__ __forceinline__ int tile_at(int l) { return tile_index(l & 7, (l >> 3) & 7, l >> 6); }
-    // the thread's pair of cells: local indices of the red (colour 0) and the black one, their tile entries
-    struct Pair {
-        int  ly, lz, px, le, lr, lb, cr, cb, offR, offB;  // le: the even one; offR, offB: tile offsets out of the pair
-        // the parent of the pair's 2x2x2 group in the parent brick, for a brick with coordinate parities odd
-        __device__ __forceinline__ int parent(int odd) const {
-            return (((odd >> 2 & 1) * 4 + lz / 2) * 8 + (odd >> 1 & 1) * 4 + ly / 2) * 8 + (odd & 1) * 4 + px;
-        }
-    };
-    // the x-adjacent pair's own coefficients, a load each (the even cell's offset is even)
+    // what a pair's rows take besides its lower neighbours' couplings
     struct Own {
         float2 diag, inv, cx, cy, cz;
     };
-    static __device__ __forceinline__ float2 two(const float* __restrict__ v, int32_t o) { return *(const float2*)(v + o); }
     static __device__ __forceinline__ Own own(const LevelDev& L, int32_t o) {
-        return Own{two(L.diag, o), two(L.invdiag, o), two(L.cx, o), two(L.cy, o), two(L.cz, o)};
+        return Own{load2(L.diag, o), load2(L.invdiag, o), load2(L.cx, o), load2(L.cy, o), load2(L.cz, o)};
     }
     // the rows of the pair's red and black cell; nb: the brick's six neighbour slots
-    static __device__ __forceinline__ void rows(const LevelDev& L, const int32_t* nb, const Own& w, int32_t s, const Pair& c, Row& R, Row& K) {
-        const int     l  = c.le;
-        const int32_t o  = s * 512 + l;
-        const int32_t nx = nb[0], ny = nb[2], nz = nb[4];
-        const bool    hx = c.px > 0 || nx >= 0, hy = c.ly > 0 || ny >= 0, hz = c.lz > 0 || nz >= 0;
-        const float   cxm = L.cx[c.px > 0 ? o - 1 : (hx ? nx * 512 + l + 7 : o)];
-        const float2  cym = two(L.cy, c.ly > 0 ? o - 8 : (hy ? ny * 512 + l + 56 : o));
-        const float2  czm = two(L.cz, c.lz > 0 ? o - 64 : (hz ? nz * 512 + l + 448 : o));
-        const bool    hX = c.px < 3 || nb[1] >= 0, hY = c.ly < 7 || nb[3] >= 0, hZ = c.lz < 7 || nb[5] >= 0;
-        const Row     E{hz ? -czm.x * w.inv.x : 0.f, hy ? -cym.x * w.inv.x : 0.f, hx ? -cxm * w.inv.x : 0.f, -w.cx.x * w.inv.x,
-                    hY ? -w.cy.x * w.inv.x : 0.f, hZ ? -w.cz.x * w.inv.x : 0.f, 0.f, w.diag.x};
-        const Row     O{hz ? -czm.y * w.inv.y : 0.f, hy ? -cym.y * w.inv.y : 0.f, hX ? -w.cx.y * w.inv.y : 0.f, -w.cx.x * w.inv.y,
-                    hY ? -w.cy.y * w.inv.y : 0.f, hZ ? -w.cz.y * w.inv.y : 0.f, 0.f, w.diag.y};
-        R = c.lr == c.le ? E : O;
-        K = c.lr == c.le ? O : E;
-    }
-    // b/d - sum (a/d) x over the neighbours of the cell at x; pair: the other cell of its pair, off: the
-    // offset out of the pair
-    static __device__ __forceinline__ float solved(const Row& R, const float* x, int off, float pair) {
-        const float p = __builtin_fmaf(R.out, x[off], __builtin_fmaf(R.ym, x[-kTileRow], __builtin_fmaf(R.zm, x[-kTilePlane], R.bs)));
-        return p + __builtin_fmaf(R.zp, x[kTilePlane], __builtin_fmaf(R.yp, x[kTileRow], R.in * pair));
+    static __device__ __forceinline__ void rows(const LevelDev& L, const int32_t* nb, const Own& w, int32_t s, const BrickPair& c, Row& R, Row& K) {
+        const PairNeighbours n(nb, s, c);
+        smooth_rows(PairCoupling{w.cx, w.cy, w.cz, load2(L.cy, n.ym), load2(L.cz, n.zm), L.cx[n.xm]}, w.inv, n, c, R, K);
+        R.diag = c.red(w.diag);
+        K.diag = c.black(w.diag);
     }
     // one half-sweep over the group's n bricks (4 tiles apart): cells of one colour read only the other.
     // own: the cells' values, pair: those of the other colour
     template<int kTurns> static __device__ __forceinline__ void half(const Row* R, float* x, int off, float* own, const float* pair, int n) {
 #pragma unroll
         for(int q = 0; q < kTurns; ++q)
-            if(q < n) own[q] = solved(R[q], x + 4 * kTile * q, off, pair[q]);
+            if(q < n) own[q] = R[q].solved(x + 4 * kTile * q, off, pair[q]);
 #pragma unroll
         for(int q = 0; q < kTurns; ++q)
             if(q < n) x[4 * kTile * q] = own[q];
@@ -3250,7 +3263,7 @@ struct k_mg_tail {
     // pre-smoother from x = 0 on the level's tiles, then the residual's 2x2x2 sums to the next level's tiles
     // (its right-hand side) and to its b (for the way up)
     template<int kTurns>
-    __device__ __forceinline__ void down(const Row* R, const Row* K, const Pair& c, float* xs, const int32_t (*nb)[8], int S, int grp, const LevelDev& C) const {
+    __device__ __forceinline__ void down(const Row* R, const Row* K, const BrickPair& c, float* xs, const int32_t (*nb)[8], int S, int grp, const LevelDev& C) const {
         const int n = (S - grp + 3) >> 2;  // bricks grp, grp + 4, ..
         float*    x = xs + kTile * grp;
         float     vr[kTurns] = {}, vb[kTurns] = {};
@@ -3261,7 +3274,7 @@ struct k_mg_tail {
                 half<kTurns>(R, x + c.cr, c.offR, vr, vb, n);
                 __syncthreads();
             }
-            half<kTurns>(K, x + c.cb, c.offB, vb, vr, n);
+            half<kTurns>(K, x + c.cb, -c.offR, vb, vr, n);
             __syncthreads();
         }
         halos(xs, nb, S);
@@ -3270,8 +3283,8 @@ struct k_mg_tail {
         for(int q = 0; q < kTurns; ++q)
             if(q < n) {
                 const float* y  = x + 4 * kTile * q;
-                const float  rr = R[q].diag * (solved(R[q], y + c.cr, c.offR, vb[q]) - vr[q]);
-                const float  rk = K[q].diag * (solved(K[q], y + c.cb, c.offB, vr[q]) - vb[q]);
+                const float  rr = R[q].diag * (R[q].solved(y + c.cr, c.offR, vb[q]) - vr[q]);
+                const float  rk = K[q].diag * (K[q].solved(y + c.cb, -c.offR, vr[q]) - vb[q]);
                 // the x pair is this thread's, the odd y lies in lane ^ 4, the odd z in lane ^ 32
                 const float e = rr + rk, ey = e + __shfl_xor(e, 4), sum = ey + __shfl_xor(ey, 32);
                 const int   par = nb[grp + 4 * q][6];
@@ -3285,7 +3298,7 @@ struct k_mg_tail {
     }
     // coarse-grid correction, then the post-smoother
     template<int kTurns>
-    __device__ __forceinline__ void up(const Row* R, const Row* K, const Pair& c, float* xs, const int32_t (*nb)[8], int S, int grp) const {
+    __device__ __forceinline__ void up(const Row* R, const Row* K, const BrickPair& c, float* xs, const int32_t (*nb)[8], int S, int grp) const {
         const int n = (S - grp + 3) >> 2;
         float*    x = xs + kTile * grp;
         float     vr[kTurns] = {}, vb[kTurns] = {};
@@ -3306,7 +3319,7 @@ struct k_mg_tail {
         halos(xs, nb, S);
         __syncthreads();
         for(int it = 0; it < sweeps; ++it) {
-            half<kTurns>(K, x + c.cb, c.offB, vb, vr, n);
+            half<kTurns>(K, x + c.cb, -c.offR, vb, vr, n);
             __syncthreads();
             half<kTurns>(R, x + c.cr, c.offR, vr, vb, n);
             __syncthreads();
@@ -3317,19 +3330,8 @@ struct k_mg_tail {
         __shared__ int32_t nb[kTiles][8];  // per brick: six neighbour slots, parent slot, parities of its coordinates
         int t = threadIdx.x;
         asm volatile("" : "+v"(t));  // keeps the batched form's loop over scenes from holding the lane's constants in registers
-        const int grp = t >> 8, tt = t & 255;
-        Pair      c;
-        c.ly = (tt >> 2) & 7;
-        c.lz = tt >> 5;
-        c.px = tt & 3;
-        c.le = (c.lz * 8 + c.ly) * 8 + 2 * c.px;
-        const int o0 = (c.ly + c.lz) & 1;  // the even cell's colour
-        c.lr = c.le + o0;
-        c.lb = c.le + 1 - o0;
-        c.cr = tile_at(c.lr);
-        c.cb = tile_at(c.lb);
-        c.offR = c.lr & 1 ? 1 : -1;
-        c.offB = -c.offR;
+        const int       grp = t >> 8;
+        const BrickPair c(t & 255);
         // the brick tables and the pairs' own coefficients of the first two levels and the coarsest, before
         // anything waits: the lower neighbours' follow when the tables are in LDS
         int32_t tab[kLevels];
@@ -3349,11 +3351,11 @@ struct k_mg_tail {
 #pragma unroll
         for(int q = 0; q < 2; ++q)
             if(grp + 4 * q < S0) {
-                own0[q] = own(lv[0], (grp + 4 * q) * 512 + c.le);
-                b0[q]   = two(lv[0].b, (grp + 4 * q) * 512 + c.le);
+                own0[q] = own(lv[0], (grp + 4 * q) * 512 + c.even);
+                b0[q]   = load2(lv[0].b, (grp + 4 * q) * 512 + c.even);
             }
-        if(nLev > 2 && grp < (int)lv[1].nSlots) own1 = own(lv[1], grp * 512 + c.le);
-        if(grp == 0) ownC = own(lv[last], c.le);
+        if(nLev > 2 && grp < (int)lv[1].nSlots) own1 = own(lv[1], grp * 512 + c.even);
+        if(grp == 0) ownC = own(lv[last], c.even);
         if(st && st->done) return;
         int base = 0;
 #pragma unroll
@@ -3371,8 +3373,8 @@ struct k_mg_tail {
             const int s = grp + 4 * q;
             if(s < S0) {
                 rows(lv[0], nb[s], own0[q], s, c, R0[q], K0[q]);
-                R0[q].rhs(c.lr == c.le ? b0[q].x : b0[q].y);
-                K0[q].rhs(c.lr == c.le ? b0[q].y : b0[q].x);
+                R0[q].rhs(c.red(b0[q]));
+                K0[q].rhs(c.black(b0[q]));
             }
         }
         const int lastAt = base - 1;  // the coarsest level's only tile
@@ -3380,7 +3382,7 @@ struct k_mg_tail {
         if(grp == 0) rows(lv[last], nb[lastAt], ownC, 0, c, RC, KC);
         // a later level's rows, when it is its turn
         auto later = [&](int l, int at) {
-            if(grp < (int)lv[l].nSlots) rows(lv[l], nb[at + grp], own(lv[l], grp * 512 + c.le), grp, c, R1[0], K1[0]);
+            if(grp < (int)lv[l].nSlots) rows(lv[l], nb[at + grp], own(lv[l], grp * 512 + c.even), grp, c, R1[0], K1[0]);
         };
         // the right-hand side that the finer level left in the tile; x starts from 0
         auto take = [&](Row& R, Row& K, int at) {
@@ -3404,8 +3406,9 @@ struct k_mg_tail {
             float     vr[1] = {0.f}, vb[1] = {0.f};
             if(n && nLev > 1) take(RC, KC, lastAt);
             else if(n) {
-                RC.rhs(lv[0].b[c.lr]);
-                KC.rhs(lv[0].b[c.lb]);
+                const float2 b = load2(lv[0].b, c.even);
+                RC.rhs(c.red(b));
+                KC.rhs(c.black(b));
             }
             first<1>(&RC, x + c.cr, vr, n);
             __syncthreads();
@@ -3414,20 +3417,19 @@ struct k_mg_tail {
                     half<1>(&RC, x + c.cr, c.offR, vr, vb, n);
                     __syncthreads();
                 }
-                half<1>(&KC, x + c.cb, c.offB, vb, vr, n);
+                half<1>(&KC, x + c.cb, -c.offR, vb, vr, n);
                 __syncthreads();
             }
             for(int it = 0; it < coarsest; ++it) {
                 if(it) {  // the black cells hold their solution already
-                    half<1>(&KC, x + c.cb, c.offB, vb, vr, n);
+                    half<1>(&KC, x + c.cb, -c.offR, vb, vr, n);
                     __syncthreads();
                 }
                 half<1>(&RC, x + c.cr, c.offR, vr, vb, n);
                 __syncthreads();
             }
             if(n && nLev == 1) {
-                lv[0].x[c.lr] = vr[0];
-                lv[0].x[c.lb] = vb[0];
+                store2(lv[0].x, c.even, c.cells(vr[0], vb[0]));
             }
         }
         for(int l = last - 1; l >= 1; --l) {
@@ -3436,8 +3438,9 @@ struct k_mg_tail {
             if(last > 2 && l < last - 1) {  // the way down used the registers for a later level
                 later(l, base);
                 if(grp < S) {
-                    R1[0].rhs(lv[l].b[grp * 512 + c.lr]);
-                    K1[0].rhs(lv[l].b[grp * 512 + c.lb]);
+                    const float2 b = load2(lv[l].b, grp * 512 + c.even);
+                    R1[0].rhs(c.red(b));
+                    K1[0].rhs(c.black(b));
                 }
             }
             up<1>(R1, K1, c, xs + kTile * base, nb + base, S, grp);
@@ -3448,8 +3451,7 @@ struct k_mg_tail {
             for(int q = 0; q < 2; ++q) {
                 const int s = grp + 4 * q;
                 if(s < S0) {
-                    lv[0].x[s * 512 + c.lr] = xs[kTile * s + c.cr];
-                    lv[0].x[s * 512 + c.lb] = xs[kTile * s + c.cb];
+                    store2(lv[0].x, s * 512 + c.even, c.cells(xs[kTile * s + c.cr], xs[kTile * s + c.cb]));
                 }
             }
         }
