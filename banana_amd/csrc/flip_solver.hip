@@ -1472,10 +1472,8 @@ public:
 
     Co<float> timestepCFL() {  // PIC_Solver.cpp:342-349
         fill32(counters.p, 0, 4);
-        DevBuf* vel[3] = {&u, &v, &w};
-        size_t  cnt[3] = {nU, nV, nW};
-        for(int d = 0; d < 3; ++d)
-            launch(k_maxabs{(const float*)vel[d]->as<float>(), cnt[d], counters.as<uint32_t>()}, std::min<unsigned>(blocks(cnt[d]), 2048));
+        launch(k_maxabs{{u.as<float>(), v.as<float>(), w.as<float>()}, {(uint32_t)nU, (uint32_t)nV, (uint32_t)nW}, counters.as<uint32_t>()},
+               std::min<unsigned>(blocks(nU + nV + nW), k_maxabs::kBlocks));
         readback(hostU32, counters.p, 4);
         co_await syncPoint();
         float m;
