@@ -618,12 +618,14 @@ public:
     }
 
     // PIC_Solver.cpp:353-373
-    void moveParticles(float dt) {
+    // keys: the binning follows at once, with keys formed here (binParticles(true))
+    void moveParticles(float dt, bool keys = false) {
         if(!np) return;
+        if(keys) fill32(occ.p, 0, occ.bytes);
         VelGrid G{u.as<float>(), v.as<float>(), w.as<float>()};
         ktBegin(BNN_KT_MOVE);
         launch(k_move{cur->view(), (uint32_t)np, G, g, bnd, dt,
-                           prm.advection_steps, prm.reflect_velocity_at_boundary, prm.boundary_reflection_multiplier}, blocks(np));
+                           prm.advection_steps, prm.reflect_velocity_at_boundary, prm.boundary_reflection_multiplier, keys ? cellKeys() : CellKeys{}}, blocks(np));
         ktEnd(BNN_KT_MOVE);
         binned = false;
     }
@@ -654,7 +656,8 @@ public:
     }
 
     // cell-sorted binning: key + count, scan, scatter, per-cell ordering, permute
-    void binParticles() {
+    CellKeys cellKeys() { return CellKeys{key.as<uint32_t>(), cellCount.as<uint32_t>(), occ.as<uint8_t>()}; }
+    void binParticles(bool keysDone = false) {
         if(!np) {
             fill32(cellStart.p, 0, (nC + 1) * 4);
             fill32(occ.p, 0, occ.bytes);
@@ -663,10 +666,10 @@ public:
             return;
         }
         const ParticleBufs& P = *cur;
-        fill32(occ.p, 0, occ.bytes);
-        launch(k_cell_key{P.px.as<float>(), P.py.as<float>(), P.pz.as<float>(), (uint32_t)np, g, key.as<uint32_t>(), cellCount.as<uint32_t>(),
-                          occ.as<uint8_t>()},
-               blocks(np));
+        if(!keysDone) {
+            fill32(occ.p, 0, occ.bytes);
+            launch(k_cell_key{P.px.as<float>(), P.py.as<float>(), P.pz.as<float>(), (uint32_t)np, g, cellKeys()}, blocks(np));
+        }
         scan(cellCount.as<uint32_t>(), cellStart.as<uint32_t>(), nC, cellStart.as<uint32_t>() + nC);
         launch(k_scatter{key.as<uint32_t>(), (uint32_t)np, cellStart.as<uint32_t>(), cellCount.as<uint32_t>(), perm.as<uint32_t>()}, blocks(np));
         launch(k_segsort{cellStart.as<uint32_t>(), (uint32_t)nC, perm.as<uint32_t>()}, blocks(nC));
@@ -1454,7 +1457,8 @@ public:
         if(!(dt > 0)) throw Error(BNN_ERR_INVALID_ARG, "dt must be > 0");
         beginStats();
         stageBegin(BNN_STAGE_MOVE);
-        moveParticles(dt);
+        const bool keys = !prm.correct_position;
+        moveParticles(dt, keys);
         stageEnd(BNN_STAGE_MOVE);
         if(prm.correct_position) {  // PIC_Solver.cpp:295 (after moveParticles, before advanceVelocity)
             stageBegin(BNN_STAGE_OTHER);
@@ -1462,7 +1466,7 @@ public:
             stageEnd(BNN_STAGE_OTHER);
         }
         stageBegin(BNN_STAGE_BIN);
-        binParticles();
+        binParticles(keys);
         stageEnd(BNN_STAGE_BIN);
         bool ok = co_await advanceVelocity(dt);
         co_await endStats(dt);
