@@ -2777,11 +2777,9 @@ __device__ __forceinline__ float mg_prolonged(float xpre, float xc, bool has, fl
     return has && inv != 0.f ? xpre + omega * xc : xpre;
 }
 
-// the brick's one-cell halo (6 faces x 64 cells) in LDS: the neighbouring bricks' starting values, 0 where
-// there is none. A wave a face, so the face and its neighbour are scalars. kProlong as in mg_smooth_one;
-// the parent of the neighbour brick is this brick's parent, or that one's neighbour across the face when
-// this brick is on the parent's face.
-template<int kProlong>
+// the brick's one-cell halo (6 faces x 64 cells) in LDS: the neighbouring bricks' corrected values, 0 where
+// there is none. A wave a face, so the face and its neighbour are scalars. The parent of the neighbour brick
+// is this brick's parent, or that one's neighbour across the face when this brick is on the parent's face.
 __device__ __forceinline__ void smooth_halo(const LevelDev& L, const LevelDev& C, float omega, int s, float* xs) {
     const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), a = threadIdx.x & 7, e = threadIdx.x >> 3 & 7;
 #pragma unroll
@@ -2795,54 +2793,29 @@ __device__ __forceinline__ void smooth_halo(const LevelDev& L, const LevelDev& C
             // the cell's coordinates in the neighbour: m across the face, a and e along it
             const int     m = d & 1 ? 0 : 7, lx = d < 2 ? m : a, ly = d < 2 ? a : (d < 4 ? m : e), lz = d < 4 ? e : m;
             const int32_t o = n * 512 + (lz * 8 + ly) * 8 + lx;
-            v               = L.r[o];
-            if(kProlong == 1) {
-                const int     own = L.ptab[8 * s + 7], odd = own ^ 1 << (d >> 1);  // parities of the brick's, the neighbour's coordinates
-                const bool    cross = (own >> (d >> 1) & 1) == (d & 1);
-                const int32_t cs = L.ptab[8 * s + (cross ? d : 6)];
-                const int     cl = (((odd >> 2 & 1) * 4 + lz / 2) * 8 + (odd >> 1 & 1) * 4 + ly / 2) * 8 + (odd & 1) * 4 + lx / 2;
-                v                = mg_prolonged(v, C.x[cs < 0 ? 0 : cs * 512 + cl], cs >= 0, L.invdiag[o], omega);
-            }
+            const int     own = L.ptab[8 * s + 7], odd = own ^ 1 << (d >> 1);  // parities of the brick's, the neighbour's coordinates
+            const bool    cross = (own >> (d >> 1) & 1) == (d & 1);
+            const int32_t cs = L.ptab[8 * s + (cross ? d : 6)];
+            const int     cl = (((odd >> 2 & 1) * 4 + lz / 2) * 8 + (odd >> 1 & 1) * 4 + ly / 2) * 8 + (odd & 1) * 4 + lx / 2;
+            v                = mg_prolonged(L.r[o], C.x[cs < 0 ? 0 : cs * 512 + cl], cs >= 0, L.invdiag[o], omega);
         }
         xs[(1 + a) * sa + (1 + e) * se + (d & 1 ? 9 : 0) * sd] = v;
     }
 }
 
-// coarse-grid correction in place: L.r (the pre-smoothed x) += omega * P x_coarse on every unknown.
-// One block per brick, a pair of cells per thread with one parent, which lies in the brick's parent brick.
-struct k_mg_prolong {
-    static constexpr int kThreads = 256;
-    LevelDev F;
-    LevelDev C;
-    float omega;
-    const PcgState* __restrict__ st;
-    __device__ void operator()(Blk blk) const {
-        if(st && st->done) return;
-        const BrickPair c(threadIdx.x);
-        for(uint32_t v = blk.id; v < F.nSlots; v += blk.n) {
-            const int     s   = (int)xcd_slot(v, F.nSlots);
-            const int32_t cs  = F.ptab[8 * s + 6], o = s * 512 + c.even;
-            const float   xc  = C.x[cs < 0 ? 0 : cs * 512 + c.parent(F.ptab[8 * s + 7])];
-            const float2  inv = F.uni.is(s) ? make_float2(F.uni.inv, F.uni.inv) : load2(F.invdiag, o), xv = load2(F.r, o);
-            store2(F.r, o, make_float2(mg_prolonged(xv.x, xc, cs >= 0, inv.x, omega), mg_prolonged(xv.y, xc, cs >= 0, inv.y, omega)));
-        }
-    }
-};
-
 // Brick-hybrid Gauss-Seidel: one block per brick runs `sweeps` red-black sweeps (pre-smoother) or
 // black-red sweeps (post-smoother) on its 512 cells in LDS, with the x of neighbouring bricks held at
 // their values on entry (Jacobi between bricks). For the brick's own system A_BB the red-black and
 // black-red sequences are transposes of each other, so the pre- and post-smoothers are adjoint and
-// the V-cycle stays symmetric. Pre-smoother (kProlong == 0): starts from x = 0 (every V-cycle does)
-// and writes L.r. Post-smoother: starts from the coarse-grid-corrected L.r + omega * P x_coarse for
-// the brick and its halo, formed on the fly (kProlong == 1: no extra launch, for the small coarse
-// levels) or already added by k_mg_prolong (kProlong == 2: the finest level, where a streaming pass
-// is cheaper than the dependent loads), and writes L.x. Input and output are different arrays, so
-// no block reads what another writes. Each of the 256 threads owns
+// the V-cycle stays symmetric. Pre-smoother: starts from x = 0 (every V-cycle does) and writes L.r.
+// Post-smoother (kPost): starts from the coarse-grid-corrected L.r + omega * P x_coarse, formed here for
+// the brick and its halo, and writes L.x. (On the finest level the correction was once a streaming pass of
+// its own, 12.9 us at 9593 bricks and a launch; with the parents from the brick tables it costs the smoother
+// 10: 33.7 -> 43.8 us, at 1309 bricks 7.7 -> 9.2 for a pass of 3.5.) Input and output are different arrays, so no block reads what another writes. Each of the 256 threads owns
 // an x-adjacent pair of cells, one of each colour, so every thread updates one cell per half-sweep.
 // kDot (finest level, post-smoother): also writes the brick's partial of z.r (z = the result,
 // r = L.b) to pz[slot], the PCG's next rho.
-template<int kProlong, int kDot>
+template<bool kPost, bool kDot>
 __device__ __forceinline__ void mg_smooth_one(const LevelDev& L, const LevelDev& C, float omega, int sweeps, double* __restrict__ pz, int s,
                                               const BrickPair& c, float2 b, float* xs, double* sh) {
     const int            t = threadIdx.x;
@@ -2852,14 +2825,12 @@ __device__ __forceinline__ void mg_smooth_one(const LevelDev& L, const LevelDev&
     const float2         inv = uni ? make_float2(L.uni.inv, L.uni.inv) : load2(L.invdiag, n.o);
     float                zr, zb;
     SmoothRow            R, K;
-    if(kProlong) {
-        float2 xv = load2(L.r, n.o);
-        if(kProlong == 1) {
-            const int32_t cs = L.ptab[8 * s + 6];
-            const float   xc = C.x[cs < 0 ? 0 : cs * 512 + c.parent(L.ptab[8 * s + 7])];
-            xv = make_float2(mg_prolonged(xv.x, xc, cs >= 0, inv.x, omega), mg_prolonged(xv.y, xc, cs >= 0, inv.y, omega));
-        }
-        smooth_halo<kProlong>(L, C, omega, s, xs);
+    if(kPost) {
+        const int32_t cs = L.ptab[8 * s + 6];
+        const float   xc = C.x[cs < 0 ? 0 : cs * 512 + c.parent(L.ptab[8 * s + 7])];
+        float2        xv = load2(L.r, n.o);
+        xv = make_float2(mg_prolonged(xv.x, xc, cs >= 0, inv.x, omega), mg_prolonged(xv.y, xc, cs >= 0, inv.y, omega));
+        smooth_halo(L, C, omega, s, xs);
         xs[c.cr] = zr = c.red(xv);
         xs[c.cb] = zb = c.black(xv);
     } else {  // x = 0, and 0 around it
@@ -2869,7 +2840,7 @@ __device__ __forceinline__ void mg_smooth_one(const LevelDev& L, const LevelDev&
     smooth_rows(w, inv, n, c, R, K);
     R.bs = c.red(b) * c.red(inv);
     K.bs = c.black(b) * c.black(inv);
-    if(!kProlong) {
+    if(!kPost) {
         xs[c.cr] = zr = R.bs;  // the first red half-sweep
         zb            = 0.f;
     }
@@ -2877,14 +2848,14 @@ __device__ __forceinline__ void mg_smooth_one(const LevelDev& L, const LevelDev&
     auto black = [&] { xs[c.cb] = zb = K.solved(xs + c.cb, -c.offR, zr); };
     __syncthreads();
     for(int it = 0; it < sweeps; ++it) {
-        if(kProlong) black();
+        if(kPost) black();
         else if(it) red();
-        if(kProlong || it) __syncthreads();
-        if(kProlong) red();
+        if(kPost || it) __syncthreads();
+        if(kPost) red();
         else black();
         __syncthreads();
     }
-    store2(kProlong ? L.x : L.r, n.o, c.cells(zr, zb));
+    store2(kPost ? L.x : L.r, n.o, c.cells(zr, zb));
     if(kDot) {
         const double d = block_sum<256>((double)zr * (double)c.red(b) + (double)zb * (double)c.black(b), sh);
         if(t == 0) pz[s] = d;
@@ -2892,7 +2863,7 @@ __device__ __forceinline__ void mg_smooth_one(const LevelDev& L, const LevelDev&
     __syncthreads();  // xs is reused by the workgroup's next brick
 }
 
-template<int kProlong, int kDot>
+template<bool kPost, bool kDot>
 struct k_mg_smooth_brick {
     static constexpr int kThreads = 256;
     LevelDev L;
@@ -2908,7 +2879,7 @@ struct k_mg_smooth_brick {
         const BrickPair c(threadIdx.x);
         for(uint32_t v = blk.id; v < L.nSlots; v += blk.n) {
             const int s = (int)xcd_slot(v, L.nSlots);
-            mg_smooth_one<kProlong, kDot>(L, C, omega, sweeps, pz, s, c, load2(L.b, s * 512 + c.even), xs, sh);
+            mg_smooth_one<kPost, kDot>(L, C, omega, sweeps, pz, s, c, load2(L.b, s * 512 + c.even), xs, sh);
         }
     }
 };
@@ -2917,7 +2888,7 @@ struct k_mg_smooth_brick {
 // x += alpha s and r -= alpha q (PCGSolver.cpp:178-181), the brick's max|r| to pm[slot], then the
 // pre-smoother on b = r, which reads only the brick's own cells (it starts from x = 0). The finest
 // level's r array is the PCG's q buffer: this brick's q is read before the smoother overwrites it.
-// Per cell the same arithmetic as k_pcg_update followed by k_mg_smooth_brick<0, 0>.
+// Per cell the same arithmetic as k_pcg_update followed by k_mg_smooth_brick<false, false>.
 // kFold (small systems): alpha (k_pcg_alpha) is formed here from nPart <= kFoldMax partials of s.q.
 template<bool kFold>
 struct k_pcg_update_pre {
@@ -2969,7 +2940,7 @@ struct k_pcg_update_pre {
             store2(L.b, o, rv);
             const double m = block_max<256>(fmax((double)fabsf(rv.x), (double)fabsf(rv.y)), sh);
             if(t == 0) pm[slot] = m;
-            mg_smooth_one<0, 0>(L, L, omega, sweeps, nullptr, slot, c, rv, xs, sh);
+            mg_smooth_one<false, false>(L, L, omega, sweeps, nullptr, slot, c, rv, xs, sh);
         }
     }
 };

@@ -986,10 +986,6 @@ public:
     // (false when the fine level is the coarsest: the caller then forms z.r itself).
     // finePreDone: the finest level's pre-smoother already ran (fused with the PCG update). stopPart: the
     // iteration's stop test runs in the finest restriction, over these per-brick partials of max|r|.
-    // The finest level's correction: formed by the post-smoother itself up to kProlongInPost bricks alone
-    // (a launch less), else as a streaming pass of its own (at 9600 bricks 14 us against the dependent
-    // loads; in a batch the launch is shared).
-    static constexpr uint32_t kProlongInPost = 1024;
     bool vcycle(PcgState* stp, bool finePreDone = false, const double* stopPart = nullptr) {
         const int   nu    = prm.mg_sweeps;
         const float omega = prm.mg_omega;
@@ -1000,7 +996,7 @@ public:
             const unsigned G = std::max<uint32_t>(L.nSlots, 1u);
             if(!(l == 0 && finePreDone)) {
                 ktBegin(l == 0 ? BNN_KT_MG_PRE : BNN_KT_MG_COARSE);
-                launch(k_mg_smooth_brick<0, 0>{L, C, omega, nu, stp, (double*)nullptr}, G);
+                launch(k_mg_smooth_brick<false, false>{L, C, omega, nu, stp, (double*)nullptr}, G);
                 ktEnd(l == 0 ? BNN_KT_MG_PRE : BNN_KT_MG_COARSE);
             }
             ktBegin(l == 0 ? BNN_KT_MG_RESTRICT : BNN_KT_MG_COARSE);
@@ -1024,20 +1020,13 @@ public:
         for(int l = down - 1; l >= 0; --l) {
             const LevelDev L = levelDev(l), C = levelDev(l + 1);
             const uint32_t G = std::max<uint32_t>(L.nSlots, 1u);
-            if(l == 0 && !rec && L.nSlots <= kProlongInPost) {
+            if(l == 0) {  // also forms z.r
                 ktBegin(BNN_KT_MG_POST);
-                launch(k_mg_smooth_brick<1, 1>{L, C, omega, nu, stp, pz.as<double>()}, G);
-                ktEnd(BNN_KT_MG_POST);
-            } else if(l == 0) {  // correction as its own streaming pass, then smooth and form z.r
-                ktBegin(BNN_KT_MG_PROLONG);
-                launch(k_mg_prolong{L, C, omega, stp}, G);
-                ktEnd(BNN_KT_MG_PROLONG);
-                ktBegin(BNN_KT_MG_POST);
-                launch(k_mg_smooth_brick<2, 1>{L, C, omega, nu, stp, pz.as<double>()}, G);
+                launch(k_mg_smooth_brick<true, true>{L, C, omega, nu, stp, pz.as<double>()}, G);
                 ktEnd(BNN_KT_MG_POST);
             } else {
                 ktBegin(BNN_KT_MG_COARSE);
-                launch(k_mg_smooth_brick<1, 0>{L, C, omega, nu, stp, (double*)nullptr}, G);
+                launch(k_mg_smooth_brick<true, false>{L, C, omega, nu, stp, (double*)nullptr}, G);
                 ktEnd(BNN_KT_MG_COARSE);
             }
         }

@@ -61,8 +61,7 @@ KERNEL_BYTES = {
                                                             # 3 couplings, 1/diag in; x, r, pre-smoothed z out
     "mg_pre": lambda Np, F, C, V, A: 24 * A,                # 3 couplings, b, 1/diag in; x out
     "mg_restrict": lambda Np, F, C, V, A: 24.5 * A,         # b, diag, 3 couplings, x in; coarse b out
-    "mg_prolong": lambda Np, F, C, V, A: 12.5 * A,          # x, 1/diag, coarse x in; x out
-    "mg_post": lambda Np, F, C, V, A: 28 * A,               # 3 couplings, b, 1/diag, x in; x out
+    "mg_post": lambda Np, F, C, V, A: 28.5 * A,             # 3 couplings, b, 1/diag, x, coarse x in; x out
     "extrap": lambda Np, F, C, V, A: 11 * F,                # three components, 4 layers: value + valid in; value, valid, extrapolated out
 }
 

@@ -212,7 +212,8 @@ typedef enum bnn_kernel_timer {
     BNN_KT_MOVE        = 5,
     BNN_KT_MG_PRE      = 6,  /* multigrid pre-smoother, finest level (the first V-cycle of a solve) */
     BNN_KT_MG_RESTRICT = 7,  /* residual + restriction, finest level */
-    BNN_KT_MG_PROLONG  = 8,  /* coarse-grid correction, finest level */
+    BNN_KT_MG_PROLONG  = 8,  /* coarse-grid correction of the finest level as a pass of its own (none:
+                                 the post-smoother forms it) */
     BNN_KT_MG_POST     = 9,  /* post-smoother (and z.r partials), finest level */
     BNN_KT_MG_COARSE   = 10, /* every V-cycle launch on the coarser levels */
     BNN_KT_EXTRAP      = 11, /* extrapolation (three components, four layers) in one launch */
