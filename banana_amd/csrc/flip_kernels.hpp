@@ -1918,25 +1918,35 @@ __device__ __forceinline__ double fold(const double* __restrict__ p, int n, bool
     return isMax ? block_max<1024>(a, sh) : block_sum<1024>(a, sh);
 }
 
-// The same fold by every workgroup of a consumer kernel (NT threads), for n <= kFoldMax partials: valid
+// The same sum by every workgroup of a consumer kernel (NT threads), for n <= kFoldMax partials: valid
 // in all threads and, with fold()'s order (64 consecutive partials per wavefront sum, then the sums in
 // order), the same bits. On small systems it replaces a one-block launch (2.5-3.5 us of an iteration of
 // about 90 at 64^3); reading the partials in every workgroup costs more than that launch on large ones.
 constexpr int kFoldMax = 512;
-template<int NT> __device__ __forceinline__ double fold_all(const double* __restrict__ p, int n, bool isMax, double* sh) {
+template<int NT> __device__ __forceinline__ double fold_all(const double* __restrict__ p, int n, double* sh) {
 #pragma unroll
     for(int k = 0; k < kFoldMax / NT; ++k) {
         const int    i = k * NT + (int)threadIdx.x;
-        double       v = i < n ? p[i] : 0.0;
-        v = isMax ? wave_maxd(v) : wave_sum(v);
+        const double v = wave_sum(i < n ? p[i] : 0.0);
         if((threadIdx.x & 63) == 0) sh[k * (NT / 64) + (threadIdx.x >> 6)] = v;
     }
     __syncthreads();
     double t = 0;
-    for(int w = 0; w < kFoldMax / 64; ++w) t = isMax ? fmax(t, sh[w]) : t + sh[w];
+    for(int w = 0; w < kFoldMax / 64; ++w) t += sh[w];
     __syncthreads();
     return t;
 }
+
+// max|r| of an iteration where the restriction needs it at once (the multigrid's fused update): 64 words, a
+// cache line each, that take the bricks' maxima by atomicMax on the bits of non-negative floats, which no
+// order changes. The SpMV before clears them. A fold of the bricks' partials took a launch of its own (2.4 us
+// at 1309 bricks, 4.6 at 9593, and the gap before the next) or, on small systems, reads in every workgroup
+// of the restriction (4.6 us at 216 bricks, now 4.3).
+constexpr int kMaxWords = 64, kMaxWordStep = 32;
+__device__ __forceinline__ void max_words_clear(uint32_t* w, Blk blk) {
+    if(w && blk.id == 0 && threadIdx.x < kMaxWords) w[kMaxWordStep * threadIdx.x] = 0u;
+}
+__device__ __forceinline__ void  max_words_put(uint32_t* w, uint32_t brick, float m) { atomicMax(w + kMaxWordStep * (brick % kMaxWords), __float_as_uint(m)); }
 
 // the stop test of an iteration (PCGSolver.cpp:182-187), B = max|r|. With the multigrid preconditioner it
 // runs before the V-cycle: the last iteration of a solve needs none (two thirds of an iteration's time, and
@@ -2056,20 +2066,19 @@ struct k_pcg_spmv {
     PcgState* next;
     const double* __restrict__ rz;
     int nPart;
+    uint32_t* maxWords;  // or null
     __device__ void operator()(Blk blk) const {
         __shared__ double sh[8];
         float             beta;
+        double            A = 0, be = 0;
         if(kFold && next) {
-            const bool   done = st->done != 0;
-            const double A = done ? 0.0 : fold_all<512>(rz, nPart, false, sh), be = A / st->rho;
-            if(blk.id == 0 && threadIdx.x == 0) {
-                *next = *st;
-                if(!done) {
-                    next->beta = be;
-                    next->rho  = A;
-                }
+            const bool done = st->done != 0;
+            A  = done ? 0.0 : fold_all<512>(rz, nPart, sh);
+            be = A / st->rho;
+            if(done) {
+                if(blk.id == 0 && threadIdx.x == 0) *next = *st;
+                return;
             }
-            if(done) return;
             beta = (float)be;
         } else {
             if(st->done) return;
@@ -2117,6 +2126,13 @@ struct k_pcg_spmv {
         }
         d = block_sum<512>(d, sh);
         if(threadIdx.x == 0) pa[blk.id] = d;
+        // stores to the state come last (see k_mg_residual_restrict)
+        max_words_clear(maxWords, blk);
+        if(kFold && next && blk.id == 0 && threadIdx.x == 0) {
+            *next      = *st;
+            next->beta = be;
+            next->rho  = A;
+        }
     }
 };
 
@@ -2885,7 +2901,7 @@ struct k_mg_smooth_brick {
 };
 
 // The PCG update fused with the V-cycle's first step on the finest level (multigrid): per brick,
-// x += alpha s and r -= alpha q (PCGSolver.cpp:178-181), the brick's max|r| to pm[slot], then the
+// x += alpha s and r -= alpha q (PCGSolver.cpp:178-181), the brick's max|r| to the max words, then the
 // pre-smoother on b = r, which reads only the brick's own cells (it starts from x = 0). The finest
 // level's r array is the PCG's q buffer: this brick's q is read before the smoother overwrites it.
 // Per cell the same arithmetic as k_pcg_update followed by k_mg_smooth_brick<false, false>.
@@ -2899,7 +2915,7 @@ struct k_pcg_update_pre {
     float omega;
     int sweeps;
     PcgState* st;
-    double* __restrict__ pm;
+    uint32_t* maxWords;
     const double* __restrict__ sq;
     int nPart;
     __device__ void operator()(Blk blk) const {
@@ -2908,22 +2924,21 @@ struct k_pcg_update_pre {
         if(st->done) return;
         const int t     = threadIdx.x;
         float     alpha = 0.f;
+        double    A = 0, al = 0;
         if(kFold) {
-            // the first workgroup records it in the state; the others read only rho, which stays, and a
-            // stop flag set meanwhile ends them just as their own sum does
-            const double A  = fold_all<256>(sq, nPart, false, sh);
-            const bool   ok = !(A < (double)kFltMin);
-            const double al = st->rho / A;
-            if(blk.id == 0 && t == 0) {
-                st->tmp = A;
-                if(ok) st->alpha = al;
-                else {
+            // the first workgroup records it in the state, at the end (see k_mg_residual_restrict); the others
+            // read only rho, which stays, and a stop flag set meanwhile ends them just as their own sum does
+            A  = fold_all<256>(sq, nPart, sh);
+            al = st->rho / A;
+            if(A < (double)kFltMin) {
+                if(blk.id == 0 && t == 0) {
+                    st->tmp     = A;
                     st->done    = 1;
                     st->success = 1;
                     st->iter += 1;
                 }
+                return;
             }
-            if(!ok) return;
             alpha = (float)al;
         } else {
             alpha = (float)st->alpha;
@@ -2939,8 +2954,12 @@ struct k_pcg_update_pre {
             store2(x, o, xv);
             store2(L.b, o, rv);
             const double m = block_max<256>(fmax((double)fabsf(rv.x), (double)fabsf(rv.y)), sh);
-            if(t == 0) pm[slot] = m;
             mg_smooth_one<false, false>(L, L, omega, sweeps, nullptr, slot, c, rv, xs, sh);
+            if(t == 0) max_words_put(maxWords, v, (float)m);
+        }
+        if(kFold && blk.id == 0 && t == 0) {
+            st->tmp   = A;
+            st->alpha = al;
         }
     }
 };
@@ -2950,24 +2969,33 @@ struct k_pcg_update_pre {
 // fine brick writes the 64 coarse cells it covers; r itself is never stored. Coarse cells without an
 // active child brick keep the zeros they get when the hierarchy is built. A thread's pair of cells and its
 // partners in the group, lanes ^ 4 and ^ 32, form the sum.
-// kStop (finest level, small systems): first the iteration's stop test over nPart <= kFoldMax partials rm
-// of max|r|; the first workgroup records it, the others read only what it leaves alone.
+// kStop (finest level, after a fused update): first the iteration's stop test, on the max words; the first
+// workgroup records it, the others read only what it leaves alone. It does so at the end: after a store to
+// the state the compiler loads the tables, which may overlap it for all it knows, by vector instructions
+// (the restriction of 9593 bricks 13.7 -> 30 us).
+// At most kMaxRedBlocks workgroups take the bricks in turn then, for the words' read before the first: 19.8 us
+// at 9593 bricks against 22.8 with a workgroup a brick.
 template<bool kStop>
 struct k_mg_residual_restrict {
     static constexpr int kThreads = 256;
     LevelDev F;
     LevelDev C;
     PcgState* st;
-    const double* __restrict__ rm;
-    int nPart;
+    const uint32_t* maxWords;
     __device__ void operator()(Blk blk) const {
-        if(st && st->done) return;
         const int t = threadIdx.x;
+        float     B = 0.f;
         if(kStop) {
-            __shared__ double sh[8];
-            const double      B = fold_all<256>(rm, nPart, true, sh);
-            if(blk.id == 0 && t == 0) pcg_stop_test(*st, B);
-            if((float)B < st->tol) return;
+            const float    w = __uint_as_float(maxWords[kMaxWordStep * (t & 63)]), tol = st->tol;
+            const uint32_t done = st->done;
+            if(done) return;
+            B = wave_max(w);
+            if(B < tol) {
+                if(blk.id == 0 && t == 0) pcg_stop_test(*st, B);
+                return;
+            }
+        } else if(st && st->done) {
+            return;
         }
         const BrickPair c(t);
         for(uint32_t v = blk.id; v < F.nSlots; v += blk.n) {
@@ -2997,6 +3025,7 @@ struct k_mg_residual_restrict {
             const int32_t cs = F.ptab[8 * s + 6];
             if(!(c.ly & 1) && !(c.lz & 1) && cs >= 0) C.b[cs * 512 + c.parent(F.ptab[8 * s + 7])] = sum;
         }
+        if(kStop && blk.id == 0 && t == 0) pcg_stop_test(*st, B);
     }
 };
 

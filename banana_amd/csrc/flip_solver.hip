@@ -294,6 +294,7 @@ public:
     DevBuf   x64prev, prevBrickSlot;  // the last refined solve's pressure and brick -> slot table
     bool     prevPressure = false;   // they hold a converged pressure of this grid
     bool     warmNext     = false;   // this solve starts from them (x64 filled by k_warm_start)
+    DevBuf   maxWords;              // max|r| of an iteration (max_words_put)
     DevBuf   pa, pb, pz, pst;       // PCG partials (per block: pa, pb; per brick: pz), device states
     DevBuf   icInv, icLx, icLy, icLz;  // IC(0) factor (BNN_PRECOND_IC0 only)
     SolveState* hostSolve = nullptr;  // pinned
@@ -421,6 +422,7 @@ public:
         slotBrick.reserve(nb * 4);
         brickSlot.reserve(nb * 4);
         pst.reserve(sizeof(SolveState));
+        maxWords.reserve(kMaxWords * kMaxWordStep * 4);
         // zero everything the reference zero-fills at resize (PIC_Data.cpp:101-117)
         for(auto* b : {&u, &v, &w, &ut, &vt, &wt, &uo, &vo, &wo, &wu, &wv, &ww, &vu, &vv, &vw, &eu, &ev_, &ew, &phi, &bsdf,
                        &cellStart, &cellCount, &counters, &pst})
@@ -447,7 +449,7 @@ public:
         nbrTab.reserve((size_t)c * 6 * 4);
         uniFlag.reserve((size_t)c * 4);
         pa.reserve((size_t)kMaxRedBlocks * 8);
-        pb.reserve((size_t)std::max<uint32_t>(kMaxRedBlocks, c) * 8);  // per block, or per brick (k_pcg_update_pre)
+        pb.reserve((size_t)kMaxRedBlocks * 8);  // per block
         pz.reserve((size_t)c * 8);
         if(prm.preconditioner == BNN_PRECOND_IC0)
             for(auto* b : {&icInv, &icLx, &icLy, &icLz}) b->reserve(nv * 4);
@@ -984,9 +986,9 @@ public:
     // One block per brick. On each level the pre-smoothed x lives in L.r and the final x in L.x.
     // Returns true when the fine level's post-smoother also wrote the per-brick partials of z.r to pz
     // (false when the fine level is the coarsest: the caller then forms z.r itself).
-    // finePreDone: the finest level's pre-smoother already ran (fused with the PCG update). stopPart: the
-    // iteration's stop test runs in the finest restriction, over these per-brick partials of max|r|.
-    bool vcycle(PcgState* stp, bool finePreDone = false, const double* stopPart = nullptr) {
+    // finePreDone: the finest level's pre-smoother already ran (fused with the PCG update);
+    // the iteration's stop test then runs in the finest restriction.
+    bool vcycle(PcgState* stp, bool finePreDone = false) {
         const int   nu    = prm.mg_sweeps;
         const float omega = prm.mg_omega;
         const int   tail  = mgTail();
@@ -1000,8 +1002,8 @@ public:
                 ktEnd(l == 0 ? BNN_KT_MG_PRE : BNN_KT_MG_COARSE);
             }
             ktBegin(l == 0 ? BNN_KT_MG_RESTRICT : BNN_KT_MG_COARSE);
-            if(l == 0 && stopPart) launch(k_mg_residual_restrict<true>{L, C, stp, stopPart, (int)L.nSlots}, G);
-            else launch(k_mg_residual_restrict<false>{L, C, stp, nullptr, 0}, G);
+            if(l == 0 && finePreDone) launch(k_mg_residual_restrict<true>{L, C, stp, maxWords.as<uint32_t>()}, redBlocks());
+            else launch(k_mg_residual_restrict<false>{L, C, stp, nullptr}, G);
             ktEnd(l == 0 ? BNN_KT_MG_RESTRICT : BNN_KT_MG_COARSE);
         }
         ktBegin(BNN_KT_MG_COARSE);
@@ -1108,11 +1110,11 @@ public:
         int           nrz = (int)G;
         const bool    ic0 = prm.preconditioner == BNN_PRECOND_IC0;
         if(ic0) formIC0();
-        auto          zr  = [&](PcgState* stp, bool finePreDone, const double* stopPart = nullptr) {
+        auto          zr  = [&](PcgState* stp, bool finePreDone) {
             if(ic0) {
                 applyIC0(r.as<float>(), z.as<float>(), stp);
                 launch(k_pcg_dot_zr{(const float*)z.as<float>(), (const float*)r.as<float>(), nSlots, stp, dpa}, G);
-            } else if(vcycle(stp, finePreDone, stopPart)) {
+            } else if(vcycle(stp, finePreDone)) {
                 rz  = pz.as<double>();
                 nrz = (int)nSlots;
             } else {
@@ -1120,8 +1122,8 @@ public:
             }
         };
         if(!jac) zr(nullptr, false);
-        // multigrid over several levels: the update is fused with the finest pre-smoother, and its
-        // max|r| partials are per brick
+        // multigrid over several levels: the update is fused with the finest pre-smoother, its max|r| goes
+        // to the max words
         const bool fuseUpdate = !jac && !ic0 && mgLevels > 1;
         // small systems alone: the folds of alpha and beta run inside the kernels that use them. In a batch
         // a launch is shared by all scenes, and mixing both forms splits it: 48 scenes took 13.65 ms a
@@ -1163,7 +1165,8 @@ public:
                 ktBegin(BNN_KT_PCG_SPMV);
                 auto spmv = [&](auto k) {
                     k = {nbrTab.as<int32_t>(), z.as<float>(), sA, sB, q.as<float>(), diag32.as<float>(), cx32.as<float>(), cy32.as<float>(),
-                         cz32.as<float>(), uniRow, nSlots, dst, dpa, endLast ? alt_ : nullptr, rz, (int)nSlots};
+                         cz32.as<float>(), uniRow, nSlots, dst, dpa, endLast ? alt_ : nullptr, rz, (int)nSlots,
+                         fuseUpdate ? maxWords.as<uint32_t>() : nullptr};
                     launch(k, G);
                 };
                 if(folded) spmv(k_pcg_spmv<true>{});
@@ -1173,7 +1176,7 @@ public:
                 if(!folded) launch(k_pcg_alpha{dst, (const double*)dpa, (int)G}, 1);
                 ktBegin(BNN_KT_PCG_UPDATE);
                 auto updatePre = [&](auto k) {
-                    k = {sB, x.as<float>(), fineLevel(), prm.mg_omega, prm.mg_sweeps, dst, dpb, dpa, (int)G};
+                    k = {sB, x.as<float>(), fineLevel(), prm.mg_omega, prm.mg_sweeps, dst, maxWords.as<uint32_t>(), dpa, (int)G};
                     launch(k, std::max<uint32_t>(nSlots, 1u));
                 };
                 if(folded) updatePre(k_pcg_update_pre<true>{});
@@ -1181,9 +1184,8 @@ public:
                 else
                     launch(k_pcg_update{(const float*)sB, (const float*)q.as<float>(), (const float*)invd.as<float>(), x.as<float>(), r.as<float>(), z.as<float>(), nSlots, (const PcgState*)dst, dpa, dpb, jac}, G);
                 ktEnd(BNN_KT_PCG_UPDATE);
-                if(fuseUpdate) {  // the stop test comes before the V-cycle
-                    if(!folded) launch(k_pcg_beta{dst, nullptr, 0, (const double*)dpb, (int)nSlots}, 1);
-                    zr(dst, true, folded ? (const double*)dpb : nullptr);
+                if(fuseUpdate) {  // the stop test is in the V-cycle's first restriction
+                    zr(dst, true);
                     if(!folded || c + 1 == n) launch(k_pcg_beta{dst, rz, nrz, nullptr, 0}, 1);
                 } else {
                     if(!jac) zr(dst, false);
