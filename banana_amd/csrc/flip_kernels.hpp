@@ -1769,9 +1769,9 @@ struct SystemOut {
 // bricks, and the kernels that stream the finest level take the row from here instead of reading it: 4 of
 // 8 words a cell of the SpMV, 32 of 52 bytes of the FP64 residual. Same values, same bits. At 256^3 (9593
 // bricks, about 60% of them uniform): SpMV 31.5 -> 27.8 us, update 38.1 -> 34.2, post-smoother 41.3 ->
-// 34.9, FP64 residual 69.7 -> 49.5. The restriction, bound by its instructions, and the prolongation keep
-// their own times, but the rows they leave unread stay out of the caches: without them in it the step
-// gained 0.24 of 14.7 ms, with them 0.44. The flag comes before the row in a dependent chain, 0.5 us of
+// 34.9, FP64 residual 69.7 -> 49.5 (before the kernels took pairs of cells). The restriction, bound by its
+// instructions, kept its own time, but the rows it leaves unread stay out of the caches: without it in this
+// the step gained 0.24 of 14.7 ms, with it 0.44. The flag comes before the row in a dependent chain, 0.5 us of
 // the 4.6 us an SpMV of 216 bricks takes: systems of up to kUniformMin bricks read every row (at 567
 // neither wins).
 constexpr uint32_t kUniformMin = 1024;
@@ -2684,12 +2684,13 @@ __device__ __forceinline__ uint32_t xcd_slot(uint32_t b, uint32_t n) {
 constexpr int kTileRow = 12, kTilePlane = 120, kTile = 1200;
 __device__ __forceinline__ int tile_index(int lx, int ly, int lz) { return (lz + 1) * kTilePlane + (ly + 1) * kTileRow + lx + 1; }
 
-// The smoothers, the restriction and the prolongation work on pairs of cells: their loads, a cell each, were
+// The smoothers and the restriction work on pairs of cells: their loads, a cell each, were
 // what bounded them (a load of 64 floats costs a CU 10 to 20 cycles however few bytes it moves; a pair takes
 // half as many), and below some hundred bricks the steps from brick to parent in a launch. As pairs, with
 // the parities and parents of the brick tables: at 216 / 9593 bricks update with pre-smoother 7.3 / 35.2 ->
-// 5.8 / 31.9 us, restriction 6.4 / 18.6 -> 4.6 / 14.1, post-smoother 6.9 / 33.7 -> 6.0 / 33.3,
-// prolongation (9593) 14.7 -> 13.2, the 64^3 step 1.90 -> 1.83 ms, 256^3 14.15 -> 13.85.
+// 5.8 / 31.9 us, restriction 6.4 / 18.6 -> 4.6 / 14.1 (before it took the stop test), post-smoother 6.9 / 33.7
+// -> 6.0 / 33.3 (before it took the correction), the 64^3 step 1.90 -> 1.83 ms, 256^3 14.15 -> 13.85. (The
+// SpMV, bound by latency and by the wavefronts in flight, lost as pairs: 27.8 -> 33.5 us.)
 
 // The x-adjacent pair of cells that thread t of a brick's 256 owns, one of each colour: even is the first
 // one's index in the brick, cr and cb the red (colour 0) and the black one's tile entries, offR the tile

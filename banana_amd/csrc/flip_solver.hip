@@ -288,7 +288,8 @@ public:
     // bricks + pressure system
     uint32_t nb = 0, nSlots = 0, slotCap = 0, nFluid = 0;
     DevBuf   bflag, brickSlot, slotBrick, nbrTab, uniFlag;
-    UniformRow uniRow{};  // the current system's
+    float    uniDt = 0.f;  // time step of the current system
+    UniformRow uniRow() const { return UniformRow(nSlots > kUniformMin ? uniFlag.as<int32_t>() : nullptr, uniDt); }
     DevBuf   x, r, z, s0, s1, q, rhs32, diag32, cx32, cy32, cz32, invd;
     DevBuf   rhs64, diag64, cx64, cy64, cz64, x64;
     DevBuf   x64prev, prevBrickSlot;  // the last refined solve's pressure and brick -> slot table
@@ -875,7 +876,7 @@ public:
         SystemOut  S{rhs64.as<double>(), refined ? diag64.as<double>() : nullptr, refined ? cx64.as<double>() : nullptr,
                     refined ? cy64.as<double>() : nullptr, refined ? cz64.as<double>() : nullptr, rhs32.as<float>(), diag32.as<float>(),
                     cx32.as<float>(), cy32.as<float>(), cz32.as<float>(), invd.as<float>(), uniFlag.as<int32_t>()};
-        uniRow = UniformRow(nSlots > kUniformMin ? uniFlag.as<int32_t>() : nullptr, dt);
+        uniDt = dt;
         VelGrid G{u.as<float>(), v.as<float>(), w.as<float>()};
         launch(k_assemble{(const int32_t*)slotBrick.as<int32_t>(), g, (const float*)phi.as<float>(), G, (const float*)wu.as<float>(), (const float*)wv.as<float>(), (const float*)ww.as<float>(), dt, S}, nSlots);
         if(warmNext) {
@@ -908,7 +909,7 @@ public:
     LevelDev fineLevel() {
         return LevelDev{g.nx, g.ny, g.nz, g.nbx, g.nby, g.nbz, brickSlot.as<int32_t>(), slotBrick.as<int32_t>(), nbrTab.as<int32_t>(),
                         diag32.as<float>(), cx32.as<float>(), cy32.as<float>(), cz32.as<float>(), invd.as<float>(),
-                        z.as<float>(), r.as<float>(), q.as<float>(), nSlots, ptab0.as<int32_t>(), uniRow};
+                        z.as<float>(), r.as<float>(), q.as<float>(), nSlots, ptab0.as<int32_t>(), uniRow()};
     }
     LevelDev levelDev(int l) {
         if(l == 0) return fineLevel();
@@ -1085,7 +1086,7 @@ public:
     // the outer pass around an inner solve: x64 += (or =, zeroX) x, then the residual's fold
     void residualPass(int zeroX, const PcgState* gate) {
         const unsigned G = redBlocks();
-        launch(k_residual64{(const int32_t*)nbrTab.as<int32_t>(), (const double*)x64.as<double>(), (const double*)rhs64.as<double>(), (const double*)diag64.as<double>(), (const double*)cx64.as<double>(), (const double*)cy64.as<double>(), (const double*)cz64.as<double>(), uniRow, rhs32.as<float>(), nSlots, pa.as<double>(), pb.as<double>(), zeroX, gate}, G);
+        launch(k_residual64{(const int32_t*)nbrTab.as<int32_t>(), (const double*)x64.as<double>(), (const double*)rhs64.as<double>(), (const double*)diag64.as<double>(), (const double*)cx64.as<double>(), (const double*)cy64.as<double>(), (const double*)cz64.as<double>(), uniRow(), rhs32.as<float>(), nSlots, pa.as<double>(), pb.as<double>(), zeroX, gate}, G);
         launch(k_residual64_fin{&pst.as<SolveState>()->outer, (const double*)pa.as<double>(), (const double*)pb.as<double>(), (int)G, gate}, 1);
     }
     void accumulatePass(int zeroX, const PcgState* gate) {
@@ -1165,7 +1166,7 @@ public:
                 ktBegin(BNN_KT_PCG_SPMV);
                 auto spmv = [&](auto k) {
                     k = {nbrTab.as<int32_t>(), z.as<float>(), sA, sB, q.as<float>(), diag32.as<float>(), cx32.as<float>(), cy32.as<float>(),
-                         cz32.as<float>(), uniRow, nSlots, dst, dpa, endLast ? alt_ : nullptr, rz, (int)nSlots,
+                         cz32.as<float>(), uniRow(), nSlots, dst, dpa, endLast ? alt_ : nullptr, rz, (int)nSlots,
                          fuseUpdate ? maxWords.as<uint32_t>() : nullptr};
                     launch(k, G);
                 };
