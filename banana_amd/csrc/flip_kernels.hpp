@@ -1920,19 +1920,29 @@ __device__ __forceinline__ double fold(const double* __restrict__ p, int n, bool
 
 // The same sum by every workgroup of a consumer kernel (NT threads), for n <= kFoldMax partials: valid
 // in all threads and, with fold()'s order (64 consecutive partials per wavefront sum, then the sums in
-// order), the same bits. On small systems it replaces a one-block launch (2.5-3.5 us of an iteration of
-// about 90 at 64^3); reading the partials in every workgroup costs more than that launch on large ones.
-constexpr int kFoldMax = 512;
+// order), the same bits; sh holds kFoldMax / 64 sums. On small systems it replaces a one-block launch
+// (2.5-3.5 us of an iteration of about 90 at 64^3). With the parts past n skipped it does so up to 1024
+// bricks: 567 bricks 2490 -> 2410 us a substep, 623 2850 -> 2800; at 1309 the launch is the cheaper
+// (a 128^3 frame 16.1 -> 16.4 ms with the limit at 2048).
+constexpr int kFoldMax = 1024;
 template<int NT> __device__ __forceinline__ double fold_all(const double* __restrict__ p, int n, double* sh) {
+    double v[kFoldMax / NT];
 #pragma unroll
     for(int k = 0; k < kFoldMax / NT; ++k) {
-        const int    i = k * NT + (int)threadIdx.x;
-        const double v = wave_sum(i < n ? p[i] : 0.0);
-        if((threadIdx.x & 63) == 0) sh[k * (NT / 64) + (threadIdx.x >> 6)] = v;
+        const int i = k * NT + (int)threadIdx.x;
+        v[k]        = 0.0;
+        if(k * NT < n) v[k] = i < n ? p[i] : 0.0;
     }
+#pragma unroll
+    for(int k = 0; k < kFoldMax / NT; ++k)
+        if(k * NT < n) {
+            const double s = wave_sum(v[k]);
+            if((threadIdx.x & 63) == 0) sh[k * (NT / 64) + (threadIdx.x >> 6)] = s;
+        }
     __syncthreads();
-    double t = 0;
-    for(int w = 0; w < kFoldMax / 64; ++w) t += sh[w];
+    double    t = 0;
+    const int m = (n + NT - 1) / NT * (NT / 64);
+    for(int w = 0; w < m; ++w) t += sh[w];
     __syncthreads();
     return t;
 }
@@ -2068,7 +2078,7 @@ struct k_pcg_spmv {
     int nPart;
     uint32_t* maxWords;  // or null
     __device__ void operator()(Blk blk) const {
-        __shared__ double sh[8];
+        __shared__ double sh[kFoldMax / 64];
         float             beta;
         double            A = 0, be = 0;
         if(kFold && next) {
@@ -2921,7 +2931,7 @@ struct k_pcg_update_pre {
     int nPart;
     __device__ void operator()(Blk blk) const {
         __shared__ __align__(16) float xs[kTile];
-        __shared__ double sh[8];
+        __shared__ double sh[kFoldMax / 64];
         if(st->done) return;
         const int t     = threadIdx.x;
         float     alpha = 0.f;
