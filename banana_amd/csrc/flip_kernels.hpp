@@ -2932,15 +2932,19 @@ struct k_pcg_update_pre {
     __device__ void operator()(Blk blk) const {
         __shared__ __align__(16) float xs[kTile];
         __shared__ double sh[kFoldMax / 64];
-        if(st->done) return;
-        const int t     = threadIdx.x;
-        float     alpha = 0.f;
-        double    A = 0, al = 0;
+        const int  t     = threadIdx.x;
+        const bool done  = st->done != 0;
+        float      alpha = 0.f;
+        double     A = 0, al = 0;
         if(kFold) {
-            // the first workgroup records it in the state, at the end (see k_mg_residual_restrict); the others
-            // read only rho, which stays, and a stop flag set meanwhile ends them just as their own sum does
+            // The first workgroup records alpha in the state, at the end (see k_mg_residual_restrict), or the
+            // stop when the sum ends the solve. That store may fall between the reads of the flag by two waves
+            // of another workgroup, so every wave takes part in the fold, whatever it read, and leaves by the
+            // sum: one that saw the stop of this launch has the same sum in front of it as one that did not.
+            // (Leaving before it, a wave would miss its part of the fold.) A stop of an earlier launch is seen by all.
             A  = fold_all<256>(sq, nPart, sh);
             al = st->rho / A;
+            if(done) return;
             if(A < (double)kFltMin) {
                 if(blk.id == 0 && t == 0) {
                     st->tmp     = A;
@@ -2952,6 +2956,7 @@ struct k_pcg_update_pre {
             }
             alpha = (float)al;
         } else {
+            if(done) return;
             alpha = (float)st->alpha;
         }
         const BrickPair c(t);
@@ -2981,9 +2986,10 @@ struct k_pcg_update_pre {
 // active child brick keep the zeros they get when the hierarchy is built. A thread's pair of cells and its
 // partners in the group, lanes ^ 4 and ^ 32, form the sum.
 // kStop (finest level, after a fused update): first the iteration's stop test, on the max words; the first
-// workgroup records it, the others read only what it leaves alone. It does so at the end: after a store to
-// the state the compiler loads the tables, which may overlap it for all it knows, by vector instructions
-// (the restriction of 9593 bricks 13.7 -> 30 us).
+// workgroup records it. A wave of another workgroup that sees the stop it records leaves early, which is no
+// matter: the V-cycle ends with this iteration, and no wave here waits for another. It records it at the end:
+// after a store to the state the compiler loads the tables, which may overlap it for all it knows, by vector
+// instructions (the restriction of 9593 bricks 13.7 -> 30 us).
 // At most kMaxRedBlocks workgroups take the bricks in turn then, for the words' read before the first: 19.8 us
 // at 9593 bricks against 22.8 with a workgroup a brick.
 template<bool kStop>
