@@ -919,14 +919,16 @@ public:
                         L.x.as<float>(), L.b.as<float>(), L.r.as<float>(), L.nSlots, L.ptab.as<int32_t>(), UniformRow{}};
     }
 
-    // the coarse levels' grids: each halves the one before until every axis fits one brick
+    // the coarse levels' grids: each halves the one before until every axis fits one brick. Kept only when
+    // every buffer was to be had: the next solve starts over otherwise
     void setupLevels() {
         if(!mg.empty()) return;
-        mg.emplace_back(nullptr);
+        decltype(mg) lv;
+        lv.emplace_back(nullptr);
         int nx = g.nx, ny = g.ny, nz = g.nz;
-        while((nx > 8 || ny > 8 || nz > 8) && (int)mg.size() < kMaxMgLevels) {
-            mg.emplace_back(new MgLevel());
-            MgLevel& L = *mg.back();
+        while((nx > 8 || ny > 8 || nz > 8) && (int)lv.size() < kMaxMgLevels) {
+            lv.emplace_back(new MgLevel());
+            MgLevel& L = *lv.back();
             nx = (nx + 1) / 2;
             ny = (ny + 1) / 2;
             nz = (nz + 1) / 2;
@@ -936,8 +938,9 @@ public:
             L.flag.reserve(L.nb * 4);
             L.brickSlot.reserve(L.nb * 4);
             L.slotBrick.reserve(L.nb * 4);
-            fill32(L.flag.p, 0, L.nb * 4);
         }
+        mg.swap(lv);
+        for(size_t l = 1; l < mg.size(); ++l) fill32(mg[l]->flag.p, 0, mg[l]->nb * 4);
     }
     // the levels in use (until one brick remains) and their buffers, from the counts in hostU32[1 + l]
     void sizeLevels(int nCand) {

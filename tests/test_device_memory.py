@@ -1,0 +1,80 @@
+"""What a scene holds of device memory, on the host alone: libbnn_flip.so over a stand-in HIP runtime
+(hip_host_stub.c) that counts allocations and makes a chosen one fail. Kernels do not run; the counts of
+active bricks that they would give are set by the test."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+
+
+@pytest.fixture(scope="module")
+def run(bnn, tmp_path_factory):
+    lib = str(tmp_path_factory.mktemp("stub") / "libhipstub.so")
+    subprocess.check_call(["gcc", "-O1", "-shared", "-fPIC", "-w", "-Wl,-soname,libamdhip64.so.7", "-o", lib,
+                           os.path.join(HERE, "hip_host_stub.c")])
+    head = f"""
+import ctypes as C, sys
+stub = C.CDLL({lib!r}, mode=C.RTLD_GLOBAL)
+stub.stub_live_bytes.restype = C.c_size_t
+sys.path.insert(0, {os.path.dirname(HERE)!r})
+import numpy as np
+import banana_amd
+from banana_amd import scenes
+from banana_amd.serving import footprint
+
+def levels(n):  # the brick grids of the multigrid levels, finest first
+    out = [n]
+    while max(n) > 8:
+        n = tuple((a + 1) // 2 for a in n)
+        out.append(n)
+    return [int(np.prod([(a + 7) // 8 for a in n])) for n in out]
+
+def all_bricks(n):  # the counters after a scene whose every brick holds fluid
+    l = levels(n)
+    c = np.array([512 * l[0]] + l, np.uint32)
+    stub.stub_set_counts(c.ctypes.data_as(C.POINTER(C.c_uint32)), len(c))
+
+def scene(cells=(40, 30, 20), **kw):
+    params = scenes.base_params(64)
+    params.update(box_max=tuple(c / 64 for c in cells), **kw)
+    return params, banana_amd.FLIPSolver(params)
+"""
+
+    def go(body):
+        r = subprocess.run([sys.executable, "-c", head + body], capture_output=True, text=True, timeout=120)
+        assert r.returncode == 0, r.stdout + r.stderr[-2000:]
+        return r.stdout
+    return go
+
+
+def test_projection_after_running_out_of_memory(run):
+    """A projection that fails for want of memory at any of its allocations, called again when there is
+    memory, holds all the buffers that one does which never failed (one left out would be a null pointer in
+    a kernel)."""
+    run("""
+def project(fail):
+    params, g = scene(pressure_mode=1)  # a zero residual ends the solve before its first iteration
+    g.set_particles(np.full((1, 3), 0.1, np.float32), np.zeros((1, 3), np.float32))
+    all_bricks(g.n)
+    stub.stub_fail_at(fail)
+    if fail >= 0:
+        try:
+            g.pressure_projection(1e-3)
+            raise SystemExit(f"allocation {fail} did not fail")
+        except banana_amd.BnnError as e:
+            assert e.status == 4, e
+        stub.stub_fail_at(-1)
+    g.pressure_projection(1e-3)
+    made, held = stub.stub_mallocs(), stub.stub_live_bytes()
+    g.close()
+    assert stub.stub_live_bytes() == 0
+    return made, held
+
+made, held = project(-1)
+assert made > 20
+for k in range(made):
+    assert project(k)[1] == held, (k, made)
+""")
