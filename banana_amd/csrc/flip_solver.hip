@@ -435,6 +435,8 @@ public:
     void ensureParticles(uint64_t n) {
         if(n <= cap) return;
         const uint64_t c = n + n / 8 + 1024;
+        cap = np = 0;  // growing gives the old buffers up: nothing is left of them where it fails
+        binned = false;
         bufA.reserve(c, affineScheme());
         bufB.reserve(c, affineScheme());
         key.reserve(c * 4);
@@ -446,6 +448,7 @@ public:
         if(n <= slotCap && slotCap) return;
         const uint32_t c  = std::max<uint32_t>(n + n / 4 + 16, 64);
         const size_t   nv = (size_t)c * 512;
+        slotCap = 0;  // set again when every buffer is there
         for(auto* b : {&x, &r, &z, &s0, &s1, &q, &rhs32, &diag32, &cx32, &cy32, &cz32, &invd}) b->reserve(nv * 4);
         nbrTab.reserve((size_t)c * 6 * 4);
         uniFlag.reserve((size_t)c * 4);
@@ -826,6 +829,7 @@ public:
             x64prev.swapWith(x64);
         }
         prevPressure = false;
+        systemValid  = false;  // until the new one stands
         // the active bricks of every level, counted with one wait
         const bool mgp = prm.preconditioner == BNN_PRECOND_MG;
         if(mgp) setupLevels();
@@ -953,6 +957,7 @@ public:
             if(L.nSlots > L.slotCap) {
                 const uint32_t c  = L.nSlots + L.nSlots / 4 + 4;
                 const size_t   nv = (size_t)c * 512 * 4;
+                L.slotCap = 0;
                 for(DevBuf* b : {&L.diag, &L.cx, &L.cy, &L.cz, &L.inv, &L.x, &L.b, &L.r}) b->reserve(nv);
                 L.nbr.reserve((size_t)c * 24);
                 L.slotCap = c;

@@ -26,6 +26,11 @@ void stub_fail_at(long n) {
 }
 long   stub_mallocs(void) { return mallocs; } /* since stub_fail_at */
 size_t stub_live_bytes(void) { return live; }
+long   stub_live_blocks(void) {
+    long n = 0;
+    for(int i = 0; i < kMaxBlocks; ++i) n += block[i] != NULL;
+    return n;
+}
 /* what a copy to the host of exactly n words reads (the active bricks' counters) */
 void stub_set_counts(const uint32_t* v, uint32_t n) {
     memcpy(counts, v, 4 * (size_t)n);

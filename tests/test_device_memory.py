@@ -37,6 +37,11 @@ def all_bricks(n):  # the counters after a scene whose every brick holds fluid
     c = np.array([512 * l[0]] + l, np.uint32)
     stub.stub_set_counts(c.ctypes.data_as(C.POINTER(C.c_uint32)), len(c))
 
+def few_bricks(n):  # ... two bricks of it, below one on each coarser level
+    c = np.ones(1 + len(levels(n)), np.uint32)
+    c[1] = 2
+    stub.stub_set_counts(c.ctypes.data_as(C.POINTER(C.c_uint32)), len(c))
+
 def scene(cells=(40, 30, 20), **kw):
     params = scenes.base_params(64)
     params.update(box_max=tuple(c / 64 for c in cells), **kw)
@@ -77,4 +82,65 @@ made, held = project(-1)
 assert made > 20
 for k in range(made):
     assert project(k)[1] == held, (k, made)
+""")
+
+
+def test_smaller_projection_after_a_larger_ran_out_of_memory(run):
+    """Buffers that a growing system gave up before it ran out are had again by the next one, however small."""
+    run("""
+def project(fail):
+    params, g = scene(pressure_mode=1)
+    g.set_particles(np.full((1, 3), 0.1, np.float32), np.zeros((1, 3), np.float32))
+    few_bricks(g.n)
+    g.pressure_projection(1e-3)
+    small = stub.stub_live_blocks()
+    all_bricks(g.n)
+    stub.stub_fail_at(fail)
+    if fail >= 0:
+        try:
+            g.pressure_projection(1e-3)
+            raise SystemExit(f"allocation {fail} did not fail")
+        except banana_amd.BnnError as e:
+            assert e.status == 4, e
+        stub.stub_fail_at(-1)
+        few_bricks(g.n)
+    g.pressure_projection(1e-3)
+    assert stub.stub_live_blocks() >= small, fail
+    made = stub.stub_mallocs()
+    g.close()
+    return made
+
+made = project(-1)
+assert made > 20
+for k in range(made):
+    project(k)
+""")
+
+
+def test_fewer_particles_after_more_ran_out_of_memory(run):
+    """The same for the particle buffers."""
+    run("""
+def put(g, n):
+    g.set_particles(np.full((n, 3), 0.1, np.float32), np.zeros((n, 3), np.float32))
+
+def fill(fail):
+    params, g = scene(transfer_scheme=2)
+    put(g, 1)
+    stub.stub_fail_at(fail)
+    if fail >= 0:
+        try:
+            put(g, 10000)
+            raise SystemExit(f"allocation {fail} did not fail")
+        except banana_amd.BnnError as e:
+            assert e.status == 4, e
+        stub.stub_fail_at(-1)
+    put(g, 1 if fail >= 0 else 10000)
+    made, held = stub.stub_mallocs(), stub.stub_live_blocks()
+    g.close()
+    return made, held
+
+made, held = fill(-1)
+assert made > 20
+for k in range(made):
+    assert fill(k)[1] == held, (k, made)
 """)
