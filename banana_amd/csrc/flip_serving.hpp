@@ -23,29 +23,42 @@
 namespace bnn {
 
 // device bytes a FlipSolver with these parameters and n particles may hold: the grid, particles
-// and the pressure system sized for every brick active (its largest size)
+// and the pressure system sized for every brick active (its largest size), as allocGrid, ensureParticles,
+// ensureSlots, the multigrid levels, the warm start and the z-sort reserve them
 static size_t scene_footprint(const bnn_flip_params& prm, uint64_t n) {
     const GridDims G = grid_dims(prm);
     const size_t   nx = G.n[0], ny = G.n[1], nz = G.n[2];
     const size_t   C = nx * ny * nz, N = (nx + 1) * (ny + 1) * (nz + 1);
     const size_t   nU = (nx + 1) * ny * nz, nV = nx * (ny + 1) * nz, nW = nx * ny * (nz + 1), F = nU + nV + nW;
-    size_t         nbx = (nx + 7) / 8, nby = (ny + 7) / 8, nbz = (nz + 7) / 8, nb = nbx * nby * nbz;
-    size_t         b = 16 * F + 2 * F + 12 * C + 4 * N + 4 + 4 * (blocks(std::max(C, nb), kScanTile) + 1) + nb +
-               256 + 12 * nb + 2 * sizeof(PcgState);
-    const size_t slotsCap = nb + nb / 4 + 16;
-    b += 12 * 4 * 512 * slotsCap + 28 * slotsCap + 2 * 8 * kMaxRedBlocks;
-    b += (prm.pressure_mode == BNN_PRESSURE_REFINED ? 6 : 1) * 8 * 512 * slotsCap;
+    const size_t   nbx = (nx + 7) / 8, nby = (ny + 7) / 8, nbz = (nz + 7) / 8, nb = nbx * nby * nbz;
+    const size_t   scanWords = blocks(std::max(C, nb), kScanTile) + 1;
+    size_t         b = 16 * F + 2 * F + 12 * C + 4 + 4 * N + 4 * scanWords + 256 + 12 * nb + (nb + 3) / 4 * 4 + sizeof(SolveState) +
+               4 * kMaxWords * kMaxWordStep;
+    const size_t slots = std::max<size_t>(nb + nb / 4 + 16, 64), vec = 512 * slots;
+    b += 12 * 4 * vec + (24 + 4 + 8) * slots + 2 * 8 * kMaxRedBlocks;  // neighbours, uniform flags, z.r partials
+    const bool refined = prm.pressure_mode == BNN_PRESSURE_REFINED;
+    b += (refined ? 6 : 1) * 8 * vec;
+    if(refined && prm.warm_start) b += 8 * vec + 4 * nb;
+    if(prm.preconditioner == BNN_PRECOND_IC0) b += 4 * 4 * vec;
     if(prm.preconditioner == BNN_PRECOND_MG) {
+        b += 32 * slots;  // parents
         size_t lx = nx, ly = ny, lz = nz;
-        while(lx > 8 || ly > 8 || lz > 8) {
+        for(int l = 1; (lx > 8 || ly > 8 || lz > 8) && l < kMaxMgLevels; ++l) {
             lx = (lx + 1) / 2, ly = (ly + 1) / 2, lz = (lz + 1) / 2;
             const size_t lnb = ((lx + 7) / 8) * ((ly + 7) / 8) * ((lz + 7) / 8), cap = lnb + lnb / 4 + 4;
-            b += 12 * lnb + 28 * cap + 8 * 4 * 512 * cap;
+            b += 12 * lnb + (24 + 32) * cap + 8 * 4 * 512 * cap;
         }
     }
-    // per particle: two sets of 6 float arrays, the 16 + 8-byte packed transfer records and the id
-    // (the binning writes the other set), the cell key and the permutation
-    if(n) b += 112 * (n + n / 8 + 1024);
+    // per particle: two sets of 6 float arrays (32 bytes longer), the 16 + 8-byte packed transfer records and
+    // the id (the binning writes the other set), the cell key and the permutation; nine floats a set of the
+    // affine schemes
+    if(n) {
+        b += (112 + (prm.transfer_scheme != BNN_TRANSFER_FLIP ? 72 : 0)) * (n + n / 8 + 1024) + 2 * 6 * 32;
+        if(prm.enable_sort_particle) {
+            const ZsortLayout L = zsort_layout(n);
+            b += 8 * L.nh + 16 + (L.partWords > scanWords ? 4 * (L.partWords - scanWords) : 0);
+        }
+    }
     return b;
 }
 
