@@ -1787,7 +1787,7 @@ struct UniformRow {
         d64 = ((((t + t) + t) + t) + t) + t;
         c   = (float)c64;
         d   = (float)d64;
-        inv = (float)(1.0 / d64);
+        inv = d64 > 0 ? (float)(1.0 / d64) : 0.f;  // as k_assemble: a projection may be given any time step
     }
     __device__ __forceinline__ bool is(int s) const { return flag && flag[s] != 0; }
 };

@@ -39,3 +39,23 @@ def test_uniform_rows(bnn, cells, precond):
     rmax, bmax, _ = host_residual(phi, g.grid("weight_u"), g.grid("weight_v"), g.grid("weight_w"), g.pressure(), g.rhs(), DT)
     g.close()
     assert bmax > 0 and rmax <= 1.01e-8 * bmax
+
+
+@pytest.mark.parametrize("dt", [0.0, -1.0 / 600.0])
+def test_uniform_rows_without_a_positive_diagonal(bnn, dt):
+    """A projection is given its time step as it is: with none or a negative one no row has a positive
+    diagonal, so every inverse is 0, the preconditioner gives zeros and the pressure stays 0, on uniform
+    bricks as on others."""
+    h = 1.0 / 64.0
+    params = scenes.base_params(64)
+    params.update(box_max=(80 * h,) * 3, max_cg_iteration=50)
+    pos = np.stack(np.meshgrid(*[(np.arange(80, dtype=np.float32) + 0.5) * np.float32(h)] * 3, indexing="ij"), -1).reshape(-1, 3)
+    g = bnn.FLIPSolver(params)
+    g.set_particles(pos, np.random.default_rng(1).normal(0, 0.5, pos.shape).astype(np.float32))
+    g.map_particles_to_grid()
+    g.pressure_projection(np.float32(dt))
+    p = g.pressure()
+    z = g.apply_preconditioner(np.random.default_rng(2).normal(0, 1, p.size))
+    assert g.stats()["pcg_success"] == 0
+    g.close()
+    assert np.all(p == 0) and np.all(z == 0)
