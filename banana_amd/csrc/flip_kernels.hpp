@@ -724,21 +724,24 @@ struct FaceOut {
 
 constexpr int kP2gSide = 16, kP2gOwn = kP2gSide - 2;  // columns of a workgroup per axis, and those it owns
 
-// one axis of a particle of cell c: n = node-aligned weights of the nodes c, c+1; h = half-shifted weights
-// of c-1, c, c+1. With f = x - c in [0, 1) these are bary()'s fractions without its branches: the base of
-// x - 0.5 is c-1 with fraction f + 0.5 when f < 0.5, else c with f - 0.5 (both exact), and 1 - fraction
-// rounds the same exact value either way. Outside the grid f clamps to 0 / 1 as bary's does.
-__device__ __forceinline__ void p2g_axis(float x, float c, float* n, float* h) {
+// one axis of a particle at fraction f of cell c: n = node-aligned weights of the nodes c, c+1; h =
+// half-shifted weights of c-1, c, c+1. With f = x - c in [0, 1) these are bary()'s fractions without its
+// branches: the base of x - 0.5 is c-1 with fraction f + 0.5 when f < 0.5, else c with f - 0.5 (both exact),
+// and 1 - fraction rounds the same exact value either way.
+__device__ __forceinline__ void p2g_axis(float f, float* n, float* h) {
 #pragma clang fp contract(off)
-    const float f = fminf(fmaxf(x - c, 0.f), 1.f);
     n[0] = 1.0f - f;
     n[1] = f;
     h[0] = fmaxf(0.5f - f, 0.f);
     h[1] = fminf(f + 0.5f, 1.5f - f);
     h[2] = fmaxf(f - 0.5f, 0.f);
 }
-// the first (lo) / last (hi) cell of an axis: the half-shifted stencil clamps onto the cell's own node
-__device__ __forceinline__ void p2g_axis_edge(bool lo, bool hi, float* h) {
+// the first (lo) / last (hi) cell of an axis: outside the grid f clamps to 0 / 1 as bary's does, the
+// half-shifted stencil onto the cell's own node. A coordinate that is not a number is binned to the first
+// cell, and its weights are not numbers either.
+__device__ __forceinline__ void p2g_axis_edge(float f, bool lo, bool hi, float* n, float* h) {
+    if(!lo && !hi) return;
+    p2g_axis(fminf(fmaxf(f, 0.f), 1.f), n, h);
     if(lo && h[0] > 0.f) {
         h[0] = 0.f;
         h[1] = 1.f;
@@ -747,6 +750,15 @@ __device__ __forceinline__ void p2g_axis_edge(bool lo, bool hi, float* h) {
         if(h[2] > 0.f) h[1] = 1.f;
         h[2] = 0.f;
     }
+    if(f != f) n[0] = n[1] = h[1] = h[2] = f;
+}
+// bary()'s weight of a node on an axis of `size` nodes, and whether the node is one of the stencil's two
+__device__ __forceinline__ bool stencil_weight(float x, int size, int node, float& w) {
+    int   b;
+    float f;
+    bary(x, size, b, f);
+    w = node == b ? 1.0f - f : f;
+    return node == b || node == b + 1;
 }
 
 // momentum and weight of kX x kY x kZ nodes: (wx * wy) * wz as the reference forms it, added node by node
@@ -833,7 +845,8 @@ struct k_p2g {
     }
     __device__ void operator()(Blk blk) const {
 #pragma clang fp contract(off)
-        __shared__ float2 part[21][kThreads];  // a complete plane's partial sums: u 2x3, v 3x2, w 3x3
+        __shared__ float2   part[21][kThreads];  // a complete plane's partial sums: u 2x3, v 3x2, w 3x3
+        __shared__ uint32_t redo[kThreads];      // per thread, the planes of its nodes whose sums are not finite
         const int ntx = (g.nx + kP2gOwn) / kP2gOwn, nty = (g.ny + kP2gOwn) / kP2gOwn, ntz = (g.nz + seg) / seg;
         int       tx, ty, tz;
         tile_of_block(blk, ntx, nty, ntz, tx, ty, tz);
@@ -858,6 +871,7 @@ struct k_p2g {
             }
             return;
         }
+        redo[t] = 0;
         const float fi = (float)i, fj = (float)j;
         const bool  edgeXY = i == 0 || i == g.nx - 1 || j == 0 || j == g.ny - 1;
         // world positions of the column's nodes (getWorldCoordinate: (index + extra) * dx + bMin)
@@ -889,14 +903,15 @@ struct k_p2g {
             for(int q = 0; q < kBatch; ++q) {
                 if(p + (uint32_t)q >= e) break;
                 float xn[2], xh[3], yn[2], yh[3], zn[2], zh[3];
-                p2g_axis(R.x[q], fi, xn, xh);
-                p2g_axis(R.y[q], fj, yn, yh);
-                p2g_axis(R.z[q], (float)z, zn, zh);
+                const float fx = R.x[q] - fi, fy = R.y[q] - fj, fz = R.z[q] - (float)z;
+                p2g_axis(fx, xn, xh);
+                p2g_axis(fy, yn, yh);
+                p2g_axis(fz, zn, zh);
                 if(edgeXY) {
-                    p2g_axis_edge(i == 0, i == g.nx - 1, xh);
-                    p2g_axis_edge(j == 0, j == g.ny - 1, yh);
+                    p2g_axis_edge(fx, i == 0, i == g.nx - 1, xn, xh);
+                    p2g_axis_edge(fy, j == 0, j == g.ny - 1, yn, yh);
                 }
-                if(z == 0 || z == g.nz - 1) p2g_axis_edge(z == 0, z == g.nz - 1, zh);
+                if(z == 0 || z == g.nz - 1) p2g_axis_edge(fz, z == 0, z == g.nz - 1, zn, zh);
                 if constexpr(kAffine) {
                     const float fz = (float)z;
                     float       dnx[2], dhx[3], dny[2], dhy[3], dnz[2], dhz[3];
@@ -982,8 +997,8 @@ struct k_p2g {
                                 b.x += s.x;
                                 b.y += s.y;
                             }
-                        emit(out.u, out.vu, a, ownU, atU);
-                        emit(out.v, out.vv, b, ownV, atV);
+                        const bool lost = emit(out.u, out.vu, a, ownU, atU) | emit(out.v, out.vv, b, ownV, atV);
+                        if(lost) redo[t] |= 1u << (z - 1 - k0);
                     }
                     if(z < k1) {
                         float2 c = make_float2(0.f, 0.f);
@@ -995,7 +1010,7 @@ struct k_p2g {
                                 c.x += s.x;
                                 c.y += s.y;
                             }
-                        emit(out.w, out.vw, c, ownW, atW);
+                        if(emit(out.w, out.vw, c, ownW, atW)) redo[t] |= 1u << (z - k0);
                     }
                 }
                 __syncthreads();
@@ -1011,13 +1026,62 @@ struct k_p2g {
 #pragma unroll
             for(int e = 0; e < 9; ++e) mw[0][e] = mw[1][e], ww[0][e] = ww[1][e], mw[1][e] = 0.f, ww[1][e] = 0.f;
         }
+        for(uint32_t r = redo[t]; r; r &= r - 1u) {
+            const int k = k0 + __builtin_ctz(r);
+            for(int d = 0; d < 3; ++d) {
+                const bool mine = d == 0 ? ownU && k < g.nz : (d == 1 ? ownV && k < g.nz : ownW);
+                if(!mine) continue;
+                float*   vel = d == 0 ? out.u : (d == 1 ? out.v : out.w);
+                uint8_t* ok  = d == 0 ? out.vu : (d == 1 ? out.vv : out.vw);
+                emit(vel, ok, node(d, i, j, k), true, lin3(i, j, k, g.nx + (d == 0), g.ny + (d == 1)));
+            }
+        }
     }
-    // node velocity = momentum / weight where the weight is positive, else 0 and invalid
-    __device__ __forceinline__ static void emit(float* __restrict__ vel, uint8_t* __restrict__ valid, float2 s, bool mine, size_t at) {
-        if(!mine) return;
+    // node velocity = momentum / weight where the weight is positive, else 0 and invalid. Returns whether the
+    // sums are not finite
+    __device__ __forceinline__ static bool emit(float* __restrict__ vel, uint8_t* __restrict__ valid, float2 s, bool mine, size_t at) {
+        if(!mine) return false;
         const bool ok = s.y > kFltMin;
         vel[at]       = ok ? s.x / s.y : 0.f;
         valid[at]     = ok ? 1 : 0;
+        return !(fabsf(s.x) + s.y < __builtin_inff());
+    }
+    // The sums of node (i, j, k) of component d over the particles whose stencil holds it. The splat takes all
+    // three nodes of a half-shifted axis and counts on a weight of 0 to add nothing, which a velocity or an
+    // affine matrix that is not finite does not: the nodes it reached are summed again here, in the splat's
+    // order, so that it reaches the eight of its stencil and the finite terms give the same bits.
+    __device__ __forceinline__ float2 node(int d, int i, int j, int k) const {
+#pragma clang fp contract(off)
+        const float hx = d == 0 ? 0.f : 0.5f, hy = d == 1 ? 0.f : 0.5f, hz = d == 2 ? 0.f : 0.5f;
+        const int   x1 = min(d == 0 ? i : i + 1, g.nx - 1), y1 = min(d == 1 ? j : j + 1, g.ny - 1), z1 = min(d == 2 ? k : k + 1, g.nz - 1);
+        float2      s = make_float2(0.f, 0.f);
+        for(int y = max(j - 1, 0); y <= y1; ++y)
+            for(int x = max(i - 1, 0); x <= x1; ++x) {
+                float2 c = make_float2(0.f, 0.f);
+                for(int z = max(k - 1, 0); z <= z1; ++z) {
+                    const size_t cell = lin3(x, y, z, g.nx, g.ny);
+                    for(uint32_t p = cell_start[cell], e = cell_start[cell + 1]; p < e; ++p) {
+                        const float4 a = P.gp[p];
+                        const float2 b = P.gv[p];
+                        float        wx, wy, wz;
+                        const bool   in = stencil_weight(a.x - hx, g.nx + (d == 0), i, wx) & stencil_weight(a.y - hy, g.ny + (d == 1), j, wy) &
+                                        stencil_weight(a.z - hz, g.nz + (d == 2), k, wz);
+                        if(!in) continue;
+                        float v = d == 0 ? a.w : (d == 1 ? b.x : b.y);
+                        if constexpr(kAffine) {
+                            const float dx = (((float)i + hx) * g.dx + g.bminx) - P.px[p], dy = (((float)j + hy) * g.dx + g.bminy) - P.py[p],
+                                        dz = (((float)k + hz) * g.dx + g.bminz) - P.pz[p];
+                            v = v + ((A.c[3 * d][p] * dx + A.c[3 * d + 1][p] * dy) + A.c[3 * d + 2][p] * dz);
+                        }
+                        const float w = (wx * wy) * wz;
+                        c.x = __builtin_fmaf(w, v, c.x);
+                        c.y += w;
+                    }
+                }
+                s.x += c.x;
+                s.y += c.y;
+            }
+        return s;
     }
 };
 
