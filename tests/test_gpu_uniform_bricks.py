@@ -10,6 +10,7 @@ import numpy as np
 import pytest
 
 from banana_amd import scenes
+from banana_amd.serving import Batch
 from test_gpu_configs import host_residual
 
 pytestmark = pytest.mark.gpu
@@ -59,3 +60,38 @@ def test_uniform_rows_without_a_positive_diagonal(bnn, dt):
     assert g.stats()["pcg_success"] == 0
     g.close()
     assert np.all(p == 0) and np.all(z == 0)
+
+
+@pytest.mark.parametrize("refined", [0, 1], ids=["fp32", "refined"])
+def test_uniform_rows_in_a_batch(bnn, refined):
+    """Scenes on both sides of the system size at which the uniform rows' constant is used (1331, 1000 and 1890
+    bricks of a full box) in one batch: every bit of the velocities and the pressure is that of the scene alone."""
+    h = 1.0 / 64.0
+    made = []
+    for cells in ((84, 84, 84), (76, 76, 76), (140, 68, 100)):
+        params = scenes.base_params(64, boundary_sdf_at_init=True)
+        params.update(box_max=tuple(c * h for c in cells), pressure_mode=refined, warm_start=refined)
+        ax = [(np.arange(2 * c, dtype=np.float32) + 0.5) * np.float32(h / 2) for c in cells]
+        pos = np.stack(np.meshgrid(*ax, indexing="ij"), -1).reshape(-1, 3)
+        vel = np.random.default_rng(sum(cells)).normal(0, 0.5, pos.shape).astype(np.float32)
+        pair = []
+        for _ in range(2):
+            g = bnn.FLIPSolver(params)
+            g.set_particles(pos, vel)
+            pair.append(g)
+        made.append(pair)
+    b = Batch()
+    for _ in range(2):
+        for alone, _ in made:
+            alone.step(DT)
+        assert np.all(b.step([g for _, g in made], DT) == 0)
+    bricks = [alone.stats()["num_active_bricks"] for alone, _ in made]
+    assert min(bricks) <= 1024 < max(bricks)
+    for alone, g in made:
+        assert np.array_equal(alone.pressure(), g.pressure())
+        for x, y in zip(alone.particles(), g.particles()):
+            assert np.array_equal(x, y)
+        for k in ("pcg_iterations", "outer_iterations", "pcg_success", "pcg_residual"):
+            assert alone.stats()[k] == g.stats()[k], k
+        alone.close()
+        g.close()
