@@ -42,3 +42,34 @@ def test_mg_tail_shapes(bnn, cells):
             assert abs(zr[0][1] - zr[1][0]) <= 1e-4 * np.sqrt(zr[0][0] * zr[1][1])
         g.close()
     assert np.linalg.norm(out[1] - out[0]) <= 1e-6 * np.linalg.norm(out[0])
+
+
+def test_mg_coarsest_of_two_bricks(bnn):
+    """An axis of more than 8 * 2^15 cells leaves the coarsest of the 16 levels with more than one brick, which
+    the tail does not take: fluid on both sides of the border between its two, and far from it."""
+    h = 1.0 / 16.0
+    nz = 8 * 2 ** 15 + 10
+    params = scenes.base_params(16)
+    params.update(box_max=(6 * h, 5 * h, nz * h), pressure_mode=1, refine_tolerance=1e-10, max_cg_iteration=20000)
+    rng = np.random.default_rng(5)
+    pos = np.concatenate([rng.uniform(0, 1, (8 * 30 * (hi - lo), 3)) * [6 * h, 5 * h, (hi - lo) * h] + [0, 0, lo * h]
+                          for lo, hi in ((nz - 30, nz - 1), (100000, 100040), (3, 20))]).astype(np.float32)
+    vel = rng.normal(0, 0.5, pos.shape).astype(np.float32)
+    out = {}
+    for precond in (1, 0):
+        g = bnn.FLIPSolver(dict(params, preconditioner=precond))
+        assert g.n[2] > 8 * 2 ** 15
+        g.set_particles(pos, vel)
+        g.map_particles_to_grid()
+        g.pressure_projection(DT)
+        assert g.stats()["pcg_success"] == 1
+        out[precond] = g.pressure()
+        if precond == 1:
+            r = rng.normal(0, 1, (2, out[1].size))
+            r[:, out[1] == 0] = 0  # empty rows
+            z = [g.apply_preconditioner(v) for v in r]
+            zr = [[float(a @ b) for b in r] for a in z]
+            assert zr[0][0] > 0 and zr[1][1] > 0
+            assert abs(zr[0][1] - zr[1][0]) <= 1e-4 * np.sqrt(zr[0][0] * zr[1][1])
+        g.close()
+    assert np.linalg.norm(out[1] - out[0]) <= 1e-6 * np.linalg.norm(out[0])
