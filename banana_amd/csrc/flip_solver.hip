@@ -360,6 +360,7 @@ public:
         HIP_OK(hipGetDevice(&device));
         HIP_OK(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
         allocGrid();
+        if(prm.preconditioner == BNN_PRECOND_MG) setupLevels();
         HIP_OK(hipHostMalloc((void**)&hostSolve, sizeof(SolveState), hipHostMallocDefault));
         HIP_OK(hipHostMalloc((void**)&hostU32, 256, hipHostMallocDefault));
         if(prm.boundary_sdf_at_init) computeBoundarySDF();
@@ -832,7 +833,6 @@ public:
         systemValid  = false;  // until the new one stands
         // the active bricks of every level, counted with one wait
         const bool mgp = prm.preconditioner == BNN_PRECOND_MG;
-        if(mgp) setupLevels();
         const int nCand = mgp ? (int)mg.size() - 1 : 0;
         uint32_t* cnt   = counters.as<uint32_t>();
         {
@@ -923,16 +923,15 @@ public:
                         L.x.as<float>(), L.b.as<float>(), L.r.as<float>(), L.nSlots, L.ptab.as<int32_t>(), UniformRow{}};
     }
 
-    // the coarse levels' grids: each halves the one before until every axis fits one brick. Kept only when
-    // every buffer was to be had: the next solve starts over otherwise
+    // the coarse levels' grids: each halves the one before until every axis fits one brick. Made with the scene,
+    // flags cleared: a projection that fails half-way, alone or in a batch whose launches are dropped, leaves
+    // them whole
     void setupLevels() {
-        if(!mg.empty()) return;
-        decltype(mg) lv;
-        lv.emplace_back(nullptr);
+        mg.emplace_back(nullptr);
         int nx = g.nx, ny = g.ny, nz = g.nz;
-        while((nx > 8 || ny > 8 || nz > 8) && (int)lv.size() < kMaxMgLevels) {
-            lv.emplace_back(new MgLevel());
-            MgLevel& L = *lv.back();
+        while((nx > 8 || ny > 8 || nz > 8) && (int)mg.size() < kMaxMgLevels) {
+            mg.emplace_back(new MgLevel());
+            MgLevel& L = *mg.back();
             nx = (nx + 1) / 2;
             ny = (ny + 1) / 2;
             nz = (nz + 1) / 2;
@@ -942,9 +941,8 @@ public:
             L.flag.reserve(L.nb * 4);
             L.brickSlot.reserve(L.nb * 4);
             L.slotBrick.reserve(L.nb * 4);
+            HIP_OK(hipMemsetAsync(L.flag.p, 0, L.nb * 4, stream));
         }
-        mg.swap(lv);
-        for(size_t l = 1; l < mg.size(); ++l) fill32(mg[l]->flag.p, 0, mg[l]->nb * 4);
     }
     // the levels in use (until one brick remains) and their buffers, from the counts in hostU32[1 + l]
     void sizeLevels(int nCand) {
