@@ -851,9 +851,9 @@ public:
                 MgLevel& L      = *mg[l];
                 f.cnbx[l]       = L.nbx;
                 f.cnby[l]       = L.nby;
-                f.flag[l]       = x_.flag[l] = L.flag.as<uint32_t>();
-                x_.brickSlot[l] = L.brickSlot.as<int32_t>();
-                x_.slotBrick[l] = L.slotBrick.as<int32_t>();
+                f.flag[l]       = x_.flag[l] = L.flag;
+                x_.brickSlot[l] = L.brickSlot;
+                x_.slotBrick[l] = L.slotBrick;
                 x_.nb[l]        = L.nb;
             }
             launch(f, k_brick_flags::blocks(nb));
@@ -903,9 +903,12 @@ public:
     struct MgLevel {
         int      nx = 0, ny = 0, nz = 0, nbx = 0, nby = 0, nbz = 0;
         uint32_t nb = 0, nSlots = 0, slotCap = 0;
-        DevBuf   flag, brickSlot, slotBrick, nbr, diag, cx, cy, cz, inv, x, b, r, ptab;
+        uint32_t* flag = nullptr;  // parts of levelTables
+        int32_t * brickSlot = nullptr, *slotBrick = nullptr;
+        DevBuf   nbr, diag, cx, cy, cz, inv, x, b, r, ptab;
     };
     DevBuf                                ptab0;  // parent table of the fine level
+    DevBuf                                levelTables;
     std::vector<std::unique_ptr<MgLevel>> mg;  // mg[0] unused (the fine level lives in the PCG buffers)
     int                                   mgLevels = 0;
     static constexpr uint32_t             kCoarsestSlots = 1;  // coarsen until one brick remains
@@ -918,7 +921,7 @@ public:
     LevelDev levelDev(int l) {
         if(l == 0) return fineLevel();
         MgLevel& L = *mg[l];
-        return LevelDev{L.nx, L.ny, L.nz, L.nbx, L.nby, L.nbz, L.brickSlot.as<int32_t>(), L.slotBrick.as<int32_t>(), L.nbr.as<int32_t>(),
+        return LevelDev{L.nx, L.ny, L.nz, L.nbx, L.nby, L.nbz, L.brickSlot, L.slotBrick, L.nbr.as<int32_t>(),
                         L.diag.as<float>(), L.cx.as<float>(), L.cy.as<float>(), L.cz.as<float>(), L.inv.as<float>(),
                         L.x.as<float>(), L.b.as<float>(), L.r.as<float>(), L.nSlots, L.ptab.as<int32_t>(), UniformRow{}};
     }
@@ -928,7 +931,8 @@ public:
     // them whole
     void setupLevels() {
         mg.emplace_back(nullptr);
-        int nx = g.nx, ny = g.ny, nz = g.nz;
+        int    nx = g.nx, ny = g.ny, nz = g.nz;
+        size_t n = 0;
         while((nx > 8 || ny > 8 || nz > 8) && (int)mg.size() < kMaxMgLevels) {
             mg.emplace_back(new MgLevel());
             MgLevel& L = *mg.back();
@@ -938,10 +942,20 @@ public:
             L.nx = nx; L.ny = ny; L.nz = nz;
             L.nbx = (nx + 7) / 8; L.nby = (ny + 7) / 8; L.nbz = (nz + 7) / 8;
             L.nb  = (uint32_t)(L.nbx * L.nby * L.nbz);
-            L.flag.reserve(L.nb * 4);
-            L.brickSlot.reserve(L.nb * 4);
-            L.slotBrick.reserve(L.nb * 4);
-            HIP_OK(hipMemsetAsync(L.flag.p, 0, L.nb * 4, stream));
+            n += L.nb;
+        }
+        if(n == 0) return;
+        levelTables.reserve(n * 12);  // one allocation: the flags of all levels, then their tables
+        HIP_OK(hipMemsetAsync(levelTables.p, 0, n * 4, stream));
+        uint32_t* f = levelTables.as<uint32_t>();
+        int32_t*  t = levelTables.as<int32_t>() + n;
+        for(size_t l = 1; l < mg.size(); ++l) {
+            MgLevel& L  = *mg[l];
+            L.flag      = f;
+            L.brickSlot = t;
+            L.slotBrick = t + n;
+            f += L.nb;
+            t += L.nb;
         }
     }
     // the levels in use (until one brick remains) and their buffers, from the counts in hostU32[1 + l]
@@ -980,8 +994,8 @@ public:
             t.nbx[l]       = L ? L->nbx : g.nbx;
             t.nby[l]       = L ? L->nby : g.nby;
             t.nbz[l]       = L ? L->nbz : g.nbz;
-            t.brickSlot[l] = (L ? L->brickSlot : brickSlot).as<int32_t>();
-            t.slotBrick[l] = (L ? L->slotBrick : slotBrick).as<int32_t>();
+            t.brickSlot[l] = L ? L->brickSlot : brickSlot.as<int32_t>();
+            t.slotBrick[l] = L ? L->slotBrick : slotBrick.as<int32_t>();
             t.nbr[l]       = (L ? L->nbr : nbrTab).as<int32_t>();
             t.ptab[l]      = l + 1 < mgLevels ? (L ? L->ptab : ptab0).as<int32_t>() : nullptr;
             n += blocks(t.nSlots[l]);
