@@ -711,11 +711,11 @@ __device__ __forceinline__ void tile_of_block(Blk blk, int ntx, int nty, int ntz
 //
 // A workgroup is 16 x 16 columns around 14 x 14 owned ones (each node needs the columns next to it:
 // 1.31 visits a particle, against 1.95 for a tile of 8^3 nodes scattered into LDS, which this
-// replaces) and a segment of `seg` node planes (seg + 2 rows read). Bound by VALU issue: 214
+// replaces) and a segment of `seg` node planes (seg + 2 rows read). Bound by VALU issue: some 210
 // instructions a particle visit, and a wavefront's row lasts as long as its fullest cell. 33M particles
-// at 256^3: 1724 -> 876 us (689 while every cell holds 8); 26k at 24^3, where the scattered tile was a
-// serial chain of 27 colour rounds in 64 wavefronts: 263 -> 33 us; affine, 1.27M: 1155 -> 180 us (a
-// gather per node column).
+// at 256^3, a settling flow: 1740 -> 880 us (690 on the initial lattice, where every cell holds 8); 26k at
+// 24^3, where the scattered tile was a serial chain of 27 colour rounds in 64 wavefronts: 263 -> 33 us;
+// affine, 1.27M: 1155 -> 180 us (a gather per node column).
 //==================================================================================================
 struct FaceOut {
     float *u, *v, *w;
@@ -1074,6 +1074,7 @@ struct k_p2g {
                             v = v + ((A.c[3 * d][p] * dx + A.c[3 * d + 1][p] * dy) + A.c[3 * d + 2][p] * dz);
                         }
                         const float w = (wx * wy) * wz;
+                        if(w != w) return make_float2(0.f, w);  // no weight, whatever else comes
                         c.x = __builtin_fmaf(w, v, c.x);
                         c.y += w;
                     }
@@ -1723,7 +1724,9 @@ struct k_brick_flags {
 // one host wait where a three-launch scan, slot, neighbour and parent table kernel per level and two waits
 // took 150 us of a 64^3 substep's 2350, and the cell counts' one atomic 121 us at 256^3): slots in ascending brick order, the
 // brick -> slot (-1: inactive) and slot -> brick tables, and the level's count to out[1 + l]. Level 0 reads
-// the cell counts and adds them up to out[0]; the coarse levels' flags return to 0 for the next time.
+// the cell counts and adds them up to out[0]; the coarse levels' flags return to 0 for the next time. Its time
+// grows with the brick grid: 41 us at 256^3, 277 at 512^3, 1490 at 900^3. With the flags and tables that is still
+// less than the flags, scans and tables before it at each (427 against 544 us at 512^3, 2230 against 2520 at 900^3).
 struct k_brick_index {
     static constexpr int kThreads = 1024, kItems = 8;
     uint32_t* flag[kMaxMgLevels];
@@ -1832,12 +1835,11 @@ struct SystemOut {
 // faces, so every coupling is -dt and the diagonal 6 dt as the assembly sums it. k_assemble flags such
 // bricks, and the kernels that stream the finest level take the row from here instead of reading it: 4 of
 // 8 words a cell of the SpMV, 32 of 52 bytes of the FP64 residual. Same values, same bits. At 256^3 (9593
-// bricks, about 60% of them uniform): SpMV 31.5 -> 27.8 us, update 38.1 -> 34.2, post-smoother 41.3 ->
-// 34.9, FP64 residual 69.7 -> 49.5 (before the kernels took pairs of cells). The restriction, bound by its
-// instructions, kept its own time, but the rows it leaves unread stay out of the caches: without it in this
-// the step gained 0.24 of 14.7 ms, with it 0.44. The flag comes before the row in a dependent chain, 0.5 us of
-// the 4.6 us an SpMV of 216 bricks takes: systems of up to kUniformMin bricks read every row (at 567
-// neither wins).
+// bricks, about 60% of them uniform): SpMV 33.7 -> 28.5 us, update 35.2 -> 32.6, restriction 24.1 -> 19.8,
+// post-smoother 47.0 -> 44.5, FP64 residual 70.3 -> 49.0. The flag comes before the row in a dependent chain,
+// 0.5 us of the 4.6 us an SpMV of 216 bricks takes, so small systems have nothing to gain: refined projections
+// of full boxes of 216 to 1000 bricks take the same time with and without, within the runs' 2%; of 1331 bricks
+// 2210 -> 2165 us, 2197 2850 -> 2770, 8000 5850 -> 5540. Up to kUniformMin bricks every row is read.
 constexpr uint32_t kUniformMin = 1024;
 
 struct UniformRow {
@@ -1985,9 +1987,9 @@ __device__ __forceinline__ double fold(const double* __restrict__ p, int n, bool
 // The same sum by every workgroup of a consumer kernel (NT threads), for n <= kFoldMax partials: valid
 // in all threads and, with fold()'s order (64 consecutive partials per wavefront sum, then the sums in
 // order), the same bits; sh holds kFoldMax / 64 sums. On small systems it replaces a one-block launch
-// (2.5-3.5 us of an iteration of about 90 at 64^3). With the parts past n skipped it does so up to 1024
-// bricks: 567 bricks 2490 -> 2410 us a substep, 623 2850 -> 2800; at 1309 the launch is the cheaper
-// (a 128^3 frame 16.1 -> 16.4 ms with the limit at 2048).
+// (2.5-3.5 us of an iteration of about 90 at 64^3). Refined projections with the launch and without it: 216
+// bricks 1510 -> 1440 us, 512 1770 -> 1690, 729 2170 -> 2100, 1000 2280 -> 2240. With more partials every
+// workgroup's fold costs more than the launch: 1331 bricks 2230 -> 2310 us, 1728 2490 -> 2730.
 constexpr int kFoldMax = 1024;
 template<int NT> __device__ __forceinline__ double fold_all(const double* __restrict__ p, int n, double* sh) {
     double v[kFoldMax / NT];
@@ -3110,8 +3112,9 @@ struct k_mg_residual_restrict {
     }
 };
 
-// coarsest level: x = 0, then `sweeps` red-black sweeps followed by `sweeps` black-red sweeps
-// (symmetric), all inside one block
+// A coarsest level of more than one brick, which only an axis of more than 8 * 2^15 cells leaves (the last of
+// kMaxMgLevels levels; k_mg_tail solves one brick): x = 0, then `sweeps` red-black sweeps followed by `sweeps`
+// black-red sweeps (symmetric), all inside one block
 struct k_mg_coarsest {
     static constexpr int kThreads = 1024;
     LevelDev L;
@@ -3136,7 +3139,6 @@ struct k_mg_coarsest {
     }
 };
 
-// partial z.r for the PCG (after the V-cycle wrote z)
 //==================================================================================================
 // The reference's preconditioner: natural-order incomplete Cholesky IC(0) with the 0.25 pivot
 // safeguard (PCGSolver.cpp:398-466, minDiagonalRatio PCGSolver.h:88-89) and its two triangular
@@ -3266,6 +3268,7 @@ struct k_ic0_upper_plane {
     }
 };
 
+// partial z.r for the PCG (after the preconditioner wrote z)
 struct k_pcg_dot_zr {
     static constexpr int kThreads = 512;
     const float* __restrict__ z;

@@ -391,8 +391,9 @@ bnn_status  bnn_io_from_json(const char* json_text, bnn_io_params* io);
 /* changes bnn_flip_params.timing of a live handle (0: no events, 1: stage events, 2: also per-kernel
  * events); takes effect at the next step */
 bnn_status  bnn_flip_set_timing(bnn_flip* h, int32_t timing);
-/* device bytes a scene with these parameters and n_particles keeps resident in HBM (what
- * bnn_flip_create + bnn_flip_set_particles allocate; stepping allocates nothing per scene) */
+/* device bytes a scene with these parameters and n_particles keeps resident in HBM at most: what
+ * bnn_flip_create and bnn_flip_set_particles allocate, the pressure system with fluid in every brick
+ * (allocated as the fluid spreads), and the z-sort's scratch when EnableSortParticle is set */
 bnn_status  bnn_flip_footprint(const bnn_flip_params* p, uint64_t n_particles, uint64_t* bytes);
 
 /* --- batching --------------------------------------------------------------------------------
