@@ -906,11 +906,11 @@ struct k_p2g {
                 const float fx = R.x[q] - fi, fy = R.y[q] - fj, fz = R.z[q] - (float)z;
                 p2g_axis(fx, xn, xh);
                 p2g_axis(fy, yn, yh);
-                p2g_axis(fz, zn, zh);
                 if(edgeXY) {
                     p2g_axis_edge(fx, i == 0, i == g.nx - 1, xn, xh);
                     p2g_axis_edge(fy, j == 0, j == g.ny - 1, yn, yh);
                 }
+                p2g_axis(fz, zn, zh);
                 if(z == 0 || z == g.nz - 1) p2g_axis_edge(fz, z == 0, z == g.nz - 1, zn, zh);
                 if constexpr(kAffine) {
                     const float fz = (float)z;
@@ -1026,14 +1026,16 @@ struct k_p2g {
 #pragma unroll
             for(int e = 0; e < 9; ++e) mw[0][e] = mw[1][e], ww[0][e] = ww[1][e], mw[1][e] = 0.f, ww[1][e] = 0.f;
         }
-        for(uint32_t r = redo[t]; r; r &= r - 1u) {
-            const int k = k0 + __builtin_ctz(r);
+        int at = t;
+        asm volatile("" : "+v"(at));  // what follows takes no register from the loops before it
+        for(uint32_t r = redo[at]; r; r &= r - 1u) {
+            const int ni = tx * kP2gOwn - 1 + at % kP2gSide, nj = ty * kP2gOwn - 1 + at / kP2gSide, nk = k0 + __builtin_ctz(r);
             for(int d = 0; d < 3; ++d) {
-                const bool mine = d == 0 ? ownU && k < g.nz : (d == 1 ? ownV && k < g.nz : ownW);
-                if(!mine) continue;
+                const int sx = g.nx + (d == 0), sy = g.ny + (d == 1), sz = g.nz + (d == 2);
+                if(ni >= sx || nj >= sy || nk >= sz) continue;
                 float*   vel = d == 0 ? out.u : (d == 1 ? out.v : out.w);
                 uint8_t* ok  = d == 0 ? out.vu : (d == 1 ? out.vv : out.vw);
-                emit(vel, ok, node(d, i, j, k), true, lin3(i, j, k, g.nx + (d == 0), g.ny + (d == 1)));
+                emit(vel, ok, node(d, ni, nj, nk), true, lin3(ni, nj, nk, sx, sy));
             }
         }
     }
