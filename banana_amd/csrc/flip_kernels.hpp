@@ -845,8 +845,7 @@ struct k_p2g {
     }
     __device__ void operator()(Blk blk) const {
 #pragma clang fp contract(off)
-        __shared__ float2   part[21][kThreads];  // a complete plane's partial sums: u 2x3, v 3x2, w 3x3
-        __shared__ uint32_t redo[kThreads];      // per thread, the planes of its nodes whose sums are not finite
+        __shared__ float2 part[21][kThreads];  // a complete plane's partial sums: u 2x3, v 3x2, w 3x3
         const int ntx = (g.nx + kP2gOwn) / kP2gOwn, nty = (g.ny + kP2gOwn) / kP2gOwn, ntz = (g.nz + seg) / seg;
         int       tx, ty, tz;
         tile_of_block(blk, ntx, nty, ntz, tx, ty, tz);
@@ -871,7 +870,6 @@ struct k_p2g {
             }
             return;
         }
-        redo[t] = 0;
         const float fi = (float)i, fj = (float)j;
         const bool  edgeXY = i == 0 || i == g.nx - 1 || j == 0 || j == g.ny - 1;
         // world positions of the column's nodes (getWorldCoordinate: (index + extra) * dx + bMin)
@@ -941,6 +939,7 @@ struct k_p2g {
         const uint32_t sU = (uint32_t)((g.nx + 1) * g.ny), sV = (uint32_t)(g.nx * (g.ny + 1)), sW = (uint32_t)(g.nx * g.ny);
         uint32_t       atU = (uint32_t)(k0 - 1) * sU + (uint32_t)(j * (g.nx + 1) + i), atV = (uint32_t)(k0 - 1) * sV + (uint32_t)(j * g.nx + i),
                  atW = (uint32_t)k0 * sW + (uint32_t)(j * g.nx + i);
+        float     lost = 0.f;                               // not 0 when a momentum of the owned nodes is not finite
         const int zs = max(k0 - 1, 0), ze = min(k1, g.nz);  // row nz holds no cells: it only completes the last planes
         uint32_t  pb, pe, nb, ne;
         Rec       cur, nxt;
@@ -997,8 +996,9 @@ struct k_p2g {
                                 b.x += s.x;
                                 b.y += s.y;
                             }
-                        const bool lost = emit(out.u, out.vu, a, ownU, atU) | emit(out.v, out.vv, b, ownV, atV);
-                        if(lost) redo[t] |= 1u << (z - 1 - k0);
+                        emit(out.u, out.vu, a, ownU, atU);
+                        emit(out.v, out.vv, b, ownV, atV);
+                        lost = __builtin_fmaf(b.x, 0.f, __builtin_fmaf(a.x, 0.f, lost));
                     }
                     if(z < k1) {
                         float2 c = make_float2(0.f, 0.f);
@@ -1010,7 +1010,8 @@ struct k_p2g {
                                 c.x += s.x;
                                 c.y += s.y;
                             }
-                        if(emit(out.w, out.vw, c, ownW, atW)) redo[t] |= 1u << (z - k0);
+                        emit(out.w, out.vw, c, ownW, atW);
+                        lost = __builtin_fmaf(c.x, 0.f, lost);
                     }
                 }
                 __syncthreads();
@@ -1026,32 +1027,31 @@ struct k_p2g {
 #pragma unroll
             for(int e = 0; e < 9; ++e) mw[0][e] = mw[1][e], ww[0][e] = ww[1][e], mw[1][e] = 0.f, ww[1][e] = 0.f;
         }
+        if(lost == 0.f) return;
         int at = t;
         asm volatile("" : "+v"(at));  // what follows takes no register from the loops before it
-        for(uint32_t r = redo[at]; r; r &= r - 1u) {
-            const int ni = tx * kP2gOwn - 1 + at % kP2gSide, nj = ty * kP2gOwn - 1 + at / kP2gSide, nk = k0 + __builtin_ctz(r);
+        const int ni = tx * kP2gOwn - 1 + at % kP2gSide, nj = ty * kP2gOwn - 1 + at / kP2gSide;
+        for(int k = k0; k < k1; ++k)
             for(int d = 0; d < 3; ++d) {
                 const int sx = g.nx + (d == 0), sy = g.ny + (d == 1), sz = g.nz + (d == 2);
-                if(ni >= sx || nj >= sy || nk >= sz) continue;
+                if(ni >= sx || nj >= sy || k >= sz) continue;
                 float*   vel = d == 0 ? out.u : (d == 1 ? out.v : out.w);
                 uint8_t* ok  = d == 0 ? out.vu : (d == 1 ? out.vv : out.vw);
-                emit(vel, ok, node(d, ni, nj, nk), true, lin3(ni, nj, nk, sx, sy));
+                emit(vel, ok, node(d, ni, nj, k), true, lin3(ni, nj, k, sx, sy));
             }
-        }
     }
-    // node velocity = momentum / weight where the weight is positive, else 0 and invalid. Returns whether the
-    // sums are not finite
-    __device__ __forceinline__ static bool emit(float* __restrict__ vel, uint8_t* __restrict__ valid, float2 s, bool mine, size_t at) {
-        if(!mine) return false;
+    // node velocity = momentum / weight where the weight is positive, else 0 and invalid
+    __device__ __forceinline__ static void emit(float* __restrict__ vel, uint8_t* __restrict__ valid, float2 s, bool mine, size_t at) {
+        if(!mine) return;
         const bool ok = s.y > kFltMin;
         vel[at]       = ok ? s.x / s.y : 0.f;
         valid[at]     = ok ? 1 : 0;
-        return !(fabsf(s.x) + s.y < __builtin_inff());
     }
     // The sums of node (i, j, k) of component d over the particles whose stencil holds it. The splat takes all
     // three nodes of a half-shifted axis and counts on a weight of 0 to add nothing, which a velocity or an
-    // affine matrix that is not finite does not: the nodes it reached are summed again here, in the splat's
-    // order, so that it reaches the eight of its stencil and the finite terms give the same bits.
+    // affine matrix that is not finite does not: the nodes of a thread that one reached (0 times their momentum
+    // is not 0: three multiply-adds a plane tell) are summed again here, in the splat's order, so that it
+    // reaches the eight of its stencil and the finite terms give the same bits.
     __device__ __forceinline__ float2 node(int d, int i, int j, int k) const {
 #pragma clang fp contract(off)
         const float hx = d == 0 ? 0.f : 0.5f, hy = d == 1 ? 0.f : 0.5f, hz = d == 2 ? 0.f : 0.5f;
